@@ -112,19 +112,32 @@ __global__ void __launch_bounds__(1024) k_mis(Ctl c, GraphDev g, int32_t* st, in
   standalone_retire(c);
 }
 
+// LONG: the graph has rows of more than kTopoEdges edges, which go on wl, two
+// lists of n entries. Both forms share one resource class (64 VGPRs, no
+// scratch): the grid is sized on the form without.
+template <bool LONG>
 __global__ void __launch_bounds__(1024, 8) k_pagerank(Ctl c, GraphDev g, float* c0, float* c1, float* rank,
-                                                   float damping, float base, float r0, int iters,
+                                                   float damping, float base, float r0, int iters, int32_t* wl,
                                                    int* iters_out) {
+  __shared__ int s_range[2];
+  __shared__ int s_cnt[3];
+  __shared__ float s_seg[kPrSegs];
   Team t;
   if (!standalone_begin(c, t)) return;
   int lo, hi;
-  block_range(g.n, t.id, t.n, &lo, &hi);
+  if (LONG) {
+    if (threadIdx.x < 3) s_cnt[threadIdx.x] = 0;
+    balanced_range(g, t.id, t.n, s_range, &lo, &hi);
+    pagerank_lists(g, lo, hi, wl, wl + g.n, s_cnt);
+  } else {
+    block_range(g.n, t.id, t.n, &lo, &hi);
+  }
   pagerank_init(g, c0, r0, lo, hi);
   xcd_barrier(c, t);
   for (int it = 0; it < iters; it++) {
     const float* cin = (it & 1) ? c1 : c0;
     float* cout = (it & 1) ? c0 : c1;
-    pagerank_iter<true>(g, cin, cout, rank, damping, base, it == iters - 1, lo, hi);
+    pagerank_pass<LONG>(g, cin, cout, rank, damping, base, it == iters - 1, lo, hi, wl, wl + g.n, s_cnt, s_seg);
     xcd_barrier(c, t);
   }
   clock_end(c, t.id);
@@ -307,7 +320,7 @@ bool wgm_app_kernel_info(int kernel, KernelInfo* out) {
     case WGM_K_SSSP: *out = KernelInfo{(const void*)&k_frontier<true>, wgm_frontier_lds}; return true;
     case WGM_K_COLOR: *out = KernelInfo{(const void*)&k_color, nullptr}; return true;
     case WGM_K_MIS: *out = KernelInfo{(const void*)&k_mis, nullptr}; return true;
-    case WGM_K_PAGERANK: *out = KernelInfo{(const void*)&k_pagerank, nullptr}; return true;
+    case WGM_K_PAGERANK: *out = KernelInfo{(const void*)&k_pagerank<false>, nullptr}; return true;
     default: return wgm_pannotia_kernel_info(kernel, out);
   }
 }
@@ -334,8 +347,8 @@ int wgm_app_probe(wgm_runtime* rt, int kernel, int grid, int wg_size) {
                          (int32_t*)nullptr, (int32_t*)nullptr, (int*)nullptr);
       return WGM_OK;
     case WGM_K_PAGERANK:
-      hipLaunchKernelGGL(k_pagerank, dim3(grid), dim3(wg_size), 0, rt->stream, rt->ctl, GraphDev{}, (float*)nullptr,
-                         (float*)nullptr, (float*)nullptr, 0.f, 0.f, 0.f, 0, (int*)nullptr);
+      hipLaunchKernelGGL(k_pagerank<false>, dim3(grid), dim3(wg_size), 0, rt->stream, rt->ctl, GraphDev{}, (float*)nullptr,
+                         (float*)nullptr, (float*)nullptr, 0.f, 0.f, 0.f, 0, (int32_t*)nullptr, (int*)nullptr);
       return WGM_OK;
     default:
       return wgm_pannotia_probe(rt, kernel, grid, wg_size);
@@ -552,6 +565,7 @@ int wgm_pagerank(wgm_runtime* rt, wgm_graph* g, float damping, int32_t iteration
   int rc = dev_alloc(rt, &g->f0, g->n);
   if (!rc) rc = dev_alloc(rt, &g->f1, g->n);
   if (!rc) rc = dev_alloc(rt, &g->f2, g->n);
+  if (!rc && g->maxdeg > kTopoEdges) rc = dev_alloc(rt, &g->wl, 2 * (size_t)g->n);
   if (rc) return rc;
   const float nf = (float)g->n;
   const float base = (1.0f - damping) / nf;
@@ -559,8 +573,12 @@ int wgm_pagerank(wgm_runtime* rt, wgm_graph* g, float damping, int32_t iteration
   int grid = 0, wg = 0;
   rc = launch_prologue(rt, WGM_K_PAGERANK, lc, &grid, &wg);
   if (rc) return rc;
-  hipLaunchKernelGGL(k_pagerank, dim3(grid), dim3(wg), 0, rt->stream, rt->ctl, wgm_graph_view(g), g->f0, g->f1, g->f2,
-                     damping, base, r0, iterations, g->iters);
+  if (g->maxdeg > kTopoEdges)
+    hipLaunchKernelGGL(k_pagerank<true>, dim3(grid), dim3(wg), 0, rt->stream, rt->ctl, wgm_graph_view(g), g->f0, g->f1,
+                       g->f2, damping, base, r0, iterations, g->wl, g->iters);
+  else
+    hipLaunchKernelGGL(k_pagerank<false>, dim3(grid), dim3(wg), 0, rt->stream, rt->ctl, wgm_graph_view(g), g->f0, g->f1,
+                       g->f2, damping, base, r0, iterations, (int32_t*)nullptr, g->iters);
   rc = launch_epilogue(rt, lc, g, st);
   if (rc) return rc;
   if (rank_out) HIPCHK(rt, hipMemcpy(rank_out, g->f2, sizeof(float) * (size_t)g->n, hipMemcpyDeviceToHost));

@@ -888,9 +888,9 @@ __device__ __forceinline__ void mis_phase_b_wl(const GraphDev& g, int32_t* st, i
 }
 
 // ------------------------------------------------------------ PageRank
-// Pull iteration r'(v) = base + d * sum_{u in N(v)} r(u)/deg(u), FP32, the sum
-// taken in CSR order by one thread, so the result is bitwise reproducible.
-// contrib holds r(u)/deg(u) (0 for deg 0).
+// Pull iteration r'(v) = base + d * sum_{u in N(v)} r(u)/deg(u), FP32, each sum
+// in a fixed order, so the result is bitwise reproducible. contrib holds
+// r(u)/deg(u) (0 for deg 0).
 __device__ __forceinline__ void pagerank_init(const GraphDev& g, float* contrib, float r0, int lo, int hi) {
   for (int v = lo + (int)threadIdx.x; v < hi; v += blockDim.x) {
     const int deg = g.row_ptr[v + 1] - g.row_ptr[v];
@@ -898,53 +898,162 @@ __device__ __forceinline__ void pagerank_init(const GraphDev& g, float* contrib,
   }
 }
 
-// GROUPED (the standalone kernel): kTopoGroup vertices per thread per pass,
-// their rows, then the first kTopoEdges edges of each, then those
-// neighbours' contributions, all in flight together (three round trips per
-// group instead of two per edge); each sum still adds its terms one by one in
-// edge order, so the result is the same bit for bit.
-template <bool GROUPED = false>
+// One row per thread (the mega-kernel's resizable task).
 __device__ __forceinline__ void pagerank_iter(const GraphDev& g, const float* cin, float* cout, float* rank,
                                               float damping, float base, bool last, int lo, int hi) {
-  if (!GROUPED) {
-    for (int v = lo + (int)threadIdx.x; v < hi; v += blockDim.x) {
-      const int beg = g.row_ptr[v], end = g.row_ptr[v + 1];
-      float sum = 0.0f;
-      for (int e = beg; e < end; e++) sum = sum + cin[g.col[e]];
-      const float r = __builtin_fmaf(damping, sum, base);
-      if (last) rank[v] = r;
-      else cout[v] = (end > beg) ? r / (float)(end - beg) : 0.0f;
-    }
-    return;
+  for (int v = lo + (int)threadIdx.x; v < hi; v += blockDim.x) {
+    const int beg = g.row_ptr[v], end = g.row_ptr[v + 1];
+    float sum = 0.0f;
+    for (int e = beg; e < end; e++) sum = sum + cin[g.col[e]];
+    const float r = __builtin_fmaf(damping, sum, base);
+    if (last) rank[v] = r;
+    else cout[v] = (end > beg) ? r / (float)(end - beg) : 0.0f;
   }
-  const int bd = blockDim.x;
-  for (int b0 = lo + (int)threadIdx.x; b0 < hi; b0 += kTopoGroup * bd) {
-    int v[kTopoGroup], beg[kTopoGroup], end[kTopoGroup];
+}
+
+// The standalone kernel's iteration. Rows of at most kTopoEdges edges are
+// summed by one thread, a few rows per pass: their rows, then their
+// edges, then those neighbours' contributions, all in flight together, the
+// terms added one by one in edge order. On a graph with longer rows (LONG)
+// those are on three lists, built once per launch (pagerank_lists):
+//   up to kPrMid edges   eight lanes a row;
+//   up to kPrSeg edges   one wave a row;
+//   longer               the workgroup, in segments of kPrSeg edges a wave.
+// A lane adds its terms in edge order (every 8th or 64th edge, four in
+// flight), the lanes' sums meet in a fixed tree and a row's segments are
+// added in a fixed order, so a rank depends on the graph alone, not on the
+// launch shape, and a long row's rounding error is that of a short sum.
+// Bound: the chain of dependent loads of the longest row a workgroup has.
+// Symmetrised RMAT scale 17 ef 16 (3.9 M edges), 50 iterations, 512 x 1024,
+// whole call: 134.1 ms with one thread a row and equal vertex counts, 1.31 ms
+// here; largest relative error against FP64 2.1e-6 there, 4.8e-8 here.
+constexpr int kPrMid = 64;
+constexpr int kPrSeg = 2048;
+constexpr int kPrSegs = 256;  // segment sums in LDS at a time
+
+// Sum of G lanes' terms cin[col[e]], e = beg + lane, + G, ...; every lane of
+// the group gets the total.
+template <int G>
+__device__ __forceinline__ float pagerank_group_sum(const int32_t* col, const float* cin, int beg, int end, int lane) {
+  float sum = 0.0f;
+  int e = beg + lane;
+  for (; e + 3 * G < end; e += 4 * G) {
+    int u[4];
+    float x[4];
 #pragma unroll
-    for (int k = 0; k < kTopoGroup; k++) {
+    for (int q = 0; q < 4; q++) u[q] = col[e + q * G];
+#pragma unroll
+    for (int q = 0; q < 4; q++) x[q] = cin[u[q]];
+#pragma unroll
+    for (int q = 0; q < 4; q++) sum = sum + x[q];
+  }
+  int u[3];
+  float x[3];
+#pragma unroll
+  for (int q = 0; q < 3; q++) u[q] = e + q * G < end ? col[e + q * G] : -1;
+#pragma unroll
+  for (int q = 0; q < 3; q++) x[q] = u[q] >= 0 ? cin[u[q]] : 0.0f;
+#pragma unroll
+  for (int q = 0; q < 3; q++)
+    if (u[q] >= 0) sum = sum + x[q];
+#pragma unroll
+  for (int o = G / 2; o > 0; o >>= 1) sum = sum + __shfl_xor(sum, o, G);
+  return sum;
+}
+
+// This workgroup's long rows: list[lo, lo + cnt[0]) those of up to kPrMid
+// edges, list[hi - cnt[1], hi) those of up to kPrSeg, list2[lo, lo + cnt[2])
+// the rest. s_cnt: three ints of LDS, zeroed by the caller before a barrier.
+__device__ __forceinline__ void pagerank_lists(const GraphDev& g, int lo, int hi, int32_t* list, int32_t* list2,
+                                               int* s_cnt) {
+  for (int v = lo + (int)threadIdx.x; v < hi; v += blockDim.x) {
+    const int deg = g.row_ptr[v + 1] - g.row_ptr[v];
+    if (deg <= kTopoEdges) continue;
+    const int k = deg <= kPrMid ? 0 : deg <= kPrSeg ? 1 : 2;
+    const int i = __hip_atomic_fetch_add(&s_cnt[k], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    if (k == 0) list[lo + i] = v;
+    else if (k == 1) list[hi - 1 - i] = v;
+    else list2[lo + i] = v;
+  }
+}
+
+template <bool LONG>
+__device__ __forceinline__ void pagerank_pass(const GraphDev& g, const float* cin, float* cout, float* rank,
+                                              float damping, float base, bool last, int lo, int hi,
+                                              const int32_t* list, const int32_t* list2, const int* cnt,
+                                              float* s_seg) {
+  auto put = [&](int v, float sum, int deg) {
+    const float r = __builtin_fmaf(damping, sum, base);
+    if (last) rank[v] = r;
+    else cout[v] = deg > 0 ? r / (float)deg : 0.0f;
+  };
+  constexpr int U = LONG ? 2 : 3;
+  const int bd = blockDim.x;
+  if (LONG) {  // the longest chains first
+    const int wave = (int)threadIdx.x >> 6, nw = bd >> 6, lane = (int)threadIdx.x & 63;
+    for (int i = 0; i < cnt[2]; i++) {
+      const int v = list2[lo + i];
+      const int beg = g.row_ptr[v], end = g.row_ptr[v + 1];
+      float total = 0.0f;
+      for (int a = beg; a < end; a += kPrSegs * kPrSeg) {
+        const int ns = min(kPrSegs, (end - a + kPrSeg - 1) / kPrSeg);
+        for (int s = wave; s < ns; s += nw) {
+          const int sb = a + s * kPrSeg;
+          const float x = pagerank_group_sum<64>(g.col, cin, sb, min(sb + kPrSeg, end), lane);
+          if (lane == 0) s_seg[s] = x;
+        }
+        __syncthreads();
+        if (wave == 0) {
+          float x = 0.0f;
+          for (int s = lane; s < ns; s += 64) x = x + s_seg[s];
+          for (int o = 32; o > 0; o >>= 1) x = x + __shfl_xor(x, o, 64);
+          total = total + x;
+        }
+        __syncthreads();
+      }
+      if (threadIdx.x == 0) put(v, total, end - beg);
+    }
+    for (int i = wave; i < cnt[1]; i += nw) {
+      const int v = list[hi - 1 - i];
+      const int beg = g.row_ptr[v], end = g.row_ptr[v + 1];
+      const float x = pagerank_group_sum<64>(g.col, cin, beg, end, lane);
+      if (lane == 0) put(v, x, end - beg);
+    }
+    for (int i = (int)threadIdx.x >> 3; i < cnt[0]; i += bd >> 3) {
+      const int v = list[lo + i];
+      const int beg = g.row_ptr[v], end = g.row_ptr[v + 1];
+      const float x = pagerank_group_sum<8>(g.col, cin, beg, end, lane & 7);
+      if ((lane & 7) == 0) put(v, x, end - beg);
+    }
+  }
+  for (int b0 = lo + (int)threadIdx.x; b0 < hi; b0 += U * bd) {
+    int v[U], beg[U], end[U];
+#pragma unroll
+    for (int k = 0; k < U; k++) {
       v[k] = b0 + k * bd;
       const bool in = v[k] < hi;
       beg[k] = in ? g.row_ptr[v[k]] : 0;
       end[k] = in ? g.row_ptr[v[k] + 1] : 0;
+      if (LONG && end[k] - beg[k] > kTopoEdges) v[k] = hi;  // summed above
     }
-    int u[kTopoGroup][kTopoEdges];
+    int u[U][kTopoEdges];
 #pragma unroll
-    for (int k = 0; k < kTopoGroup; k++)
+    for (int k = 0; k < U; k++)
 #pragma unroll
-      for (int j = 0; j < kTopoEdges; j++) u[k][j] = beg[k] + j < end[k] ? g.col[beg[k] + j] : -1;
-    float cu[kTopoGroup][kTopoEdges];
+      for (int j = 0; j < kTopoEdges; j++)
+        u[k][j] = (!LONG || v[k] < hi) && beg[k] + j < end[k] ? g.col[beg[k] + j] : -1;
+    float cu[U][kTopoEdges];
 #pragma unroll
-    for (int k = 0; k < kTopoGroup; k++)
+    for (int k = 0; k < U; k++)
 #pragma unroll
       for (int j = 0; j < kTopoEdges; j++) cu[k][j] = u[k][j] >= 0 ? cin[u[k][j]] : 0.0f;
 #pragma unroll
-    for (int k = 0; k < kTopoGroup; k++) {
+    for (int k = 0; k < U; k++) {
       if (v[k] >= hi) continue;
       float sum = 0.0f;
 #pragma unroll
       for (int j = 0; j < kTopoEdges; j++)
         if (u[k][j] >= 0) sum = sum + cu[k][j];
-      for (int e = beg[k] + kTopoEdges; e < end[k]; e++) sum = sum + cin[g.col[e]];
       const float r = __builtin_fmaf(damping, sum, base);
       if (last) rank[v[k]] = r;
       else cout[v[k]] = (end[k] > beg[k]) ? r / (float)(end[k] - beg[k]) : 0.0f;
@@ -961,6 +1070,45 @@ __device__ __forceinline__ void block_range(int n, int rank, int nteam, int* lo,
   if (b > n) b = n;
   *lo = (int)a;
   *hi = (int)b;
+}
+
+// First vertex whose rows and edges before it, counted kRowCost a row and one
+// an edge, reach `target`; called by a whole wave, 64 probes a round.
+constexpr int kRowCost = 4;
+__device__ __forceinline__ int balanced_split(const int32_t* row_ptr, int n, long long target) {
+  const int lane = (int)threadIdx.x & 63;
+  int a = 0, b = n;  // the answer is in [a, b]
+  while (a < b) {
+    const int step = (b - a + 63) >> 6;
+    const long long p = (long long)a + (long long)lane * step;  // probe: still below the target
+    const bool below = p < b && (long long)row_ptr[p] + (long long)kRowCost * p < target;
+    const int k = __popcll(__ballot(below));  // cost grows with the vertex: the first k probes are below
+    if (k == 0) break;
+    const int last = a + (k - 1) * step;
+    b = min(b, last + step);
+    a = last + 1;
+  }
+  return a;
+}
+
+// Contiguous vertex range of workgroup `rank` among `nteam` with an even share
+// of rows and edges (merge-path split): on a graph with long rows, equal
+// vertex counts would leave most edges with the workgroups that drew the hubs
+// (RMAT scale 17: the first of 512 blocks holds a third of the edges).
+// s_range: two ints of LDS.
+__device__ __forceinline__ void balanced_range(const GraphDev& g, int rank, int nteam, int* s_range, int* lo, int* hi) {
+  if (threadIdx.x < 64) {
+    const long long total = (long long)g.m + (long long)kRowCost * g.n;
+    const int a = rank == 0 ? 0 : balanced_split(g.row_ptr, g.n, total * rank / nteam);
+    const int b = rank == nteam - 1 ? g.n : balanced_split(g.row_ptr, g.n, total * (rank + 1) / nteam);
+    if (threadIdx.x == 0) {
+      s_range[0] = a;
+      s_range[1] = b;
+    }
+  }
+  __syncthreads();
+  *lo = __builtin_amdgcn_readfirstlane(s_range[0]);
+  *hi = __builtin_amdgcn_readfirstlane(s_range[1]);
 }
 
 }  // namespace wgm
