@@ -52,60 +52,126 @@ __global__ void __launch_bounds__(1024) k_frontier(Ctl c, GraphDev g, FrontierDe
   standalone_retire(c);
 }
 
-// wl: two lists of n entries; a workgroup uses [lo, hi) of each for the open
-// vertices of its block (worklist rounds). The open count of round r is
-// s_wl[r % 3]: reset two rounds after its last read.
-__global__ void __launch_bounds__(1024) k_color(Ctl c, GraphDev g, int32_t* color, int32_t* wl, int* iters_out) {
-  __shared__ int s_wl[3];
+// Colouring without rounds. The rounds give a vertex the colour 1 + the
+// largest colour among its neighbours of priority not below its own (1
+// without one, or with exactly one neighbour), whenever each is reached, so
+// the workgroups sweep their open vertices on their own until none is left:
+// a vertex takes its colour once its last blocker has one, and colours travel
+// through agent-scope accesses, which need no barrier. Two barriers remain:
+// after the first pass, which writes every state, and before the round count,
+// which is what the rounds' stop flag gives -- the largest colour R, or R + 1
+// where a vertex coloured last, with more than one neighbour, has a neighbour
+// coloured last too (possible where an edge has no reverse).
+// Every participant is resident and the highest open vertex is never blocked,
+// so the sweeps end.
+// Bound: the first pass by the graph's bytes, then the longest chain of
+// dependent colours (one trip beyond the L2 each) and the sweeps' list
+// traffic. 2048^2 grid, 14 colours, 256 x 1024, kernel: 410 us in rounds (of
+// about 12 us each for draining the stores, the slowest workgroup and the
+// barrier), 285 us here.
+// wl: two lists of n entries (16 bytes with LONG, the graphs with rows of more
+// than kTopoEdges edges, 8 without); a workgroup uses [lo, hi) of each.
+template <bool LONG>
+__global__ void __launch_bounds__(1024) k_color(Ctl c, GraphDev g, int32_t* color, void* wl, int* iters_out) {
+  extern __shared__ int lds[];
+  __shared__ int s_cnt[2];
+  __shared__ int s_n[2];
+  __shared__ int s_top;
   Team t;
   if (!standalone_begin(c, t)) return;
   int lo, hi;
-  block_range(g.n, t.id, t.n, &lo, &hi);
-  if (threadIdx.x == 0) s_wl[0] = s_wl[1] = s_wl[2] = 0;
+  if (LONG) balanced_range(g, t.id, t.n, s_n, &lo, &hi);
+  else block_range(g.n, t.id, t.n, &lo, &hi);
+  if (threadIdx.x == 0) s_cnt[0] = s_cnt[1] = s_top = 0;
   __syncthreads();
-  int* flags = c.lines;
-  int round = 1, cnt = hi - lo;
-  const int32_t* lin = nullptr;
-  for (;; round++) {
-    if (threadIdx.x == 0) s_wl[(round + 1) % 3] = 0;
-    int32_t* lout = (round & 1) ? wl : wl + g.n;
-    const bool any = color_round_wl(g, color, round, lo, cnt, lin, lout, &s_wl[round % 3]);
-    if (__syncthreads_or(any) && threadIdx.x == 0) st_relaxed(&flags[(round % 3) * kLine], 1);
-    if (t.id == 0 && threadIdx.x == 0) st_relaxed(&flags[((round + 1) % 3) * kLine], 0);
-    xcd_barrier(c, t);
-    if (ld_relaxed(&flags[(round % 3) * kLine]) == 0) break;
-    cnt = s_wl[round % 3];
-    lin = lout;
+  const size_t half = (size_t)g.n * (LONG ? sizeof(int4) : sizeof(int2));
+  int top = 0;  // largest colour this thread gave
+  auto decide = [&](int v, int acc) {
+    st_agent(&color[v], acc + 1);
+    top = max(top, acc + 1);
+  };
+  auto keep = [&](int v) { st_agent(&color[v], -1); };
+  open_pass<LONG>(g, FirstProbe<true>{g.prio}, true, lo, hi - lo, nullptr, wl, &s_cnt[0], lds, s_n, decide, keep);
+  xcd_barrier<false>(c, t);
+  int which = 0, cnt = __builtin_amdgcn_readfirstlane(s_cnt[0]);
+  while (cnt > 0) {  // list `which` to the other, whose count was cleared a sweep ago
+    open_pass<LONG>(g, ColorProbe{color, g.prio}, true, lo, cnt, (char*)wl + which * half,
+                    (char*)wl + (1 - which) * half, &s_cnt[1 - which], lds, s_n, decide, keep);
+    __syncthreads();
+    const int left = __builtin_amdgcn_readfirstlane(s_cnt[1 - which]);
+    if (threadIdx.x == 0) s_cnt[which] = 0;
+    __syncthreads();
+    if (left == cnt) spin_pause();
+    cnt = left;
+    which = 1 - which;
   }
+  // the round count
+  for (int o = 32; o > 0; o >>= 1) top = max(top, __shfl_xor(top, o, 64));
+  if ((threadIdx.x & 63) == 0)
+    __hip_atomic_fetch_max(&s_top, top, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+  __syncthreads();
+  int* largest = &c.lines[0];
+  int* again = &c.lines[kLine];
+  const int mine = s_top;
+  if (threadIdx.x == 0) __hip_atomic_fetch_max(largest, mine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  xcd_barrier<false>(c, t);
+  const int last = ld_relaxed(largest);
+  if (mine == last) {
+    const int lane = (int)threadIdx.x & 63;
+    for (int v0 = lo + ((int)threadIdx.x & ~63); v0 < hi; v0 += blockDim.x) {
+      unsigned long long m = __ballot(v0 + lane < hi && ld_agent(&color[min(v0 + lane, hi - 1)]) == last);
+      for (; m; m &= m - 1) {  // the wave walks each row
+        const int v = v0 + __ffsll((long long)m) - 1;
+        const int beg = g.row_ptr[v], end = g.row_ptr[v + 1];
+        if (end - beg == 1) continue;
+        bool hit = false;
+        for (int e = beg + lane; e < end; e += 64) hit |= ld_agent(&color[g.col[e]]) == last;
+        if (hit) st_relaxed(again, 1);
+      }
+    }
+  }
+  xcd_barrier<false>(c, t);
   clock_end(c, t.id);
-  if (t.id == 0 && threadIdx.x == 0) *iters_out = round;
+  if (t.id == 0 && threadIdx.x == 0) *iters_out = last + ld_relaxed(again);
   standalone_retire(c);
 }
 
-__global__ void __launch_bounds__(1024) k_mis(Ctl c, GraphDev g, int32_t* st, int32_t* s_out, int32_t* wl,
+// Phase A moves the open vertices from the first list to the second, phase B
+// those that stay open back to the first (first round: the whole range). Their
+// counts are s_a and s_b, each cleared in the other phase.
+template <bool LONG>
+__global__ void __launch_bounds__(1024) k_mis(Ctl c, GraphDev g, int32_t* st, int32_t* s_out, void* wl,
                                              int* iters_out) {
-  __shared__ int s_wl[3];
+  extern __shared__ int lds[];
+  __shared__ int s_a, s_b;
+  __shared__ int s_n[2];
   Team t;
   if (!standalone_begin(c, t)) return;
   int lo, hi;
-  block_range(g.n, t.id, t.n, &lo, &hi);
-  if (threadIdx.x == 0) s_wl[0] = s_wl[1] = s_wl[2] = 0;
+  if (LONG) balanced_range(g, t.id, t.n, s_n, &lo, &hi);
+  else block_range(g.n, t.id, t.n, &lo, &hi);
+  if (threadIdx.x == 0) s_a = s_b = 0;
   __syncthreads();
+  void* la = wl;
+  void* lb = (char*)wl + (size_t)g.n * (LONG ? sizeof(int4) : sizeof(int2));
   int* flags = c.lines;
   int round = 1, cnt = hi - lo;
-  const int32_t* lin = nullptr;
   for (;; round++) {
-    if (threadIdx.x == 0) s_wl[(round + 1) % 3] = 0;
-    int32_t* lout = (round & 1) ? wl : wl + g.n;
-    const bool any = mis_phase_a_wl(g, st, s_out, round, lo, cnt, lin);
-    if (__syncthreads_or(any) && threadIdx.x == 0) st_relaxed(&flags[(round % 3) * kLine], 1);
+    // a vertex is open: not the last round
+    if (cnt > 0 && threadIdx.x == 0) st_relaxed(&flags[(round % 3) * kLine], 1);
+    mis_phase_a_wl<LONG>(g, st, s_out, round, lo, cnt, round == 1 ? nullptr : la, lb, &s_a, lds, s_n);
     if (t.id == 0 && threadIdx.x == 0) st_relaxed(&flags[((round + 1) % 3) * kLine], 0);
     xcd_barrier(c, t);
     if (ld_relaxed(&flags[(round % 3) * kLine]) == 0) break;
-    mis_phase_b_wl(g, st, round, lo, cnt, lin, lout, &s_wl[round % 3]);
+    const int left = __builtin_amdgcn_readfirstlane(s_a);  // scalar: the passes' loops hold barriers
+    if (threadIdx.x == 0) s_b = 0;
+    __syncthreads();
+    if (LONG) mis_phase_b_long(g, st, round, lo, left, (const int4*)lb, (int4*)la, &s_b, lds, s_n);
+    else mis_phase_b_low(g, st, round, lo, left, (const int2*)lb, (int2*)la, &s_b);
     xcd_barrier(c, t);
-    cnt = s_wl[round % 3];
-    lin = lout;
+    cnt = __builtin_amdgcn_readfirstlane(s_b);
+    if (threadIdx.x == 0) s_a = 0;
+    __syncthreads();
   }
   clock_end(c, t.id);
   if (t.id == 0 && threadIdx.x == 0) *iters_out = round;
@@ -154,12 +220,6 @@ __global__ void k_reached_edges(GraphDev g, const uint32_t* dist, unsigned long 
   if ((threadIdx.x & 63) == 0 && local) atomicAdd(out, local);
 }
 
-
-
-__global__ void k_fill_i32(int32_t* p, int n, int32_t v) {
-  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) p[i] = v;
-}
-
 }  // namespace wgm
 
 
@@ -178,6 +238,11 @@ int dev_alloc(wgm_runtime* rt, T** p, size_t count) {
   }
   return WGM_OK;
 }
+
+// Words of the graph's worklists: two lists of n entries of 16 bytes on graphs
+// with rows of more than kTopoEdges edges (PageRank takes the first 2 n
+// words), 8 bytes on the others.
+size_t wl_words(const wgm_graph* g) { return (g->maxdeg > kTopoEdges ? 8 : 4) * (size_t)g->n; }
 
 int launch_prologue(wgm_runtime* rt, int kernel, const wgm_launch* lc, int* grid, int* wg) {
   wgm_launch def{256, 0, 0, 0};
@@ -314,12 +379,16 @@ int wgm_graph_reached_edges(wgm_graph* g, int64_t* out) {
   return WGM_OK;
 }
 
+// Both forms of the colour and MIS kernels are launched with the long-row
+// form's LDS, so that the grid found for one holds for the other.
+static int scan_lds(int wg) { return scan_lds_bytes(wg); }
+
 bool wgm_app_kernel_info(int kernel, KernelInfo* out) {
   switch (kernel) {
     case WGM_K_BFS: *out = KernelInfo{(const void*)&k_frontier<false>, wgm_frontier_lds}; return true;
     case WGM_K_SSSP: *out = KernelInfo{(const void*)&k_frontier<true>, wgm_frontier_lds}; return true;
-    case WGM_K_COLOR: *out = KernelInfo{(const void*)&k_color, nullptr}; return true;
-    case WGM_K_MIS: *out = KernelInfo{(const void*)&k_mis, nullptr}; return true;
+    case WGM_K_COLOR: *out = KernelInfo{(const void*)&k_color<false>, scan_lds}; return true;
+    case WGM_K_MIS: *out = KernelInfo{(const void*)&k_mis<false>, scan_lds}; return true;
     case WGM_K_PAGERANK: *out = KernelInfo{(const void*)&k_pagerank<false>, nullptr}; return true;
     default: return wgm_pannotia_kernel_info(kernel, out);
   }
@@ -339,12 +408,12 @@ int wgm_app_probe(wgm_runtime* rt, int kernel, int grid, int wg_size) {
                          FrontierDev{}, NearFar{}, 0, (int*)nullptr);
       return WGM_OK;
     case WGM_K_COLOR:
-      hipLaunchKernelGGL(k_color, dim3(grid), dim3(wg_size), 0, rt->stream, rt->ctl, GraphDev{}, (int32_t*)nullptr,
-                         (int32_t*)nullptr, (int*)nullptr);
+      hipLaunchKernelGGL(k_color<false>, dim3(grid), dim3(wg_size), lds, rt->stream, rt->ctl, GraphDev{},
+                         (int32_t*)nullptr, (void*)nullptr, (int*)nullptr);
       return WGM_OK;
     case WGM_K_MIS:
-      hipLaunchKernelGGL(k_mis, dim3(grid), dim3(wg_size), 0, rt->stream, rt->ctl, GraphDev{}, (int32_t*)nullptr,
-                         (int32_t*)nullptr, (int32_t*)nullptr, (int*)nullptr);
+      hipLaunchKernelGGL(k_mis<false>, dim3(grid), dim3(wg_size), lds, rt->stream, rt->ctl, GraphDev{},
+                         (int32_t*)nullptr, (int32_t*)nullptr, (void*)nullptr, (int*)nullptr);
       return WGM_OK;
     case WGM_K_PAGERANK:
       hipLaunchKernelGGL(k_pagerank<false>, dim3(grid), dim3(wg_size), 0, rt->stream, rt->ctl, GraphDev{}, (float*)nullptr,
@@ -523,14 +592,13 @@ int wgm_color(wgm_runtime* rt, wgm_graph* g, const wgm_launch* lc, int32_t* colo
   if (!rt || !g || g->rt != rt) return fail(rt, WGM_ERR_INVALID, "bad runtime/graph");
   if (!g->prio) return fail(rt, WGM_ERR_INVALID, "colouring needs vertex priorities");
   int rc = dev_alloc(rt, &g->i32a, g->n);
-  if (!rc) rc = dev_alloc(rt, &g->wl, 2 * (size_t)g->n);
+  if (!rc) rc = dev_alloc(rt, &g->wl, wl_words(g));
   if (rc) return rc;
-  hipLaunchKernelGGL(k_fill_i32, dim3(256), dim3(256), 0, rt->stream, g->i32a, g->n, -1);
   int grid = 0, wg = 0;
   rc = launch_prologue(rt, WGM_K_COLOR, lc, &grid, &wg);
   if (rc) return rc;
-  hipLaunchKernelGGL(k_color, dim3(grid), dim3(wg), 0, rt->stream, rt->ctl, wgm_graph_view(g), g->i32a, g->wl,
-                     g->iters);
+  hipLaunchKernelGGL(g->maxdeg > kTopoEdges ? k_color<true> : k_color<false>, dim3(grid), dim3(wg), scan_lds_bytes(wg),
+                     rt->stream, rt->ctl, wgm_graph_view(g), g->i32a, (void*)g->wl, g->iters);
   rc = launch_epilogue(rt, lc, g, st);
   if (rc) return rc;
   if (color_out) HIPCHK(rt, hipMemcpy(color_out, g->i32a, sizeof(int32_t) * (size_t)g->n, hipMemcpyDeviceToHost));
@@ -542,15 +610,13 @@ int wgm_mis(wgm_runtime* rt, wgm_graph* g, const wgm_launch* lc, int32_t* s_out,
   if (!g->prio) return fail(rt, WGM_ERR_INVALID, "MIS needs vertex priorities");
   int rc = dev_alloc(rt, &g->i32a, g->n);
   if (!rc) rc = dev_alloc(rt, &g->i32b, g->n);
-  if (!rc) rc = dev_alloc(rt, &g->wl, 2 * (size_t)g->n);
+  if (!rc) rc = dev_alloc(rt, &g->wl, wl_words(g));
   if (rc) return rc;
-  hipLaunchKernelGGL(k_fill_i32, dim3(256), dim3(256), 0, rt->stream, g->i32a, g->n, -1);
-  hipLaunchKernelGGL(k_fill_i32, dim3(256), dim3(256), 0, rt->stream, g->i32b, g->n, 0);
   int grid = 0, wg = 0;
   rc = launch_prologue(rt, WGM_K_MIS, lc, &grid, &wg);
   if (rc) return rc;
-  hipLaunchKernelGGL(k_mis, dim3(grid), dim3(wg), 0, rt->stream, rt->ctl, wgm_graph_view(g), g->i32a, g->i32b, g->wl,
-                     g->iters);
+  hipLaunchKernelGGL(g->maxdeg > kTopoEdges ? k_mis<true> : k_mis<false>, dim3(grid), dim3(wg), scan_lds_bytes(wg),
+                     rt->stream, rt->ctl, wgm_graph_view(g), g->i32a, g->i32b, (void*)g->wl, g->iters);
   rc = launch_epilogue(rt, lc, g, st);
   if (rc) return rc;
   if (s_out) HIPCHK(rt, hipMemcpy(s_out, g->i32b, sizeof(int32_t) * (size_t)g->n, hipMemcpyDeviceToHost));
@@ -565,7 +631,7 @@ int wgm_pagerank(wgm_runtime* rt, wgm_graph* g, float damping, int32_t iteration
   int rc = dev_alloc(rt, &g->f0, g->n);
   if (!rc) rc = dev_alloc(rt, &g->f1, g->n);
   if (!rc) rc = dev_alloc(rt, &g->f2, g->n);
-  if (!rc && g->maxdeg > kTopoEdges) rc = dev_alloc(rt, &g->wl, 2 * (size_t)g->n);
+  if (!rc && g->maxdeg > kTopoEdges) rc = dev_alloc(rt, &g->wl, wl_words(g));
   if (rc) return rc;
   const float nf = (float)g->n;
   const float base = (1.0f - damping) / nf;

@@ -609,16 +609,14 @@ __device__ __forceinline__ void frontier_heavy(const GraphDev& g, const Frontier
 // (`start != end - 1`, src/pannotia/graph_apps/color/device/color.cl:46) is kept:
 // a vertex with exactly one neighbour ignores it. The stop flag of round c is
 // line c % 3 of `flags`.
-// The standalone kernels (the worklist rounds below) take vertices
-// kTopoGroup to a thread per pass (i, i + bd, i + 2 bd, ...: each load
-// coalesced across the wave) and issue the group's work level by level --
-// their rows and priorities, then the first kTopoEdges edges of each, then
-// those neighbours' states and priorities -- so a thread waits for a few
-// memory round trips per group instead of a dependent chain per vertex and
-// per edge. Edges past the first kTopoEdges of a vertex are walked one by one
-// afterwards. The registers this takes (~90 VGPRs) would spill in the
-// mega-kernel, whose resizable tasks keep one vertex at a time (color_round,
-// mis_phase_a / _b).
+// On low-degree graphs the standalone kernels (the worklist rounds below) take
+// vertices kTopoGroup to a thread per pass (i, i + bd, i + 2 bd, ...: each
+// load coalesced across the wave) and issue the group's work level by level --
+// rows and priorities, then the kTopoEdges edges of each, then those
+// neighbours' states and priorities -- so a thread waits for a few memory
+// round trips per group instead of a dependent chain per vertex and per edge.
+// The registers this takes (~90 VGPRs) would spill in the mega-kernel, whose
+// resizable tasks keep one vertex at a time (color_round, mis_phase_a / _b).
 constexpr int kTopoGroup = 4;
 constexpr int kTopoEdges = 4;
 
@@ -652,8 +650,6 @@ __device__ __forceinline__ bool color_round(const GraphDev& g, int32_t* color, i
 // undecided vertex with a neighbour that joined this round is removed.
 // Two barriers per round instead of three; the sets are those of
 // src/pannotia/graph_apps/mis/device/mis.cl:21-124.
-// The standalone kernel's forms (mis_phase_a_wl / _b_wl) group their loads
-// as the colour rounds do.
 __device__ __forceinline__ bool mis_phase_a(const GraphDev& g, int32_t* st, int32_t* s_out, int round,
                                             int lo, int hi) {
   bool any = false;
@@ -691,183 +687,435 @@ __device__ __forceinline__ void mis_phase_b(const GraphDev& g, int32_t* st, int 
   }
 }
 
-// ------------------------------------------------------- worklist rounds
-// The standalone colour and MIS kernels visit only the vertices still open:
-// a workgroup keeps the open vertices of its block in its share ([lo, ...))
-// of one of two lists, visits that list in the next round and writes the
-// vertices that stay open to the other. A vertex's decision depends only on
-// its neighbours' states, read as in the topology-driven rounds, and only its
-// own workgroup writes it, so the colours, sets and round counts are the same.
-// On the 2048^2 grid colour's 16 rounds visit 13.9 M vertices instead of
-// 67.1 M. The first round visits the whole block (no list).
-__device__ __forceinline__ void wl_push(bool stay, int v, int32_t* lout, int lo, int* cnt) {
-  const unsigned long long mask = __ballot(stay);
-  if (mask) {
-    const int lane = threadIdx.x & 63;
-    const int leader = __ffsll((long long)mask) - 1;
-    int base = 0;
-    if (lane == leader) base = __hip_atomic_fetch_add(cnt, __popcll(mask), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-    base = __builtin_amdgcn_readlane(base, leader);
-    if (stay) lout[lo + base + __popcll(mask & ((1ull << lane) - 1ull))] = v;
+// ------------------------------------------------------------- worklists
+// The standalone colour and MIS kernels visit only the vertices still open,
+// and most of those with one load. An open vertex is held back by a blocker:
+// a neighbour still undecided whose priority decides against it (colour: not
+// below its own; MIS: not above). A decided neighbour stays decided and
+// priorities are fixed, so as long as the blocker is undecided the vertex
+// stays open without a look at its row, and once it is not, the row's edges
+// before it need no second look. A workgroup keeps the open vertices of its
+// range, each with its blocker, in its share ([lo, ...)) of one of two lists
+// and writes those that stay open to the other. Only a vertex's own workgroup
+// writes its state. The first pass reads no states (all are undecided) and
+// writes every one.
+//
+// Two forms. Graphs of out-degree at most kTopoEdges: entries {vertex,
+// blocker}, four per thread with their loads in flight together, and a
+// vertex that lost its blocker reads its whole row again. The others (long
+// rows): entries {vertex, blocker's edge, blocker, value so far}; the scan for
+// the next blocker goes on from its edge, four edges by the thread, kScanMid
+// by eight lanes, the rest by a wave, each stage's unfinished rows queued in
+// LDS for the next, in ranges of equal rows and edges (balanced_range).
+constexpr int kScanMid = 64;
+constexpr int kScanU = 2;  // entries per thread and chunk of the long-row form
+// LDS of the long-row form: two queues of kScanU * bd {vertex or entry, edge, value}.
+__host__ __device__ constexpr int scan_lds_bytes(int bd) { return 2 * kScanU * bd * 3 * 4; }
+
+// A slot of a list for each lane of the wave that wants one.
+__device__ __forceinline__ int wl_slot(bool want, int* cnt) {
+  const unsigned long long mask = __ballot(want);
+  if (!mask) return 0;
+  const int lane = threadIdx.x & 63;
+  const int leader = __ffsll((long long)mask) - 1;
+  int base = 0;
+  if (lane == leader) base = __hip_atomic_fetch_add(cnt, __popcll(mask), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+  return __builtin_amdgcn_readlane(base, leader) + __popcll(mask & ((1ull << lane) - 1ull));
+}
+__device__ __forceinline__ int wl_slot1(int* cnt) {
+  return __hip_atomic_fetch_add(cnt, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+
+// Probes: test(u, pv, valid, acc) says whether neighbour u blocks a vertex of
+// priority pv; held(w, acc) whether blocker w still does. acc collects what the
+// vertex's decision needs from its decided neighbours (colour: the largest
+// colour). The loads are issued for every call (u is a valid vertex also where
+// the lane has no edge), so several calls overlap.
+//
+// Colour: a vertex is coloured one above the largest colour among the
+// neighbours whose priority is not below its own, once they all have theirs
+// (negative: uncoloured).
+struct ColorProbe {
+  const int32_t* color;
+  const uint32_t* prio;
+  __device__ __forceinline__ bool test(int u, uint32_t pv, bool valid, int& acc) const {
+    const uint32_t p = prio[u];
+    const int c = ld_agent(&color[u]);
+    const bool above = valid & (p >= pv);
+    acc = above && c > acc ? c : acc;
+    return above & (c < 0);
+  }
+  __device__ __forceinline__ bool held(int w, int& acc) const {
+    const int c = ld_agent(&color[w]);
+    acc = c > acc ? c : acc;
+    return c < 0;
+  }
+};
+// MIS phase A: undecided at the round's start (-1, or 2 * round: joined in it).
+struct MisProbe {
+  const int32_t* st;
+  const uint32_t* prio;
+  int joined;
+  __device__ __forceinline__ bool test(int u, uint32_t pv, bool valid, int&) const {
+    const uint32_t p = prio[u];
+    const int s = st[u];
+    return valid & (p <= pv) & ((s == -1) | (s == joined));
+  }
+  __device__ __forceinline__ bool held(int w, int&) const {
+    const int s = st[w];
+    return (s == -1) | (s == joined);
+  }
+};
+// First pass of either: every neighbour is undecided.
+template <bool ABOVE>
+struct FirstProbe {
+  const uint32_t* prio;
+  __device__ __forceinline__ bool test(int u, uint32_t pv, bool valid, int&) const {
+    const uint32_t p = prio[u];
+    return valid & (ABOVE ? p >= pv : p <= pv);
+  }
+  __device__ __forceinline__ bool held(int, int&) const { return false; }
+};
+// MIS phase B: joined this round.
+struct JoinedProbe {
+  const int32_t* st;
+  int joined;
+  __device__ __forceinline__ bool test(int u, uint32_t, bool valid, int&) const { return valid & (st[u] == joined); }
+};
+
+// First edge in [e, stop) whose target blocks, or -1; *w its target. Called by
+// the G lanes of a group together, Q edges a lane per round; every lane gets
+// the group's largest acc.
+template <int G, int Q, class Probe>
+__device__ __forceinline__ int scan_row(const int32_t* col, int e, int stop, int lane, uint32_t pv, const Probe& probe,
+                                        int* w, int& acc) {
+  const int shift = ((int)threadIdx.x & 63) & ~(G - 1);
+  int at = -1;
+  for (; e < stop && at < 0; e += G * Q) {
+    int u[Q];
+    bool hit[Q];
+#pragma unroll
+    for (int q = 0; q < Q; q++) u[q] = e + q * G + lane < stop ? col[e + q * G + lane] : -1;
+#pragma unroll
+    for (int q = 0; q < Q; q++) hit[q] = probe.test(max(u[q], 0), pv, u[q] >= 0, acc);
+#pragma unroll
+    for (int q = 0; q < Q; q++) {
+      unsigned long long m = __ballot(hit[q]) >> shift;
+      if (G < 64) m &= (1ull << (G & 63)) - 1ull;
+      if (m && at < 0) {
+        const int first = __ffsll((long long)m) - 1;
+        *w = __shfl(u[q], first, G);
+        at = e + q * G + first;
+      }
+    }
+  }
+  // Without this the compiler reuses the loop's exit mask for a caller's
+  // `at >= 0`, and that mask holds only the lanes of the last iteration:
+  // groups that found their edge earlier are then taken for not having one.
+  opaque(at);
+#pragma unroll
+  for (int o = G / 2; o > 0; o >>= 1) acc = max(acc, __shfl_xor(acc, o, G));
+  return at;
+}
+
+// Stages 1 and 2 of a long-row chunk over the queue entries {id, edge, value}
+// of s_q[0 .. s_n[0]): row(id) is the id's vertex, done(id, v, edge or -1,
+// target, value) takes the result on one lane. Ends with a barrier where the
+// queue was not empty.
+template <class Probe, class Row, class Done>
+__device__ __forceinline__ void scan_queued(const GraphDev& g, int* s_q, int* s_n, const Probe& probe, const Row& row,
+                                            const Done& done) {
+  const int bd = blockDim.x, cap = kScanU * bd, lane = (int)threadIdx.x & 63;
+  int* q1 = s_q;
+  int* q2 = s_q + 3 * cap;
+  __syncthreads();
+  const int n1 = __builtin_amdgcn_readfirstlane(s_n[0]);
+  if (n1 == 0) return;
+  for (int i = (int)threadIdx.x >> 3; i < n1; i += bd >> 3) {
+    const int id = q1[i], e = q1[cap + i];
+    int acc = q1[2 * cap + i], w = -1;
+    const int v = row(id);
+    const int end = g.row_ptr[v + 1], stop = min(end, e + kScanMid);
+    const int hit = scan_row<8, 2>(g.col, e, stop, lane & 7, g.prio[v], probe, &w, acc);
+    if ((lane & 7) == 0) {
+      if (hit >= 0 || stop == end) {
+        done(id, v, hit, w, acc);
+      } else {
+        const int k = wl_slot1(&s_n[1]);
+        q2[k] = id;
+        q2[cap + k] = stop;
+        q2[2 * cap + k] = acc;
+      }
+    }
+  }
+  __syncthreads();
+  const int n2 = __builtin_amdgcn_readfirstlane(s_n[1]);
+  for (int i = (int)threadIdx.x >> 6; i < n2; i += bd >> 6) {
+    const int id = q2[i], e = q2[cap + i];
+    int acc = q2[2 * cap + i], w = -1;
+    const int v = row(id);
+    const int hit = scan_row<64, 4>(g.col, e, g.row_ptr[v + 1], lane, g.prio[v], probe, &w, acc);
+    if (lane == 0) done(id, v, hit, w, acc);
+  }
+  __syncthreads();
+}
+
+// One pass over the open vertices that decides those without a blocker, on a
+// graph with long rows. decide(v, acc) writes a vertex's state, keep(v) the
+// first pass's undecided one (lin is null there: the vertices are lo + i).
+// skip1: a vertex with exactly one neighbour has no blocker (colour). s_n: two
+// ints of LDS; ocnt counts the entries written to lout.
+template <class Probe, class Decide, class Keep>
+__device__ __forceinline__ void open_pass_long(const GraphDev& g, const Probe& probe, bool skip1, int lo, int cnt,
+                                               const int4* lin, int4* lout, int* ocnt, int* s_q, int* s_n,
+                                               const Decide& decide, const Keep& keep) {
+  const int bd = blockDim.x, cap = kScanU * bd;
+  for (int base = 0; base < cnt; base += kScanU * bd) {
+    if (threadIdx.x == 0) s_n[0] = s_n[1] = 0;
+    __syncthreads();
+    bool in[kScanU], scan[kScanU];
+    int4 en[kScanU];
+    int e[kScanU], end[kScanU];
+    uint32_t pv[kScanU];
+#pragma unroll
+    for (int k = 0; k < kScanU; k++) {
+      const int i = base + k * bd + (int)threadIdx.x;
+      in[k] = i < cnt;
+      en[k] = int4{0, 0, 0, 0};
+      if (in[k]) {
+        if (lin) en[k] = lin[lo + i];
+        else en[k].x = lo + i;
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < kScanU; k++) scan[k] = in[k] && !(lin && probe.held(en[k].z, en[k].w));
+#pragma unroll
+    for (int k = 0; k < kScanU; k++) {
+      e[k] = scan[k] ? lin ? en[k].y + 1 : g.row_ptr[en[k].x] : 0;
+      end[k] = scan[k] ? g.row_ptr[en[k].x + 1] : 0;
+      pv[k] = scan[k] ? g.prio[en[k].x] : 0u;
+    }
+    int u[kScanU][4];
+#pragma unroll
+    for (int k = 0; k < kScanU; k++) {
+      if (skip1 && !lin && end[k] - e[k] == 1) end[k] = e[k];
+#pragma unroll
+      for (int j = 0; j < 4; j++) u[k][j] = e[k] + j < end[k] ? g.col[e[k] + j] : -1;
+    }
+    bool hit[kScanU][4];
+#pragma unroll
+    for (int k = 0; k < kScanU; k++)
+#pragma unroll
+      for (int j = 0; j < 4; j++) hit[k][j] = probe.test(max(u[k][j], 0), pv[k], u[k][j] >= 0, en[k].w);
+#pragma unroll
+    for (int k = 0; k < kScanU; k++) {
+      bool held = in[k] && !scan[k];
+#pragma unroll
+      for (int j = 3; j >= 0; j--)
+        if (hit[k][j]) {
+          held = true;
+          en[k].y = e[k] + j;
+          en[k].z = u[k][j];
+        }
+      const bool more = scan[k] && !held && e[k] + 4 < end[k];
+      if (in[k] && !held && !more) decide(en[k].x, en[k].w);
+      if (held && !lin) keep(en[k].x);
+      const int slot = wl_slot(held, ocnt);
+      if (held) lout[lo + slot] = en[k];
+      const int qs = wl_slot(more, &s_n[0]);
+      if (more) {
+        s_q[qs] = en[k].x;
+        s_q[cap + qs] = e[k] + 4;
+        s_q[2 * cap + qs] = en[k].w;
+      }
+    }
+    scan_queued(
+        g, s_q, s_n, probe, [&](int id) { return id; },
+        [&](int, int v, int edge, int w, int acc) {
+          if (edge < 0) {
+            decide(v, acc);
+          } else {
+            if (!lin) keep(v);
+            lout[lo + wl_slot1(ocnt)] = int4{v, edge, w, acc};
+          }
+        });
   }
 }
 
-// The i-th open vertex of the block: list entry, or lo + i in the first round.
-__device__ __forceinline__ int wl_vertex(const int32_t* lin, int lo, int i) { return lin ? lin[lo + i] : lo + i; }
-
-__device__ __forceinline__ bool color_round_wl(const GraphDev& g, int32_t* color, int round, int lo, int cnt,
-                                               const int32_t* lin, int32_t* lout, int* ocnt) {
-  bool any = false;
+// The same on a graph of out-degree at most kTopoEdges.
+template <class Probe, class Decide, class Keep>
+__device__ __forceinline__ void open_pass_low(const GraphDev& g, const Probe& probe, bool skip1, int lo, int cnt,
+                                              const int2* lin, int2* lout, int* ocnt, const Decide& decide,
+                                              const Keep& keep) {
   const int bd = blockDim.x;
   for (int base = (int)threadIdx.x; base < cnt; base += kTopoGroup * bd) {
-    int v[kTopoGroup], beg[kTopoGroup], deg[kTopoGroup];
+    int2 en[kTopoGroup];
+    bool in[kTopoGroup], scan[kTopoGroup];
+    int beg[kTopoGroup], deg[kTopoGroup], acc[kTopoGroup];
     uint32_t pv[kTopoGroup];
-    bool open[kTopoGroup];
 #pragma unroll
     for (int k = 0; k < kTopoGroup; k++) {
-      open[k] = base + k * bd < cnt;
-      v[k] = open[k] ? wl_vertex(lin, lo, base + k * bd) : 0;
+      in[k] = base + k * bd < cnt;
+      en[k] = int2{0, 0};
+      if (in[k]) {
+        if (lin) en[k] = lin[lo + base + k * bd];
+        else en[k].x = lo + base + k * bd;
+      }
     }
 #pragma unroll
     for (int k = 0; k < kTopoGroup; k++) {
-      beg[k] = open[k] ? g.row_ptr[v[k]] : 0;
-      const int end = open[k] ? g.row_ptr[v[k] + 1] : 0;
-      pv[k] = open[k] ? g.prio[v[k]] : 0u;
+      acc[k] = 0;
+      scan[k] = in[k] && !(lin && probe.held(en[k].y, acc[k]));
+    }
+#pragma unroll
+    for (int k = 0; k < kTopoGroup; k++) {
+      beg[k] = scan[k] ? g.row_ptr[en[k].x] : 0;
+      const int end = scan[k] ? g.row_ptr[en[k].x + 1] : 0;
+      pv[k] = scan[k] ? g.prio[en[k].x] : 0u;
       deg[k] = end - beg[k];
-      if (deg[k] == 1) deg[k] = 0;  // a vertex with exactly one neighbour ignores it
+      if (skip1 && deg[k] == 1) deg[k] = 0;
     }
     int u[kTopoGroup][kTopoEdges];
 #pragma unroll
     for (int k = 0; k < kTopoGroup; k++)
 #pragma unroll
       for (int j = 0; j < kTopoEdges; j++) u[k][j] = j < deg[k] ? g.col[beg[k] + j] : -1;
-    int cu[kTopoGroup][kTopoEdges];
-    uint32_t pu[kTopoGroup][kTopoEdges];
+    bool hit[kTopoGroup][kTopoEdges];
 #pragma unroll
     for (int k = 0; k < kTopoGroup; k++)
 #pragma unroll
-      for (int j = 0; j < kTopoEdges; j++) {
-        cu[k][j] = u[k][j] >= 0 ? color[u[k][j]] : 0;
-        pu[k][j] = u[k][j] >= 0 ? g.prio[u[k][j]] : 0u;
-      }
+      for (int j = 0; j < kTopoEdges; j++) hit[k][j] = probe.test(max(u[k][j], 0), pv[k], u[k][j] >= 0, acc[k]);
 #pragma unroll
     for (int k = 0; k < kTopoGroup; k++) {
-      bool coloured = false;
-      if (open[k]) {
-        long long mx = -1;
+      bool held = in[k] && !scan[k];
 #pragma unroll
-        for (int j = 0; j < kTopoEdges; j++) {
-          if (u[k][j] >= 0 && (cu[k][j] == -1 || cu[k][j] == round)) {
-            any = true;
-            mx = (long long)pu[k][j] > mx ? (long long)pu[k][j] : mx;
-          }
+      for (int j = kTopoEdges - 1; j >= 0; j--)
+        if (hit[k][j]) {
+          held = true;
+          en[k].y = u[k][j];
         }
-        for (int e = beg[k] + kTopoEdges; e < beg[k] + deg[k]; e++) {
-          const int w = g.col[e];
-          const int cw = color[w];
-          if (cw == -1 || cw == round) {
-            any = true;
-            const long long pw = (long long)g.prio[w];
-            mx = pw > mx ? pw : mx;
-          }
-        }
-        coloured = (long long)pv[k] > mx;
-        if (coloured) color[v[k]] = round;
-      }
-      wl_push(open[k] && !coloured, v[k], lout, lo, ocnt);
+      if (in[k] && !held) decide(en[k].x, acc[k]);
+      if (held && !lin) keep(en[k].x);
+      const int slot = wl_slot(held, ocnt);
+      if (held) lout[lo + slot] = en[k];
     }
   }
-  return any;
+}
+
+template <bool LONG, class Probe, class Decide, class Keep>
+__device__ __forceinline__ void open_pass(const GraphDev& g, const Probe& probe, bool skip1, int lo, int cnt,
+                                          const void* lin, void* lout, int* ocnt, int* s_q, int* s_n,
+                                          const Decide& decide, const Keep& keep) {
+  if constexpr (LONG)
+    open_pass_long(g, probe, skip1, lo, cnt, (const int4*)lin, (int4*)lout, ocnt, s_q, s_n, decide, keep);
+  else
+    open_pass_low(g, probe, skip1, lo, cnt, (const int2*)lin, (int2*)lout, ocnt, decide, keep);
 }
 
 // MIS phase A over the open list: an open vertex joins if its priority is
-// below every neighbour undecided at the round start (state -1 or 2r).
-__device__ __forceinline__ bool mis_phase_a_wl(const GraphDev& g, int32_t* st, int32_t* s_out, int round, int lo,
-                                               int cnt, const int32_t* lin) {
-  bool any = false;
-  const int joined = 2 * round;
-  const int bd = blockDim.x;
-  for (int base = (int)threadIdx.x; base < cnt; base += kTopoGroup * bd) {
-    int v[kTopoGroup], beg[kTopoGroup], deg[kTopoGroup];
-    uint32_t pv[kTopoGroup];
-    bool open[kTopoGroup];
-#pragma unroll
-    for (int k = 0; k < kTopoGroup; k++) {
-      open[k] = base + k * bd < cnt;
-      v[k] = open[k] ? wl_vertex(lin, lo, base + k * bd) : 0;
-    }
-#pragma unroll
-    for (int k = 0; k < kTopoGroup; k++) {
-      beg[k] = open[k] ? g.row_ptr[v[k]] : 0;
-      deg[k] = (open[k] ? g.row_ptr[v[k] + 1] : 0) - beg[k];
-      pv[k] = open[k] ? g.prio[v[k]] : 0u;
-    }
-    int u[kTopoGroup][kTopoEdges];
-#pragma unroll
-    for (int k = 0; k < kTopoGroup; k++)
-#pragma unroll
-      for (int j = 0; j < kTopoEdges; j++) u[k][j] = j < deg[k] ? g.col[beg[k] + j] : -1;
-    int su[kTopoGroup][kTopoEdges];
-    uint32_t pu[kTopoGroup][kTopoEdges];
-#pragma unroll
-    for (int k = 0; k < kTopoGroup; k++)
-#pragma unroll
-      for (int j = 0; j < kTopoEdges; j++) {
-        su[k][j] = u[k][j] >= 0 ? st[u[k][j]] : 0;
-        pu[k][j] = u[k][j] >= 0 ? g.prio[u[k][j]] : 0u;
-      }
-#pragma unroll
-    for (int k = 0; k < kTopoGroup; k++) {
-      if (!open[k]) continue;
-      any = true;
-      long long mn = 0x100000000LL;  // above every uint32 priority
-#pragma unroll
-      for (int j = 0; j < kTopoEdges; j++)
-        if (u[k][j] >= 0 && (su[k][j] == -1 || su[k][j] == joined))
-          mn = (long long)pu[k][j] < mn ? (long long)pu[k][j] : mn;
-      for (int e = beg[k] + kTopoEdges; e < beg[k] + deg[k]; e++) {
-        const int w = g.col[e];
-        const int sw = st[w];
-        if (sw == -1 || sw == joined) {
-          const long long pw = (long long)g.prio[w];
-          mn = pw < mn ? pw : mn;
-        }
-      }
-      if ((long long)pv[k] < mn) {
-        st[v[k]] = joined;
-        s_out[v[k]] = 2;
-      }
-    }
-  }
-  return any;
+// below every neighbour undecided at the round start (state -1 or 2r; one
+// that joins within the round is read as either).
+template <bool LONG>
+__device__ __forceinline__ void mis_phase_a_wl(const GraphDev& g, int32_t* st, int32_t* s_out, int round, int lo,
+                                               int cnt, const void* lin, void* lout, int* ocnt, int* s_q, int* s_n) {
+  auto decide = [&](int v, int) {
+    st[v] = 2 * round;
+    s_out[v] = 2;
+  };
+  auto keep = [&](int v) {
+    st[v] = -1;
+    s_out[v] = 0;
+  };
+  if (round == 1)
+    open_pass<LONG>(g, FirstProbe<false>{g.prio}, false, lo, cnt, nullptr, lout, ocnt, s_q, s_n, decide, keep);
+  else
+    open_pass<LONG>(g, MisProbe{st, g.prio, 2 * round}, false, lo, cnt, lin, lout, ocnt, s_q, s_n, decide, keep);
 }
 
-// MIS phase B over the same list: a vertex that did not join and has a
-// neighbour that joined this round is removed; the rest stay open.
-__device__ __forceinline__ void mis_phase_b_wl(const GraphDev& g, int32_t* st, int round, int lo, int cnt,
-                                               const int32_t* lin, int32_t* lout, int* ocnt) {
+// MIS phase B over the vertices phase A left: one with a neighbour that
+// joined this round is removed; the rest stay open. Its blocker is looked at
+// first: it is the neighbour most likely to have joined.
+__device__ __forceinline__ void mis_phase_b_long(const GraphDev& g, int32_t* st, int round, int lo, int cnt,
+                                                 const int4* lin, int4* lout, int* ocnt, int* s_q, int* s_n) {
+  const int joined = 2 * round, bd = blockDim.x, cap = kScanU * bd;
+  const JoinedProbe probe{st, joined};
+  for (int base = 0; base < cnt; base += kScanU * bd) {
+    if (threadIdx.x == 0) s_n[0] = s_n[1] = 0;
+    __syncthreads();
+    bool in[kScanU], gone[kScanU];
+    int4 en[kScanU];
+    int beg[kScanU], end[kScanU];
+#pragma unroll
+    for (int k = 0; k < kScanU; k++) {
+      const int i = base + k * bd + (int)threadIdx.x;
+      in[k] = i < cnt;
+      en[k] = in[k] ? lin[lo + i] : int4{0, 0, 0, 0};
+    }
+#pragma unroll
+    for (int k = 0; k < kScanU; k++) {
+      gone[k] = in[k] && st[en[k].z] == joined;
+      beg[k] = in[k] ? g.row_ptr[en[k].x] : 0;
+      end[k] = in[k] ? g.row_ptr[en[k].x + 1] : 0;
+    }
+    int u[kScanU][4];
+#pragma unroll
+    for (int k = 0; k < kScanU; k++)
+#pragma unroll
+      for (int j = 0; j < 4; j++) u[k][j] = !gone[k] && beg[k] + j < end[k] ? g.col[beg[k] + j] : -1;
+    int none = 0;
+#pragma unroll
+    for (int k = 0; k < kScanU; k++)
+#pragma unroll
+      for (int j = 0; j < 4; j++) u[k][j] = (int)probe.test(max(u[k][j], 0), 0u, u[k][j] >= 0, none);
+#pragma unroll
+    for (int k = 0; k < kScanU; k++) {
+#pragma unroll
+      for (int j = 0; j < 4; j++) gone[k] = gone[k] || u[k][j] != 0;
+      if (gone[k]) st[en[k].x] = joined + 1;
+      const bool more = in[k] && !gone[k] && beg[k] + 4 < end[k];
+      const bool stay = in[k] && !gone[k] && !more;
+      const int slot = wl_slot(stay, ocnt);
+      if (stay) lout[lo + slot] = en[k];
+      const int qs = wl_slot(more, &s_n[0]);
+      if (more) {
+        s_q[qs] = base + k * bd + (int)threadIdx.x;
+        s_q[cap + qs] = beg[k] + 4;
+        s_q[2 * cap + qs] = 0;
+      }
+    }
+    scan_queued(
+        g, s_q, s_n, probe, [&](int id) { return lin[lo + id].x; },
+        [&](int id, int v, int edge, int, int) {
+          if (edge >= 0) st[v] = joined + 1;
+          else lout[lo + wl_slot1(ocnt)] = lin[lo + id];
+        });
+  }
+}
+
+__device__ __forceinline__ void mis_phase_b_low(const GraphDev& g, int32_t* st, int round, int lo, int cnt,
+                                                const int2* lin, int2* lout, int* ocnt) {
   const int joined = 2 * round;
   const int bd = blockDim.x;
   for (int base = (int)threadIdx.x; base < cnt; base += kTopoGroup * bd) {
-    int v[kTopoGroup], sv[kTopoGroup], beg[kTopoGroup], deg[kTopoGroup];
-    bool open[kTopoGroup];
+    int2 en[kTopoGroup];
+    bool in[kTopoGroup], gone[kTopoGroup];
+    int beg[kTopoGroup], deg[kTopoGroup];
 #pragma unroll
     for (int k = 0; k < kTopoGroup; k++) {
-      const bool in = base + k * bd < cnt;
-      v[k] = in ? wl_vertex(lin, lo, base + k * bd) : 0;
-      sv[k] = in ? st[v[k]] : 0;
-      open[k] = in && sv[k] == -1;
+      in[k] = base + k * bd < cnt;
+      en[k] = in[k] ? lin[lo + base + k * bd] : int2{0, 0};
     }
 #pragma unroll
     for (int k = 0; k < kTopoGroup; k++) {
-      beg[k] = open[k] ? g.row_ptr[v[k]] : 0;
-      deg[k] = (open[k] ? g.row_ptr[v[k] + 1] : 0) - beg[k];
+      gone[k] = in[k] && st[en[k].y] == joined;
+      beg[k] = in[k] ? g.row_ptr[en[k].x] : 0;
+      deg[k] = (in[k] ? g.row_ptr[en[k].x + 1] : 0) - beg[k];
     }
     int u[kTopoGroup][kTopoEdges];
 #pragma unroll
     for (int k = 0; k < kTopoGroup; k++)
 #pragma unroll
-      for (int j = 0; j < kTopoEdges; j++) u[k][j] = j < deg[k] ? g.col[beg[k] + j] : -1;
+      for (int j = 0; j < kTopoEdges; j++) u[k][j] = j < deg[k] && !gone[k] ? g.col[beg[k] + j] : -1;
     int su[kTopoGroup][kTopoEdges];
 #pragma unroll
     for (int k = 0; k < kTopoGroup; k++)
@@ -875,14 +1123,12 @@ __device__ __forceinline__ void mis_phase_b_wl(const GraphDev& g, int32_t* st, i
       for (int j = 0; j < kTopoEdges; j++) su[k][j] = u[k][j] >= 0 ? st[u[k][j]] : 0;
 #pragma unroll
     for (int k = 0; k < kTopoGroup; k++) {
-      bool hit = false;
-      if (open[k]) {
 #pragma unroll
-        for (int j = 0; j < kTopoEdges; j++) hit = hit || (u[k][j] >= 0 && su[k][j] == joined);
-        for (int e = beg[k] + kTopoEdges; e < beg[k] + deg[k] && !hit; e++) hit = st[g.col[e]] == joined;
-        if (hit) st[v[k]] = joined + 1;
-      }
-      wl_push(open[k] && !hit, v[k], lout, lo, ocnt);
+      for (int j = 0; j < kTopoEdges; j++) gone[k] = gone[k] || (u[k][j] >= 0 && su[k][j] == joined);
+      if (gone[k]) st[en[k].x] = joined + 1;
+      const bool stay = in[k] && !gone[k];
+      const int slot = wl_slot(stay, ocnt);
+      if (stay) lout[lo + slot] = en[k];
     }
   }
 }

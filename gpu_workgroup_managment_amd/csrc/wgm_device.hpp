@@ -36,6 +36,14 @@ __device__ __forceinline__ void st_relaxed(int* p, int v) {
 __device__ __forceinline__ void st_release(int* p, int v) {
   __hip_atomic_store(p, v, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
 }
+template <class T>
+__device__ __forceinline__ T ld_agent(const T* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <class T>
+__device__ __forceinline__ void st_agent(T* p, T v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
 __device__ __forceinline__ int add_relaxed(int* p, int v) {
   return __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
@@ -331,8 +339,9 @@ __device__ __forceinline__ void global_barrier_disc(const Ctl& c, int id, int n,
 // L1-only invalidate (buffer_inv sc0) does not act outside threadgroup-split
 // mode, so members keep the full agent-scope acquire.
 // MAINT = false drops the write-back and the acquires: for callers whose
-// shared state goes only through agent-scope atomics (run_team), where the
-// barrier need only order arrivals after this workgroup's drained accesses.
+// shared state goes only through agent-scope atomics (run_team, k_color),
+// where the barrier need only order arrivals after this workgroup's drained
+// accesses.
 template <bool MAINT = true, class Spin = SpinForever>
 __device__ __forceinline__ void xcd_barrier(const Ctl& c, Team& t, const Spin& sp = Spin()) {
   drain_vmem();

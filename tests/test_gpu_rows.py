@@ -42,3 +42,66 @@ def test_pagerank_row_classes(rt):
         base = r if base is None else base
         assert np.array_equal(r.view(np.uint32), base.view(np.uint32)), (wg, wgs)
     dg.close()
+
+
+def _symmetric(g):
+    return G.from_edges(g.n, np.repeat(np.arange(g.n), g.degrees()), g.col, symmetric=True)
+
+
+# rows at the edges of the scan's stages: 4 edges by the thread, 64 by eight lanes, the rest by a wave (256 a round)
+STAGES = (1, 2, 4, 5, 12, 67, 68, 69, 132, 324, 325, 3000)
+
+
+def _stage_graph():
+    n, src, dst = 6007, [], []
+    rng = np.random.default_rng(8)
+    for v, deg in enumerate(STAGES):
+        src.append(np.full(deg, v))
+        dst.append(len(STAGES) + rng.permutation(n - len(STAGES))[:deg])
+    return _symmetric(G.from_edges(n, np.concatenate(src), np.concatenate(dst)))
+
+
+def _complete(n):
+    i, j = np.divmod(np.arange(n * n), n)
+    return G.from_edges(n, i[i != j], j[i != j])
+
+
+OPEN_GRAPHS = {
+    "stages": _stage_graph,
+    "rmat": lambda: _symmetric(G.rmat(13, 16, seed=2)),
+    "complete": lambda: _complete(131),  # as many colours as vertices: one long chain
+    "mesh": lambda: G.grid(61, 83),
+    "path": lambda: G.grid(1, 4099),
+    "no edges": lambda: G.CSR(np.zeros(71, np.int32), np.zeros(0, np.int32)),
+}
+
+
+@pytest.mark.parametrize("name", list(OPEN_GRAPHS))
+@pytest.mark.parametrize("wg,wgs", [(64, 1), (192, 19), (1024, 0)])
+def test_color_mis_worklists(rt, name, wg, wgs):
+    """Colours, sets and round counts of both forms of the worklist kernels."""
+    g = OPEN_GRAPHS[name]()
+    if name == "no edges":
+        g.prio = np.arange(g.n, dtype=np.uint32)
+    else:
+        G.add_priorities(g)
+    dg = rt.graph(g)
+    ref, rounds = oracle.color(g.row_ptr, g.col, g.prio)
+    out, st = dg.color(wg_size=wg, num_wgs=wgs)
+    assert np.array_equal(out, ref) and st["iterations"] == rounds
+    ref, rounds = oracle.mis(g.row_ptr, g.col, g.prio)
+    out, st = dg.mis(wg_size=wg, num_wgs=wgs)
+    assert np.array_equal(out, ref) and st["iterations"] == rounds
+    dg.close()
+
+
+@pytest.mark.parametrize("degree", [3, 9])
+def test_color_directed_round_count(rt, degree):
+    """Edges without a reverse: two neighbours may take the last colour in the
+    same round, and the round count is one more."""
+    n = 4001
+    rng = np.random.default_rng(degree)
+    g = G.add_priorities(G.from_edges(n, np.repeat(np.arange(n), degree), rng.integers(0, n, degree * n)))
+    ref, rounds = oracle.color(g.row_ptr, g.col, g.prio)
+    out, st = rt.graph(g).color(wg_size=256, num_wgs=24)
+    assert np.array_equal(out, ref) and st["iterations"] == rounds
