@@ -47,6 +47,8 @@ struct wgm_graph {
   int32_t ntasks = 0;
   // BC per-slot state and the result
   int32_t bc_slots = 0;
+  int32_t bc_rows = 0;  // dependency rows in bc_del
+  int32_t* bc_srcs = nullptr;
   int32_t* bc_d = nullptr;
   double* bc_sig = nullptr;
   double* bc_del = nullptr;

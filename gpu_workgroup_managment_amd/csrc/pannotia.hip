@@ -19,9 +19,8 @@
 // Here each workgroup takes a whole source: BFS levels with a workgroup queue,
 // path counts pulled over in-edges in in-edge order, dependencies pulled over
 // out-edges in CSR order, all in FP64 with no atomics on the sums. The
-// dependencies of one batch of sources (one per workgroup) land in per-slot
-// rows that, after one barrier, every workgroup adds to bc in source order for
-// its share of the vertices. The result does not depend on the grid and
+// dependencies of a batch of sources land in a row each; after one barrier the
+// rows are added to bc in source order. The result does not depend on the grid and
 // equals the FP64 oracle bit for bit.
 
 #include "apps_internal.hpp"
@@ -34,7 +33,8 @@ using namespace wgm;
 namespace wgm {
 
 constexpr int32_t kBigNum = WGM_BIG_NUM;
-// Cap on BC's per-slot state (28 bytes a vertex per slot): the grid shrinks to fit.
+// Cap on BC's per-slot state (28 bytes a vertex per slot, its row included): the
+// grid shrinks to fit.
 constexpr unsigned long long kBcSlotBytes = 8ull << 30;
 
 struct MinplusDev {
@@ -126,7 +126,9 @@ struct BcDev {
   int32_t slots;     // per-slot arrays allocated (>= participants)
   int32_t* d;        // [slots][n] BFS level, -1 unreached
   double* sig;       // [slots][n] shortest-path counts
-  double* del;       // [slots][n] dependencies of the slot's source (zero between batches)
+  double* del;       // [rows][n] dependencies, a row per source of a batch
+  int32_t rows;      // sources per batch
+  const int32_t* srcs;  // [nsrc] sources with an out-edge; [nsrc]: their count
   int32_t* q;        // [slots][n] vertices in level order
   int32_t* lvl;      // [slots][n + 2] level starts in q
   double* bc;        // [n]
@@ -137,97 +139,400 @@ __device__ __forceinline__ int wg_ld(const int* p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
+// State of one source. In global memory: levels in d. In LDS, for graphs that
+// fit: level membership as bitmaps, of which three levels' are kept in turn
+// (bit set l % 3 is cleared while level l + 1 is the current one of the
+// forward pass, or level l - 2 of the backward pass), since a pass only asks
+// for the levels next to its own; 18 bytes a vertex, two workgroups per CU up
+// to 4300 vertices.
+struct BcGlobal {
+  static constexpr int kRow = 16;
+  int32_t* d;
+  double* sig;
+  double* del;
+  int32_t* q;
+  __device__ __forceinline__ void init(int n) const {
+    for (int v = (int)threadIdx.x; v < n; v += blockDim.x) {
+      d[v] = -1;
+      del[v] = 0.0;
+    }
+  }
+  __device__ __forceinline__ void set(int v, int l) const { d[v] = l; }
+  __device__ __forceinline__ bool fresh(int w) const { return wg_ld(&d[w]) == -1; }
+  __device__ __forceinline__ bool claim(int w, int l) const {
+    int expect = -1;
+    return __hip_atomic_compare_exchange_strong(&d[w], &expect, l, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                                __HIP_MEMORY_SCOPE_WORKGROUP);
+  }
+  __device__ __forceinline__ bool at(int v, int l) const { return wg_ld(&d[v]) == l; }
+  __device__ __forceinline__ void mark(int, int) const {}
+  __device__ __forceinline__ void clear(int) const {}
+};
+
+typedef __attribute__((address_space(3))) double lds_f64;
+typedef __attribute__((address_space(3))) uint16_t lds_u16;
+
+struct BcLds {
+  static constexpr int kRow = 8;
+  lds_f64* sig;
+  lds_f64* del;
+  lds_u16* q;
+  lds_u32* seen;
+  lds_u32* bits;  // three bit sets
+  int words;
+  __device__ __forceinline__ void init(int n) const {
+    for (int v = (int)threadIdx.x; v < n; v += blockDim.x) del[v] = 0.0;
+    for (int i = (int)threadIdx.x; i < words; i += blockDim.x) seen[i] = bits[i] = bits[words + i] = bits[2 * words + i] = 0u;
+  }
+  __device__ __forceinline__ void set(int v, int l) const {
+    seen[v >> 5] = 1u << (v & 31);
+    bits[(l % 3) * words + (v >> 5)] = 1u << (v & 31);
+  }
+  __device__ __forceinline__ bool fresh(int w) const { return !((seen[w >> 5] >> (w & 31)) & 1u); }
+  __device__ __forceinline__ bool claim(int w, int l) const {
+    const uint32_t bit = 1u << (w & 31);
+    if (__hip_atomic_fetch_or(&seen[w >> 5], bit, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) & bit) return false;
+    mark(w, l);
+    return true;
+  }
+  __device__ __forceinline__ bool at(int v, int l) const {
+    return (bits[(l % 3) * words + (v >> 5)] >> (v & 31)) & 1u;
+  }
+  __device__ __forceinline__ void mark(int v, int l) const {
+    __hip_atomic_fetch_or(&bits[(l % 3) * words + (v >> 5)], 1u << (v & 31), __ATOMIC_RELAXED,
+                          __HIP_MEMORY_SCOPE_WORKGROUP);
+  }
+  __device__ __forceinline__ void clear(int l) const {
+    for (int i = (int)threadIdx.x; i < words; i += blockDim.x) bits[((l + 3) % 3) * words + i] = 0u;
+  }
+};
+
+__host__ __device__ constexpr int bc_words(int n) { return (n + 31) / 32; }
+__host__ __device__ constexpr long long bc_lds_bytes(long long n) {
+  return 16 * n + (2 * n + 3) / 4 * 4 + 4 * 4 * ((n + 31) / 32);
+}
+
+// Rows of up to State::kRow edges are walked by one thread, all its edges in
+// flight; up to kBcMid by 16 lanes (one DPP row), four rows a wave at a time;
+// longer ones by the wave. (kRow: 16 where an edge's lookups go to memory and
+// want to be many in flight, 8 where they stay in LDS and the kernel is to fit
+// 64 VGPRs.)
+constexpr int kBcMid = 64;
+
+// The rows of the wave's lanes in `m`, 16 lanes a row: the groups take the
+// rows in turn, 16 edges a step, step(v, this lane's target or -1, first step,
+// last step). The next step's targets are loaded before a step is taken.
+template <class Step>
+__device__ __forceinline__ void bc_mid(unsigned long long m, int v, int beg, int end, const int32_t* col,
+                                       const Step& step) {
+  if (!m) return;
+  const int lane = (int)threadIdx.x & 63, sub = lane & 15;
+  const int count = __popcll(m);
+  // lane k: the lane of the k-th row
+  const int rank = __popcll(m & ((1ull << lane) - 1ull));
+  const bool mine = (m >> lane) & 1ull;
+  const int from = __builtin_amdgcn_ds_permute(4 * (mine ? rank : count + lane - rank), lane);
+  auto open = [&](int k, int& vv, int& e, int& b1) {
+    const int src = __shfl(from, k & 63, 64);
+    vv = __shfl(v, src, 64);
+    e = __shfl(beg, src, 64);
+    b1 = __shfl(end, src, 64);
+    if (k >= count) e = b1 = 0;
+  };
+  int k = lane >> 4;  // this group's row, and its next one
+  int vv, e, b1, ov, oe, ob1;
+  open(k, vv, e, b1);
+  int w = e + sub < b1 ? col[e + sub] : -1;
+  open(k + 4, ov, oe, ob1);
+  bool first = true;
+  while (__ballot(e < b1)) {  // every lane takes part in the moves between lanes
+    const bool last = e + 16 >= b1;
+    const int cv = vv, cw = w;
+    const bool live = e < b1;
+    vv = last ? ov : vv;
+    e = last ? oe : e + 16;
+    b1 = last ? ob1 : b1;
+    k = last ? k + 4 : k;
+    w = e + sub < b1 ? col[e + sub] : -1;
+    if (__ballot(last)) open(k + 4, ov, oe, ob1);
+    if (live) step(cv, cw, first, last);
+    first = last;
+  }
+}
+
+// The rows of the wave's lanes in `m`, one after the other, 64 edges a step:
+// step(lane of the row, this lane's target or -1, first step, last step). The
+// next step's targets are loaded before a step is taken.
+template <class Step>
+__device__ __forceinline__ void bc_wide(unsigned long long m, int beg, int end, const int32_t* col, const Step& step) {
+  if (!m) return;
+  const int lane = (int)threadIdx.x & 63;
+  int l = __ffsll((long long)m) - 1;
+  int e = __builtin_amdgcn_readlane(beg, l), b1 = __builtin_amdgcn_readlane(end, l);
+  int w = e + lane < b1 ? col[e + lane] : -1;
+  bool first = true;
+  while (true) {
+    const int cl = l, cw = w;
+    const bool last = e + 64 >= b1;
+    e += 64;
+    if (last) {
+      m &= m - 1;
+      if (m) {
+        l = __ffsll((long long)m) - 1;
+        e = __builtin_amdgcn_readlane(beg, l);
+        b1 = __builtin_amdgcn_readlane(end, l);
+      }
+    }
+    w = m && e + lane < b1 ? col[e + lane] : -1;
+    step(cl, cw, first, last);
+    if (!m) break;
+    first = last;
+  }
+}
+
+// acc plus the wave's terms in lane order (lanes outside h have none).
+__device__ __forceinline__ double bc_add_wave(double acc, double t, unsigned long long h) {
+  const long long bits = __double_as_longlong(t);
+  const int tl = (int)bits, th = (int)(bits >> 32);
+  auto lane_value = [&](int k) {
+    const unsigned lo = (unsigned)__builtin_amdgcn_readlane(tl, k), hi = (unsigned)__builtin_amdgcn_readlane(th, k);
+    return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+  };
+  if (__popcll(h) < 24) {
+    for (; h; h &= h - 1) acc += lane_value(__ffsll((long long)h) - 1);
+  } else {
+#pragma unroll
+    for (int k = 0; k < 64; k++) acc += lane_value(k);  // a lane without a term adds zero
+  }
+  return acc;
+}
+
+// acc plus the terms of the 16 lanes of this lane's DPP row, in lane order.
+template <int K = 0>
+__device__ __forceinline__ double bc_add_row(double acc, double t) {
+  if constexpr (K < 16) {
+    const long long bits = __double_as_longlong(t);
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)bits, 0x150 + K, 0xf, 0xf, false);  // row_newbcast:K
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(bits >> 32), 0x150 + K, 0xf, 0xf, false);
+    return bc_add_row<K + 1>(
+        acc + __longlong_as_double((long long)(((unsigned long long)(unsigned)hi << 32) | (unsigned)lo)), t);
+  } else {
+    return acc;
+  }
+}
+
+// For every vertex v of q[a, z): the terms of its row's edges that have one
+// (term(v, w, &t), never negative), added in edge order whoever computes them
+// (an edge without a term adds zero), then put(v, sum). Consecutive entries go
+// to different waves, so that the hubs, which are found early in a level,
+// spread over the workgroup.
+template <class State, class Term, class Put>
+__device__ __forceinline__ void bc_rows(const State& st, const int32_t* row, const int32_t* col, int a, int z,
+                                        const Term& term, const Put& put) {
+  const int lane = (int)threadIdx.x & 63, wave = (int)threadIdx.x >> 6, nw = (int)blockDim.x >> 6;
+  for (int base = a; base < z; base += blockDim.x) {
+    const int i = base + lane * nw + wave;
+    const bool in = i < z;
+    const int v = in ? (int)st.q[i] : 0;
+    const int beg = in ? row[v] : 0, end = in ? row[v + 1] : 0;
+    const int deg = end - beg;
+    int w[State::kRow];
+#pragma unroll
+    for (int k = 0; k < State::kRow; k++) w[k] = deg <= State::kRow && beg + k < end ? col[beg + k] : -1;
+    if (in && deg <= State::kRow) {
+      double acc = 0.0;
+#pragma unroll
+      for (int k = 0; k < State::kRow; k++) {
+        double t;
+        if (w[k] >= 0 && term(v, w[k], &t)) acc += t;
+      }
+      put(v, acc);
+    }
+    double acc = 0.0;
+    bc_wide(__ballot(deg > kBcMid), beg, end, col, [&](int l, int u, bool first, bool last) {
+      const int vv = __builtin_amdgcn_readlane(v, l);
+      double t = 0.0;
+      const bool has = u >= 0 && term(vv, u, &t);
+      acc = bc_add_wave(first ? 0.0 : acc, has ? t : 0.0, __ballot(has));
+      if (last && lane == 0) put(vv, acc);
+    });
+    bc_mid(__ballot(deg > State::kRow && deg <= kBcMid), v, beg, end, col, [&](int vv, int u, bool first, bool last) {
+      double t = 0.0;
+      if (u < 0 || !term(vv, u, &t)) t = 0.0;
+      acc = bc_add_row(first ? 0.0 : acc, t);
+      if (last && (lane & 15) == 0) put(vv, acc);
+    });
+  }
+}
+
 // One source on one workgroup; returns its number of BFS levels.
-__device__ int bc_source(const BcDev& b, int s, int32_t* d, double* sig, double* del, int32_t* q, int32_t* lvl,
-                         int* s_tail) {
-  for (int v = (int)threadIdx.x; v < b.n; v += blockDim.x) d[v] = -1;
+template <class State>
+__device__ __forceinline__ int bc_source(const BcDev& b, int s, const State& st, int32_t* lvl, int* s_tail) {
+  st.init(b.n);
   __syncthreads();
   if (threadIdx.x == 0) {
-    d[s] = 0;
-    sig[s] = 1.0;
-    q[0] = s;
+    st.set(s, 0);
+    st.sig[s] = 1.0;
+    st.q[0] = s;
     lvl[0] = 0;
     lvl[1] = 1;
     *s_tail = 1;
   }
   __syncthreads();
+  const int lane = (int)threadIdx.x & 63, wave = (int)threadIdx.x >> 6, nw = (int)blockDim.x >> 6;
   int L = 0, lo = 0, hi = 1;
   while (lo < hi) {
     // discover level L + 1 (mega_bfs_kernel_func, bc.cl:17-104)
-    for (int i = lo + (int)threadIdx.x; i < hi; i += blockDim.x) {
-      const int v = q[i];
-      for (int e = b.row_ptr[v]; e < b.row_ptr[v + 1]; e++) {
-        const int w = b.col[e];
-        if (wg_ld(&d[w]) == -1) {
-          int expect = -1;
-          if (__hip_atomic_compare_exchange_strong(&d[w], &expect, L + 1, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
-                                                   __HIP_MEMORY_SCOPE_WORKGROUP))
-            q[atomicAdd(s_tail, 1)] = w;
-        }
-      }
+    auto reach = [&](int w) {
+      if (st.claim(w, L + 1)) st.q[atomicAdd(s_tail, 1)] = w;
+    };
+    st.clear(L - 1);
+    for (int base = lo; base < hi; base += blockDim.x) {
+      const int i = base + lane * nw + wave;
+      const bool in = i < hi;
+      const int v = in ? (int)st.q[i] : 0;
+      const int beg = in ? b.row_ptr[v] : 0, end = in ? b.row_ptr[v + 1] : 0;
+      const int deg = end - beg;
+      int w[State::kRow];
+      bool open[State::kRow];
+#pragma unroll
+      for (int k = 0; k < State::kRow; k++) w[k] = deg <= State::kRow && beg + k < end ? b.col[beg + k] : -1;
+#pragma unroll
+      for (int k = 0; k < State::kRow; k++) open[k] = w[k] >= 0 && st.fresh(w[k]);
+#pragma unroll
+      for (int k = 0; k < State::kRow; k++)
+        if (open[k]) reach(w[k]);
+      bc_wide(__ballot(deg > kBcMid), beg, end, b.col, [&](int, int u, bool, bool) {
+        if (u >= 0 && st.fresh(u)) reach(u);
+      });
+      bc_mid(__ballot(deg > State::kRow && deg <= kBcMid), v, beg, end, b.col, [&](int, int u, bool, bool) {
+        if (u >= 0 && st.fresh(u)) reach(u);
+      });
     }
     __syncthreads();
     // the same for every lane: keep the level loop's control uniform
     const int tail = __builtin_amdgcn_readfirstlane(*s_tail);
     // path counts of level L + 1, pulled over in-edges in order
-    for (int i = hi + (int)threadIdx.x; i < tail; i += blockDim.x) {
-      const int w = q[i];
-      double acc = 0.0;
-      for (int j = b.rrow[w]; j < b.rrow[w + 1]; j++) {
-        const int u = b.rcol[j];
-        if (wg_ld(&d[u]) == L) acc += sig[u];
-      }
-      sig[w] = acc;
-    }
+    bc_rows(
+        st, b.rrow, b.rcol, hi, tail,
+        [&](int, int u, double* t) {
+          if (!st.at(u, L)) return false;
+          *t = st.sig[u];
+          return true;
+        },
+        [&](int w, double acc) { st.sig[w] = acc; });
     if (threadIdx.x == 0) lvl[L + 2] = tail;
     __syncthreads();
     lo = hi;
     hi = tail;
     L++;
   }
-  // dependencies, deepest level first (mega_backtrack_kernel_func, bc.cl:106-183)
-  for (int l = L - 1; l >= 0; l--) {
-    const int a = lvl[l], z = lvl[l + 1];
-    for (int i = a + (int)threadIdx.x; i < z; i += blockDim.x) {
-      const int v = q[i];
-      const double sv = sig[v];
-      double acc = 0.0;
-      for (int e = b.row_ptr[v]; e < b.row_ptr[v + 1]; e++) {
-        const int w = b.col[e];
-        if (wg_ld(&d[w]) == l + 1) acc += sv / sig[w] * (1.0 + del[w]);
-      }
-      del[v] = v == s ? 0.0 : acc;
-    }
+  // dependencies, deepest level first (mega_backtrack_kernel_func, bc.cl:106-183);
+  // the last level's are zero, as initialised
+  for (int l = L - 2; l >= 0; l--) {
+    const int a = __builtin_amdgcn_readfirstlane(lvl[l]), z = __builtin_amdgcn_readfirstlane(lvl[l + 1]);
+    st.clear(l - 1);
+    bc_rows(
+        st, b.row_ptr, b.col, a, z,
+        [&](int v, int w, double* t) {
+          if (!st.at(w, l + 1)) return false;
+          *t = st.sig[v] / st.sig[w] * (1.0 + st.del[w]);
+          return true;
+        },
+        [&](int v, double acc) {
+          if (v != s) st.del[v] = acc;
+          st.mark(v, l);
+        });
     __syncthreads();
   }
   return L;
 }
 
-__global__ void __launch_bounds__(1024) k_bc(Ctl c, BcDev b, int* iters_out) {
-  __shared__ int s_tail;
+// The sources that reach something (an out-edge), in order, by one workgroup;
+// the others have one level and no dependencies. out[nsrc] = their count.
+__global__ void __launch_bounds__(1024) k_bc_sources(const int32_t* row_ptr, int nsrc, int32_t* out) {
+  __shared__ int s_wave[17];
+  int total = 0;
+  for (int base = 0; base < nsrc; base += blockDim.x) {
+    const int s = base + (int)threadIdx.x;
+    const bool take = s < nsrc && row_ptr[s + 1] > row_ptr[s];
+    int cnt;
+    const int at = wg_exclusive_scan(take ? 1 : 0, s_wave, &cnt);
+    if (take) out[total + at] = s;
+    total += cnt;
+  }
+  if (threadIdx.x == 0) out[nsrc] = total;
+}
+
+// The workgroups claim sources one by one and leave each one's dependencies in
+// its row; after a barrier the rows are added to bc in source order, 64
+// vertices a workgroup: every wave stages kBcAhead rows in LDS, one wave adds
+// them. As many sources share a barrier as the rows hold (one row per source
+// where memory allows).
+// Bound: RMAT 12 (ef 8, 4096 sources): the rows' dependent loads and ordered
+// additions in a workgroup. One thread a row, the state in global memory, a
+// barrier per source and workgroup, and the rows added with one load in
+// flight: 11.3 ms a call (1024 x 256), 1.35 ms here.
+constexpr int kBcAhead = 8;
+__host__ __device__ constexpr long long bc_stage_bytes(int wg) { return (long long)wg * kBcAhead * 8; }
+
+template <bool LDS>
+__global__ void __launch_bounds__(1024, LDS ? 8 : 4) k_bc(Ctl c, BcDev b, int* iters_out) {
+  extern __shared__ double lds_bc[];
+  __shared__ int s_tail, s_claim;
   Team t;
   if (!standalone_begin(c, t)) return;
-  const int S = t.n < b.slots ? t.n : b.slots;
   const size_t off = (size_t)t.id * (size_t)b.n;
-  unsigned long long levels = 0;
+  int32_t* lvl = b.lvl + (size_t)t.id * ((size_t)b.n + 2);
+  const int lane = (int)threadIdx.x & 63, wave = (int)threadIdx.x >> 6, nw = (int)blockDim.x >> 6;
+  const int count = __builtin_amdgcn_readfirstlane(b.srcs[b.nsrc]);
+  unsigned long long levels = t.id == 0 ? (unsigned long long)(b.nsrc - count) : 0;
   int batches = 0;
-  for (int base = 0; base < b.nsrc; base += S, batches++) {
-    const int s = base + t.id;
-    if (t.id < S && s < b.nsrc)
-      levels += (unsigned long long)bc_source(b, s, b.d + off, b.sig + off, b.del + off, b.q + off,
-                                              b.lvl + (size_t)t.id * ((size_t)b.n + 2), &s_tail);
-    xcd_barrier(c, t);
-    // bc[v] += delta of each source of the batch, in source order; the rows
-    // are cleared for the next batch on the way
-    const int cnt = b.nsrc - base < S ? b.nsrc - base : S;
-    for (int v = t.id * (int)blockDim.x + (int)threadIdx.x; v < b.n; v += t.n * (int)blockDim.x) {
-      double acc = b.bc[v];
-      for (int j = 0; j < cnt; j++) {
-        double* row = b.del + (size_t)j * (size_t)b.n;
-        acc += row[v];
-        row[v] = 0.0;
+  for (int base = 0; base < count; base += b.rows, batches++) {
+    const int stop = min(count, base + b.rows);
+    int* claim = &c.lines[(batches & 1) * kLine];  // the other one is cleared for the next batch
+    while (t.id < b.slots) {
+      if (threadIdx.x == 0) s_claim = add_relaxed(claim, 1);
+      __syncthreads();
+      const int k = base + __builtin_amdgcn_readfirstlane(s_claim);
+      if (k >= stop) break;
+      const int s = __builtin_amdgcn_readfirstlane(b.srcs[k]);
+      double* del = b.del + (size_t)(k - base) * (size_t)b.n;
+      if constexpr (LDS) {
+        lds_f64* p = (lds_f64*)lds_bc;
+        lds_u16* q = (lds_u16*)(p + 2 * b.n);
+        lds_u32* w = (lds_u32*)q + (b.n + 1) / 2;
+        const int words = bc_words(b.n);
+        const BcLds st{p, p + b.n, q, w, w + words, words};
+        levels += (unsigned long long)bc_source(b, s, st, lvl, &s_tail);
+        for (int v = (int)threadIdx.x; v < b.n; v += blockDim.x) del[v] = st.del[v];
+      } else {
+        const BcGlobal st{b.d + off, b.sig + off, del, b.q + off};
+        levels += (unsigned long long)bc_source(b, s, st, lvl, &s_tail);
       }
-      b.bc[v] = acc;
+      __syncthreads();
+    }
+    if (t.id == 0 && threadIdx.x == 0) st_relaxed(&c.lines[((batches + 1) & 1) * kLine], 0);
+    xcd_barrier(c, t);
+    double* stage = lds_bc;  // [nw * kBcAhead][64]
+    for (int v0 = t.id * 64; v0 < b.n; v0 += t.n * 64) {
+      const int v = v0 + lane;
+      double acc = wave == 0 && v < b.n ? b.bc[v] : 0.0;
+      for (int j0 = base; j0 < stop; j0 += nw * kBcAhead) {
+        const int j = j0 + wave * kBcAhead;
+        const double* x = b.del + (size_t)(j - base) * (size_t)b.n + v;
+        double y[kBcAhead];
+#pragma unroll
+        for (int k = 0; k < kBcAhead; k++) y[k] = j + k < stop && v < b.n ? x[(size_t)k * (size_t)b.n] : 0.0;
+        __syncthreads();  // the last round's sums are done
+#pragma unroll
+        for (int k = 0; k < kBcAhead; k++) stage[(wave * kBcAhead + k) * 64 + lane] = y[k];
+        __syncthreads();
+        if (wave == 0)
+          for (int k = 0; k < nw * kBcAhead; k++) acc += stage[k * 64 + lane];  // rows past the end add zero
+      }
+      if (wave == 0 && v < b.n) b.bc[v] = acc;
+      __syncthreads();
     }
     xcd_barrier(c, t);
   }
@@ -310,7 +615,7 @@ const void* minplus_kernel(int lanes) {
 // grid from the occupancy of `kernel` (capped at max_grid), optional host
 // handshake, bounded wait.
 int launch_standalone_app(wgm_runtime* rt, int kernel, const void* fn, const wgm_launch* lc, Ctl* ctl, void** args,
-                          int max_grid, wgm_run_stats* st) {
+                          int max_grid, wgm_run_stats* st, size_t lds = 0) {
   wgm_launch def{256, 0, 0, 0};
   const wgm_launch& l = lc ? *lc : def;
   const int wg = l.wg_size > 0 ? l.wg_size : 256;
@@ -322,7 +627,7 @@ int launch_standalone_app(wgm_runtime* rt, int kernel, const void* fn, const wgm
   if (rc) return rc;
   *ctl = rt->ctl;
   HIPCHK(rt, hipEventRecord(rt->ev0, rt->stream));
-  HIPCHK(rt, hipLaunchKernel(fn, dim3(grid), dim3(wg), args, 0, rt->stream));
+  HIPCHK(rt, hipLaunchKernel(fn, dim3(grid), dim3(wg), args, lds, rt->stream));
   double host_ms = 0.0;
   if (l.handshake) {
     rc = wgm_host_handshake(rt, &host_ms);
@@ -334,9 +639,28 @@ int launch_standalone_app(wgm_runtime* rt, int kernel, const void* fn, const wgm
   return WGM_OK;
 }
 
+// LDS a BC workgroup may use, and what it takes besides its state (statics and
+// allocation granularity, rounded up).
+constexpr long long kBcLds = 160 << 10;
+constexpr long long kBcLdsFixed = 1536;
+constexpr int kCuThreads = 2048;  // 32 waves
+constexpr size_t kBcRowBytes = 1ull << 30;
+
+// Whether a source's state fits LDS: 18 bytes a vertex, up to about 8900
+// vertices. Below that the state is always in LDS, also where only one
+// workgroup then fits a CU (RMAT 13, ef 8, 1500 sources, kernel: 1.28 ms; 3.14
+// ms in global memory at 1024 x 256, 2.27 at 256 x 1024).
+bool bc_in_lds(const wgm_graph* g) { return bc_lds_bytes(g->n) + kBcLdsFixed <= kBcLds; }
+long long bc_lds(const wgm_graph* g, int wg) {
+  return std::max(bc_stage_bytes(wg), bc_in_lds(g) ? bc_lds_bytes(g->n) : 0ll);
+}
+
 // Grid of the BC launch: the occupancy grid, capped so the per-slot state
-// stays within kBcSlotBytes.
-int bc_grid(wgm_runtime* rt, const wgm_graph* g, const wgm_launch* lc, int* grid) {
+// stays within kBcSlotBytes. With the state in LDS, which then bounds the
+// workgroups on a CU, the threads asked for are taken in as many larger
+// workgroups as fit (RMAT 12, 1024 x 256 asked, kernel: 1.73 ms as 512 x 256,
+// 1.25 ms as 512 x 512).
+int bc_grid(wgm_runtime* rt, const wgm_graph* g, const wgm_launch* lc, int* grid, int* wg) {
   wgm_launch def{256, 0, 0, 0};
   const wgm_launch& l = lc ? *lc : def;
   int rc = wgm_resolve_grid(rt, WGM_K_BC, l.wg_size > 0 ? l.wg_size : 256, l.num_wgs, grid);
@@ -345,6 +669,20 @@ int bc_grid(wgm_runtime* rt, const wgm_graph* g, const wgm_launch* lc, int* grid
   const size_t cap = (size_t)kBcSlotBytes / per_slot;
   if (cap < 1) return fail(rt, WGM_ERR_NOMEM, "one BC slot needs %zu bytes", per_slot);
   if ((size_t)*grid > cap) *grid = (int)cap;
+  *wg = l.wg_size > 0 ? l.wg_size : 256;
+  if (bc_in_lds(g)) {
+    const int per_cu = (int)std::min(kBcLds / (bc_lds(g, *wg) + kBcLdsFixed), (long long)kCuThreads / *wg);
+    const int fit = std::max(per_cu, 1) * rt->info.num_cus;
+    if (*grid > fit) {
+      *wg = std::min({1024, *wg * (*grid / fit), kCuThreads / std::max(per_cu, 1) / 64 * 64});
+      *grid = fit;
+    }
+  } else {  // more than can be resident would only cost the discovery window
+    int per_cu = 0;
+    rc = wgm_occupancy(rt, WGM_K_BC, *wg, &per_cu);
+    if (rc) return rc;
+    *grid = std::min(*grid, std::max(per_cu, 1) * rt->info.num_cus);
+  }
   return WGM_OK;
 }
 
@@ -352,10 +690,12 @@ int bc_grid(wgm_runtime* rt, const wgm_graph* g, const wgm_launch* lc, int* grid
 
 int wgm_graph_in_edges(wgm_graph* g) { return graph_reverse(g); }
 
+static int bc_stage(int wg) { return (int)bc_stage_bytes(wg); }
+
 bool wgm_pannotia_kernel_info(int kernel, KernelInfo* out) {
   switch (kernel) {
     case WGM_K_MINPLUS: *out = KernelInfo{(const void*)&k_minplus<16>, nullptr}; return true;
-    case WGM_K_BC: *out = KernelInfo{(const void*)&k_bc, nullptr}; return true;
+    case WGM_K_BC: *out = KernelInfo{(const void*)&k_bc<false>, bc_stage}; return true;
     default: return false;
   }
 }
@@ -367,7 +707,7 @@ int wgm_pannotia_probe(wgm_runtime* rt, int kernel, int grid, int wg_size) {
                          (int*)nullptr);
       return WGM_OK;
     case WGM_K_BC:
-      hipLaunchKernelGGL(k_bc, dim3(grid), dim3(wg_size), 0, rt->stream, rt->ctl, BcDev{}, (int*)nullptr);
+      hipLaunchKernelGGL(k_bc<false>, dim3(grid), dim3(wg_size), (size_t)bc_stage_bytes(wg_size), rt->stream, rt->ctl, BcDev{}, (int*)nullptr);
       return WGM_OK;
     default:
       return WGM_ERR_INVALID;
@@ -375,7 +715,7 @@ int wgm_pannotia_probe(wgm_runtime* rt, int kernel, int grid, int wg_size) {
 }
 
 void wgm_pannotia_release(wgm_graph* g) {
-  void* ptrs[] = {g->rrow, g->rcol, g->rwt, g->tasks, g->bc_d, g->bc_sig, g->bc_del, g->bc_q, g->bc_lvl, g->bc_sum};
+  void* ptrs[] = {g->rrow, g->rcol, g->rwt, g->tasks, g->bc_d, g->bc_sig, g->bc_del, g->bc_q, g->bc_lvl, g->bc_sum, g->bc_srcs};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
 }
@@ -440,36 +780,44 @@ int wgm_bc(wgm_runtime* rt, wgm_graph* g, int32_t num_sources, const wgm_launch*
   const int32_t nsrc = num_sources > 0 ? num_sources : g->n;
   int rc = graph_reverse(g);
   if (rc) return rc;
-  int grid = 0;
-  rc = bc_grid(rt, g, lc, &grid);
+  int grid = 0, wg = 0;
+  rc = bc_grid(rt, g, lc, &grid, &wg);
   if (rc) return rc;
-  if (g->bc_slots < grid) {
+  // a row per source where kBcRowBytes hold them, at least one per workgroup
+  const int32_t rows = (int32_t)std::min<size_t>((size_t)nsrc, std::max<size_t>((size_t)grid, kBcRowBytes / (8 * (size_t)g->n)));
+  if (g->bc_slots < grid || g->bc_rows < rows) {
     void* old[] = {g->bc_d, g->bc_sig, g->bc_del, g->bc_q, g->bc_lvl};
     for (void* p : old)
       if (p) (void)hipFree(p);
     g->bc_d = g->bc_q = g->bc_lvl = nullptr;
     g->bc_sig = g->bc_del = nullptr;
-    g->bc_slots = 0;
-    const size_t sn = (size_t)grid * (size_t)g->n;
-    hipError_t e = hipMalloc((void**)&g->bc_d, sizeof(int32_t) * sn);
-    if (e == hipSuccess) e = hipMalloc((void**)&g->bc_sig, sizeof(double) * sn);
-    if (e == hipSuccess) e = hipMalloc((void**)&g->bc_del, sizeof(double) * sn);
-    if (e == hipSuccess) e = hipMalloc((void**)&g->bc_q, sizeof(int32_t) * sn);
-    if (e == hipSuccess) e = hipMalloc((void**)&g->bc_lvl, sizeof(int32_t) * (size_t)grid * ((size_t)g->n + 2));
+    const int32_t slots = std::max(g->bc_slots, grid), nrows = std::max(g->bc_rows, rows);
+    g->bc_slots = g->bc_rows = 0;
+    const size_t sn = (size_t)slots * (size_t)g->n;
+    hipError_t e = hipMalloc((void**)&g->bc_del, sizeof(double) * (size_t)nrows * (size_t)g->n);
+    if (e == hipSuccess) e = hipMalloc((void**)&g->bc_lvl, sizeof(int32_t) * (size_t)slots * ((size_t)g->n + 2));
+    if (!bc_in_lds(g)) {
+      if (e == hipSuccess) e = hipMalloc((void**)&g->bc_d, sizeof(int32_t) * sn);
+      if (e == hipSuccess) e = hipMalloc((void**)&g->bc_sig, sizeof(double) * sn);
+      if (e == hipSuccess) e = hipMalloc((void**)&g->bc_q, sizeof(int32_t) * sn);
+    }
     if (e != hipSuccess) return wgm_hip_fail(rt, e, "hipMalloc(BC slots)");
-    // dependency rows start at zero; each batch's reduction clears them again
-    HIPCHK(rt, hipMemsetAsync(g->bc_del, 0, sizeof(double) * sn, rt->stream));
-    g->bc_slots = grid;
+    g->bc_slots = slots;
+    g->bc_rows = nrows;
   }
+  if (!g->bc_srcs) HIPCHK(rt, hipMalloc((void**)&g->bc_srcs, sizeof(int32_t) * ((size_t)g->n + 1)));
   if (!g->bc_sum) HIPCHK(rt, hipMalloc((void**)&g->bc_sum, sizeof(double) * ((size_t)g->n + 1)));
   unsigned long long* levels = (unsigned long long*)(g->bc_sum + g->n);
   HIPCHK(rt, hipMemsetAsync(g->bc_sum, 0, sizeof(double) * ((size_t)g->n + 1), rt->stream));
   BcDev b{g->row_ptr, g->col, g->rrow, g->rcol, g->n, nsrc, g->bc_slots, g->bc_d, g->bc_sig, g->bc_del,
-          g->bc_q, g->bc_lvl, g->bc_sum, levels};
+          rows, g->bc_srcs, g->bc_q, g->bc_lvl, g->bc_sum, levels};
+  hipLaunchKernelGGL(k_bc_sources, dim3(1), dim3(1024), 0, rt->stream, g->row_ptr, nsrc, g->bc_srcs);
   Ctl ctl{};
   void* args[] = {&ctl, &b, &g->iters};
   wgm_run_stats local{};
-  rc = launch_standalone_app(rt, WGM_K_BC, (const void*)&k_bc, lc, &ctl, args, grid, &local);
+  const wgm_launch shape{wg, grid, lc ? lc->handshake : 0, 0};
+  rc = launch_standalone_app(rt, WGM_K_BC, bc_in_lds(g) ? (const void*)&k_bc<true> : (const void*)&k_bc<false>, &shape, &ctl, args, grid,
+                             &local, (size_t)bc_lds(g, wg));
   if (rc) return rc;
   unsigned long long lv = 0;
   HIPCHK(rt, hipMemcpy(&lv, levels, sizeof(lv), hipMemcpyDeviceToHost));

@@ -105,3 +105,44 @@ def test_color_directed_round_count(rt, degree):
     ref, rounds = oracle.color(g.row_ptr, g.col, g.prio)
     out, st = rt.graph(g).color(wg_size=256, num_wgs=24)
     assert np.array_equal(out, ref) and st["iterations"] == rounds
+
+
+def _lds_limit():
+    """Largest vertex count whose BC state is kept in LDS (18 bytes a vertex and four bitmaps in 160 KB - 1536)."""
+    n = 8000
+    while 16 * (n + 1) + (2 * (n + 1) + 3) // 4 * 4 + 16 * ((n + 32) // 32) + 1536 <= 160 << 10:
+        n += 1
+    return n
+
+
+def _random_arcs(n, m, seed):
+    rng = np.random.default_rng(seed)
+    return G.from_edges(n, rng.integers(0, n, m), rng.integers(0, n, m))
+
+
+BC_GRAPHS = {
+    "lds limit": (lambda: _random_arcs(_lds_limit(), 30000, 1), 70),
+    "above lds": (lambda: _random_arcs(_lds_limit() + 1, 30000, 1), 70),
+    "row stages": (_stage_graph, 40),  # rows of 8, 9, 16, 17, 64, 65 edges and more, in both directions
+    "stages, global": (lambda: _symmetric(G.from_edges(9001, np.r_[np.zeros(700, int), np.ones(64, int), np.full(17, 2)],
+                                                       np.r_[np.arange(10, 710), np.arange(300, 364), np.arange(5, 22)])), 30),
+    "many levels": (lambda: G.grid(1, 301), 301),
+    "large counts": (lambda: G.grid(40, 41), 50),  # path counts far above 2^53
+    "one vertex": (lambda: G.CSR(np.zeros(2, np.int32), np.zeros(0, np.int32)), 1),
+    "no edges": (lambda: G.CSR(np.zeros(34, np.int32), np.zeros(0, np.int32)), 33),
+    "two batches": (lambda: G.from_edges(12001, np.zeros(12000, int), np.arange(1, 12001), symmetric=True), 12001),
+}
+
+
+@pytest.mark.parametrize("name", list(BC_GRAPHS))
+def test_bc_state_and_row_classes(rt, name):
+    """Bit-exact sums wherever the state of a source is kept and whoever walks
+    its rows, level count included."""
+    make, sources = BC_GRAPHS[name]
+    g = make()
+    ref, levels = oracle.bc(g.row_ptr, g.col, sources)
+    dg = rt.graph(g)
+    for wg, wgs in ((64, 9), (256, 1024)) if g.n < 12000 else ((256, 1024),):
+        out, st = dg.bc(sources, wg_size=wg, num_wgs=wgs)
+        assert np.array_equal(out, ref) and st["iterations"] == levels, (wg, wgs)
+    dg.close()
