@@ -10,9 +10,10 @@
 // resident and only the per-run state is re-initialised on the device.
 
 #include "apps_internal.hpp"
-#include "team_frontier.hpp"
+#include "low_degree.hpp"
 
 #include <algorithm>
+#include <cstdlib>
 #include <cstring>
 
 using namespace wgm;
@@ -50,6 +51,55 @@ __global__ void __launch_bounds__(1024) k_frontier(Ctl c, GraphDev g, FrontierDe
                                               [&]() { xcd_barrier<false>(c, t); });
   clock_end(c, t.id);
   standalone_retire(c);
+}
+
+// BFS / push SSSP on a low-degree graph of narrow levels (a mesh or road
+// network of up to kLowMaxN vertices): one workgroup runs the degree-bounded
+// step of the batched launch, its queues, visited or far bits and combine
+// tables in LDS, on packed rows (k_low_rows). A team's cross-workgroup barrier
+// costs more than a narrow level's work. Bound: two dependent loads and one or
+// two workgroup barriers a level (1.1 us BFS, 2.3 us SSSP).
+// Rule: no edge spans more than kLowSpan places of the (circular) vertex
+// order, so that k levels reach at most 2 k kLowSpan + 1 vertices; or the whole
+// graph is small. Kernel times, team -> one workgroup, 64 x 512: 361 x 415 grid
+// BFS 3508 -> 606 us, SSSP 7293 -> 2591; 10^5 vertices of 4 random edges within
+// span 300: 2608 -> 408 and 6428 -> 1777, span 1000: 502 -> 243 and 1392 ->
+// 1422, so the line lies at 768; random targets, 8192 vertices: 75 -> 32 and
+// 209 -> 122, 16384: 93 -> 50 and 254 -> 237, 20000: SSSP 272 -> 300 and more,
+// so it lies at 16384. Whole calls, 361 x 415 SSSP: 8106 -> 2903 us.
+constexpr int32_t kLowSpan = 768;
+constexpr int32_t kLowAnySpan = 16384;
+constexpr int32_t kLowMaxN = 32 * kFarBitWords;
+// Band width of the low-degree SSSP (weights in [0, 255]), as in the batched
+// launch.
+constexpr uint32_t kLowDelta = 512;
+
+template <bool SSSP>
+__global__ void __launch_bounds__(1024) k_low(Ctl c, GraphDev g, FrontierDev s, NearFar nf, int src,
+                                              const uint32_t* ell, int* iters_out) {
+  extern __shared__ __attribute__((aligned(16))) int lds_low[];  // the combine tables hold 64-bit words
+  __shared__ int s_cnt[3];
+  Team t;
+  if (!standalone_begin(c, t)) return;
+  if (t.id == 0) {
+    nf.delta = SSSP ? kLowDelta : 0u;
+    run_low<SSSP, kLowDegree, SSSP ? kCombU : kLowSlots, true, SSSP>(g, s, nf, src, lds_low, s_cnt, iters_out, true, ell);
+    __syncthreads();
+    if (threadIdx.x == 0) clock_end(c, 0);
+  }
+  standalone_retire(c);
+}
+
+// Packed rows of a low-degree graph: kLowDegree words a vertex, (target << 8) |
+// weight, kEllNone past the degree.
+__global__ void k_low_rows(GraphDev g, uint32_t* ell) {
+  for (int v = blockIdx.x * blockDim.x + threadIdx.x; v < g.n; v += gridDim.x * blockDim.x) {
+    const int beg = g.row_ptr[v], deg = g.row_ptr[v + 1] - beg;
+#pragma unroll
+    for (int k = 0; k < kLowDegree; k++)
+      ell[(size_t)v * kLowDegree + k] =
+          k < deg ? ((uint32_t)g.col[beg + k] << 8) | (g.wt ? (uint32_t)g.wt[beg + k] & 255u : 0u) : kEllNone;
+  }
 }
 
 // Colouring without rounds. The rounds give a vertex the colour 1 + the
@@ -444,6 +494,18 @@ int wgm_graph_create(wgm_runtime* rt, const wgm_csr* h, const uint32_t* prio, wg
   g->n = h->n;
   g->m = h->m;
   g->maxdeg = maxdeg;
+  if (maxdeg <= kLowDegree && h->n <= kLowMaxN) {
+    int32_t span = 0;
+    for (int32_t v = 0; h->n > kLowAnySpan && v < h->n; v++)
+      for (int32_t e = h->row_ptr[v], end = h->row_ptr[v + 1]; e < end; e++) {
+        const int32_t d = std::abs(h->col[e] - v);
+        span = std::max(span, std::min(d, h->n - d));
+      }
+    uint32_t bits = 0;
+    for (int64_t e = 0; h->wt && e < h->m; e++) bits |= (uint32_t)h->wt[e];
+    g->low = span <= kLowSpan;
+    g->low_weights = g->low && h->wt && bits <= 255u;
+  }
   auto bail = [&](int rc) { wgm_graph_destroy(g); return rc; };
   int rc = dev_alloc(rt, &g->row_ptr, (size_t)h->n + 1);
   if (!rc) rc = dev_alloc(rt, &g->col, (size_t)h->m);
@@ -465,7 +527,7 @@ int wgm_graph_destroy(wgm_graph* g) {
   wgm_pannotia_release(g);
   void* ptrs[] = {g->row_ptr, g->col, g->wt, g->prio, g->dist, g->stamp, g->q0, g->q1, g->counts,
                   g->i32a, g->i32b, g->f0, g->f1, g->f2, g->iters, g->tq, g->tqa, g->claims, g->far,
-                  g->in_far, g->fcnt, g->hv, g->hdu, g->hclaim, g->hcnt, g->wl};
+                  g->in_far, g->fcnt, g->hv, g->hdu, g->hclaim, g->hcnt, g->wl, g->ell};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
   delete g;
@@ -477,6 +539,7 @@ int64_t wgm_graph_bytes(const wgm_graph* g) {
   int64_t b = 4 * ((int64_t)g->n + 1) + 4 * g->m;
   if (g->wt) b += 4 * g->m;
   if (g->prio) b += 4 * (int64_t)g->n;
+  if (g->ell) b += 4 * kLowDegree * (int64_t)g->n;
   if (g->rrow) b += 4 * ((int64_t)g->n + 1) + (g->rwt ? 8 : 4) * g->m + 16 * (int64_t)g->ntasks;
   return b;
 }
@@ -504,12 +567,13 @@ int wgm_enqueue_frontier(wgm_runtime* rt, const GraphDev& g, FrontierDev s, cons
   return WGM_OK;
 }
 
-int wgm_launch_frontier(wgm_runtime* rt, const GraphDev& g, FrontierDev s, const NearFar& nf, bool sssp, int src,
-                        int grid, int wg, int handshake, int* iters_dev, wgm_run_stats* st) {
+template <class Enqueue>
+static int launch_and_finish(wgm_runtime* rt, int handshake, int* iters_dev, const Enqueue& enqueue,
+                             wgm_run_stats* st) {
   int rc = wgm_reset_ctl(rt, 0, handshake ? 1 : 0);
   if (rc) return rc;
   HIPCHK(rt, hipEventRecord(rt->ev0, rt->stream));
-  rc = wgm_enqueue_frontier(rt, g, s, nf, sssp, src, grid, wg, iters_dev);
+  rc = enqueue();
   if (rc) return rc;
   double host_ms = 0.0;
   if (handshake) rc = wgm_host_handshake(rt, &host_ms);
@@ -522,6 +586,39 @@ int wgm_launch_frontier(wgm_runtime* rt, const GraphDev& g, FrontierDev s, const
   local.iterations = iters;
   local.host_ms = host_ms;
   if (st) *st = local;
+  return WGM_OK;
+}
+
+int wgm_launch_frontier(wgm_runtime* rt, const GraphDev& g, FrontierDev s, const NearFar& nf, bool sssp, int src,
+                        int grid, int wg, int handshake, int* iters_dev, wgm_run_stats* st) {
+  return launch_and_finish(
+      rt, handshake, iters_dev, [&]() { return wgm_enqueue_frontier(rt, g, s, nf, sssp, src, grid, wg, iters_dev); }, st);
+}
+
+// The packed rows of a low-degree graph, laid out once.
+static int low_rows(wgm_runtime* rt, wgm_graph* g) {
+  if (g->ell) return WGM_OK;
+  int rc = dev_alloc(rt, &g->ell, (size_t)kLowDegree * (size_t)g->n);
+  if (rc) return rc;
+  hipLaunchKernelGGL(k_low_rows, dim3(256), dim3(256), 0, rt->stream, wgm_graph_view(g), g->ell);
+  HIPCHK(rt, hipGetLastError());
+  return WGM_OK;
+}
+
+// Enqueue k_low: the threads asked for, in workgroups of up to 1024 (one fits a
+// CU beside its LDS).
+static int enqueue_low(wgm_runtime* rt, const wgm_graph* g, const FrontierDev& s, const NearFar& nf, bool sssp, int src,
+                       int grid, int wg) {
+  const GraphDev view = wgm_graph_view(g);
+  const long long threads = (long long)grid * wg;
+  const int lwg = (int)std::min<long long>(1024, threads);
+  const int lgrid = (int)std::min<long long>(threads / lwg, rt->info.num_cus);
+  const size_t lds = sssp ? (size_t)kLowSsspLds : (size_t)low_bfs_lds_bytes(lwg);
+  if (sssp)
+    hipLaunchKernelGGL(k_low<true>, dim3(lgrid), dim3(lwg), lds, rt->stream, rt->ctl, view, s, nf, src, g->ell, g->iters);
+  else
+    hipLaunchKernelGGL(k_low<false>, dim3(lgrid), dim3(lwg), lds, rt->stream, rt->ctl, view, s, nf, src, g->ell, g->iters);
+  HIPCHK(rt, hipGetLastError());
   return WGM_OK;
 }
 
@@ -560,16 +657,25 @@ static int run_frontier(wgm_runtime* rt, wgm_graph* g, int32_t src, const wgm_la
   int grid = 0;
   rc = wgm_resolve_grid(rt, kernel, wg, lc ? lc->num_wgs : 0, &grid);
   if (rc) return rc;
-  // BFS takes its wide levels bottom-up over the in-edges
+  const bool low = sssp ? g->low_weights : g->low;
   GraphDev view = wgm_graph_view(g);
-  if (!sssp) {
+  if (low) {
+    rc = low_rows(rt, g);
+    if (rc) return rc;
+  } else if (!sssp) {
+    // BFS takes its wide levels bottom-up over the in-edges
     rc = wgm_graph_in_edges(g);
     if (rc) return rc;
     view.rrow = g->rrow;
     view.rcol = g->rcol;
   }
   wgm_run_stats local{};
-  rc = wgm_launch_frontier(rt, view, s, nf, sssp, src, grid, wg, lc ? lc->handshake : 0, g->iters, &local);
+  if (low) {
+    auto enqueue = [&]() { return enqueue_low(rt, g, s, nf, sssp, src, grid, wg); };
+    rc = launch_and_finish(rt, lc ? lc->handshake : 0, g->iters, enqueue, &local);
+  } else {
+    rc = wgm_launch_frontier(rt, view, s, nf, sssp, src, grid, wg, lc ? lc->handshake : 0, g->iters, &local);
+  }
   if (rc) return rc;
   rc = wgm_graph_reached_edges(g, &local.edges_scanned);
   if (rc) return rc;

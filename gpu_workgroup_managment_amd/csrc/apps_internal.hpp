@@ -25,6 +25,11 @@ struct wgm_graph {
   float* f2 = nullptr;
   int* iters = nullptr;
   int32_t* wl = nullptr;  // colour / MIS worklists, PageRank's long rows (wl_words in apps.hip)
+  // low-degree graphs (k_low): BFS may run on one workgroup; the weights also
+  // fit the packed rows; the rows, laid out on first use
+  bool low = false;
+  bool low_weights = false;
+  uint32_t* ell = nullptr;
   // standalone BFS / SSSP (one team of every participant): two queues of
   // tcap entries with distance tags (SSSP), claim counters, near-far queues
   // and flags

@@ -146,3 +146,46 @@ def test_bc_state_and_row_classes(rt, name):
         out, st = dg.bc(sources, wg_size=wg, num_wgs=wgs)
         assert np.array_equal(out, ref) and st["iterations"] == levels, (wg, wgs)
     dg.close()
+
+
+def _spans(n, span, seed):
+    """Four out-edges a vertex (some fewer), none longer than `span` on the ring of n vertices."""
+    rng = np.random.default_rng(seed)
+    src = np.repeat(np.arange(n), rng.integers(0, 5, n))
+    g = G.from_edges(n, src, (src + rng.integers(-span, span + 1, len(src))) % n)
+    g.wt = rng.integers(0, 256, g.m).astype(np.int32)
+    return g
+
+
+LOW = {
+    "one": lambda: G.CSR(np.zeros(2, np.int32), np.zeros(0, np.int32), np.zeros(0, np.int32)),
+    "path": lambda: G.grid(1, 300),
+    "spill": lambda: _spans(16384, 8192, 1),  # levels past the queues in LDS, any span
+    "above": lambda: _spans(16385, 769, 2),  # past both lines
+    "ring": lambda: _spans(40000, 768, 3),
+    "bits": lambda: G.grid(512, 512),         # the last bit of the LDS bitmaps
+    "past": lambda: G.grid(437, 600),         # 2^18 + 56 vertices
+}
+
+
+@pytest.mark.parametrize("name", LOW)
+def test_low_degree_graphs(rt, name):
+    """BFS and push SSSP where a low-degree graph moves to one workgroup, on
+    both sides of each line; weights of 0 and 255, then one above the packed
+    rows' 8 bits."""
+    g = LOW[name]()
+    if g.m and g.wt is None:
+        g.wt = np.random.default_rng(5).integers(0, 256, g.m).astype(np.int32)
+    src = g.n // 2 if name != "bits" else 0
+    for top in (255, 256):
+        if g.m:
+            g.wt[g.m // 2] = top
+        levels, n_levels = oracle.bfs(g.row_ptr, g.col, src)
+        ref = oracle.sssp(g.row_ptr, g.col, g.wt, src)
+        dg = rt.graph(g)
+        for wg, wgs in ((64, 1), (320, 3), (512, 64), (1024, 0)):
+            d, st = dg.bfs(src, wg_size=wg, num_wgs=wgs)
+            assert np.array_equal(d, levels) and st["iterations"] == n_levels, (wg, wgs)
+            d, _ = dg.sssp(src, wg_size=wg, num_wgs=wgs, mode=1)
+            assert np.array_equal(d, ref), (wg, wgs)
+        dg.close()
