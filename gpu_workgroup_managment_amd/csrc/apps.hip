@@ -48,7 +48,8 @@ __global__ void __launch_bounds__(1024) k_frontier(Ctl c, GraphDev g, FrontierDe
   Team t;
   if (!standalone_begin(c, t)) return;
   run_team<SSSP, SSSP ? kEdgeSlots : 1, true>(g, s, nf, src, t.id, t.n, lds, iters_out,
-                                              [&]() { xcd_barrier<false>(c, t); });
+                                              [&]() { xcd_barrier<false>(c, t); },
+                                              lds + standalone_pass_lds_bytes(blockDim.x) / 4);
   clock_end(c, t.id);
   standalone_retire(c);
 }
@@ -403,6 +404,7 @@ static int team_frontier_state(wgm_graph* g, bool sssp, FrontierDev* s, NearFar*
   s->hdu = g->hdu;
   s->hclaim = g->hclaim;
   s->hcnt = g->hcnt;
+  s->fine = g->maxdeg > kFineDegree ? 1 : 0;
   *nf = NearFar{};
   if (sssp) {
     nf->q[0] = g->far;
@@ -431,6 +433,7 @@ int wgm_graph_reached_edges(wgm_graph* g, int64_t* out) {
 
 // Both forms of the colour and MIS kernels are launched with the long-row
 // form's LDS, so that the grid found for one holds for the other.
+static int wgm_frontier_lds(int wg) { return standalone_frontier_lds_bytes(wg); }
 static int scan_lds(int wg) { return scan_lds_bytes(wg); }
 
 bool wgm_app_kernel_info(int kernel, KernelInfo* out) {
@@ -558,7 +561,7 @@ int wgm_enqueue_frontier(wgm_runtime* rt, const GraphDev& g, FrontierDev s, cons
                          int grid, int wg, int* iters_dev) {
   s.chunk = wg;  // frontier entries a workgroup claims at a time
   s.heavy = heavy_threshold(wg);
-  const size_t lds = frontier_lds_bytes(wg);
+  const size_t lds = standalone_frontier_lds_bytes(wg);
   if (sssp)
     hipLaunchKernelGGL(k_frontier<true>, dim3(grid), dim3(wg), lds, rt->stream, rt->ctl, g, s, nf, src, iters_dev);
   else

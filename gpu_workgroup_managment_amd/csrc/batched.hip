@@ -975,6 +975,7 @@ int wgm_batch_run_standalone(wgm_runtime* rt, wgm_batch* b, const wgm_launch* lc
     s.hdu = (uint32_t*)(b->sa_heavy + b->sa_hcap);
     s.hclaim = b->sa_heavy + 2 * b->sa_hcap;
     s.hcnt = b->sa_heavy + 3 * b->sa_hcap;
+    s.fine = j.maxdeg > kFineDegree ? 1 : 0;
     NearFar nf{};
     if (sssp) {
       nf.q[0] = b->far + j.f_off;

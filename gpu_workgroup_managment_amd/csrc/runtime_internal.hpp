@@ -43,8 +43,6 @@ struct KernelInfo {
   int (*lds)(int wg_size);  // dynamic LDS bytes at a workgroup size (nullptr: none)
 };
 
-inline int wgm_frontier_lds(int wg) { return wgm::frontier_lds_bytes(wg); }
-
 const KernelInfo& wgm_kernel_info(int kernel);
 size_t wgm_kernel_lds(int kernel, int wg_size);
 int wgm_hip_fail(wgm_runtime* rt, hipError_t e, const char* what);

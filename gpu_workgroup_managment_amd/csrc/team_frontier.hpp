@@ -63,55 +63,115 @@ __device__ __forceinline__ void team_barrier(int* cnt, int* gen, int k, int& epo
   __syncthreads();
 }
 
+// LDS of the standalone frontier kernels: a frontier pass (frontier_batch) or a
+// bottom-up pass (the scan queues and its found vertices), then
+// kStandaloneWords words that outlast a pass.
+constexpr int kStandaloneWords = 4;
+__host__ __device__ constexpr int bottom_up_lds_bytes(int bd) { return scan_lds_bytes(bd) + kScanU * bd * 4; }
+__host__ __device__ constexpr int standalone_pass_lds_bytes(int bd) {
+  return frontier_lds_bytes(bd) > bottom_up_lds_bytes(bd) ? frontier_lds_bytes(bd) : bottom_up_lds_bytes(bd);
+}
+__host__ __device__ constexpr int standalone_frontier_lds_bytes(int bd) {
+  return standalone_pass_lds_bytes(bd) + 4 * kStandaloneWords;
+}
+
+// Frontier membership (bottom-up): a vertex of distance `level`.
+struct FrontProbe {
+  const uint32_t* dist;
+  uint32_t level;
+  __device__ __forceinline__ bool test(int u, uint32_t, bool valid, int&) const {
+    return valid & (ld_agent(&dist[u]) == level);
+  }
+};
+
 // A BFS level taken bottom-up (direction-optimizing BFS, Beamer et al.,
 // SC 2012): every unvisited vertex of the member's range looks for an
-// in-neighbour in the frontier (dist == level), four in-edges per round with
-// an early exit, and if it finds one takes level + 1 and queues itself. A
-// vertex is written only by its own thread, so no atomic on dist is needed;
-// the distances are read and written with agent-scope accesses (coherent
-// across the XCDs' L2s, as the top-down step's). The set of vertices it
-// discovers is the top-down level's: the unvisited vertices with an in-edge
-// from the frontier. The level's counters are rotated as frontier_level
-// rotates them.
+// in-neighbour in the frontier (dist == level) and if it finds one takes
+// level + 1 and queues itself. The first four in-edges are the thread's; the
+// rows still open then go on in LDS queues, eight lanes a row, then a wave
+// (scan_queued): a few vertices whose long rows meet no frontier would
+// otherwise hold back their waves, edge after edge. The vertices found are
+// gathered in LDS and queued with one counter atomic per chunk. A vertex is
+// written only by its own workgroup, so no atomic on dist is needed; the
+// distances are read and written with agent-scope accesses (coherent across
+// the XCDs' L2s, as the top-down step's). The set of vertices it discovers is
+// the top-down level's: the unvisited vertices with an in-edge from the
+// frontier. The level's counters are rotated as frontier_level rotates them.
+// s_n: four LDS words, the first three zero at the call and at the return.
 // A level runs bottom-up while the frontier holds more than n / kBottomUpDiv
 // vertices, or more than the vertices not yet reached (the tail of a BFS,
 // where a few unvisited vertices scan their in-edges instead of the frontier
-// its out-edges).
+// its out-edges), or where a smaller one has so many out-edges that scanning
+// is cheaper (bottom_up_pays).
 constexpr int kBottomUpDiv = 16;
 
 __device__ __forceinline__ void frontier_bottom_up(const GraphDev& g, const FrontierDev& s, int level, int rank,
-                                                   int nteam) {
-  const int bd = blockDim.x, tid = threadIdx.x, lane = tid & 63;
+                                                   int nteam, int* lds, int* s_n) {
+  const int bd = blockDim.x, tid = threadIdx.x;
   int32_t* out_q = (level & 1) ? s.q0 : s.q1;
   int* out_cnt = &s.counts[((level + 1) % 3) * kLine];
-  const uint32_t cur = (uint32_t)level, next = (uint32_t)level + 1u;
+  const uint32_t next = (uint32_t)level + 1u;
+  const FrontProbe probe{s.dist, (uint32_t)level};
+  GraphDev in = g;  // rows of in-edges
+  in.row_ptr = g.rrow;
+  in.col = g.rcol;
+  int* s_found = lds + scan_lds_bytes(bd) / 4;
   int lo, hi;
   block_range(g.n, rank, nteam, &lo, &hi);
-  for (int base = lo; base < hi; base += bd) {
-    const int v = base + tid;
-    bool found = false;
-    if (v < hi && __hip_atomic_load(&s.dist[v], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == kInf) {
-      const int b = g.rrow[v], e = g.rrow[v + 1];
-      for (int j = b; j < e && !found; j += 4) {
-        int u[4];
+  for (int base = lo; base < hi; base += kScanU * bd) {
+    if (base > lo) __syncthreads();  // the last chunk's found vertices are stored
+    int v[kScanU], e[kScanU], end[kScanU], u[kScanU][4], none = 0;
+    bool open[kScanU], hit[kScanU][4];
 #pragma unroll
-        for (int q = 0; q < 4; q++) u[q] = j + q < e ? g.rcol[j + q] : -1;
-        uint32_t du[4];
-#pragma unroll
-        for (int q = 0; q < 4; q++)
-          du[q] = u[q] >= 0 ? __hip_atomic_load(&s.dist[u[q]], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : kInf;
-#pragma unroll
-        for (int q = 0; q < 4; q++) found = found || du[q] == cur;
-      }
-      if (found) __hip_atomic_store(&s.dist[v], next, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    for (int k = 0; k < kScanU; k++) {
+      v[k] = base + k * bd + tid;
+      open[k] = v[k] < hi && ld_agent(&s.dist[min(v[k], hi - 1)]) == kInf;
     }
-    const unsigned long long mask = __ballot(found);
-    if (mask) {
-      const int leader = __ffsll((long long)mask) - 1;
-      int pos = 0;
-      if (lane == leader) pos = __hip_atomic_fetch_add(out_cnt, __popcll(mask), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      pos = __builtin_amdgcn_readlane(pos, leader) + __popcll(mask & ((1ull << lane) - 1ull));
-      if (found) __hip_atomic_store(&out_q[pos], v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+    for (int k = 0; k < kScanU; k++) {
+      e[k] = open[k] ? in.row_ptr[v[k]] : 0;
+      end[k] = open[k] ? in.row_ptr[v[k] + 1] : 0;
+    }
+#pragma unroll
+    for (int k = 0; k < kScanU; k++)
+#pragma unroll
+      for (int j = 0; j < 4; j++) u[k][j] = e[k] + j < end[k] ? in.col[e[k] + j] : -1;
+#pragma unroll
+    for (int k = 0; k < kScanU; k++)
+#pragma unroll
+      for (int j = 0; j < 4; j++) hit[k][j] = u[k][j] >= 0 && probe.test(max(u[k][j], 0), 0u, true, none);
+#pragma unroll
+    for (int k = 0; k < kScanU; k++) {
+      const bool found = hit[k][0] || hit[k][1] || hit[k][2] || hit[k][3];
+      const bool more = !found && e[k] + 4 < end[k];
+      const int fs = wl_slot(found, &s_n[2]);
+      if (found) s_found[fs] = v[k];
+      const int qs = wl_slot(more, &s_n[0]);
+      if (more) {
+        lds[qs] = v[k];
+        lds[kScanU * bd + qs] = e[k] + 4;
+        lds[2 * kScanU * bd + qs] = 0;
+      }
+    }
+    scan_queued(
+        in, lds, s_n, probe, [&](int id) { return id; },
+        [&](int, int w, int edge, int, int) {
+          if (edge >= 0) s_found[wl_slot1(&s_n[2])] = w;
+        });
+    // scan_queued passed a barrier after the last use of what is read here, and
+    // every thread reads the count before the barrier below
+    const int nf = __builtin_amdgcn_readfirstlane(s_n[2]);
+    if (tid == 0) s_n[0] = s_n[1] = 0;
+    if (nf > 0) {
+      if (tid == 0) s_n[3] = add_relaxed(out_cnt, nf);
+      __syncthreads();
+      if (tid == 0) s_n[2] = 0;
+      const int at = __builtin_amdgcn_readfirstlane(s_n[3]);
+      for (int i = tid; i < nf; i += bd) {
+        const int w = s_found[i];
+        st_agent(&s.dist[w], next);
+        st_agent(&out_q[at + i], w);
+      }
     }
   }
   if (rank == 0 && tid == 0) {
@@ -119,6 +179,46 @@ __device__ __forceinline__ void frontier_bottom_up(const GraphDev& g, const Fron
     if (s.chunk > 0 && s.claims) st_relaxed(&s.claims[((level + 2) % 3) * kLine], 0);
     if (s.heavy > 0) st_relaxed(&s.hcnt[((level + 1) % 3) * kLine], 0);
   }
+}
+
+// Out-edges of the frontier q[0, in_n), estimated from kSamples of its entries,
+// evenly spaced, by the first wave: every member reads the same entries and
+// gets the same sum, so none has to be told. word: an LDS word.
+constexpr int kSamples = 256;
+__device__ __forceinline__ float front_edges(const GraphDev& g, const int32_t* q, int in_n, int* word) {
+  const int samples = min(kSamples, in_n);
+  if (threadIdx.x < 64) {
+    int v[kSamples / 64], deg = 0;
+#pragma unroll
+    for (int k = 0; k < kSamples / 64; k++) {
+      const int i = (int)threadIdx.x + 64 * k;
+      v[k] = i < samples ? ld_agent(&q[(int)((long long)i * in_n / samples)]) : -1;
+    }
+#pragma unroll
+    for (int k = 0; k < kSamples / 64; k++) deg += v[k] >= 0 ? g.row_ptr[v[k] + 1] - g.row_ptr[v[k]] : 0;
+    for (int o = 32; o > 0; o >>= 1) deg += __shfl_xor(deg, o, 64);
+    if (threadIdx.x == 0) *word = deg;
+  }
+  __syncthreads();
+  const float sum = (float)__builtin_amdgcn_readfirstlane(*word);
+  return sum * ((float)in_n / (float)samples);
+}
+
+// Whether a level of `edges` frontier edges is cheaper bottom-up: there the
+// unreached vertices scan until they meet the frontier, about m / edges edges
+// each, if they have so many. A frontier edge is taken at kFrontierEdge
+// scanned ones (its claim is performed beyond the L2). Asked on graphs of
+// skewed degrees (FrontierDev.fine) for frontiers of more than n / kSampleDiv
+// vertices: elsewhere edges go with vertices, and the question's two dependent
+// loads (2 us) would only cost (ER 2^16, 64 x 512: 97 -> 100 us). RMAT scale
+// 20 (ef 16), 512 x 1024, kernel: the second level, 1.5 to 5% of the vertices
+// with 41% of the edges, took 1.3 of the BFS's 1.72 ms top-down; 0.16 ms in
+// all with it bottom-up.
+constexpr int kSampleDiv = 128;
+constexpr float kFrontierEdge = 2.0f;
+__device__ __forceinline__ bool bottom_up_pays(const GraphDev& g, float edges, int unreached) {
+  const float m = (float)g.m;
+  return (float)unreached * fminf(m / (float)g.n, m / fmaxf(edges, 1.0f)) < kFrontierEdge * edges;
 }
 
 // A graph served by a team of k workgroups (rank 0..k-1). Everything the
@@ -129,12 +229,13 @@ __device__ __forceinline__ void frontier_bottom_up(const GraphDev& g, const Fron
 // Bellman-Ford), with the far counters and band minimum in device lines.
 // U: edges per thread per frontier pass (frontier_batch). HEAVY: teams whose
 // FrontierDev sets heavy > 0 (the standalone kernels) run the heavy-entry
-// pass; the batched kernel's teams (heavy = 0) are built without it.
+// pass; the batched kernel's teams (heavy = 0) are built without it. s_words:
+// kStandaloneWords LDS words (with HEAVY).
 // Reference: drelax2 (src/lonestar/graph_apps/bfs/device/bfs.cl:214-302,
 // src/lonestar/graph_apps/sssp/device/sssp.cl:262-318).
 template <bool SSSP, int U = 1, bool HEAVY = false, class Barrier>
 __device__ void run_team(const GraphDev& g, const FrontierDev& s, const NearFar& nf, int src, int rank, int k,
-                         int* lds, int* iters_out, Barrier&& bar) {
+                         int* lds, int* iters_out, Barrier&& bar, int* s_words = nullptr) {
   const bool near_far = SSSP && nf.delta > 0;
   int lo, hi;
   block_range(g.n, rank, k, &lo, &hi);
@@ -159,6 +260,7 @@ __device__ void run_team(const GraphDev& g, const FrontierDev& s, const NearFar&
       st_relaxed(&nf.cnt[2 * kLine], INT32_MAX);
     }
   }
+  if (HEAVY && threadIdx.x < kStandaloneWords) s_words[threadIdx.x] = 0;
   bar();
   const int bd = blockDim.x;
   int level = 0, fi = 0;
@@ -169,8 +271,11 @@ __device__ void run_team(const GraphDev& g, const FrontierDev& s, const NearFar&
     while ((in_n = ld_relaxed(&s.counts[(level % 3) * kLine])) != 0) {
       // every member read the same counts after the barriers: the same choice
       seen += in_n;
-      if (!SSSP && g.rrow && (in_n > g.n / kBottomUpDiv || in_n > g.n - seen))
-        frontier_bottom_up(g, s, level, rank, k);
+      bool up = !SSSP && HEAVY && g.rrow && (in_n > g.n / kBottomUpDiv || in_n > g.n - seen);
+      if (!SSSP && HEAVY && g.rrow && s.fine && !up && in_n > g.n / kSampleDiv)
+        up = bottom_up_pays(g, front_edges(g, (level & 1) ? s.q1 : s.q0, in_n, s_words + 3), g.n - seen);
+      if (up)
+        frontier_bottom_up(g, s, level, rank, k, lds, s_words);
       else
         frontier_level<SSSP, true, SSSP, U>(g, s, level, rank, k, lds, thr, near_far ? nf.far(fi) : nullptr,
                                             &nf.cnt[fi * kLine], nf.flag);

@@ -189,3 +189,31 @@ def test_low_degree_graphs(rt, name):
             d, _ = dg.sssp(src, wg_size=wg, num_wgs=wgs, mode=1)
             assert np.array_equal(d, ref), (wg, wgs)
         dg.close()
+
+
+def _reverse(g):
+    return G.from_edges(g.n, g.col, np.repeat(np.arange(g.n), g.degrees()))
+
+
+BFS = {
+    "hubs_out": lambda: _rows_graph(seed=6),             # few entries hold a level's edges
+    "hubs_in": lambda: _reverse(_rows_graph(seed=7)),    # long rows scanned bottom-up
+    "stages_in": lambda: _reverse(_stage_graph()),
+    "rmat": lambda: G.rmat(12, 16, seed=11),
+    "er": lambda: G.erdos_renyi(5003, 40000, seed=12),   # even degrees: no estimate
+    "star": lambda: G.from_edges(3001, np.zeros(3000, int), np.arange(1, 3001), symmetric=True),
+}
+
+
+@pytest.mark.parametrize("name", BFS)
+def test_bfs_bottom_up(rt, name):
+    """Levels and their count where a level runs bottom-up, from one wave (many
+    chunks of its range) to the whole grid."""
+    g = BFS[name]()
+    dg = rt.graph(g)
+    for src in (0, g.n // 2, g.n - 1):
+        levels, n_levels = oracle.bfs(g.row_ptr, g.col, src)
+        for wg, wgs in ((64, 1), (192, 3), (512, 64), (1024, 0)):
+            d, st = dg.bfs(src, wg_size=wg, num_wgs=wgs)
+            assert np.array_equal(d, levels) and st["iterations"] == n_levels, (src, wg, wgs)
+    dg.close()
