@@ -497,6 +497,12 @@ int wgm_graph_create(wgm_runtime* rt, const wgm_csr* h, const uint32_t* prio, wg
   g->n = h->n;
   g->m = h->m;
   g->maxdeg = maxdeg;
+  int32_t lo = 0, hi = 0;
+  for (int64_t e = 0; h->wt && e < h->m; e++) {
+    lo = std::min(lo, h->wt[e]);
+    hi = std::max(hi, h->wt[e]);
+  }
+  g->wild_weights = lo < 0 || hi > INT32_MAX - (int32_t)kInf;
   if (maxdeg <= kLowDegree && h->n <= kLowMaxN) {
     int32_t span = 0;
     for (int32_t v = 0; h->n > kLowAnySpan && v < h->n; v++)
@@ -504,10 +510,8 @@ int wgm_graph_create(wgm_runtime* rt, const wgm_csr* h, const uint32_t* prio, wg
         const int32_t d = std::abs(h->col[e] - v);
         span = std::max(span, std::min(d, h->n - d));
       }
-    uint32_t bits = 0;
-    for (int64_t e = 0; h->wt && e < h->m; e++) bits |= (uint32_t)h->wt[e];
     g->low = span <= kLowSpan;
-    g->low_weights = g->low && h->wt && bits <= 255u;
+    g->low_weights = g->low && h->wt && lo >= 0 && hi <= 255;
   }
   auto bail = [&](int rc) { wgm_graph_destroy(g); return rc; };
   int rc = dev_alloc(rt, &g->row_ptr, (size_t)h->n + 1);
@@ -543,7 +547,8 @@ int64_t wgm_graph_bytes(const wgm_graph* g) {
   if (g->wt) b += 4 * g->m;
   if (g->prio) b += 4 * (int64_t)g->n;
   if (g->ell) b += 4 * kLowDegree * (int64_t)g->n;
-  if (g->rrow) b += 4 * ((int64_t)g->n + 1) + (g->rwt ? 8 : 4) * g->m + 16 * (int64_t)g->ntasks;
+  if (g->rrow) b += 4 * ((int64_t)g->n + 1) + (g->rwt ? 8 : 4) * g->m;
+  if (g->mp_sid) b += 5 * g->m + 4 * (g->m / 256 + (int64_t)g->n + g->mp_rows + 3 * (int64_t)g->mp_words);
   return b;
 }
 

@@ -44,12 +44,20 @@ struct wgm_graph {
   uint32_t* hdu = nullptr;
   int32_t* hclaim = nullptr;
   int* hcnt = nullptr;    // 3 lines
-  // in-edge CSR and min-plus tasks (Pannotia SSSP / BC), built on first use
+  // in-edge CSR, built on first use
   int32_t* rrow = nullptr;
   int32_t* rcol = nullptr;
   int32_t* rwt = nullptr;
-  void* tasks = nullptr;  // int4 {row, begin, end, 0}
-  int32_t ntasks = 0;
+  // min-plus graph (MinplusDev in pannotia.hip) and its state, on first use
+  int32_t* mp_sid = nullptr;
+  uint8_t* mp_roff = nullptr;
+  int32_t* mp_start = nullptr;
+  int32_t* mp_cid = nullptr;
+  int32_t* mp_d = nullptr;
+  uint32_t* mp_bits = nullptr;
+  int32_t mp_rows = 0;
+  int32_t mp_words = 0;
+  bool wild_weights = false;  // a weight is negative, or wraps when added to an unreached distance
   // BC per-slot state and the result
   int32_t bc_slots = 0;
   int32_t bc_rows = 0;  // dependency rows in bc_del

@@ -37,63 +37,241 @@ constexpr int32_t kBigNum = WGM_BIG_NUM;
 // grid shrinks to fit.
 constexpr unsigned long long kBcSlotBytes = 8ull << 30;
 
+// Min-plus graph: the vertices with an in-edge ("rows") numbered in order, the
+// in-edges in row order in blocks of 256, the last one padded.
+constexpr int kMpBlock = 256;
 struct MinplusDev {
-  const int4* tasks;  // {row, begin, end, 0}
-  int32_t ntasks;
-  int32_t max_sweeps;  // n + 1 sweeps settle any graph without a negative cycle
-  const int32_t* rcol;
-  const int32_t* rwt;
-  int32_t* dist;
+  const int32_t* sid;    // row of an edge's source; nrows: a vertex without in-edges, or padding
+  const int32_t* wt;
+  const uint8_t* roff;   // row of an edge less the block's first
+  const int32_t* bstart; // [nblk + 1] first row of a block; the last one: nrows
+  const int32_t* cid;    // [n] row of a vertex, -1: none
+  const int32_t* row_ptr;
+  const int32_t* col;
+  const int32_t* owt;    // weights of the out-edges
+  int32_t nblk;
+  int32_t nrows;
+  int32_t n;
+  int32_t src;
+  int32_t big;           // distance of an unreached vertex
+  int32_t all;           // the first sweep follows every vertex's edges (minplus_first)
+  int32_t max_sweeps;    // n + 1 sweeps settle any graph without a negative cycle
+  int32_t shift;         // rows per bit of the LDS map: 1 << shift
+  int32_t map_words;
+  int32_t bit_words;     // words of one bit set
+  int32_t* d;            // [nrows + 1] distances of the rows; the last one stays at big
+  uint32_t* bits;        // three bit sets: rows lowered in sweep s in set s % 3
+  int32_t* dist;         // [n] result
 };
 
-template <int G>
+typedef __attribute__((address_space(3))) int lds_i32;
+typedef int i32x4 __attribute__((ext_vector_type(4)));
+
+// Marks the lowered rows row0 + i (bit i of mask) for the next sweep.
+__device__ __forceinline__ void mp_mark(uint32_t* next, int row0, unsigned long long mask) {
+  if (!mask) return;
+  const int lane = (int)threadIdx.x & 63, sh = row0 & 31;
+  const unsigned long long lo = mask << sh, hi = sh ? mask >> (64 - sh) : 0ull;
+  const uint32_t w = lane == 0 ? (uint32_t)lo : lane == 1 ? (uint32_t)(lo >> 32) : lane == 2 ? (uint32_t)hi : 0u;
+  if (w) __hip_atomic_fetch_or(&next[(row0 >> 5) + lane], w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// The bit set into the LDS map: bit j of the map is the union of the bits
+// j << shift .. ((j + 1) << shift) - 1. (Sets and map are whole 16-byte units.)
+__device__ __forceinline__ void mp_load_map(const MinplusDev& p, const uint32_t* set, lds_u32* map) {
+  if (p.shift == 0) {
+    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+    typedef __attribute__((address_space(3))) u32x4 lds_u32x4;
+#pragma unroll 4
+    for (int i = (int)threadIdx.x; i < p.map_words / 4; i += blockDim.x) ((lds_u32x4*)map)[i] = ((const u32x4*)set)[i];
+    return;
+  }
+  for (int i = (int)threadIdx.x; i < p.map_words; i += blockDim.x) {
+    uint32_t out = 0;
+    for (int b = 0; b < 32; b++) {
+      const long long r0 = (32ll * i + b) << p.shift, r1 = r0 + (1ll << p.shift);
+      uint32_t any = 0;
+      if (p.shift < 5) {
+        if ((r0 >> 5) < p.bit_words) any = (set[r0 >> 5] >> (r0 & 31)) & ((1u << (1 << p.shift)) - 1u);
+      } else {
+        for (long long w = r0 >> 5; w < min(r1 >> 5, (long long)p.bit_words); w++) any |= set[w];
+      }
+      out |= any ? 1u << b : 0u;
+    }
+    map[i] = out;
+  }
+}
+
+// The first sweep: from a cleared state only the source's edges lower
+// anything, unless a weight is negative or so large that it wraps (p.all).
+__device__ __forceinline__ bool minplus_first(const MinplusDev& p, int id, int nteam) {
+  uint32_t* next = p.bits + p.bit_words;
+  const int tid = id * (int)blockDim.x + (int)threadIdx.x, stride = nteam * (int)blockDim.x;
+  bool any = false;
+  auto relax = [&](int e, int du) {
+    const int c = p.cid[p.col[e]], cand = (int)((uint32_t)du + (uint32_t)p.owt[e]);
+    if (cand < p.big && cand < __hip_atomic_fetch_min(&p.d[c], cand, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
+      __hip_atomic_fetch_or(&next[c >> 5], 1u << (c & 31), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      any = true;
+    }
+  };
+  if (p.all) {
+    for (int u = tid; u < p.n; u += stride)
+      for (int e = p.row_ptr[u]; e < p.row_ptr[u + 1]; e++) relax(e, u == p.src ? 0 : p.big);
+  } else {
+    const int end = p.row_ptr[p.src + 1];
+    for (int e = p.row_ptr[p.src] + tid; e < end; e += stride) relax(e, 0);
+  }
+  return any;
+}
+
+// A step of a sweep: the blocks [b, b1), kMpU at most, by one wave, which
+// follows the edges whose source is set in `map`. A block's candidates meet in
+// the wave's LDS table, an entry per row of the block; a row that goes on in
+// the next block is carried there. All rows but those at the step's ends are
+// this wave's alone, so they are lowered by plain stores; a row at an end by an
+// atomic minimum, and each wave that lowers it below what it was before the
+// sweep marks it. The blocks' loads are in flight together.
+constexpr int kMpU = 4;
+__device__ __forceinline__ bool minplus_step(const MinplusDev& p, int b, int b1, lds_i32* tab, const lds_u32* map,
+                                             uint32_t* next) {
+  const int lane = (int)threadIdx.x & 63;
+  i32x4 s[kMpU];
+  int c0[kMpU + 1];
+#pragma unroll
+  for (int u = 0; u < kMpU; u++)
+    s[u] = b + u < b1 ? ((const i32x4*)p.sid)[(size_t)(b + u) * 64 + lane] : i32x4{p.nrows, p.nrows, p.nrows, p.nrows};
+#pragma unroll
+  for (int u = 0; u <= kMpU; u++) c0[u] = p.bstart[min(b + u, b1)];
+  const int first = c0[0], last = c0[kMpU];  // rows that other waves may lower too
+  unsigned hit[kMpU], some = 0;
+#pragma unroll
+  for (int u = 0; u < kMpU; u++) {
+    const int id[4] = {s[u].x, s[u].y, s[u].z, s[u].w};
+    hit[u] = 0;
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      const unsigned r = (unsigned)id[j] >> p.shift;
+      hit[u] |= ((map[r >> 5] >> (r & 31)) & 1u) << j;
+    }
+    some |= hit[u];
+  }
+  if (!__ballot(some != 0)) return false;
+  i32x4 w[kMpU];
+  int du[kMpU][4], dv[kMpU][4];
+  uint32_t ro[kMpU];
+#pragma unroll
+  for (int u = 0; u < kMpU; u++) {
+    w[u] = i32x4{0, 0, 0, 0};
+    ro[u] = 0;
+    if (hit[u]) {
+      w[u] = ((const i32x4*)p.wt)[(size_t)(b + u) * 64 + lane];
+      ro[u] = ((const uint32_t*)p.roff)[(size_t)(b + u) * 64 + lane];
+    }
+    const int id[4] = {s[u].x, s[u].y, s[u].z, s[u].w};
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      du[u][j] = 0;
+      if ((hit[u] >> j) & 1u) du[u][j] = __hip_atomic_load(&p.d[id[j]], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    }
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      dv[u][q] = 0;
+      if (c0[u + 1] - c0[u] >= 64 * q)
+        dv[u][q] = __hip_atomic_load(&p.d[min(c0[u] + 64 * q + lane, p.nrows)], __ATOMIC_RELAXED,
+                                     __HIP_MEMORY_SCOPE_WORKGROUP);
+    }
+  }
+  bool any = false;
+  int carry = INT32_MAX;
+#pragma unroll
+  for (int u = 0; u < kMpU; u++) {
+    if (b + u >= b1) break;
+    if (!__ballot(hit[u] != 0) && carry == INT32_MAX) continue;
+    // a lane's candidates of one row, which is the ordinary case, go in as one
+    const int wj[4] = {w[u].x, w[u].y, w[u].z, w[u].w};
+    int best = INT32_MAX;
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      if ((hit[u] >> j) & 1u) best = min(best, (int)((uint32_t)wj[j] + (uint32_t)du[u][j]));
+      const unsigned row = (ro[u] >> (8 * j)) & 255u;
+      if (best != INT32_MAX && (j == 3 || row != ((ro[u] >> (8 * j + 8)) & 255u))) {
+        __hip_atomic_fetch_min(&tab[row], best, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        best = INT32_MAX;
+      }
+    }
+    // entry `rows` (if there is one) is the row that the next block begins in
+    const int rows = c0[u + 1] - c0[u];
+    const bool on = u + 1 < kMpU && b + u + 1 < b1;
+    int carried = INT32_MAX;
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      if (rows < 64 * q) break;
+      const int i = 64 * q + lane, c = c0[u] + i;
+      int val = INT32_MAX;
+      if (i <= rows) {
+        val = __hip_atomic_load(&tab[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        if (val != INT32_MAX) __hip_atomic_store(&tab[i], INT32_MAX, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      }
+      if (i == 0) val = min(val, carry);
+      if (on && rows < 64 * (q + 1)) {
+        carried = __builtin_amdgcn_readlane(val, rows & 63);
+        if (i == rows) val = INT32_MAX;
+      }
+      const bool lower = val < dv[u][q];
+      if (lower) {
+        if (c == first || c == last)
+          __hip_atomic_fetch_min(&p.d[c], val, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        else
+          __hip_atomic_store(&p.d[c], val, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      }
+      any |= lower;
+      mp_mark(next, c0[u] + 64 * q, __ballot(lower));
+    }
+    carry = carried;
+  }
+  return any;
+}
+
+// Bound: in the sweeps that follow most edges the L1's limit of lines on their
+// way (55 a CU measured, 450 cycles each), which the gathers of sources'
+// distances take; elsewhere the barrier and three dependent loads a sweep. A
+// sweep over all edges read 8 bytes and gathered a distance an edge, though
+// over the 11 sweeps of RMAT scale 20 (ef 16) a source is lowered 3.3 times:
+// 1575 -> 590 us (kernel, 512 x 1024 asked); RMAT 17, 64 x 1024: 620 -> 256;
+// ER 2^18 of degree 16: 1001 -> 553; ER 4096 of degree 8, 64 x 512: 116 -> 100.
+// Not better: steps dealt out over all workgroups (613 us: several XCDs then
+// write a line of distances), rows in the order of their out-degree (610).
 __global__ void __launch_bounds__(1024) k_minplus(Ctl c, MinplusDev p, int* iters_out) {
+  extern __shared__ __attribute__((aligned(16))) int lds_mp[];
   Team t;
   if (!standalone_begin(c, t)) return;
-  const int lane = (int)threadIdx.x % G, grp = (int)threadIdx.x / G, ngrp = (int)blockDim.x / G;
-  // tasks interleaved over every lane group of the grid: the consecutive
-  // tasks of a hub's row spread over many workgroups
-  const int first = t.id * ngrp + grp, stride = t.n * ngrp;
+  const int wave = (int)threadIdx.x >> 6, nw = (int)blockDim.x >> 6;
+  lds_i32* tab = (lds_i32*)lds_mp + wave * kMpBlock;
+  lds_u32* map = (lds_u32*)lds_mp + nw * kMpBlock;
+  for (int i = (int)threadIdx.x & 63; i < kMpBlock; i += 64) tab[i] = INT32_MAX;
+  // a workgroup's blocks, in steps that its waves take in turn
+  int lo, hi;
+  block_range(p.nblk, t.id, t.n, &lo, &hi);
+  const int per = min(kMpU, max(1, (hi - lo) / nw));
+  const int b0 = __builtin_amdgcn_readfirstlane(lo + wave * per);
+  int clo, chi;
+  block_range(p.bit_words, t.id, t.n, &clo, &chi);
   int* flags = c.lines;
   int sweep = 1;
   for (;; sweep++) {
-    bool any = false;
-    for (int i = first; i < p.ntasks; i += stride) {
-      const int4 tk = p.tasks[i];
-      int best = INT32_MAX;
-      // a plain (workgroup-scope) read of dist: a value another workgroup
-      // lowers during this sweep may be seen late; the barrier makes it
-      // current. Four of the lane's edges per round: their sources and
-      // weights, then the four gathers, so the lane waits for two memory
-      // round trips per four edges rather than per edge.
-      int e = tk.y + lane;
-      for (; e + 3 * G < tk.z; e += 4 * G) {
-        int sv[4], wv[4], dv[4];
-#pragma unroll
-        for (int q = 0; q < 4; q++) {
-          sv[q] = p.rcol[e + q * G];
-          wv[q] = p.rwt[e + q * G];
-        }
-#pragma unroll
-        for (int q = 0; q < 4; q++) dv[q] = __hip_atomic_load(&p.dist[sv[q]], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-#pragma unroll
-        for (int q = 0; q < 4; q++) best = wv[q] + dv[q] < best ? wv[q] + dv[q] : best;
-      }
-      for (; e < tk.z; e += G) {
-        const int du = __hip_atomic_load(&p.dist[p.rcol[e]], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-        const int cand = p.rwt[e] + du;
-        best = cand < best ? cand : best;
-      }
-#pragma unroll
-      for (int o = G / 2; o > 0; o >>= 1) {
-        const int other = __shfl_xor(best, o, G);
-        best = other < best ? other : best;
-      }
-      if (lane == 0 && best < __hip_atomic_load(&p.dist[tk.x], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)) {
-        const int old = __hip_atomic_fetch_min(&p.dist[tk.x], best, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        any |= best < old;
-      }
+    bool any;
+    uint32_t* next = p.bits + (size_t)(sweep % 3) * p.bit_words;
+    if (sweep == 1) {
+      any = minplus_first(p, t.id, t.n);
+    } else {
+      mp_load_map(p, p.bits + (size_t)((sweep - 1) % 3) * p.bit_words, map);
+      __syncthreads();
+      any = false;
+      for (int b = b0; b < hi; b += nw * per) any |= minplus_step(p, b, min(b + per, hi), tab, map, next);
     }
+    uint32_t* clear = p.bits + (size_t)((sweep + 1) % 3) * p.bit_words;
+    for (int i = clo + (int)threadIdx.x; i < chi; i += blockDim.x) clear[i] = 0u;
     if (__syncthreads_or(any) && threadIdx.x == 0) st_relaxed(&flags[(sweep % 3) * kLine], 1);
     if (t.id == 0 && threadIdx.x == 0) st_relaxed(&flags[((sweep + 1) % 3) * kLine], 0);
     xcd_barrier(c, t);
@@ -103,17 +281,48 @@ __global__ void __launch_bounds__(1024) k_minplus(Ctl c, MinplusDev p, int* iter
       break;
     }
   }
+  for (int v = t.id * (int)blockDim.x + (int)threadIdx.x; v < p.n; v += t.n * (int)blockDim.x) {
+    const int r = p.cid[v];
+    p.dist[v] = r >= 0 ? p.d[r] : v == p.src ? 0 : p.big;
+  }
   clock_end(c, t.id);
   if (t.id == 0 && threadIdx.x == 0) *iters_out = sweep;
   standalone_retire(c);
 }
 
-// Unreached vertices start at `big` (BIG_NUM for Pannotia SSSP, MYINFINITY
-// for Lonestar SSSP's pull direction): big + 255 stays below INT32_MAX, so a
-// candidate through an unreached vertex never lowers anything.
-__global__ void k_minplus_init(int32_t* dist, int n, int src, int32_t big) {
-  for (int v = blockIdx.x * blockDim.x + threadIdx.x; v < n; v += gridDim.x * blockDim.x)
-    dist[v] = v == src ? 0 : big;
+// Distances of the rows (unreached ones at `big`: BIG_NUM for Pannotia SSSP,
+// MYINFINITY for Lonestar SSSP's pull direction) and the first two bit sets.
+__global__ void k_minplus_init(MinplusDev p) {
+  const int tid = blockIdx.x * blockDim.x + threadIdx.x, stride = gridDim.x * blockDim.x;
+  const int s = p.cid[p.src];
+  for (int r = tid; r <= p.nrows; r += stride) p.d[r] = r == s ? 0 : p.big;
+  for (int i = tid; i < 3 * p.bit_words; i += stride) p.bits[i] = 0u;
+}
+
+// First rows of the blocks; one wave a vertex.
+__global__ void k_minplus_starts(const int32_t* rrow, const int32_t* cid, int n, int nblk, int nrows, int32_t* bstart) {
+  const int waves = (int)(gridDim.x * blockDim.x) >> 6, lane = (int)threadIdx.x & 63;
+  for (int v = (int)(blockIdx.x * blockDim.x + threadIdx.x) >> 6; v < n; v += waves)
+    for (long long b = ((long long)rrow[v] + kMpBlock - 1) / kMpBlock + lane; b * kMpBlock < rrow[v + 1]; b += 64)
+      bstart[b] = cid[v];
+  if (blockIdx.x == 0 && threadIdx.x == 0) bstart[nblk] = nrows;
+}
+
+// Rows of the edges and of their sources; one wave a vertex.
+__global__ void k_minplus_edges(const int32_t* rrow, const int32_t* rcol, const int32_t* cid, const int32_t* bstart,
+                                int n, int nblk, int nrows, int32_t* sid, uint8_t* roff) {
+  const int waves = (int)(gridDim.x * blockDim.x) >> 6, lane = (int)threadIdx.x & 63;
+  for (int v = (int)(blockIdx.x * blockDim.x + threadIdx.x) >> 6; v < n; v += waves)
+    for (int e = rrow[v] + lane; e < rrow[v + 1]; e += 64) {
+      const int c = cid[rcol[e]];
+      sid[e] = c < 0 ? nrows : c;
+      roff[e] = (uint8_t)(cid[v] - bstart[e / kMpBlock]);
+    }
+  if (blockIdx.x == 0)
+    for (long long e = (long long)rrow[n] + threadIdx.x; e < (long long)nblk * kMpBlock; e += blockDim.x) {
+      sid[e] = nrows;
+      roff[e] = 0;
+    }
 }
 
 struct BcDev {
@@ -549,16 +758,13 @@ __global__ void __launch_bounds__(1024, LDS ? 8 : 4) k_bc(Ctl c, BcDev b, int* i
 
 namespace {
 
-constexpr int kTaskEdgesPerLane = 16;
-
-int minplus_lanes(const wgm_graph* g) {
-  const double avg = g->n ? (double)g->m / (double)g->n : 0.0;
-  return avg < 8.0 ? 4 : avg < 32.0 ? 16 : 64;
-}
+// Edges of the min-plus graph, padding included.
+int64_t mp_edges(int64_t m) { return (m + kMpBlock - 1) / kMpBlock * kMpBlock; }
 
 // In-edge CSR (sources ascending within a row, the order of
-// parseCOO_transpose's stable sort) and the min-plus task list, built once on
-// the host from the device copy of the graph and kept resident.
+// parseCOO_transpose's stable sort), built once on the host from the device
+// copy of the graph and kept resident; the weights padded to whole blocks of
+// the min-plus sweeps.
 int graph_reverse(wgm_graph* g) {
   if (g->rrow) return WGM_OK;
   wgm_runtime* rt = g->rt;
@@ -568,7 +774,7 @@ int graph_reverse(wgm_graph* g) {
   HIPCHK(rt, hipMemcpy(rp.data(), g->row_ptr, sizeof(int32_t) * ((size_t)n + 1), hipMemcpyDeviceToHost));
   if (m) HIPCHK(rt, hipMemcpy(col.data(), g->col, sizeof(int32_t) * (size_t)m, hipMemcpyDeviceToHost));
   if (g->wt && m) HIPCHK(rt, hipMemcpy(wt.data(), g->wt, sizeof(int32_t) * (size_t)m, hipMemcpyDeviceToHost));
-  std::vector<int32_t> rrow((size_t)n + 1, 0), rcol((size_t)m), rwt(g->wt ? (size_t)m : 0);
+  std::vector<int32_t> rrow((size_t)n + 1, 0), rcol((size_t)m), rwt(g->wt ? (size_t)mp_edges(m) : 0);
   for (int64_t e = 0; e < m; e++) rrow[(size_t)col[(size_t)e] + 1]++;
   for (int32_t v = 0; v < n; v++) rrow[(size_t)v + 1] += rrow[(size_t)v];
   std::vector<int32_t> pos(rrow.begin(), rrow.end() - 1);
@@ -578,36 +784,18 @@ int graph_reverse(wgm_graph* g) {
       rcol[(size_t)p] = u;
       if (g->wt) rwt[(size_t)p] = wt[(size_t)e];
     }
-  const int chunk = kTaskEdgesPerLane * minplus_lanes(g);
-  std::vector<int4> tasks;
-  tasks.reserve((size_t)n + (size_t)(m / chunk) + 1);
-  for (int32_t v = 0; v < n; v++)
-    for (int32_t a = rrow[(size_t)v]; a < rrow[(size_t)v + 1]; a += chunk)
-      tasks.push_back(int4{v, a, std::min(a + chunk, rrow[(size_t)v + 1]), 0});
   auto alloc = [&](void** p, size_t bytes) -> int {
     hipError_t e = hipMalloc(p, bytes ? bytes : 4);
     return e == hipSuccess ? WGM_OK : wgm_hip_fail(rt, e, "hipMalloc(in-edge CSR)");
   };
   int rc = alloc((void**)&g->rrow, sizeof(int32_t) * ((size_t)n + 1));
   if (!rc) rc = alloc((void**)&g->rcol, sizeof(int32_t) * (size_t)m);
-  if (!rc && g->wt) rc = alloc((void**)&g->rwt, sizeof(int32_t) * (size_t)m);
-  if (!rc) rc = alloc((void**)&g->tasks, sizeof(int4) * tasks.size());
+  if (!rc && g->wt) rc = alloc((void**)&g->rwt, sizeof(int32_t) * rwt.size());
   if (rc) return rc;
   HIPCHK(rt, hipMemcpy(g->rrow, rrow.data(), sizeof(int32_t) * ((size_t)n + 1), hipMemcpyHostToDevice));
   if (m) HIPCHK(rt, hipMemcpy(g->rcol, rcol.data(), sizeof(int32_t) * (size_t)m, hipMemcpyHostToDevice));
-  if (g->wt && m) HIPCHK(rt, hipMemcpy(g->rwt, rwt.data(), sizeof(int32_t) * (size_t)m, hipMemcpyHostToDevice));
-  if (!tasks.empty())
-    HIPCHK(rt, hipMemcpy(g->tasks, tasks.data(), sizeof(int4) * tasks.size(), hipMemcpyHostToDevice));
-  g->ntasks = (int32_t)tasks.size();
+  if (g->wt && m) HIPCHK(rt, hipMemcpy(g->rwt, rwt.data(), sizeof(int32_t) * rwt.size(), hipMemcpyHostToDevice));
   return WGM_OK;
-}
-
-const void* minplus_kernel(int lanes) {
-  switch (lanes) {
-    case 4: return (const void*)&k_minplus<4>;
-    case 16: return (const void*)&k_minplus<16>;
-    default: return (const void*)&k_minplus<64>;
-  }
 }
 
 // Launch of a standalone persistent kernel whose first argument is the
@@ -638,6 +826,43 @@ int launch_standalone_app(wgm_runtime* rt, int kernel, const void* fn, const wgm
   st->host_ms = host_ms;
   return WGM_OK;
 }
+
+// The min-plus graph, built once from the in-edge CSR and kept resident.
+int minplus_rows(wgm_graph* g) {
+  int rc = graph_reverse(g);
+  if (rc || g->mp_sid) return rc;
+  wgm_runtime* rt = g->rt;
+  const int32_t n = g->n;
+  std::vector<int32_t> rrow((size_t)n + 1), cid((size_t)n);
+  HIPCHK(rt, hipMemcpy(rrow.data(), g->rrow, sizeof(int32_t) * rrow.size(), hipMemcpyDeviceToHost));
+  int32_t rows = 0;
+  for (int32_t v = 0; v < n; v++) cid[(size_t)v] = rrow[(size_t)v + 1] > rrow[(size_t)v] ? rows++ : -1;
+  const size_t edges = (size_t)mp_edges(g->m);
+  const int32_t nblk = (int32_t)(edges / kMpBlock);
+  g->mp_rows = rows;
+  g->mp_words = (rows / 32 + 4) / 4 * 4;
+  auto alloc = [&](auto** p, size_t count) {
+    if (*p) return hipSuccess;  // of an earlier try
+    return hipMalloc((void**)p, sizeof(**p) * std::max<size_t>(count, 1));
+  };
+  int32_t* sid = nullptr;
+  hipError_t e = alloc(&g->mp_cid, (size_t)n);
+  if (e == hipSuccess) e = alloc(&g->mp_start, (size_t)nblk + 1);
+  if (e == hipSuccess) e = alloc(&g->mp_roff, edges);
+  if (e == hipSuccess) e = alloc(&g->mp_d, (size_t)rows + 1);
+  if (e == hipSuccess) e = alloc(&g->mp_bits, 3 * (size_t)g->mp_words);
+  if (e == hipSuccess) e = hipMemcpy(g->mp_cid, cid.data(), sizeof(int32_t) * cid.size(), hipMemcpyHostToDevice);
+  if (e == hipSuccess) e = alloc(&sid, edges);
+  if (e != hipSuccess) return wgm_hip_fail(rt, e, "min-plus graph");
+  g->mp_sid = sid;
+  hipLaunchKernelGGL(k_minplus_starts, dim3(1024), dim3(256), 0, rt->stream, g->rrow, g->mp_cid, n, nblk, rows, g->mp_start);
+  hipLaunchKernelGGL(k_minplus_edges, dim3(1024), dim3(256), 0, rt->stream, g->rrow, g->rcol, g->mp_cid, g->mp_start, n,
+                     nblk, rows, g->mp_sid, g->mp_roff);
+  HIPCHK(rt, hipGetLastError());
+  return WGM_OK;
+}
+
+int minplus_tables(int wg) { return wg / 64 * kMpBlock * 4; }
 
 // LDS a BC workgroup may use, and what it takes besides its state (statics and
 // allocation granularity, rounded up).
@@ -686,6 +911,71 @@ int bc_grid(wgm_runtime* rt, const wgm_graph* g, const wgm_launch* lc, int* grid
   return WGM_OK;
 }
 
+// Min-plus sweeps from src into dist (device, n entries; `big` where
+// unreached). The LDS map has a bit a row up to kMpMapBytes, above that a bit
+// for each 2, 4, ... rows. It takes a CU for a workgroup: more workgroups than
+// that are taken as one larger one on each CU, which also shortens the barrier.
+constexpr long long kMpMapBytes = 128 << 10;
+
+int run_minplus(wgm_runtime* rt, wgm_graph* g, int32_t src, int32_t big, const wgm_launch* lc, int32_t* dist, int* iters,
+                wgm_run_stats* st) {
+  int rc = minplus_rows(g);
+  if (rc) return rc;
+  MinplusDev p{};
+  p.sid = g->mp_sid;
+  p.wt = g->rwt;
+  p.roff = g->mp_roff;
+  p.bstart = g->mp_start;
+  p.cid = g->mp_cid;
+  p.row_ptr = g->row_ptr;
+  p.col = g->col;
+  p.owt = g->wt;
+  p.nblk = (int32_t)(mp_edges(g->m) / kMpBlock);
+  p.nrows = g->mp_rows;
+  p.n = g->n;
+  p.src = src;
+  p.big = big;
+  p.all = g->wild_weights ? 1 : 0;
+  p.max_sweeps = g->n + 1;
+  while (4ll * ((p.nrows >> p.shift) / 32 + 4) > kMpMapBytes) p.shift++;
+  p.map_words = ((p.nrows >> p.shift) / 32 + 4) / 4 * 4;
+  p.bit_words = g->mp_words;
+  p.d = g->mp_d;
+  p.bits = g->mp_bits;
+  p.dist = dist;
+  wgm_launch shape{256, 0, 0, 0};
+  if (lc) shape = *lc;
+  if (shape.wg_size <= 0) shape.wg_size = 256;
+  int grid = 0;
+  rc = wgm_resolve_grid(rt, WGM_K_MINPLUS, shape.wg_size, shape.num_wgs, &grid);
+  if (rc) return rc;
+  if (grid > rt->info.num_cus) {
+    shape.wg_size = std::min(1024, shape.wg_size * ((grid + rt->info.num_cus - 1) / rt->info.num_cus));
+    grid = rt->info.num_cus;
+  }
+  // Small graphs: every further workgroup lengthens each sweep's barrier, more
+  // waves its reductions. Eight waves with a block each on up to 64 workgroups,
+  // more of them only where a wave has four (kernel, 128 blocks asked as 1024
+  // threads on a workgroup a CU: 169 -> 102 us; 2048 blocks: 328 -> 231).
+  const auto wanted = [&](int wg) {
+    const int waves = wg / 64, one = (p.nblk + waves - 1) / waves;
+    return std::max({std::min(64, one), (one + 3) / 4, g->n / (8 * wg) + 1});
+  };
+  const int few = std::min(512, shape.wg_size);
+  if (wanted(few) <= grid) shape.wg_size = few;
+  grid = std::min(grid, wanted(shape.wg_size));
+  shape.num_wgs = grid;
+  hipLaunchKernelGGL(k_minplus_init, dim3(256), dim3(256), 0, rt->stream, p);
+  Ctl ctl{};
+  void* args[] = {&ctl, &p, &g->iters};
+  rc = launch_standalone_app(rt, WGM_K_MINPLUS, (const void*)&k_minplus, &shape, &ctl, args, 0, st,
+                             (size_t)minplus_tables(shape.wg_size) + 4 * (size_t)p.map_words);
+  if (rc) return rc;
+  HIPCHK(rt, hipMemcpy(iters, g->iters, sizeof(int), hipMemcpyDeviceToHost));
+  if (*iters < 0) return fail(rt, WGM_ERR_INVALID, "distances still fall after %d sweeps: negative cycle", g->n + 1);
+  return WGM_OK;
+}
+
 }  // namespace
 
 int wgm_graph_in_edges(wgm_graph* g) { return graph_reverse(g); }
@@ -694,7 +984,7 @@ static int bc_stage(int wg) { return (int)bc_stage_bytes(wg); }
 
 bool wgm_pannotia_kernel_info(int kernel, KernelInfo* out) {
   switch (kernel) {
-    case WGM_K_MINPLUS: *out = KernelInfo{(const void*)&k_minplus<16>, nullptr}; return true;
+    case WGM_K_MINPLUS: *out = KernelInfo{(const void*)&k_minplus, minplus_tables}; return true;
     case WGM_K_BC: *out = KernelInfo{(const void*)&k_bc<false>, bc_stage}; return true;
     default: return false;
   }
@@ -703,8 +993,8 @@ bool wgm_pannotia_kernel_info(int kernel, KernelInfo* out) {
 int wgm_pannotia_probe(wgm_runtime* rt, int kernel, int grid, int wg_size) {
   switch (kernel) {
     case WGM_K_MINPLUS:
-      hipLaunchKernelGGL(k_minplus<16>, dim3(grid), dim3(wg_size), 0, rt->stream, rt->ctl, MinplusDev{},
-                         (int*)nullptr);
+      hipLaunchKernelGGL(k_minplus, dim3(grid), dim3(wg_size), (size_t)minplus_tables(wg_size), rt->stream, rt->ctl,
+                         MinplusDev{}, (int*)nullptr);
       return WGM_OK;
     case WGM_K_BC:
       hipLaunchKernelGGL(k_bc<false>, dim3(grid), dim3(wg_size), (size_t)bc_stage_bytes(wg_size), rt->stream, rt->ctl, BcDev{}, (int*)nullptr);
@@ -715,7 +1005,7 @@ int wgm_pannotia_probe(wgm_runtime* rt, int kernel, int grid, int wg_size) {
 }
 
 void wgm_pannotia_release(wgm_graph* g) {
-  void* ptrs[] = {g->rrow, g->rcol, g->rwt, g->tasks, g->bc_d, g->bc_sig, g->bc_del, g->bc_q, g->bc_lvl, g->bc_sum, g->bc_srcs};
+  void* ptrs[] = {g->rrow, g->rcol, g->rwt, g->mp_sid, g->mp_roff, g->mp_start, g->mp_cid, g->mp_d, g->mp_bits, g->bc_d, g->bc_sig, g->bc_del, g->bc_q, g->bc_lvl, g->bc_sum, g->bc_srcs};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
 }
@@ -727,22 +1017,13 @@ int wgm_sssp_minplus(wgm_runtime* rt, wgm_graph* g, int32_t src, const wgm_launc
   if (!rt || !g || g->rt != rt) return fail(rt, WGM_ERR_INVALID, "bad runtime/graph");
   if (src < 0 || src >= g->n) return fail(rt, WGM_ERR_INVALID, "source %d out of range", src);
   if (!g->wt) return fail(rt, WGM_ERR_INVALID, "SSSP needs edge weights");
-  int rc = graph_reverse(g);
-  if (rc) return rc;
   if (!g->i32a) HIPCHK(rt, hipMalloc((void**)&g->i32a, sizeof(int32_t) * (size_t)g->n));
-  hipLaunchKernelGGL(k_minplus_init, dim3(256), dim3(256), 0, rt->stream, g->i32a, g->n, src, kBigNum);
-  MinplusDev p{(const int4*)g->tasks, g->ntasks, g->n + 1, g->rcol, g->rwt, g->i32a};
-  Ctl ctl{};
-  void* args[] = {&ctl, &p, &g->iters};
-  // the three lane widths share one resource class; the grid is sized on G = 16
   wgm_run_stats local{};
-  rc = launch_standalone_app(rt, WGM_K_MINPLUS, minplus_kernel(minplus_lanes(g)), lc, &ctl, args, 0, &local);
-  if (rc) return rc;
   int iters = 0;
-  HIPCHK(rt, hipMemcpy(&iters, g->iters, sizeof(int), hipMemcpyDeviceToHost));
-  if (iters < 0) return fail(rt, WGM_ERR_INVALID, "distances still fall after %d sweeps: negative cycle", g->n + 1);
+  int rc = run_minplus(rt, g, src, kBigNum, lc, g->i32a, &iters, &local);
+  if (rc) return rc;
   local.iterations = iters;
-  local.edges_scanned = (int64_t)iters * g->m;  // every sweep reads every in-edge
+  local.edges_scanned = (int64_t)iters * g->m;  // every sweep passes every in-edge
   if (dist_out) HIPCHK(rt, hipMemcpy(dist_out, g->i32a, sizeof(int32_t) * (size_t)g->n, hipMemcpyDeviceToHost));
   if (st) *st = local;
   return WGM_OK;
@@ -754,19 +1035,10 @@ int wgm_sssp_minplus(wgm_runtime* rt, wgm_graph* g, int32_t src, const wgm_launc
 // graph's own distance array with MYINFINITY for unreached vertices, so the
 // result is wgm_sssp's uint32 distances.
 int wgm_sssp_pull(wgm_runtime* rt, wgm_graph* g, int32_t src, const wgm_launch* lc, wgm_run_stats* st) {
-  int rc = graph_reverse(g);
-  if (rc) return rc;
   if (!g->dist) HIPCHK(rt, hipMalloc((void**)&g->dist, sizeof(uint32_t) * (size_t)g->n));
-  hipLaunchKernelGGL(k_minplus_init, dim3(256), dim3(256), 0, rt->stream, (int32_t*)g->dist, g->n, src,
-                     (int32_t)kInf);
-  MinplusDev p{(const int4*)g->tasks, g->ntasks, g->n + 1, g->rcol, g->rwt, (int32_t*)g->dist};
-  Ctl ctl{};
-  void* args[] = {&ctl, &p, &g->iters};
-  rc = launch_standalone_app(rt, WGM_K_MINPLUS, minplus_kernel(minplus_lanes(g)), lc, &ctl, args, 0, st);
-  if (rc) return rc;
   int iters = 0;
-  HIPCHK(rt, hipMemcpy(&iters, g->iters, sizeof(int), hipMemcpyDeviceToHost));
-  if (iters < 0) return fail(rt, WGM_ERR_INVALID, "distances still fall after %d sweeps", g->n + 1);
+  int rc = run_minplus(rt, g, src, (int32_t)kInf, lc, (int32_t*)g->dist, &iters, st);
+  if (rc) return rc;
   st->iterations = iters;
   return WGM_OK;
 }

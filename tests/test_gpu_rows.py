@@ -217,3 +217,59 @@ def test_bfs_bottom_up(rt, name):
             d, st = dg.bfs(src, wg_size=wg, num_wgs=wgs)
             assert np.array_equal(d, levels) and st["iterations"] == n_levels, (src, wg, wgs)
     dg.close()
+
+
+def _in_rows(degrees, seed, lo=1, n=9001):
+    """Vertex i has degrees[i % len] in-edges from random vertices; one vertex in 64 has none."""
+    rng = np.random.default_rng(seed)
+    deg = np.resize(np.asarray(degrees), n)
+    deg[::64] = 0
+    g = G.from_edges(n, rng.integers(0, n, deg.sum()), np.repeat(np.arange(n), deg))
+    g.wt = rng.integers(lo, 256, g.m).astype(np.int32)
+    return g
+
+
+def _dag(n=3000, m=12000):
+    rng = np.random.default_rng(31)
+    a, b = rng.integers(0, n, (2, m))
+    g = G.from_edges(n, np.minimum(a, b)[a != b], np.maximum(a, b)[a != b])
+    g.wt = rng.integers(-5, 256, g.m).astype(np.int32)  # also lowers vertices that the source does not reach
+    return g
+
+
+def _fan(n):
+    """Vertex 0 to all others, every 64th of those to its successor."""
+    tail = np.arange(64, n - 1, 64)
+    deg = np.zeros(n, np.int64)
+    deg[0], deg[tail] = n - 1, 1
+    col = np.concatenate([np.arange(1, n), tail + 1]).astype(np.int32)
+    wt = np.concatenate([np.arange(1, n) % 251 + 1, tail % 7]).astype(np.int32)
+    return G.CSR(np.concatenate([[0], np.cumsum(deg)]).astype(np.int32), col, wt)
+
+
+MINPLUS = {
+    "ones": lambda: _in_rows([1], 21),                     # 256 rows a block
+    "blocks": lambda: _in_rows([255, 256, 257, 1, 2], 22, n=701),  # rows that end, begin and go on at a block's edge
+    "steps": lambda: _in_rows([1025, 3, 64, 5000], 23, n=301),     # rows of several steps and waves
+    "mixed": lambda: _in_rows([0, 3, 0, 0, 70, 17], 24),
+    "edge": lambda: G.CSR(np.array([0, 1, 1], np.int32), np.array([1], np.int32), np.array([7], np.int32)),
+    "none": lambda: G.CSR(np.zeros(4, np.int32), np.zeros(0, np.int32), np.zeros(0, np.int32)),
+    "negative": _dag,
+    "two_rows_a_bit": lambda: _in_rows([1, 3, 2], 25, n=1200007),
+    "words_a_bit": lambda: _fan(33600000),
+}
+
+
+@pytest.mark.parametrize("name", MINPLUS)
+def test_minplus_rows(rt, name):
+    """Min-plus sweeps at the edges of blocks, steps and the LDS map; the
+    number of sweeps stays within the Jacobi one's."""
+    g = MINPLUS[name]()
+    src = int(np.argmax(g.degrees()))
+    ref, sweeps = oracle.sssp_minplus(g.row_ptr, g.col, g.wt, src)
+    dg = rt.graph(g)
+    for wg, wgs in ((1024, 0),) if g.n > 10 ** 6 else ((64, 1), (192, 7), (512, 64), (1024, 0)):
+        d, st = dg.sssp_minplus(src, wg_size=wg, num_wgs=wgs)
+        assert np.array_equal(d, ref), (wg, wgs)
+        assert 1 <= st["iterations"] <= sweeps
+    dg.close()
