@@ -262,15 +262,6 @@ __global__ void __launch_bounds__(1024, 8) k_pagerank(Ctl c, GraphDev g, float* 
   standalone_retire(c);
 }
 
-// Sum of out-degrees of reached vertices (dist != INF): the TEPS numerator.
-__global__ void k_reached_edges(GraphDev g, const uint32_t* dist, unsigned long long* out) {
-  unsigned long long local = 0;
-  for (int v = blockIdx.x * blockDim.x + threadIdx.x; v < g.n; v += gridDim.x * blockDim.x)
-    if (dist[v] != kInf) local += (unsigned long long)(g.row_ptr[v + 1] - g.row_ptr[v]);
-  for (int d = 32; d > 0; d >>= 1) local += __shfl_down(local, d, 64);
-  if ((threadIdx.x & 63) == 0 && local) atomicAdd(out, local);
-}
-
 }  // namespace wgm
 
 
@@ -307,21 +298,16 @@ int launch_prologue(wgm_runtime* rt, int kernel, const wgm_launch* lc, int* grid
   return WGM_OK;
 }
 
-int launch_epilogue(wgm_runtime* rt, const wgm_launch* lc, wgm_graph* g, wgm_run_stats* st) {
+// The finish of an app whose result is n elements from `src`.
+template <typename T>
+int launch_epilogue(wgm_runtime* rt, const wgm_launch* lc, wgm_graph* g, const T* src, T* dst, wgm_run_stats* st) {
   HIPCHK(rt, hipGetLastError());
-  int rc = WGM_OK;
-  double host_ms = 0.0;
-  if (lc && lc->handshake) rc = wgm_host_handshake(rt, &host_ms);
-  wgm_run_stats local{};
-  int rc2 = wgm_finish_launch(rt, &local);
-  if (rc == WGM_OK) rc = rc2;
-  if (rc) return rc;
-  int iters = 0;
-  HIPCHK(rt, hipMemcpy(&iters, g->iters, sizeof(int), hipMemcpyDeviceToHost));
-  local.iterations = iters;
-  local.host_ms = host_ms;
-  if (st) *st = local;
-  return WGM_OK;
+  AppOut out;
+  out.iters = g->iters;
+  out.src = src;
+  out.dst = dst;
+  out.bytes = sizeof(T) * (size_t)g->n;
+  return wgm_finish_app(rt, lc ? lc->handshake : 0, out, st);
 }
 
 }  // namespace
@@ -413,21 +399,6 @@ static int team_frontier_state(wgm_graph* g, bool sssp, FrontierDev* s, NearFar*
     nf->cnt = g->fcnt;
     nf->delta = wgm_standalone_delta(g->maxdeg);
   }
-  return WGM_OK;
-}
-
-int wgm_graph_reached_edges(wgm_graph* g, int64_t* out) {
-  wgm_runtime* rt = g->rt;
-  unsigned long long* d = nullptr;
-  HIPCHK(rt, hipMalloc(&d, sizeof(unsigned long long)));
-  (void)hipMemsetAsync(d, 0, sizeof(unsigned long long), rt->stream);
-  hipLaunchKernelGGL(k_reached_edges, dim3(256), dim3(256), 0, rt->stream, wgm_graph_view(g), g->dist, d);
-  unsigned long long h = 0;
-  hipError_t e = hipMemcpyAsync(&h, d, sizeof(h), hipMemcpyDeviceToHost, rt->stream);
-  if (e == hipSuccess) e = hipStreamSynchronize(rt->stream);
-  (void)hipFree(d);
-  if (e != hipSuccess) return wgm_hip_fail(rt, e, "reached edges");
-  *out = (int64_t)h;
   return WGM_OK;
 }
 
@@ -575,32 +546,13 @@ int wgm_enqueue_frontier(wgm_runtime* rt, const GraphDev& g, FrontierDev s, cons
   return WGM_OK;
 }
 
-template <class Enqueue>
-static int launch_and_finish(wgm_runtime* rt, int handshake, int* iters_dev, const Enqueue& enqueue,
-                             wgm_run_stats* st) {
+int wgm_launch_frontier(wgm_runtime* rt, const GraphDev& g, FrontierDev s, const NearFar& nf, bool sssp, int src,
+                        int grid, int wg, int handshake, const AppOut& out, wgm_run_stats* st) {
   int rc = wgm_reset_ctl(rt, 0, handshake ? 1 : 0);
   if (rc) return rc;
   HIPCHK(rt, hipEventRecord(rt->ev0, rt->stream));
-  rc = enqueue();
-  if (rc) return rc;
-  double host_ms = 0.0;
-  if (handshake) rc = wgm_host_handshake(rt, &host_ms);
-  wgm_run_stats local{};
-  const int rc2 = wgm_finish_launch(rt, &local);
-  if (rc == WGM_OK) rc = rc2;
-  if (rc) return rc;
-  int iters = 0;
-  HIPCHK(rt, hipMemcpy(&iters, iters_dev, sizeof(int), hipMemcpyDeviceToHost));
-  local.iterations = iters;
-  local.host_ms = host_ms;
-  if (st) *st = local;
-  return WGM_OK;
-}
-
-int wgm_launch_frontier(wgm_runtime* rt, const GraphDev& g, FrontierDev s, const NearFar& nf, bool sssp, int src,
-                        int grid, int wg, int handshake, int* iters_dev, wgm_run_stats* st) {
-  return launch_and_finish(
-      rt, handshake, iters_dev, [&]() { return wgm_enqueue_frontier(rt, g, s, nf, sssp, src, grid, wg, iters_dev); }, st);
+  rc = wgm_enqueue_frontier(rt, g, s, nf, sssp, src, grid, wg, (int*)out.iters);
+  return rc ? rc : wgm_finish_app(rt, handshake, out, st);
 }
 
 // The packed rows of a low-degree graph, laid out once.
@@ -630,14 +582,6 @@ static int enqueue_low(wgm_runtime* rt, const wgm_graph* g, const FrontierDev& s
   return WGM_OK;
 }
 
-// Sum of out-degrees of the vertices with dist != INF into *out (a device
-// cell the caller has cleared), on the runtime's stream.
-int wgm_enqueue_reached_edges(wgm_runtime* rt, const GraphDev& g, const uint32_t* dist, unsigned long long* out) {
-  hipLaunchKernelGGL(k_reached_edges, dim3(256), dim3(256), 0, rt->stream, g, dist, out);
-  HIPCHK(rt, hipGetLastError());
-  return WGM_OK;
-}
-
 extern "C" {
 
 static int run_frontier(wgm_runtime* rt, wgm_graph* g, int32_t src, const wgm_launch* lc, uint32_t* dist_out,
@@ -648,13 +592,7 @@ static int run_frontier(wgm_runtime* rt, wgm_graph* g, int32_t src, const wgm_la
   const int mode = lc ? lc->mode : WGM_SSSP_AUTO;
   if (mode < WGM_SSSP_AUTO || mode > WGM_SSSP_PULL) return fail(rt, WGM_ERR_INVALID, "unknown SSSP mode %d", mode);
   if (sssp && (mode == WGM_SSSP_PULL || (mode == WGM_SSSP_AUTO && g->maxdeg > 4))) {
-    wgm_run_stats local{};
-    int rc = wgm_sssp_pull(rt, g, src, lc, &local);
-    if (!rc) rc = wgm_graph_reached_edges(g, &local.edges_scanned);
-    if (rc) return rc;
-    if (dist_out) HIPCHK(rt, hipMemcpy(dist_out, g->dist, sizeof(uint32_t) * (size_t)g->n, hipMemcpyDeviceToHost));
-    if (st) *st = local;
-    return WGM_OK;
+    return wgm_sssp_pull(rt, g, src, lc, dist_out, st);
   }
   FrontierDev s{};
   NearFar nf{};
@@ -677,19 +615,20 @@ static int run_frontier(wgm_runtime* rt, wgm_graph* g, int32_t src, const wgm_la
     view.rrow = g->rrow;
     view.rcol = g->rcol;
   }
-  wgm_run_stats local{};
-  if (low) {
-    auto enqueue = [&]() { return enqueue_low(rt, g, s, nf, sssp, src, grid, wg); };
-    rc = launch_and_finish(rt, lc ? lc->handshake : 0, g->iters, enqueue, &local);
-  } else {
-    rc = wgm_launch_frontier(rt, view, s, nf, sssp, src, grid, wg, lc ? lc->handshake : 0, g->iters, &local);
-  }
+  const int handshake = lc ? lc->handshake : 0;
+  AppOut out;
+  out.iters = g->iters;
+  out.reached = g->dist;
+  out.g = view;
+  out.src = g->dist;
+  out.dst = dist_out;
+  out.bytes = sizeof(uint32_t) * (size_t)g->n;
+  if (!low) return wgm_launch_frontier(rt, view, s, nf, sssp, src, grid, wg, handshake, out, st);
+  rc = wgm_reset_ctl(rt, 0, handshake ? 1 : 0);
   if (rc) return rc;
-  rc = wgm_graph_reached_edges(g, &local.edges_scanned);
-  if (rc) return rc;
-  if (dist_out) HIPCHK(rt, hipMemcpy(dist_out, g->dist, sizeof(uint32_t) * (size_t)g->n, hipMemcpyDeviceToHost));
-  if (st) *st = local;
-  return WGM_OK;
+  HIPCHK(rt, hipEventRecord(rt->ev0, rt->stream));
+  rc = enqueue_low(rt, g, s, nf, sssp, src, grid, wg);
+  return rc ? rc : wgm_finish_app(rt, handshake, out, st);
 }
 
 int wgm_bfs(wgm_runtime* rt, wgm_graph* g, int32_t src, const wgm_launch* lc, uint32_t* dist_out,
@@ -713,10 +652,7 @@ int wgm_color(wgm_runtime* rt, wgm_graph* g, const wgm_launch* lc, int32_t* colo
   if (rc) return rc;
   hipLaunchKernelGGL(g->maxdeg > kTopoEdges ? k_color<true> : k_color<false>, dim3(grid), dim3(wg), scan_lds_bytes(wg),
                      rt->stream, rt->ctl, wgm_graph_view(g), g->i32a, (void*)g->wl, g->iters);
-  rc = launch_epilogue(rt, lc, g, st);
-  if (rc) return rc;
-  if (color_out) HIPCHK(rt, hipMemcpy(color_out, g->i32a, sizeof(int32_t) * (size_t)g->n, hipMemcpyDeviceToHost));
-  return WGM_OK;
+  return launch_epilogue(rt, lc, g, g->i32a, color_out, st);
 }
 
 int wgm_mis(wgm_runtime* rt, wgm_graph* g, const wgm_launch* lc, int32_t* s_out, wgm_run_stats* st) {
@@ -731,10 +667,7 @@ int wgm_mis(wgm_runtime* rt, wgm_graph* g, const wgm_launch* lc, int32_t* s_out,
   if (rc) return rc;
   hipLaunchKernelGGL(g->maxdeg > kTopoEdges ? k_mis<true> : k_mis<false>, dim3(grid), dim3(wg), scan_lds_bytes(wg),
                      rt->stream, rt->ctl, wgm_graph_view(g), g->i32a, g->i32b, (void*)g->wl, g->iters);
-  rc = launch_epilogue(rt, lc, g, st);
-  if (rc) return rc;
-  if (s_out) HIPCHK(rt, hipMemcpy(s_out, g->i32b, sizeof(int32_t) * (size_t)g->n, hipMemcpyDeviceToHost));
-  return WGM_OK;
+  return launch_epilogue(rt, lc, g, g->i32b, s_out, st);
 }
 
 int wgm_pagerank(wgm_runtime* rt, wgm_graph* g, float damping, int32_t iterations, const wgm_launch* lc,
@@ -759,10 +692,7 @@ int wgm_pagerank(wgm_runtime* rt, wgm_graph* g, float damping, int32_t iteration
   else
     hipLaunchKernelGGL(k_pagerank<false>, dim3(grid), dim3(wg), 0, rt->stream, rt->ctl, wgm_graph_view(g), g->f0, g->f1,
                        g->f2, damping, base, r0, iterations, (int32_t*)nullptr, g->iters);
-  rc = launch_epilogue(rt, lc, g, st);
-  if (rc) return rc;
-  if (rank_out) HIPCHK(rt, hipMemcpy(rank_out, g->f2, sizeof(float) * (size_t)g->n, hipMemcpyDeviceToHost));
-  return WGM_OK;
+  return launch_epilogue(rt, lc, g, g->f2, rank_out, st);
 }
 
 }  // extern "C"

@@ -79,13 +79,12 @@ int wgm_graph_frontier_state(wgm_graph* g, bool sssp, wgm::FrontierDev* s);
 // per-run arrays of a topology-driven app: 1 colour (i32a), 2 MIS (i32a,
 // i32b), 3 PageRank (f0, f1, f2); 0 nothing
 int wgm_graph_app_state(wgm_graph* g, int app);
-int wgm_graph_reached_edges(wgm_graph* g, int64_t* out);
 int wgm_launch_frontier(wgm_runtime* rt, const wgm::GraphDev& g, wgm::FrontierDev s, const wgm::NearFar& nf, bool sssp,
-                        int src, int grid, int wg, int handshake, int* iters_dev, wgm_run_stats* st);
+                        int src, int grid, int wg, int handshake, const AppOut& out, wgm_run_stats* st);
 int wgm_enqueue_frontier(wgm_runtime* rt, const wgm::GraphDev& g, wgm::FrontierDev s, const wgm::NearFar& nf, bool sssp,
                          int src, int grid, int wg, int* iters_dev);
 uint32_t wgm_standalone_delta(int maxdeg);
-int wgm_sssp_pull(wgm_runtime* rt, wgm_graph* g, int32_t src, const wgm_launch* lc, wgm_run_stats* st);
+int wgm_sssp_pull(wgm_runtime* rt, wgm_graph* g, int32_t src, const wgm_launch* lc, uint32_t* dist_out,
+                  wgm_run_stats* st);
 // the graph's in-edge CSR (g->rrow, g->rcol), built once and kept resident
 int wgm_graph_in_edges(wgm_graph* g);
-int wgm_enqueue_reached_edges(wgm_runtime* rt, const wgm::GraphDev& g, const uint32_t* dist, unsigned long long* out);

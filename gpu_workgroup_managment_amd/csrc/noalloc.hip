@@ -24,7 +24,7 @@ namespace {
 constexpr size_t kLineBytes = kLine * sizeof(int);
 constexpr size_t kHeavyCap = (size_t)(WGM_NOALLOC_MAX_M / kHeavyMin) + 2;  // heavy-list entries
 // layout: 11 counter lines (level counts 3, claims 3, heavy-list counts 3,
-// the level count 1, the reached-edge sum 1), two queues of n + 1 entries,
+// the level count 1, a spare one), two queues of n + 1 entries,
 // three heavy lists of kHeavyCap entries
 constexpr size_t kCounterLines = 11;
 constexpr size_t kQueueOff = kCounterLines * kLineBytes;
@@ -39,12 +39,6 @@ unsigned char* g_scratch[kMaxDevices] = {};
 }  // namespace
 
 static __device__ __align__(256) unsigned char scratch[kScratchBytes];
-
-namespace wgm {
-__global__ void k_noalloc_clear(unsigned long long* cell) {
-  if (blockIdx.x == 0 && threadIdx.x == 0) *cell = 0ull;
-}
-}  // namespace wgm
 
 // Called by wgm_create with `device` current: the device address of this
 // GPU's copy of the array.
@@ -100,7 +94,6 @@ int wgm_bfs_noalloc(wgm_runtime* rt, const int32_t* row_ptr, const int32_t* col,
   s.claims = lines + 3 * kLine;
   s.hcnt = lines + 6 * kLine;
   int* iters = lines + 9 * kLine;
-  unsigned long long* reached = (unsigned long long*)(lines + 10 * kLine);
   s.q0 = (int32_t*)(base + kQueueOff);
   s.q1 = s.q0 + n + 1;
   s.hv = (int32_t*)(base + kHeavyOff);
@@ -111,19 +104,11 @@ int wgm_bfs_noalloc(wgm_runtime* rt, const int32_t* row_ptr, const int32_t* col,
   g.col = col;
   g.n = n;
   g.m = (int32_t)m;
-  wgm_run_stats local{};
-  rc = wgm_launch_frontier(rt, g, s, NearFar{}, false, src, grid, wg, lc ? lc->handshake : 0, iters, &local);
-  if (rc) return rc;
-  hipLaunchKernelGGL(k_noalloc_clear, dim3(1), dim3(64), 0, rt->stream, reached);
-  WGM_HIPCHK(rt, hipGetLastError());
-  rc = wgm_enqueue_reached_edges(rt, g, dist, reached);
-  if (rc) return rc;
-  unsigned long long edges = 0;
-  WGM_HIPCHK(rt, hipMemcpyAsync(&edges, reached, sizeof(edges), hipMemcpyDeviceToHost, rt->stream));
-  WGM_HIPCHK(rt, hipStreamSynchronize(rt->stream));
-  local.edges_scanned = (int64_t)edges;
-  if (st) *st = local;
-  return WGM_OK;
+  AppOut out;
+  out.iters = iters;
+  out.reached = dist;
+  out.g = g;
+  return wgm_launch_frontier(rt, g, s, NearFar{}, false, src, grid, wg, lc ? lc->handshake : 0, out, st);
 }
 
 }  // extern "C"

@@ -803,7 +803,8 @@ int graph_reverse(wgm_graph* g) {
 // grid from the occupancy of `kernel` (capped at max_grid), optional host
 // handshake, bounded wait.
 int launch_standalone_app(wgm_runtime* rt, int kernel, const void* fn, const wgm_launch* lc, Ctl* ctl, void** args,
-                          int max_grid, wgm_run_stats* st, size_t lds = 0) {
+                          int max_grid, const AppOut& out, wgm_run_stats* st, size_t lds,
+                          unsigned long long* extra = nullptr) {
   wgm_launch def{256, 0, 0, 0};
   const wgm_launch& l = lc ? *lc : def;
   const int wg = l.wg_size > 0 ? l.wg_size : 256;
@@ -816,15 +817,7 @@ int launch_standalone_app(wgm_runtime* rt, int kernel, const void* fn, const wgm
   *ctl = rt->ctl;
   HIPCHK(rt, hipEventRecord(rt->ev0, rt->stream));
   HIPCHK(rt, hipLaunchKernel(fn, dim3(grid), dim3(wg), args, lds, rt->stream));
-  double host_ms = 0.0;
-  if (l.handshake) {
-    rc = wgm_host_handshake(rt, &host_ms);
-    if (rc) return rc;
-  }
-  rc = wgm_finish_launch(rt, st);
-  if (rc) return rc;
-  st->host_ms = host_ms;
-  return WGM_OK;
+  return wgm_finish_app(rt, l.handshake, out, st, extra);
 }
 
 // The min-plus graph, built once from the in-edge CSR and kept resident.
@@ -917,8 +910,8 @@ int bc_grid(wgm_runtime* rt, const wgm_graph* g, const wgm_launch* lc, int* grid
 // that are taken as one larger one on each CU, which also shortens the barrier.
 constexpr long long kMpMapBytes = 128 << 10;
 
-int run_minplus(wgm_runtime* rt, wgm_graph* g, int32_t src, int32_t big, const wgm_launch* lc, int32_t* dist, int* iters,
-                wgm_run_stats* st) {
+int run_minplus(wgm_runtime* rt, wgm_graph* g, int32_t src, int32_t big, const wgm_launch* lc, int32_t* dist,
+                bool reached, void* dst, wgm_run_stats* st) {
   int rc = minplus_rows(g);
   if (rc) return rc;
   MinplusDev p{};
@@ -968,11 +961,21 @@ int run_minplus(wgm_runtime* rt, wgm_graph* g, int32_t src, int32_t big, const w
   hipLaunchKernelGGL(k_minplus_init, dim3(256), dim3(256), 0, rt->stream, p);
   Ctl ctl{};
   void* args[] = {&ctl, &p, &g->iters};
-  rc = launch_standalone_app(rt, WGM_K_MINPLUS, (const void*)&k_minplus, &shape, &ctl, args, 0, st,
+  AppOut out;
+  out.iters = g->iters;
+  out.g = wgm_graph_view(g);
+  out.reached = reached ? (const uint32_t*)dist : nullptr;
+  out.src = dist;
+  out.dst = dst;
+  out.bytes = sizeof(int32_t) * (size_t)g->n;
+  wgm_run_stats local{};
+  rc = launch_standalone_app(rt, WGM_K_MINPLUS, (const void*)&k_minplus, &shape, &ctl, args, 0, out, &local,
                              (size_t)minplus_tables(shape.wg_size) + 4 * (size_t)p.map_words);
   if (rc) return rc;
-  HIPCHK(rt, hipMemcpy(iters, g->iters, sizeof(int), hipMemcpyDeviceToHost));
-  if (*iters < 0) return fail(rt, WGM_ERR_INVALID, "distances still fall after %d sweeps: negative cycle", g->n + 1);
+  if (local.iterations < 0)
+    return fail(rt, WGM_ERR_INVALID, "distances still fall after %d sweeps: negative cycle", g->n + 1);
+  if (!reached) local.edges_scanned = (int64_t)local.iterations * g->m;  // every sweep passes every in-edge
+  if (st) *st = local;
   return WGM_OK;
 }
 
@@ -1018,15 +1021,7 @@ int wgm_sssp_minplus(wgm_runtime* rt, wgm_graph* g, int32_t src, const wgm_launc
   if (src < 0 || src >= g->n) return fail(rt, WGM_ERR_INVALID, "source %d out of range", src);
   if (!g->wt) return fail(rt, WGM_ERR_INVALID, "SSSP needs edge weights");
   if (!g->i32a) HIPCHK(rt, hipMalloc((void**)&g->i32a, sizeof(int32_t) * (size_t)g->n));
-  wgm_run_stats local{};
-  int iters = 0;
-  int rc = run_minplus(rt, g, src, kBigNum, lc, g->i32a, &iters, &local);
-  if (rc) return rc;
-  local.iterations = iters;
-  local.edges_scanned = (int64_t)iters * g->m;  // every sweep passes every in-edge
-  if (dist_out) HIPCHK(rt, hipMemcpy(dist_out, g->i32a, sizeof(int32_t) * (size_t)g->n, hipMemcpyDeviceToHost));
-  if (st) *st = local;
-  return WGM_OK;
+  return run_minplus(rt, g, src, kBigNum, lc, g->i32a, false, dist_out, st);
 }
 
 }  // extern "C"
@@ -1034,13 +1029,10 @@ int wgm_sssp_minplus(wgm_runtime* rt, wgm_graph* g, int32_t src, const wgm_launc
 // Lonestar SSSP in the pull direction: the min-plus sweeps above on the
 // graph's own distance array with MYINFINITY for unreached vertices, so the
 // result is wgm_sssp's uint32 distances.
-int wgm_sssp_pull(wgm_runtime* rt, wgm_graph* g, int32_t src, const wgm_launch* lc, wgm_run_stats* st) {
+int wgm_sssp_pull(wgm_runtime* rt, wgm_graph* g, int32_t src, const wgm_launch* lc, uint32_t* dist_out,
+                  wgm_run_stats* st) {
   if (!g->dist) HIPCHK(rt, hipMalloc((void**)&g->dist, sizeof(uint32_t) * (size_t)g->n));
-  int iters = 0;
-  int rc = run_minplus(rt, g, src, (int32_t)kInf, lc, (int32_t*)g->dist, &iters, st);
-  if (rc) return rc;
-  st->iterations = iters;
-  return WGM_OK;
+  return run_minplus(rt, g, src, (int32_t)kInf, lc, (int32_t*)g->dist, true, dist_out, st);
 }
 
 extern "C" {
@@ -1088,15 +1080,19 @@ int wgm_bc(wgm_runtime* rt, wgm_graph* g, int32_t num_sources, const wgm_launch*
   void* args[] = {&ctl, &b, &g->iters};
   wgm_run_stats local{};
   const wgm_launch shape{wg, grid, lc ? lc->handshake : 0, 0};
-  rc = launch_standalone_app(rt, WGM_K_BC, bc_in_lds(g) ? (const void*)&k_bc<true> : (const void*)&k_bc<false>, &shape, &ctl, args, grid,
-                             &local, (size_t)bc_lds(g, wg));
-  if (rc) return rc;
+  AppOut out;
+  out.iters = g->iters;
+  out.extra = levels;
+  out.src = g->bc_sum;
+  out.dst = bc_out;
+  out.bytes = sizeof(double) * (size_t)g->n;
   unsigned long long lv = 0;
-  HIPCHK(rt, hipMemcpy(&lv, levels, sizeof(lv), hipMemcpyDeviceToHost));
+  rc = launch_standalone_app(rt, WGM_K_BC, bc_in_lds(g) ? (const void*)&k_bc<true> : (const void*)&k_bc<false>, &shape, &ctl, args, grid,
+                             out, &local, (size_t)bc_lds(g, wg), &lv);
+  if (rc) return rc;
   local.iterations = (int32_t)std::min<unsigned long long>(lv, INT32_MAX);  // BFS levels over all sources
   // TEPS convention for BC: each source traverses every edge once forward
   local.edges_scanned = (int64_t)nsrc * g->m;
-  if (bc_out) HIPCHK(rt, hipMemcpy(bc_out, g->bc_sum, sizeof(double) * (size_t)g->n, hipMemcpyDeviceToHost));
   if (st) *st = local;
   return WGM_OK;
 }

@@ -4,12 +4,45 @@
 #include <hip/hip_runtime.h>
 
 #include <map>
+#include <mutex>
 #include <string>
 
 #include "graph_apps.hpp"
 #include "wgm.h"
 
 struct wgm_extras;  // scheduler / batched / serving state (other units)
+
+// What a standalone launch reports, written by k_finish into a coherent cell.
+struct AppReport {
+  unsigned long long clock[2];
+  unsigned long long edges;  // out-edges of the reached vertices
+  unsigned long long extra;
+  int count;
+  int iters;
+};
+
+// The end of a standalone launch: cells to report and the result to copy out
+// (null: none).
+struct AppOut {
+  const int* iters = nullptr;
+  const unsigned long long* extra = nullptr;
+  const uint32_t* reached = nullptr;  // distances of `g` to sum the reached edges of
+  wgm::GraphDev g{};
+  const void* src = nullptr;  // device
+  void* dst = nullptr;        // host
+  size_t bytes = 0;
+};
+
+// Pinned staging of the standalone launches' results (wgm_finish_app), of one
+// copy at a time.
+constexpr size_t kStageBytes = 16u << 20;
+constexpr size_t kStageChunk = 2u << 20;  // smaller ones pay 30 us each
+struct HostStage {
+  std::mutex mu;
+  char* buf = nullptr;
+  size_t size = 0;
+  hipEvent_t ev[kStageBytes / kStageChunk] = {};
+};
 
 struct wgm_runtime {
   int device = 0;
@@ -32,10 +65,13 @@ struct wgm_runtime {
   std::map<int, int> disc_cache;  // discovered occupancy per (kernel, wg)
   std::string last_error;
   wgm_extras* extras = nullptr;
+  HostStage stage;
 
   int* host_sched_flag() { return h_cells; }
   int* host_persistent_flag() { return h_cells + wgm::kLine; }
   int* host_participating() { return h_cells + 2 * wgm::kLine; }
+  AppReport* host_report() { return (AppReport*)(h_cells + 3 * wgm::kLine); }
+  AppReport* report_dev() { return (AppReport*)(h_cells_dev + 3 * wgm::kLine); }
 };
 
 struct KernelInfo {
@@ -53,6 +89,7 @@ int wgm_occupancy(wgm_runtime* rt, int kernel, int wg_size, int* per_cu);
 int wgm_resolve_grid(wgm_runtime* rt, int kernel, int wg_size, int requested, int* grid);
 int wgm_host_handshake(wgm_runtime* rt, double* host_ms);
 int wgm_finish_launch(wgm_runtime* rt, wgm_run_stats* st);
+int wgm_finish_app(wgm_runtime* rt, int handshake, const AppOut& out, wgm_run_stats* st, unsigned long long* extra = nullptr);
 bool wgm_wait_cell(const int* cell, int value, bool equal, double timeout_s);
 // defined by the app unit (apps.hip): true / WGM_OK when `kernel` is one of its kernels
 bool wgm_app_kernel_info(int kernel, KernelInfo* out);

@@ -273,3 +273,17 @@ def test_minplus_rows(rt, name):
         assert np.array_equal(d, ref), (wg, wgs)
         assert 1 <= st["iterations"] <= sweeps
     dg.close()
+
+
+@pytest.mark.parametrize("n", [1, 16384, 16385, (1 << 19) - 1, (1 << 19) + 1, (1 << 22) + (1 << 19) + 3])
+def test_results_arrive_whole(rt, n):
+    """Results below and above a staging size, a chunk and the whole staging
+    (4 bytes a vertex)."""
+    g = _fan(n)
+    ref, _ = oracle.sssp_minplus(g.row_ptr, g.col, g.wt, 0)
+    dg = rt.graph(g)
+    a, _ = dg.sssp_minplus(0)
+    b, st = dg.sssp(0, mode=2)
+    assert np.array_equal(a, ref) and np.array_equal(b, ref)
+    assert st["edges_scanned"] == g.m
+    dg.close()
