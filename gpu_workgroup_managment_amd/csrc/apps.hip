@@ -59,15 +59,15 @@ __global__ void __launch_bounds__(1024) k_frontier(Ctl c, GraphDev g, FrontierDe
 // step of the batched launch, its queues, visited or far bits and combine
 // tables in LDS, on packed rows (k_low_rows). A team's cross-workgroup barrier
 // costs more than a narrow level's work. Bound: two dependent loads and one or
-// two workgroup barriers a level (1.1 us BFS, 2.3 us SSSP).
+// two workgroup barriers a level (1.1 us BFS, 2.2 us SSSP).
 // Rule: no edge spans more than kLowSpan places of the (circular) vertex
 // order, so that k levels reach at most 2 k kLowSpan + 1 vertices; or the whole
 // graph is small. Kernel times, team -> one workgroup, 64 x 512: 361 x 415 grid
-// BFS 3508 -> 606 us, SSSP 7293 -> 2591; 10^5 vertices of 4 random edges within
-// span 300: 2608 -> 408 and 6428 -> 1777, span 1000: 502 -> 243 and 1392 ->
+// BFS 3508 -> 604 us, SSSP 7293 -> 2193; 10^5 vertices of 4 random edges within
+// span 300: 2608 -> 408 and 6428 -> 1455, span 1000: 502 -> 243 and 1392 ->
 // 1422, so the line lies at 768; random targets, 8192 vertices: 75 -> 32 and
 // 209 -> 122, 16384: 93 -> 50 and 254 -> 237, 20000: SSSP 272 -> 300 and more,
-// so it lies at 16384. Whole calls, 361 x 415 SSSP: 8106 -> 2903 us.
+// so it lies at 16384. Whole calls, 361 x 415 SSSP: 8093 -> 2507 us.
 constexpr int32_t kLowSpan = 768;
 constexpr int32_t kLowAnySpan = 16384;
 constexpr int32_t kLowMaxN = 32 * kFarBitWords;
@@ -84,7 +84,8 @@ __global__ void __launch_bounds__(1024) k_low(Ctl c, GraphDev g, FrontierDev s, 
   if (!standalone_begin(c, t)) return;
   if (t.id == 0) {
     nf.delta = SSSP ? kLowDelta : 0u;
-    run_low<SSSP, kLowDegree, SSSP ? kCombU : kLowSlots, true, SSSP>(g, s, nf, src, lds_low, s_cnt, iters_out, true, ell);
+    if constexpr (SSSP) run_low_comb(g, s, nf, src, lds_low, s_cnt, iters_out, ell);
+    else run_low<false, kLowDegree, kLowSlots, true>(g, s, nf, src, lds_low, s_cnt, iters_out, true, ell);
     __syncthreads();
     if (threadIdx.x == 0) clock_end(c, 0);
   }

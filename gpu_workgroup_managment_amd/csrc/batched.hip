@@ -253,7 +253,7 @@ __global__ void __launch_bounds__(1024) k_batched(Ctl c, BatchDev b) {
           // the combine tables hold a pass's candidates at most half full
           // and candidate ids fit 11 bits
           if (sssp && b.low_ell == 2 && lds_flags && nf.delta && (int)blockDim.x * kCombU <= kCombSlots / 2)
-            run_low<true, kLowDegree, kCombU, true, true>(g, s, nf, jb.src, lds, s_cnt, &b.iters[j], true, ell);
+            run_low_comb(g, s, nf, jb.src, lds, s_cnt, &b.iters[j], ell);
           else if (sssp) run_low<true, kLowDegree, kLowSlots, true>(g, s, nf, jb.src, lds, s_cnt, &b.iters[j], lds_flags, ell);
           else run_low<false, kLowDegree, kLowSlots, true>(g, s, nf, jb.src, lds, s_cnt, &b.iters[j], lds_flags, ell);
         } else {

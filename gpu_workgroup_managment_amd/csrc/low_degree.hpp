@@ -2,6 +2,8 @@
 // batched launch's small graphs and the standalone apps' narrow ones).
 #pragma once
 
+#include <type_traits>
+
 #include "team_frontier.hpp"
 
 namespace wgm {
@@ -175,27 +177,17 @@ struct LowQueues {
 // vertex, word k = (target << 8) | weight of its k-th edge, kEllNone past its
 // degree -- so the K threads of an entry load one 4K-byte row together, an
 // entry needs no row_info, and the second round trip is the atomic alone.
-// COMB (SSSP on packed rows with the LDS bitmap): no atomic on dist at all.
-// A pass loads each candidate target's distance with a plain load and folds
-// its candidates per target in an LDS combine table (comb_insert); after an
-// LDS-only barrier the one winner of each slot, if below the loaded
-// distance, stores it and queues the target. The workgroup is the only
-// writer of the graph's distances, so its L2 holds them and the second round
-// trip is an L2 hit instead of an atomic beyond the L2. A level of several
-// passes orders one pass's stores before the next pass's loads with a full
-// barrier.
-template <bool SSSP, int K, int U, bool ELL, bool COMB = false>
+template <bool SSSP, int K, int U, bool ELL>
 __device__ void run_low(const GraphDev& g, const FrontierDev& s, const NearFar& nf, int src, int* lds, int* s_cnt,
                         int* iters_out, bool lds_flags, const uint32_t* ell) {
   const bool near_far = SSSP && nf.delta > 0;
   __shared__ int s_far[3];  // far counts of q[0], q[1]; band minimum
-  const LowQueues lq = COMB ? LowQueues{(lds_u32*)lds, kCombCap, &s, 2}
-                            : LowQueues{(lds_u32*)(reinterpret_cast<uint32_t*>(lds) + frontier_lds_bytes((int)blockDim.x) / 4),
-                                        low_lds_cap((int)blockDim.x), &s, 3};
+  const LowQueues lq{(lds_u32*)(reinterpret_cast<uint32_t*>(lds) + frontier_lds_bytes((int)blockDim.x) / 4),
+                     low_lds_cap((int)blockDim.x), &s, 3};
   // one bit per vertex in LDS (lds_flags): SSSP's far flags (else a word per
   // vertex in HBM); BFS's visited marks, which then replace the atomic on
   // dist (else the atomic minimum decides the discovery)
-  lds_u32* fbits = COMB ? comb_bits(lds) : batch_bits(lds);
+  lds_u32* fbits = batch_bits(lds);
   const bool bits = near_far && lds_flags;
   const bool vis = !SSSP && lds_flags;
   for (int v = threadIdx.x; v < g.n; v += blockDim.x) {
@@ -205,9 +197,6 @@ __device__ void run_low(const GraphDev& g, const FrontierDev& s, const NearFar& 
   if (bits || vis)
     for (int w = threadIdx.x; w < (g.n + 31) / 32; w += blockDim.x)
       fbits[w] = vis && w == (src >> 5) ? 1u << (src & 31) : 0u;
-  lds_u64* comb = batch_comb(lds);
-  if (COMB)
-    for (int i = threadIdx.x; i < 3 * kCombSlots; i += blockDim.x) comb[i] = kCombEmpty;
   if (threadIdx.x == 0) {
     lq.store(0, 0, src, ELL ? 0u : row_info(g, src), 0u, SSSP, !ELL);
     s_cnt[0] = 1;
@@ -225,16 +214,6 @@ __device__ void run_low(const GraphDev& g, const FrontierDev& s, const NearFar& 
   int level = 0, fi = 0;
   uint32_t thr = near_far ? nf.delta : 0xffffffffu;
   uint32_t nrel = 0;  // edges this thread relaxed (live entries' edges)
-  int tcur = 0;       // COMB: this pass's table
-  // COMB: a queued target's packed row is loaded as it is queued, so that the
-  // next level finds it in the cache; the loads complete by the level's
-  // barrier and their values are only folded into pfacc (never read)
-  uint32_t pfv[U], pfacc = 0;
-#pragma unroll
-  for (int x = 0; x < U; x++) pfv[x] = 0u;
-  int clr[U];         // COMB: slot this thread won in the previous pass (cleared after this pass's barrier)
-#pragma unroll
-  for (int x = 0; x < U; x++) clr[x] = -1;
   while (true) {
     for (;; level++) {
       const int in_n = __builtin_amdgcn_readfirstlane(s_cnt[level % 3]);
@@ -248,18 +227,9 @@ __device__ void run_low(const GraphDev& g, const FrontierDev& s, const NearFar& 
         // slot x holds entries of this wave only while a + x per + its first
         // slot < in_n: a scalar test, so a wave runs no code for empty slots
         // (most levels fill one slot, and only some waves of it) -- issue
-        // time, not memory, bounds a narrow level. COMB passes have barriers:
-        // every wave runs them, and the per-slot tests below skip the rest.
+        // time, not memory, bounds a narrow level.
         const int wslot = __builtin_amdgcn_readfirstlane((int)threadIdx.x & ~63) / K;
-        if (COMB && a > 0) {
-          __syncthreads();  // the last pass's stores before this pass's loads
-#pragma unroll
-          for (int x = 0; x < U; x++) {
-            pfacc ^= pfv[x];
-            pfv[x] = 0u;
-          }
-        }
-        if (!COMB && a + wslot >= in_n) continue;
+        if (a + wslot >= in_n) continue;
         bool lv[U];
 #pragma unroll
         for (int x = 0; x < U; x++) lv[x] = a + x * per + wslot < in_n;
@@ -301,10 +271,8 @@ __device__ void run_low(const GraphDev& g, const FrontierDev& s, const NearFar& 
         // Only the memory operations sit under each slot's condition; what
         // reads their results comes after every slot has issued.
         uint32_t alt[U], old[U], r0[U], r1[U];
-        int hs[U];  // COMB: the target's slot in this pass's table
 #pragma unroll
         for (int x = 0; x < U; x++) {
-          hs[x] = -1;
           const bool live = ok[x] && (!SSSP || dv[x] == du[x]);
           nrel += live ? 1u : 0u;
           alt[x] = SSSP ? du[x] + w[x] : next;
@@ -321,12 +289,7 @@ __device__ void run_low(const GraphDev& g, const FrontierDev& s, const NearFar& 
             r1[x] = (uint32_t)g.row_ptr[uu + 1];
           }
           if (live) {
-            if (COMB) {
-              // the target's distance (plain load, in flight across the
-              // barrier) and the candidate into the combine table
-              old[x] = s.dist[u[x]];
-              hs[x] = comb_insert(comb + tcur * kCombSlots, u[x], comb_word(u[x], alt[x], x * bd + (int)threadIdx.x));
-            } else if (vis) {
+            if (vis) {
               // BFS with visited bits: the first to set u's bit discovers it
               const uint32_t bit = 1u << (u[x] & 31);
               old[x] = (__hip_atomic_fetch_or(&fbits[u[x] >> 5], bit, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) &
@@ -339,27 +302,6 @@ __device__ void run_low(const GraphDev& g, const FrontierDev& s, const NearFar& 
             }
           }
         }
-        bool won[U];
-#pragma unroll
-        for (int x = 0; x < U; x++) won[x] = false;
-        if constexpr (COMB) {
-          // every candidate is in the table; the slot's word is the minimum
-          // over its target's candidates, and the candidate whose word it is
-          // wins it (the thread bits break ties)
-          lds_barrier();
-          lds_u64* tb = comb + tcur * kCombSlots;
-          lds_u64* tp = comb + (tcur == 0 ? 2 : tcur - 1) * kCombSlots;
-#pragma unroll
-          for (int x = 0; x < U; x++) {
-            if (clr[x] >= 0) tp[clr[x]] = kCombEmpty;
-            clr[x] = -1;
-            if (hs[x] >= 0) {
-              won[x] = tb[hs[x]] == comb_word(u[x], alt[x], x * bd + (int)threadIdx.x);
-              if (won[x]) clr[x] = hs[x];
-            }
-          }
-          tcur = tcur == 2 ? 0 : tcur + 1;
-        }
 #pragma unroll
         for (int x = 0; x < U; x++) {
           opaque(old[x]);
@@ -371,13 +313,11 @@ __device__ void run_low(const GraphDev& g, const FrontierDev& s, const NearFar& 
 #pragma unroll
         for (int x = 0; x < U; x++) {
           ru[x] = (r0[x] << 3) | (r1[x] - r0[x]);
-          const bool better = COMB ? won[x] && alt[x] < old[x] : SSSP ? alt[x] < old[x] : old[x] == kInf;
+          const bool better = SSSP ? alt[x] < old[x] : old[x] == kInf;
           want[x] = better && (!SSSP || alt[x] < thr);
           far_cand[x] = SSSP && better && alt[x] >= thr;
           // the discoverer writes the level: nothing reads dist during a BFS
           if (vis && want[x]) s.dist[u[x]] = alt[x];
-          if (COMB && better) s.dist[u[x]] = alt[x];
-          if (COMB && want[x]) pfv[x] = ell[(size_t)u[x] * K];
         }
 #pragma unroll
         for (int x = 0; x < U; x++) {
@@ -408,11 +348,6 @@ __device__ void run_low(const GraphDev& g, const FrontierDev& s, const NearFar& 
         }
       }
       __syncthreads();
-#pragma unroll
-      for (int x = 0; x < U; x++) {
-        pfacc ^= pfv[x];
-        pfv[x] = 0u;
-      }
     }
     if (!near_far) break;
     // uniform: read after the level's barrier (scalar, so the branches
@@ -492,7 +427,260 @@ __device__ void run_low(const GraphDev& g, const FrontierDev& s, const NearFar& 
     fi = 1 - fi;
     __syncthreads();
   }
-  asm volatile("" ::"v"(pfacc));  // keeps the row loads (their values are unused)
+  for (int d = 32; d > 0; d >>= 1) nrel += __shfl_down(nrel, d, 64);
+  if ((threadIdx.x & 63) == 0 && nrel && s.relaxed) atomicAdd(s.relaxed, (unsigned long long)nrel);
+  if (threadIdx.x == 0) *iters_out = level;
+}
+
+// SSSP on packed rows with everything but the graph and the distances in LDS
+// (the combine layout): no atomic on dist at all. A pass loads each candidate
+// target's distance with a plain load and folds its candidates per target in
+// an LDS combine table (comb_insert); after an LDS barrier the one winner of
+// each slot, if below the loaded distance, stores it and queues the target.
+// The workgroup is the only writer of the graph's distances, so its L2 holds
+// them. Entry, bands and far queues are run_low's, four lanes an entry. A level
+// of up to blockDim.x / 4 entries is one pass of a slot per lane group, a wider
+// one takes passes of two, with a barrier between the stores of one pass and
+// the loads of the next. Only a level of several passes can queue a vertex
+// twice, so only the entries after one are compared with their vertices'
+// distances.
+// Bound: the chain of a level -- its entries from LDS, their rows and their
+// targets' distances from the L2, the table, the queue -- 2.2 us at 200 entries.
+// As a case of run_low, whose queue reads may also come from memory, every level
+// waited for the stores of the one before (361 x 415 grid, kernel: 2720 us; 2270
+// here). A queued target's row is not fetched ahead: wherever its register or LDS
+// word lay, a wait for it came before the level's end (2440 us).
+__device__ void run_low_comb(const GraphDev& g, const FrontierDev& s, const NearFar& nf, int src, int* lds, int* s_cnt,
+                             int* iters_out, const uint32_t* ell) {
+  constexpr int K = kLowDegree;
+  __shared__ int s_far[3];  // far counts of q[0], q[1]; band minimum
+  // uniform values in scalar registers: the loops and the barriers in them stay
+  // uniform for the compiler
+  const int bd = __builtin_amdgcn_readfirstlane((int)blockDim.x), per = bd / K;
+  const LowQueues lq{(lds_u32*)lds, kCombCap, &s, 2};
+  lds_u32* fbits = comb_bits(lds);
+  lds_u64* comb = batch_comb(lds);
+  for (int v = threadIdx.x; v < g.n; v += bd) s.dist[v] = (v == src) ? 0u : kInf;
+  for (int w = threadIdx.x; w < (g.n + 31) / 32; w += bd) fbits[w] = 0u;
+  for (int i = threadIdx.x; i < 3 * kCombSlots; i += bd) comb[i] = kCombEmpty;
+  if (threadIdx.x == 0) {
+    lq.store(0, 0, src, 0u, 0u, true, false);
+    s_cnt[0] = 1;
+    s_cnt[1] = 0;
+    s_cnt[2] = 0;
+    s_far[0] = 0;
+    s_far[1] = 0;
+    s_far[2] = INT32_MAX;
+  }
+  __syncthreads();
+  const int lane = (int)threadIdx.x & 63, slot = (int)threadIdx.x / K, k = (int)threadIdx.x % K;
+  const int wslot = __builtin_amdgcn_readfirstlane((int)threadIdx.x & ~63) / K;  // the wave's first slot
+  const unsigned long long below = (1ull << lane) - 1ull;
+  int level = 0, fi = 0, tcur = 0;
+  uint32_t thr = nf.delta, nrel = 0;
+  bool twice = false;         // the level's queue may hold a vertex twice
+  int clr[kCombU];            // slots this thread won in the previous pass, cleared after this pass's barrier
+#pragma unroll
+  for (int x = 0; x < kCombU; x++) clr[x] = -1;
+
+  auto pass = [&](auto slots, int a, int in_n, int p, int* out_cnt) {
+    constexpr int N = decltype(slots)::value;
+    tcur = __builtin_amdgcn_readfirstlane(tcur);
+    lds_u64* tb = comb + tcur * kCombSlots;
+    lds_u64* tp = comb + (tcur == 0 ? 2 : tcur - 1) * kCombSlots;
+    uint32_t du[N], word[N], dv[N], alt[N], old[N];
+    int v[N], u[N], hs[N];
+    bool on[N], ok[N];
+#pragma unroll
+    for (int x = 0; x < N; x++) {
+      on[x] = a + x * per + wslot < in_n;  // scalar: this wave has entries in the slot
+      ok[x] = false;
+      hs[x] = -1;
+    }
+    if (on[0]) {
+#pragma unroll
+      for (int x = 0; x < N; x++) {
+        const int i = a + x * per + slot;
+        ok[x] = i < in_n;
+        uint32_t none;
+        v[x] = 0;
+        du[x] = 0;
+        if (in_n <= kCombCap) {  // scalar: the queue is in LDS as a whole
+          const lds_u32* q = lq.lds + p * 2 * kCombCap + min(i, in_n - 1);
+          v[x] = (int)q[0];
+          du[x] = q[kCombCap];
+        } else if (ok[x]) {
+          lq.load(p, i, v[x], none, du[x], true, false);
+        }
+      }
+      // round trip 1: the edges (and the entries' distances)
+#pragma unroll
+      for (int x = 0; x < N; x++) word[x] = ell[(uint32_t)v[x] * K + k];
+#pragma unroll
+      for (int x = 0; x < N; x++) dv[x] = twice ? s.dist[v[x]] : du[x];
+      // round trip 2: the targets' distances, in flight across the barrier
+#pragma unroll
+      for (int x = 0; x < N; x++) {
+        ok[x] = ok[x] && word[x] != kEllNone && dv[x] == du[x];
+        u[x] = ok[x] ? (int)(word[x] >> 8) : 0;
+        alt[x] = du[x] + (word[x] & 255u);
+        nrel += ok[x] ? 1u : 0u;
+      }
+#pragma unroll
+      for (int x = 0; x < N; x++) old[x] = s.dist[u[x]];
+#pragma unroll
+      for (int x = 0; x < N; x++)
+        if (ok[x]) hs[x] = comb_insert(tb, u[x], comb_word(u[x], alt[x], x * bd + (int)threadIdx.x));
+    }
+    lds_barrier();
+    // every candidate is in the table; the slot's word is the minimum over its
+    // target's candidates, and the candidate whose word it is wins it (the
+    // thread bits break ties)
+#pragma unroll
+    for (int x = 0; x < kCombU; x++) {
+      if (clr[x] >= 0) tp[clr[x]] = kCombEmpty;
+      clr[x] = -1;
+    }
+    tcur = tcur == 2 ? 0 : tcur + 1;
+    if (!on[0]) return;
+    bool won[N];
+#pragma unroll
+    for (int x = 0; x < N; x++) {
+      won[x] = false;
+      if (hs[x] >= 0) {
+        won[x] = tb[hs[x]] == comb_word(u[x], alt[x], x * bd + (int)threadIdx.x);
+        if (won[x]) clr[x] = hs[x];
+      }
+    }
+#pragma unroll
+    for (int x = 0; x < N; x++) {
+      const bool better = won[x] && alt[x] < old[x];
+      if (!__ballot(better)) continue;
+      const bool near = better && alt[x] < thr, far = better && alt[x] >= thr;
+      if (better) s.dist[u[x]] = alt[x];
+      const unsigned long long mask = __ballot(near);
+      if (mask) {
+        const int leader = __ffsll((long long)mask) - 1, count = __popcll(mask);
+        int base = 0;
+        // (opaque: one lane's addition, which needs no combining over the wave)
+        int at = 0;
+        opaque(at);
+        if (lane == leader)
+          base = __hip_atomic_fetch_add(out_cnt + at, count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        base = __builtin_amdgcn_readlane(base, leader);
+        const int i = base + __popcll(mask & below);
+        if (base + count <= kCombCap) {  // scalar
+          lds_u32* q = lq.lds + (1 - p) * 2 * kCombCap + i;
+          if (near) {
+            q[0] = (uint32_t)u[x];
+            q[kCombCap] = alt[x];
+          }
+        } else if (near) {
+          lq.store(1 - p, i, u[x], 0u, alt[x], true, false);
+        }
+      }
+      if (__ballot(far)) {
+        const uint32_t bit = 1u << (u[x] & 31);
+        const bool fresh = far && (__hip_atomic_fetch_or(&fbits[u[x] >> 5], bit, __ATOMIC_RELAXED,
+                                                         __HIP_MEMORY_SCOPE_WORKGROUP) & bit) == 0u;
+        push_item<false>(fresh, u[x], nf.far(fi), &s_far[fi], __HIP_MEMORY_SCOPE_WORKGROUP);
+      }
+    }
+  };
+
+  while (true) {
+    for (;; level++) {
+      const int in_n = __builtin_amdgcn_readfirstlane(s_cnt[level % 3]);
+      if (in_n == 0) break;
+      // counter (level + 2) % 3 was last read at the start of level - 1
+      if (threadIdx.x == 0) s_cnt[(level + 2) % 3] = 0;
+      int* out_cnt = &s_cnt[(level + 1) % 3];
+      const int p = level & 1;  // in queue; 1 - p is the out queue
+      if (in_n <= per) {
+        pass(std::integral_constant<int, 1>{}, 0, in_n, p, out_cnt);
+        twice = false;
+      } else {
+        for (int a = 0; a < in_n; a += kCombU * per) {
+          if (a > 0) __syncthreads();  // the last pass's stores before this pass's loads
+          pass(std::integral_constant<int, kCombU>{}, a, in_n, p, out_cnt);
+        }
+        twice = in_n > kCombU * per;
+      }
+      __syncthreads();
+    }
+    // uniform: read after the level's barrier (scalar, so the branches
+    // around the barriers below stay uniform for the compiler too)
+    const int fn = __builtin_amdgcn_readfirstlane(s_far[fi]);
+    if (fn == 0) break;
+    const int p = level & 1;  // this level's (empty) queue
+    // move a far entry below the new threshold to the near queue, else to the other far queue
+    const uint32_t t_old = thr;  // far entries below it were relaxed in the band (dropped)
+    twice = false;
+    auto split = [&](bool in, int v, uint32_t dv) {
+      bool to_near = false, to_far = false;
+      if (in) {
+        if (dv < thr) {
+          // each deferred vertex is in one far queue once: it moves once
+          __hip_atomic_fetch_and(&fbits[v >> 5], ~(1u << (v & 31)), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+          to_near = dv >= t_old;
+        } else {
+          to_far = true;  // stays flagged in the other far queue
+        }
+      }
+      const unsigned long long mask = __ballot(to_near);
+      if (mask) {
+        const int leader = __ffsll((long long)mask) - 1;
+        int nb = 0;
+        if (lane == leader)
+          nb = __hip_atomic_fetch_add(&s_cnt[level % 3], __popcll(mask), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        nb = __builtin_amdgcn_readlane(nb, leader);
+        if (to_near) lq.store(p, nb + __popcll(mask & below), v, 0u, dv, true, false);
+      }
+      push_item<false>(to_far, v, nf.far(1 - fi), &s_far[1 - fi], __HIP_MEMORY_SCOPE_WORKGROUP);
+    };
+    if (fn <= bd) {
+      const bool in = (int)threadIdx.x < fn;
+      int v = 0;
+      uint32_t dv = 0;
+      if (in) {
+        v = nf.far(fi)[threadIdx.x];
+        dv = s.dist[v];
+      }
+      const int mn = wave_min_int(in && dv >= t_old ? (int)dv : INT32_MAX);
+      if (lane == 0) atomicMin(&s_far[2], mn);
+      __syncthreads();
+      thr = (uint32_t)__builtin_amdgcn_readfirstlane(s_far[2]) + nf.delta;
+      split(in, v, dv);
+    } else {
+      int mn = INT32_MAX;
+      for (int i = threadIdx.x; i < fn; i += bd) {
+        const uint32_t d = s.dist[nf.far(fi)[i]];
+        if (d >= t_old) mn = min(mn, (int)d);
+      }
+      mn = wave_min_int(mn);
+      if (lane == 0) atomicMin(&s_far[2], mn);
+      __syncthreads();
+      thr = (uint32_t)__builtin_amdgcn_readfirstlane(s_far[2]) + nf.delta;
+      for (int base = 0; base < fn; base += bd) {
+        const int i = base + (int)threadIdx.x;
+        const bool in = i < fn;
+        int v = 0;
+        uint32_t dv = 0;
+        if (in) {
+          v = nf.far(fi)[i];
+          dv = s.dist[v];
+        }
+        split(in, v, dv);
+      }
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      s_far[fi] = 0;
+      s_far[2] = INT32_MAX;
+    }
+    fi = 1 - fi;
+    __syncthreads();
+  }
   for (int d = 32; d > 0; d >>= 1) nrel += __shfl_down(nrel, d, 64);
   if ((threadIdx.x & 63) == 0 && nrel && s.relaxed) atomicAdd(s.relaxed, (unsigned long long)nrel);
   if (threadIdx.x == 0) *iters_out = level;
