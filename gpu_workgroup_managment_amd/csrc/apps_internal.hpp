@@ -30,6 +30,9 @@ struct wgm_graph {
   bool low = false;
   bool low_weights = false;
   uint32_t* ell = nullptr;
+  // PageRank's 16-bit rows (k_near_rows): 0 not looked at yet, 1 there, -1 none
+  int near = 0;
+  uint2* near_rows = nullptr;
   // standalone BFS / SSSP (one team of every participant): two queues of
   // tcap entries with distance tags (SSSP), claim counters, near-far queues
   // and flags

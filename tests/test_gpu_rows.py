@@ -287,3 +287,33 @@ def test_results_arrive_whole(rt, n):
     assert np.array_equal(a, ref) and np.array_equal(b, ref)
     assert st["edges_scanned"] == g.m
     dg.close()
+
+
+def _steps(n, span, seed):
+    """Up to four out-edges a vertex, one of them as long as `span` allows."""
+    rng = np.random.default_rng(seed)
+    src = np.repeat(np.arange(n), rng.integers(0, 5, n))
+    dst = np.clip(src + rng.integers(-min(span, n - 1), min(span, n - 1) + 1, len(src)), 0, n - 1)
+    src, dst = np.append(src, n // 2), np.append(dst, max(n // 2 - span, 0))
+    g = G.from_edges(n, src, dst)
+    keep = np.arange(g.m) - np.repeat(g.row_ptr[:-1], g.degrees()) < 4
+    return G.from_edges(n, np.repeat(np.arange(n), g.degrees())[keep], g.col[keep])
+
+
+@pytest.mark.parametrize("n,span", [(1, 0), (63, 9), (90001, 32767), (90001, 32768), (700001, 5000)])
+def test_pagerank_low_degree(rt, n, span):
+    """Ranks of graphs on both sides of the 16-bit rows' reach, with all of a
+    range's rows in LDS and a part of them, the same bits for every launch
+    shape. A term takes at most four additions, the product with the addition
+    and the division of the contribution: 6 units of 2^-24 an iteration, damped
+    by 0.85."""
+    g = _steps(n, span, 4)
+    ref = oracle.pagerank_f64(g.row_ptr, g.col, 0.85, 30)
+    dg = rt.graph(g)
+    base = None
+    for wg, wgs in ((64, 3), (192, 40), (1024, 1), (1024, 0)):
+        r, _ = dg.pagerank(0.85, 30, wg_size=wg, num_wgs=wgs)
+        assert np.abs(r / ref - 1).max() <= 6 * 2.0 ** -24 / (1 - 0.85)
+        base = r if base is None else base
+        assert np.array_equal(r.view(np.uint32), base.view(np.uint32)), (wg, wgs)
+    dg.close()
