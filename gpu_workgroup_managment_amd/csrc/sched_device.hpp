@@ -89,6 +89,9 @@ __device__ __forceinline__ void sched_unlock(int* m) { st_release(m, 0); }
 
 __device__ __forceinline__ int k_num_groups(const KCtx& k) { return ld_relaxed(k.num_groups); }
 
+// Workgroups besides the scheduler's, in its own mailbox (which no task uses).
+__device__ __forceinline__ int participants(const SchedDev& s) { return ld_relaxed(&s.task_array[0]); }
+
 // ------------------------------------------------------------- get_task
 // Thread 0 spins on this workgroup's mailbox; the restoration context is
 // copied through LDS to every thread (src/scheduler_rt/rt_device/cl_scheduler.cl:31-50).
@@ -157,7 +160,15 @@ __device__ __forceinline__ int offer_fork_thread0(const SchedDev& s, const R& to
   *after = pre;
   if (ld_relaxed(s.available) > 0 && try_lock(s.pool_lock)) {
     const int groups = k_num_groups(s.p);
-    const int snapshot = ld_relaxed(s.available);
+    // Free ids above the persistent range, up to the last workgroup: a member
+    // that returned by itself (a work queue that ran dry) is free too, but its
+    // id lies inside the range, and a mailbox past the last workgroup would be
+    // waited for without end.
+    const int snapshot = min(ld_relaxed(s.available), participants(s) - groups);
+    if (snapshot <= 0) {
+      sched_unlock(s.pool_lock);
+      return pre;
+    }
     for (int i = groups; i < groups + snapshot; i++) {
       s.p.group_ids[i + 1] = i;
       while (ld_relaxed(&s.task_array[(i + 1) * kLine]) != TASK_WAIT) {
@@ -243,6 +254,7 @@ __device__ __forceinline__ bool resize_barrier(const SchedDev& s, int vid, const
 // src/scheduler_rt/rt_device/cl_scheduler.cl:54-64
 __device__ __forceinline__ void scheduler_init(const SchedDev& s, int count) {
   sys_st_release(s.participating, count - 1);
+  st_relaxed(&s.task_array[0], count - 1);
   st_release(s.pool_lock, 0);
   st_release(s.np.executing, 0);
   st_release(s.p.executing, 0);
