@@ -89,5 +89,9 @@ int wgm_enqueue_frontier(wgm_runtime* rt, const wgm::GraphDev& g, wgm::FrontierD
 uint32_t wgm_standalone_delta(int maxdeg);
 int wgm_sssp_pull(wgm_runtime* rt, wgm_graph* g, int32_t src, const wgm_launch* lc, uint32_t* dist_out,
                   wgm_run_stats* st);
-// the graph's in-edge CSR (g->rrow, g->rcol), built once and kept resident
+// the graph's in-edge CSR (g->rrow, g->rcol, g->rwt), built once and kept
+// resident (reverse.hip); the weights padded with zeros to a multiple of kRwtPad
+constexpr int kRwtPad = 256;
 int wgm_graph_in_edges(wgm_graph* g);
+size_t wgm_row_id_words(int32_t n);
+int wgm_row_ids(wgm_graph* g, int32_t* id, int32_t* rows);

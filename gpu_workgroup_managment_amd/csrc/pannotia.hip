@@ -39,7 +39,7 @@ constexpr unsigned long long kBcSlotBytes = 8ull << 30;
 
 // Min-plus graph: the vertices with an in-edge ("rows") numbered in order, the
 // in-edges in row order in blocks of 256, the last one padded.
-constexpr int kMpBlock = 256;
+constexpr int kMpBlock = kRwtPad;
 struct MinplusDev {
   const int32_t* sid;    // row of an edge's source; nrows: a vertex without in-edges, or padding
   const int32_t* wt;
@@ -761,43 +761,6 @@ namespace {
 // Edges of the min-plus graph, padding included.
 int64_t mp_edges(int64_t m) { return (m + kMpBlock - 1) / kMpBlock * kMpBlock; }
 
-// In-edge CSR (sources ascending within a row, the order of
-// parseCOO_transpose's stable sort), built once on the host from the device
-// copy of the graph and kept resident; the weights padded to whole blocks of
-// the min-plus sweeps.
-int graph_reverse(wgm_graph* g) {
-  if (g->rrow) return WGM_OK;
-  wgm_runtime* rt = g->rt;
-  const int32_t n = g->n;
-  const int64_t m = g->m;
-  std::vector<int32_t> rp((size_t)n + 1), col((size_t)m), wt(g->wt ? (size_t)m : 0);
-  HIPCHK(rt, hipMemcpy(rp.data(), g->row_ptr, sizeof(int32_t) * ((size_t)n + 1), hipMemcpyDeviceToHost));
-  if (m) HIPCHK(rt, hipMemcpy(col.data(), g->col, sizeof(int32_t) * (size_t)m, hipMemcpyDeviceToHost));
-  if (g->wt && m) HIPCHK(rt, hipMemcpy(wt.data(), g->wt, sizeof(int32_t) * (size_t)m, hipMemcpyDeviceToHost));
-  std::vector<int32_t> rrow((size_t)n + 1, 0), rcol((size_t)m), rwt(g->wt ? (size_t)mp_edges(m) : 0);
-  for (int64_t e = 0; e < m; e++) rrow[(size_t)col[(size_t)e] + 1]++;
-  for (int32_t v = 0; v < n; v++) rrow[(size_t)v + 1] += rrow[(size_t)v];
-  std::vector<int32_t> pos(rrow.begin(), rrow.end() - 1);
-  for (int32_t u = 0; u < n; u++)
-    for (int32_t e = rp[(size_t)u]; e < rp[(size_t)u + 1]; e++) {
-      const int32_t p = pos[(size_t)col[(size_t)e]]++;
-      rcol[(size_t)p] = u;
-      if (g->wt) rwt[(size_t)p] = wt[(size_t)e];
-    }
-  auto alloc = [&](void** p, size_t bytes) -> int {
-    hipError_t e = hipMalloc(p, bytes ? bytes : 4);
-    return e == hipSuccess ? WGM_OK : wgm_hip_fail(rt, e, "hipMalloc(in-edge CSR)");
-  };
-  int rc = alloc((void**)&g->rrow, sizeof(int32_t) * ((size_t)n + 1));
-  if (!rc) rc = alloc((void**)&g->rcol, sizeof(int32_t) * (size_t)m);
-  if (!rc && g->wt) rc = alloc((void**)&g->rwt, sizeof(int32_t) * rwt.size());
-  if (rc) return rc;
-  HIPCHK(rt, hipMemcpy(g->rrow, rrow.data(), sizeof(int32_t) * ((size_t)n + 1), hipMemcpyHostToDevice));
-  if (m) HIPCHK(rt, hipMemcpy(g->rcol, rcol.data(), sizeof(int32_t) * (size_t)m, hipMemcpyHostToDevice));
-  if (g->wt && m) HIPCHK(rt, hipMemcpy(g->rwt, rwt.data(), sizeof(int32_t) * rwt.size(), hipMemcpyHostToDevice));
-  return WGM_OK;
-}
-
 // Launch of a standalone persistent kernel whose first argument is the
 // control block (*ctl, refreshed after the reset), as the apps launch theirs:
 // grid from the occupancy of `kernel` (capped at max_grid), optional host
@@ -822,29 +785,28 @@ int launch_standalone_app(wgm_runtime* rt, int kernel, const void* fn, const wgm
 
 // The min-plus graph, built once from the in-edge CSR and kept resident.
 int minplus_rows(wgm_graph* g) {
-  int rc = graph_reverse(g);
+  int rc = wgm_graph_in_edges(g);
   if (rc || g->mp_sid) return rc;
   wgm_runtime* rt = g->rt;
   const int32_t n = g->n;
-  std::vector<int32_t> rrow((size_t)n + 1), cid((size_t)n);
-  HIPCHK(rt, hipMemcpy(rrow.data(), g->rrow, sizeof(int32_t) * rrow.size(), hipMemcpyDeviceToHost));
-  int32_t rows = 0;
-  for (int32_t v = 0; v < n; v++) cid[(size_t)v] = rrow[(size_t)v + 1] > rrow[(size_t)v] ? rows++ : -1;
   const size_t edges = (size_t)mp_edges(g->m);
   const int32_t nblk = (int32_t)(edges / kMpBlock);
-  g->mp_rows = rows;
-  g->mp_words = (rows / 32 + 4) / 4 * 4;
   auto alloc = [&](auto** p, size_t count) {
     if (*p) return hipSuccess;  // of an earlier try
     return hipMalloc((void**)p, sizeof(**p) * std::max<size_t>(count, 1));
   };
   int32_t* sid = nullptr;
-  hipError_t e = alloc(&g->mp_cid, (size_t)n);
-  if (e == hipSuccess) e = alloc(&g->mp_start, (size_t)nblk + 1);
+  hipError_t e = alloc(&g->mp_cid, wgm_row_id_words(n));
+  if (e != hipSuccess) return wgm_hip_fail(rt, e, "min-plus graph");
+  int32_t rows = 0;
+  rc = wgm_row_ids(g, g->mp_cid, &rows);
+  if (rc) return rc;
+  g->mp_rows = rows;
+  g->mp_words = (rows / 32 + 4) / 4 * 4;
+  e = alloc(&g->mp_start, (size_t)nblk + 1);
   if (e == hipSuccess) e = alloc(&g->mp_roff, edges);
   if (e == hipSuccess) e = alloc(&g->mp_d, (size_t)rows + 1);
   if (e == hipSuccess) e = alloc(&g->mp_bits, 3 * (size_t)g->mp_words);
-  if (e == hipSuccess) e = hipMemcpy(g->mp_cid, cid.data(), sizeof(int32_t) * cid.size(), hipMemcpyHostToDevice);
   if (e == hipSuccess) e = alloc(&sid, edges);
   if (e != hipSuccess) return wgm_hip_fail(rt, e, "min-plus graph");
   g->mp_sid = sid;
@@ -981,8 +943,6 @@ int run_minplus(wgm_runtime* rt, wgm_graph* g, int32_t src, int32_t big, const w
 
 }  // namespace
 
-int wgm_graph_in_edges(wgm_graph* g) { return graph_reverse(g); }
-
 static int bc_stage(int wg) { return (int)bc_stage_bytes(wg); }
 
 bool wgm_pannotia_kernel_info(int kernel, KernelInfo* out) {
@@ -1042,7 +1002,7 @@ int wgm_bc(wgm_runtime* rt, wgm_graph* g, int32_t num_sources, const wgm_launch*
   if (!rt || !g || g->rt != rt) return fail(rt, WGM_ERR_INVALID, "bad runtime/graph");
   if (num_sources > g->n) return fail(rt, WGM_ERR_INVALID, "%d sources for %d vertices", num_sources, g->n);
   const int32_t nsrc = num_sources > 0 ? num_sources : g->n;
-  int rc = graph_reverse(g);
+  int rc = wgm_graph_in_edges(g);
   if (rc) return rc;
   int grid = 0, wg = 0;
   rc = bc_grid(rt, g, lc, &grid, &wg);

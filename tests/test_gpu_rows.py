@@ -317,3 +317,19 @@ def test_pagerank_low_degree(rt, n, span):
         base = r if base is None else base
         assert np.array_equal(r.view(np.uint32), base.view(np.uint32)), (wg, wgs)
     dg.close()
+
+
+@pytest.mark.parametrize("n,m", [(1, 40000), (250, 32768), (257, 32767), (65537, 90000), (70001, 300007)])
+def test_in_edges(rt, n, m):
+    """The in-edge CSR of one, two and three sort passes, partial tiles and
+    groups of tiles: betweenness needs its order bit for bit, the min-plus sweeps
+    the weights beside it."""
+    rng = np.random.default_rng(n)
+    row = np.concatenate([[0], np.cumsum(np.bincount(rng.integers(0, n, m), minlength=n))]).astype(np.int32)
+    g = G.CSR(row, (rng.integers(0, n, m) ** 2 % n).astype(np.int32), rng.integers(0, 256, m).astype(np.int32))
+    dg = rt.graph(g)
+    d, _ = dg.sssp_minplus(n // 2)
+    assert np.array_equal(d, oracle.sssp_minplus(g.row_ptr, g.col, g.wt, n // 2)[0])
+    b, _ = dg.bc(min(n, 9))
+    assert np.array_equal(b, oracle.bc(g.row_ptr, g.col, min(n, 9))[0])
+    dg.close()
