@@ -13,7 +13,6 @@
 #include "low_degree.hpp"
 
 #include <algorithm>
-#include <cstdlib>
 #include <cstring>
 
 using namespace wgm;
@@ -93,15 +92,21 @@ __global__ void __launch_bounds__(1024) k_low(Ctl c, GraphDev g, FrontierDev s, 
 }
 
 // Packed rows of a low-degree graph: kLowDegree words a vertex, (target << 8) |
-// weight, kEllNone past the degree.
-__global__ void k_low_rows(GraphDev g, uint32_t* ell) {
+// weight, kEllNone past the degree. *flags: bit 0 where an edge spans more than
+// kLowSpan of more than kLowAnySpan vertices, bit 1 where a weight does not fit.
+__global__ void k_low_rows(GraphDev g, uint32_t* ell, int* flags) {
+  int bad = 0;
   for (int v = blockIdx.x * blockDim.x + threadIdx.x; v < g.n; v += gridDim.x * blockDim.x) {
     const int beg = g.row_ptr[v], deg = g.row_ptr[v + 1] - beg;
 #pragma unroll
-    for (int k = 0; k < kLowDegree; k++)
-      ell[(size_t)v * kLowDegree + k] =
-          k < deg ? ((uint32_t)g.col[beg + k] << 8) | (g.wt ? (uint32_t)g.wt[beg + k] & 255u : 0u) : kEllNone;
+    for (int k = 0; k < kLowDegree; k++) {
+      const int u = k < deg ? g.col[beg + k] : v, d = u > v ? u - v : v - u;
+      const uint32_t w = k < deg && g.wt ? (uint32_t)g.wt[beg + k] : 0u;
+      bad |= (g.n > kLowAnySpan && min(d, g.n - d) > kLowSpan ? 1 : 0) | (w > 255u ? 2 : 0);
+      ell[(size_t)v * kLowDegree + k] = k < deg ? ((uint32_t)u << 8) | (w & 255u) : kEllNone;
+    }
   }
+  if (bad) __hip_atomic_fetch_or(flags, bad, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // Colouring without rounds. The rounds give a vertex the colour 1 + the
@@ -554,22 +559,6 @@ int wgm_graph_create(wgm_runtime* rt, const wgm_csr* h, const uint32_t* prio, wg
   g->n = h->n;
   g->m = h->m;
   g->maxdeg = maxdeg;
-  int32_t lo = 0, hi = 0;
-  for (int64_t e = 0; h->wt && e < h->m; e++) {
-    lo = std::min(lo, h->wt[e]);
-    hi = std::max(hi, h->wt[e]);
-  }
-  g->wild_weights = lo < 0 || hi > INT32_MAX - (int32_t)kInf;
-  if (maxdeg <= kLowDegree && h->n <= kLowMaxN) {
-    int32_t span = 0;
-    for (int32_t v = 0; h->n > kLowAnySpan && v < h->n; v++)
-      for (int32_t e = h->row_ptr[v], end = h->row_ptr[v + 1]; e < end; e++) {
-        const int32_t d = std::abs(h->col[e] - v);
-        span = std::max(span, std::min(d, h->n - d));
-      }
-    g->low = span <= kLowSpan;
-    g->low_weights = g->low && h->wt && lo >= 0 && hi <= 255;
-  }
   auto bail = [&](int rc) { wgm_graph_destroy(g); return rc; };
   int rc = dev_alloc(rt, &g->row_ptr, (size_t)h->n + 1);
   if (!rc) rc = dev_alloc(rt, &g->col, (size_t)h->m);
@@ -642,13 +631,28 @@ int wgm_launch_frontier(wgm_runtime* rt, const GraphDev& g, FrontierDev s, const
   return rc ? rc : wgm_finish_app(rt, handshake, out, st);
 }
 
-// The packed rows of a low-degree graph, laid out once.
+// The packed rows of a low-degree graph, laid out once, and whether BFS and the
+// push SSSP take them (g->low, g->low_weights).
 static int low_rows(wgm_runtime* rt, wgm_graph* g) {
-  if (g->ell) return WGM_OK;
+  if (g->low_known) return WGM_OK;
+  if (g->maxdeg > kLowDegree || g->n > kLowMaxN) {
+    g->low_known = true;
+    return WGM_OK;
+  }
   int rc = dev_alloc(rt, &g->ell, (size_t)kLowDegree * (size_t)g->n);
   if (rc) return rc;
-  hipLaunchKernelGGL(k_low_rows, dim3(256), dim3(256), 0, rt->stream, wgm_graph_view(g), g->ell);
-  HIPCHK(rt, hipGetLastError());
+  int flags = 0;
+  HIPCHK(rt, hipMemcpyAsync(g->iters, &flags, sizeof(int), hipMemcpyHostToDevice, rt->stream));
+  hipLaunchKernelGGL(k_low_rows, dim3(256), dim3(256), 0, rt->stream, wgm_graph_view(g), g->ell, g->iters);
+  HIPCHK(rt, hipMemcpyAsync(&flags, g->iters, sizeof(int), hipMemcpyDeviceToHost, rt->stream));
+  HIPCHK(rt, hipStreamSynchronize(rt->stream));
+  g->low = !(flags & 1);
+  g->low_weights = !flags && g->wt;
+  g->low_known = true;
+  if (!g->low) {
+    (void)hipFree(g->ell);
+    g->ell = nullptr;
+  }
   return WGM_OK;
 }
 
@@ -690,12 +694,11 @@ static int run_frontier(wgm_runtime* rt, wgm_graph* g, int32_t src, const wgm_la
   int grid = 0;
   rc = wgm_resolve_grid(rt, kernel, wg, lc ? lc->num_wgs : 0, &grid);
   if (rc) return rc;
+  rc = low_rows(rt, g);
+  if (rc) return rc;
   const bool low = sssp ? g->low_weights : g->low;
   GraphDev view = wgm_graph_view(g);
-  if (low) {
-    rc = low_rows(rt, g);
-    if (rc) return rc;
-  } else if (!sssp) {
+  if (!sssp && !low) {
     // BFS takes its wide levels bottom-up over the in-edges
     rc = wgm_graph_in_edges(g);
     if (rc) return rc;

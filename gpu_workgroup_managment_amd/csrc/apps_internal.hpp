@@ -25,8 +25,9 @@ struct wgm_graph {
   float* f2 = nullptr;
   int* iters = nullptr;
   int32_t* wl = nullptr;  // colour / MIS worklists, PageRank's long rows (wl_words in apps.hip)
-  // low-degree graphs (k_low): BFS may run on one workgroup; the weights also
-  // fit the packed rows; the rows, laid out on first use
+  // low-degree graphs (k_low), looked at on first use: BFS may run on one
+  // workgroup; the weights also fit the packed rows; the rows
+  bool low_known = false;
   bool low = false;
   bool low_weights = false;
   uint32_t* ell = nullptr;
