@@ -307,26 +307,20 @@ __global__ void k_minplus_starts(const int32_t* rrow, const int32_t* cid, int n,
   if (blockIdx.x == 0 && threadIdx.x == 0) bstart[nblk] = nrows;
 }
 
-// Rows of the edges and of their sources; one wave a vertex. *wild: 1 where a
+// Rows of the edges and of their sources, padding included. *wild: 1 where a
 // weight is negative, or wraps when added to an unreached distance.
 __global__ void k_minplus_edges(const int32_t* rrow, const int32_t* rcol, const int32_t* rwt, const int32_t* cid,
                                 const int32_t* bstart, int n, int nblk, int nrows, int32_t* sid, uint8_t* roff,
                                 int* wild) {
   bool bad = false;
-  const int waves = (int)(gridDim.x * blockDim.x) >> 6, lane = (int)threadIdx.x & 63;
-  for (int v = (int)(blockIdx.x * blockDim.x + threadIdx.x) >> 6; v < n; v += waves)
-    for (int e = rrow[v] + lane; e < rrow[v + 1]; e += 64) {
-      const int c = cid[rcol[e]];
-      sid[e] = c < 0 ? nrows : c;
-      roff[e] = (uint8_t)(cid[v] - bstart[e / kMpBlock]);
-      bad |= (uint32_t)rwt[e] > (uint32_t)(INT32_MAX - (int32_t)kInf);
-    }
+  const int64_t m = rrow[n], stride = (int64_t)gridDim.x * blockDim.x;
+  for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < (int64_t)nblk * kMpBlock; e += stride) {
+    const int c = e < m ? cid[rcol[e]] : -1;
+    sid[e] = c < 0 ? nrows : c;
+    roff[e] = e < m ? (uint8_t)(cid[row_of(rrow, n, e)] - bstart[e / kMpBlock]) : 0;
+    bad |= e < m && (uint32_t)rwt[e] > (uint32_t)(INT32_MAX - (int32_t)kInf);
+  }
   if (bad) st_relaxed(wild, 1);
-  if (blockIdx.x == 0)
-    for (long long e = (long long)rrow[n] + threadIdx.x; e < (long long)nblk * kMpBlock; e += blockDim.x) {
-      sid[e] = nrows;
-      roff[e] = 0;
-    }
 }
 
 struct BcDev {
@@ -816,7 +810,7 @@ int minplus_rows(wgm_graph* g) {
   int wild = 0;
   e = hipMemcpyAsync(g->iters, &wild, sizeof(int), hipMemcpyHostToDevice, rt->stream);
   hipLaunchKernelGGL(k_minplus_starts, dim3(1024), dim3(256), 0, rt->stream, g->rrow, g->mp_cid, n, nblk, rows, g->mp_start);
-  hipLaunchKernelGGL(k_minplus_edges, dim3(1024), dim3(256), 0, rt->stream, g->rrow, g->rcol, g->rwt, g->mp_cid,
+  hipLaunchKernelGGL(k_minplus_edges, dim3(4096), dim3(256), 0, rt->stream, g->rrow, g->rcol, g->rwt, g->mp_cid,
                      g->mp_start, n, nblk, rows, sid, g->mp_roff, g->iters);
   if (e == hipSuccess) e = hipGetLastError();
   if (e == hipSuccess) e = hipMemcpyAsync(&wild, g->iters, sizeof(int), hipMemcpyDeviceToHost, rt->stream);

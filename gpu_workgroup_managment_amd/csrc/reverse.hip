@@ -19,7 +19,7 @@ namespace wgm {
 // passes): 174 -> 3.0 ms with all allocations (by counting on the host between
 // two copies before); RMAT 17: 7.9 -> 0.48; ER 2^16 of degree 16: 3.8 -> 0.31.
 constexpr int kSortWg = 1024;
-constexpr int kSortPer = 8;                      // edges a thread takes in turn
+constexpr int kSortPer = 16;                     // edges a thread takes in turn
 constexpr int kSortTile = kSortWg * kSortPer;
 constexpr int kSortBits = 8;                     // digit width, at most
 constexpr int kSortBins = 1 << kSortBits;
@@ -30,11 +30,10 @@ struct SortEdges {
   int32_t* wt;   // null: unweighted
 };
 
-// Source of every out-edge; one wave a vertex.
-__global__ void k_sort_sources(const int32_t* row_ptr, int n, int32_t* src) {
-  const int waves = (int)(gridDim.x * blockDim.x) >> 6, lane = (int)threadIdx.x & 63;
-  for (int v = (int)(blockIdx.x * blockDim.x + threadIdx.x) >> 6; v < n; v += waves)
-    for (int e = row_ptr[v] + lane; e < row_ptr[v + 1]; e += 64) src[e] = v;
+// Source of every out-edge.
+__global__ void k_sort_sources(const int32_t* row_ptr, int n, int64_t m, int32_t* src) {
+  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+  for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < m; e += stride) src[e] = row_of(row_ptr, n, e);
 }
 
 __global__ void __launch_bounds__(kSortWg) k_sort_count(const int32_t* key, int64_t m, int shift, int mask, int* counts) {
@@ -192,7 +191,7 @@ bool reverse_on_device(wgm_graph* g, int32_t* rrow, int32_t* rcol, int32_t* rwt,
   // sources of the first lie where the second writes
   SortEdges a{p, rcol, rwt}, b{p + m, p + 2 * m, g->wt ? p + 3 * m : nullptr};
   SortEdges in{g->col, passes % 2 ? b.src : a.src, g->wt}, out = passes % 2 ? a : b;
-  hipLaunchKernelGGL(k_sort_sources, dim3(1024), dim3(256), 0, st, g->row_ptr, n, in.src);
+  hipLaunchKernelGGL(k_sort_sources, dim3(4096), dim3(256), 0, st, g->row_ptr, n, m, in.src);
   for (int k = 0; k < passes; k++) {
     const int shift = k * digit;
     hipLaunchKernelGGL(k_sort_count, dim3(nb), dim3(kSortWg), 0, st, in.key, m, shift, (1 << digit) - 1, counts);
