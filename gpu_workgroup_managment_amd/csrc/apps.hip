@@ -381,7 +381,7 @@ int launch_prologue(wgm_runtime* rt, int kernel, const wgm_launch* lc, int* grid
   wgm_launch def{256, 0, 0, 0};
   const wgm_launch& l = lc ? *lc : def;
   *wg = l.wg_size > 0 ? l.wg_size : 256;
-  int rc = wgm_resolve_grid(rt, kernel, *wg, l.num_wgs, grid);
+  int rc = wgm_resolve_resident(rt, kernel, *wg, l.num_wgs, grid);
   if (rc) return rc;
   rc = wgm_reset_ctl(rt, 0, l.handshake ? 1 : 0);
   if (rc) return rc;
@@ -692,7 +692,7 @@ static int run_frontier(wgm_runtime* rt, wgm_graph* g, int32_t src, const wgm_la
   const int kernel = sssp ? WGM_K_SSSP : WGM_K_BFS;
   const int wg = lc && lc->wg_size > 0 ? lc->wg_size : 256;
   int grid = 0;
-  rc = wgm_resolve_grid(rt, kernel, wg, lc ? lc->num_wgs : 0, &grid);
+  rc = wgm_resolve_resident(rt, kernel, wg, lc ? lc->num_wgs : 0, &grid);
   if (rc) return rc;
   rc = low_rows(rt, g);
   if (rc) return rc;

@@ -928,8 +928,8 @@ int wgm_batch_run_standalone(wgm_runtime* rt, wgm_batch* b, const wgm_launch* lc
   if (!rt || !b || b->rt != rt) return fail(rt, WGM_ERR_INVALID, "bad runtime/batch");
   const int wg = lc && lc->wg_size > 0 ? lc->wg_size : 1024;
   int grid_bfs = 0, grid_sssp = 0;
-  int rc = wgm_resolve_grid(rt, WGM_K_BFS, wg, lc ? lc->num_wgs : 0, &grid_bfs);
-  if (!rc && b->weighted) rc = wgm_resolve_grid(rt, WGM_K_SSSP, wg, lc ? lc->num_wgs : 0, &grid_sssp);
+  int rc = wgm_resolve_resident(rt, WGM_K_BFS, wg, lc ? lc->num_wgs : 0, &grid_bfs);
+  if (!rc && b->weighted) rc = wgm_resolve_resident(rt, WGM_K_SSSP, wg, lc ? lc->num_wgs : 0, &grid_sssp);
   if (rc) return rc;
   if (b->jobs.empty()) {  // a job table (queue and far-queue offsets) is needed, in any order
     wgm_batch_config cfg;

@@ -15,6 +15,7 @@
 #include "apps_internal.hpp"
 #include "team_frontier.hpp"
 
+#include <algorithm>
 #include <mutex>
 
 using namespace wgm;
@@ -71,20 +72,20 @@ int wgm_bfs_noalloc(wgm_runtime* rt, const int32_t* row_ptr, const int32_t* col,
   const int wg = lc && lc->wg_size > 0 ? lc->wg_size : 256;
   int rc = wgm_check_wg(rt, wg);
   if (rc) return rc;
-  // grid: the caller's, else an occupancy this runtime discovered earlier for
-  // the BFS kernel at this size, else the HIP occupancy bound (discovery then
-  // drops the workgroups that are not co-resident); no cache is filled here
+  // grid: the caller's, as far as it can be resident, else an occupancy this
+  // runtime discovered earlier for the BFS kernel at this size, else the HIP
+  // occupancy bound (discovery then drops the workgroups that are not
+  // co-resident); no cache is filled here
   int grid = lc && lc->num_wgs > 0 ? lc->num_wgs : 0;
-  if (grid <= 0) {
-    auto it = rt->disc_cache.find(WGM_K_BFS * 17 + wg / 64);
-    if (it != rt->disc_cache.end()) {
-      grid = it->second;
-    } else {
-      int per_cu = 0;
-      WGM_HIPCHK(rt, hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, wgm_kernel_info(WGM_K_BFS).fn, wg,
-                                                                  wgm_kernel_lds(WGM_K_BFS, wg)));
-      grid = per_cu * rt->info.num_cus;
-    }
+  if (grid > rt->max_grid) return wgm_fail(rt, WGM_ERR_INVALID, "grid %d out of range", grid);
+  auto it = rt->disc_cache.find(WGM_K_BFS * 17 + wg / 64);
+  if (grid <= 0 && it != rt->disc_cache.end()) {
+    grid = it->second;
+  } else if (grid <= 0 || grid > rt->info.num_cus) {
+    int per_cu = 0;
+    WGM_HIPCHK(rt, hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, wgm_kernel_info(WGM_K_BFS).fn, wg,
+                                                                wgm_kernel_lds(WGM_K_BFS, wg)));
+    grid = grid <= 0 ? per_cu * rt->info.num_cus : std::min(grid, per_cu * rt->info.num_cus);
   }
   if (grid < 1 || grid > rt->max_grid) return wgm_fail(rt, WGM_ERR_INVALID, "grid %d out of range", grid);
   int* lines = (int*)base;

@@ -228,6 +228,17 @@ int wgm_resolve_grid(wgm_runtime* rt, int kernel, int wg_size, int requested, in
   return WGM_OK;
 }
 
+// As above, but no more than the HIP occupancy bound where more are requested:
+// the others could not take part and would only cost the discovery window (BFS,
+// ER 2^16, 512 x 1024 asked of the 256 that fit: 1080 us for 81).
+int wgm_resolve_resident(wgm_runtime* rt, int kernel, int wg_size, int requested, int* grid) {
+  int per_cu = 0;
+  int rc = wgm_resolve_grid(rt, kernel, wg_size, requested, grid);
+  if (!rc) rc = wgm_occupancy(rt, kernel, wg_size, &per_cu);
+  if (!rc) *grid = std::min(*grid, per_cu * rt->info.num_cus);
+  return rc;
+}
+
 // Bounded host wait on a coherent host cell.
 bool wgm_wait_cell(const int* cell, int value, bool equal, double timeout_s) {
   const auto t0 = std::chrono::steady_clock::now();
@@ -395,7 +406,7 @@ int wgm_finish_app(wgm_runtime* rt, int handshake, const AppOut& out, wgm_run_st
   double host_ms = 0.0;
   if (handshake) rc = wgm_host_handshake(rt, &host_ms);
   HIPCHK(rt, hipEventRecord(rt->ev1, rt->stream));
-  const int blocks = out.reached ? std::min(256, out.g.n / 1024 + 1) : 1;
+  const int blocks = out.reached ? std::min(1024, out.g.n / 1024 + 1) : 1;
   hipLaunchKernelGGL(k_finish, dim3(blocks), dim3(256), 0, rt->stream, rt->ctl, out.g, out.reached, out.iters, out.extra,
                      rt->report_dev());
   HIPCHK(rt, hipGetLastError());

@@ -87,6 +87,7 @@ int wgm_check_wg(wgm_runtime* rt, int wg_size);
 int wgm_reset_ctl(wgm_runtime* rt, int im_exit, int handshake);
 int wgm_occupancy(wgm_runtime* rt, int kernel, int wg_size, int* per_cu);
 int wgm_resolve_grid(wgm_runtime* rt, int kernel, int wg_size, int requested, int* grid);
+int wgm_resolve_resident(wgm_runtime* rt, int kernel, int wg_size, int requested, int* grid);
 int wgm_host_handshake(wgm_runtime* rt, double* host_ms);
 int wgm_finish_launch(wgm_runtime* rt, wgm_run_stats* st);
 int wgm_finish_app(wgm_runtime* rt, int handshake, const AppOut& out, wgm_run_stats* st, unsigned long long* extra = nullptr);
