@@ -16,8 +16,8 @@ namespace wgm {
 // workgroup's waves by a prefix over their counts, so the order within a digit
 // is kept. Bound: 28 bytes an edge and pass, written in runs of a tile's edges
 // of a digit. First BFS of a graph, RMAT scale 20 (1.6e7 weighted edges, three
-// passes): 174 -> 3.0 ms with all allocations (by counting on the host between
-// two copies before); RMAT 17: 7.9 -> 0.48; ER 2^16 of degree 16: 3.8 -> 0.31.
+// passes): 174 -> 2.0 ms with all allocations (by counting on the host between
+// two copies before); RMAT 17: 7.9 -> 0.40; ER 2^16 of degree 16: 3.8 -> 0.36.
 constexpr int kSortWg = 1024;
 constexpr int kSortPer = 16;                     // edges a thread takes in turn
 constexpr int kSortTile = kSortWg * kSortPer;

@@ -367,28 +367,37 @@ int stage_drain(wgm_runtime* rt, void* dst, size_t bytes) {
 }  // namespace
 
 // The report of a standalone launch: the cells it left, and the out-edges of
-// the reached vertices. The sum and the count of finished workgroups lie in the
-// last two control lines, which the reset clears and no standalone kernel uses.
-__global__ void k_finish(Ctl c, GraphDev g, const uint32_t* reached, const int* iters, const unsigned long long* extra,
-                         AppReport* out) {
-  unsigned long long* sum = (unsigned long long*)&c.lines[(kNumLines - 2) * kLine];
+// the reached vertices. Their sum and, above it, the count of workgroups that
+// have added to it are one word of the last control line, which the reset
+// clears and no standalone kernel uses: one atomic a workgroup, and few
+// workgroups, since these are performed one after the other (10^6 vertices: 29
+// us with 1024 workgroups and two atomics each, 15 with 256, 6.6 here).
+constexpr int kFinishWgs = 64;
+constexpr int kFinishShift = 40;
+__global__ void __launch_bounds__(1024) k_finish(Ctl c, GraphDev g, const uint32_t* reached, const int* iters,
+                                                 const unsigned long long* extra, AppReport* out) {
+  unsigned long long* cell = (unsigned long long*)&c.lines[(kNumLines - 1) * kLine];
   __shared__ unsigned long long s_part;
   if (threadIdx.x == 0) s_part = 0;
   __syncthreads();
   if (reached) {
     unsigned long long local = 0;
-    for (int v = blockIdx.x * blockDim.x + threadIdx.x; v < g.n; v += gridDim.x * blockDim.x)
-      if (reached[v] != kInf) local += (unsigned long long)(g.row_ptr[v + 1] - g.row_ptr[v]);
+    const int stride = (int)(gridDim.x * blockDim.x);
+#pragma unroll 4
+    for (int v = (int)(blockIdx.x * blockDim.x + threadIdx.x); v < g.n; v += stride) {
+      const int deg = g.row_ptr[v + 1] - g.row_ptr[v];
+      local += reached[v] != kInf ? (unsigned long long)deg : 0ull;
+    }
     for (int d = 32; d > 0; d >>= 1) local += __shfl_down(local, d, 64);
     if ((threadIdx.x & 63) == 0 && local) atomicAdd(&s_part, local);
   }
   __syncthreads();
   if (threadIdx.x) return;
-  if (s_part) atomicAdd(sum, s_part);
-  if (add_acq_rel(&c.lines[(kNumLines - 1) * kLine], 1) != (int)gridDim.x - 1) return;
+  const unsigned long long before = atomicAdd(cell, (1ull << kFinishShift) + s_part);
+  if ((before >> kFinishShift) != gridDim.x - 1) return;
   out->clock[0] = c.clock[0];
   out->clock[1] = c.clock[1];
-  out->edges = __hip_atomic_load(sum, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  out->edges = (before & ((1ull << kFinishShift) - 1)) + s_part;
   out->extra = extra ? *extra : 0ull;
   out->count = *c.count;
   out->iters = iters ? *iters : 0;
@@ -406,8 +415,8 @@ int wgm_finish_app(wgm_runtime* rt, int handshake, const AppOut& out, wgm_run_st
   double host_ms = 0.0;
   if (handshake) rc = wgm_host_handshake(rt, &host_ms);
   HIPCHK(rt, hipEventRecord(rt->ev1, rt->stream));
-  const int blocks = out.reached ? std::min(1024, out.g.n / 1024 + 1) : 1;
-  hipLaunchKernelGGL(k_finish, dim3(blocks), dim3(256), 0, rt->stream, rt->ctl, out.g, out.reached, out.iters, out.extra,
+  const int blocks = out.reached ? std::min(kFinishWgs, out.g.n / 4096 + 1) : 1;
+  hipLaunchKernelGGL(k_finish, dim3(blocks), dim3(out.reached ? 1024 : 64), 0, rt->stream, rt->ctl, out.g, out.reached, out.iters, out.extra,
                      rt->report_dev());
   HIPCHK(rt, hipGetLastError());
   std::unique_lock<std::mutex> lock(rt->stage.mu, std::defer_lock);
