@@ -601,14 +601,11 @@ int64_t wgm_graph_bytes(const wgm_graph* g) {
 
 }  // extern "C"
 
-// The standalone frontier kernel on any state: prologue (grid, control
-// reset, start event), launch on `grid` workgroups of `wg` threads, then the
-// finish (HIP event time, device clock, participants); *iters_dev is the
-// device cell the kernel writes its level count to. Allocates nothing.
 uint32_t wgm_standalone_delta(int maxdeg) { return maxdeg > 4 ? kStandaloneDeltaHighDegree : kStandaloneDelta; }
 
-// Enqueue the standalone frontier kernel (no wait): chunked claims of one
-// workgroup's width, heavy entries above heavy_threshold(wg).
+// Enqueue the standalone frontier kernel (no wait, nothing allocated): chunked
+// claims of one workgroup's width, heavy entries above heavy_threshold(wg);
+// *iters_dev is the device cell the kernel writes its level count to.
 int wgm_enqueue_frontier(wgm_runtime* rt, const GraphDev& g, FrontierDev s, const NearFar& nf, bool sssp, int src,
                          int grid, int wg, int* iters_dev) {
   s.chunk = wg;  // frontier entries a workgroup claims at a time
