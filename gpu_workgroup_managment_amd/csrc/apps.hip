@@ -235,13 +235,21 @@ __global__ void __launch_bounds__(1024) k_mis(Ctl c, GraphDev g, int32_t* st, in
   standalone_retire(c);
 }
 
-// LONG: the graph has rows of more than kTopoEdges edges, which go on wl, two
-// lists of n entries. Both forms share one resource class (64 VGPRs, no
-// scratch): the grid is sized on the form without.
+// LONG: the graph has rows of more than kTopoEdges edges, which go on lists. A
+// workgroup whose range's row starts, columns and lists fit `words` words of
+// dynamic LDS holds them there for all iterations (a barrier leaves nothing of
+// them in the caches, and each was a load that the next waited for); the
+// others read them from memory, the lists from wl, two of n entries. Whole
+// calls of 50 iterations, memory -> LDS: symmetrised RMAT scale 17 ef 16, 512 x
+// 1024, 1255 -> 1098 us; ER n = 131072 of degree 8, 64 x 1024, 1127 -> 833; RMAT
+// scale 19, whose ranges do not fit, 4054 -> 3994. Both forms
+// share one resource class (64 VGPRs, no scratch): the grid is sized on the form
+// without.
 template <bool LONG>
 __global__ void __launch_bounds__(1024, 8) k_pagerank(Ctl c, GraphDev g, float* c0, float* c1, float* rank,
                                                    float damping, float base, float r0, int iters, int32_t* wl,
-                                                   int* iters_out) {
+                                                   int words, int* iters_out) {
+  extern __shared__ __attribute__((aligned(16))) int lds_pr[];
   __shared__ int s_range[2];
   __shared__ int s_cnt[3];
   __shared__ float s_seg[kPrSegs];
@@ -251,17 +259,41 @@ __global__ void __launch_bounds__(1024, 8) k_pagerank(Ctl c, GraphDev g, float* 
   if (LONG) {
     if (threadIdx.x < 3) s_cnt[threadIdx.x] = 0;
     balanced_range(g, t.id, t.n, s_range, &lo, &hi);
-    pagerank_lists(g, lo, hi, wl, wl + g.n, s_cnt);
   } else {
     block_range(g.n, t.id, t.n, &lo, &hi);
   }
-  pagerank_init(g, c0, r0, lo, hi);
-  xcd_barrier(c, t);
-  for (int it = 0; it < iters; it++) {
-    const float* cin = (it & 1) ? c1 : c0;
-    float* cout = (it & 1) ? c0 : c1;
-    pagerank_pass<LONG>(g, cin, cout, rank, damping, base, it == iters - 1, lo, hi, wl, wl + g.n, s_cnt, s_seg);
+  auto run = [&](const auto& rows) {
     xcd_barrier(c, t);
+    for (int it = 0; it < iters; it++) {
+      const float* cin = (it & 1) ? c1 : c0;
+      float* cout = (it & 1) ? c0 : c1;
+      pagerank_pass<LONG>(rows, cin, cout, rank, damping, base, it == iters - 1, lo, hi, s_cnt, s_seg);
+      xcd_barrier(c, t);
+    }
+  };
+  pagerank_init(g, c0, r0, lo, hi);
+  if constexpr (LONG) {
+    const int nr = hi - lo;
+    const int e0 = __builtin_amdgcn_readfirstlane(g.row_ptr[lo]);
+    const int ne = __builtin_amdgcn_readfirstlane(g.row_ptr[hi]) - e0;
+    const int n2 = ne / kPrSeg;  // rows of more than kPrSeg edges at most
+    if ((long long)ne + 2 * (long long)nr + 1 + n2 <= words) {
+      lds_i32* mem = (lds_i32*)lds_pr;
+      const PrRows<lds_i32*> rows{mem + ne, mem, mem + ne + nr + 1, mem + ne + 2 * nr + 1, lo, 0};
+      const int bd = blockDim.x;
+#pragma unroll 4
+      for (int i = threadIdx.x; i < ne; i += bd) mem[i] = g.col[e0 + i];
+      for (int i = threadIdx.x; i <= nr; i += bd) rows.row_ptr[i] = g.row_ptr[lo + i] - e0;
+      __syncthreads();
+      pagerank_lists(rows, lo, hi, s_cnt);
+      run(rows);
+    } else {
+      const PrRows<int32_t*> rows{(int32_t*)g.row_ptr, (int32_t*)g.col, wl, wl + g.n, 0, lo};
+      pagerank_lists(rows, lo, hi, s_cnt);
+      run(rows);
+    }
+  } else {
+    run(PrRows<const int32_t*>{g.row_ptr, g.col, nullptr, nullptr, 0, 0});
   }
   clock_end(c, t.id);
   if (t.id == 0 && threadIdx.x == 0) *iters_out = iters;
@@ -532,7 +564,7 @@ int wgm_app_probe(wgm_runtime* rt, int kernel, int grid, int wg_size) {
       return WGM_OK;
     case WGM_K_PAGERANK:
       hipLaunchKernelGGL(k_pagerank<false>, dim3(grid), dim3(wg_size), 0, rt->stream, rt->ctl, GraphDev{}, (float*)nullptr,
-                         (float*)nullptr, (float*)nullptr, 0.f, 0.f, 0.f, 0, (int32_t*)nullptr, (int*)nullptr);
+                         (float*)nullptr, (float*)nullptr, 0.f, 0.f, 0.f, 0, (int32_t*)nullptr, 0, (int*)nullptr);
       return WGM_OK;
     default:
       return wgm_pannotia_probe(rt, kernel, grid, wg_size);
@@ -779,11 +811,16 @@ static int near_rows(wgm_runtime* rt, wgm_graph* g) {
   return WGM_OK;
 }
 
+// LDS of a workgroup where 2048 threads of a CU stay resident, or the one
+// workgroup that each CU has.
+static int lds_share(const wgm_runtime* rt, int grid, int wg) {
+  return grid > rt->info.num_cus ? (160 << 10) / (2048 / wg) : 160 << 10;
+}
+
 // Rows that a workgroup holds in LDS: its range, within the share of a CU's 160
 // KB that leaves 2048 threads (or the workgroup each CU has) resident.
 static int near_held(const wgm_runtime* rt, int n, int grid, int wg) {
-  const int lds = (grid > rt->info.num_cus ? (160 << 10) / (2048 / wg) : 160 << 10) - 1536;
-  return std::min(lds / 8, (n + grid - 1) / grid);
+  return std::min((lds_share(rt, grid, wg) - 1536) / 8, (n + grid - 1) / grid);
 }
 
 int wgm_pagerank(wgm_runtime* rt, wgm_graph* g, float damping, int32_t iterations, const wgm_launch* lc,
@@ -807,12 +844,15 @@ int wgm_pagerank(wgm_runtime* rt, wgm_graph* g, float damping, int32_t iteration
     hipLaunchKernelGGL(k_pagerank_near, dim3(grid), dim3(wg), 8 * (size_t)near_held(rt, g->n, grid, wg), rt->stream, rt->ctl,
                        wgm_graph_view(g), g->near_rows, near_held(rt, g->n, grid, wg), g->f0, g->f1, g->f2, damping, base,
                        r0, iterations, g->iters);
-  else if (g->maxdeg > kTopoEdges)
-    hipLaunchKernelGGL(k_pagerank<true>, dim3(grid), dim3(wg), 0, rt->stream, rt->ctl, wgm_graph_view(g), g->f0, g->f1,
-                       g->f2, damping, base, r0, iterations, g->wl, g->iters);
-  else
+  else if (g->maxdeg > kTopoEdges) {
+    // no more than an even share of the rows and edges could need, and a half of that
+    const int64_t even = (g->m + kRowCost * (int64_t)g->n) / grid;
+    const int words = (int)std::min<int64_t>((lds_share(rt, grid, wg) - 3072) / 4, even + even / 2 + 64);
+    hipLaunchKernelGGL(k_pagerank<true>, dim3(grid), dim3(wg), 4 * (size_t)words, rt->stream, rt->ctl, wgm_graph_view(g),
+                       g->f0, g->f1, g->f2, damping, base, r0, iterations, g->wl, words, g->iters);
+  } else
     hipLaunchKernelGGL(k_pagerank<false>, dim3(grid), dim3(wg), 0, rt->stream, rt->ctl, wgm_graph_view(g), g->f0, g->f1,
-                       g->f2, damping, base, r0, iterations, (int32_t*)nullptr, g->iters);
+                       g->f2, damping, base, r0, iterations, (int32_t*)nullptr, 0, g->iters);
   return launch_epilogue(rt, lc, g, g->f2, rank_out, st);
 }
 

@@ -1177,18 +1177,31 @@ __device__ __forceinline__ void pagerank_iter(const GraphDev& g, const float* ci
 // flight), the lanes' sums meet in a fixed tree and a row's segments are
 // added in a fixed order, so a rank depends on the graph alone, not on the
 // launch shape, and a long row's rounding error is that of a short sum.
-// Bound: the chain of dependent loads of the longest row a workgroup has.
+// Bound: chains of dependent loads, one after another for the classes of rows a
+// wave has, each from beyond the L2 after a barrier: contributions only, where
+// the rest lies in LDS (PrRows). Contributions held in LDS as well, the most
+// read ones first, took longer: their copy is one chain more.
 // Symmetrised RMAT scale 17 ef 16 (3.9 M edges), 50 iterations, 512 x 1024,
-// whole call: 134.1 ms with one thread a row and equal vertex counts, 1.31 ms
+// whole call: 134.1 ms with one thread a row and equal vertex counts, 1.10 ms
 // here; largest relative error against FP64 2.1e-6 there, 4.8e-8 here.
 constexpr int kPrMid = 64;
 constexpr int kPrSeg = 2048;
 constexpr int kPrSegs = 256;  // segment sums in LDS at a time
 
+// Rows as the iterations read them: in memory, or, what a workgroup's range
+// needs, in its LDS (P a pointer there). v0: the row that row_ptr begins with;
+// l0: where the lists of the range begin.
+template <class P>
+struct PrRows {
+  P row_ptr, col, list, list2;
+  int v0, l0;
+};
+typedef __attribute__((address_space(3))) int32_t lds_i32;
+
 // Sum of G lanes' terms cin[col[e]], e = beg + lane, + G, ...; every lane of
 // the group gets the total.
-template <int G>
-__device__ __forceinline__ float pagerank_group_sum(const int32_t* col, const float* cin, int beg, int end, int lane) {
+template <int G, class P>
+__device__ __forceinline__ float pagerank_group_sum(P col, const float* cin, int beg, int end, int lane) {
   float sum = 0.0f;
   int e = beg + lane;
   for (; e + 3 * G < end; e += 4 * G) {
@@ -1215,27 +1228,28 @@ __device__ __forceinline__ float pagerank_group_sum(const int32_t* col, const fl
   return sum;
 }
 
-// This workgroup's long rows: list[lo, lo + cnt[0]) those of up to kPrMid
-// edges, list[hi - cnt[1], hi) those of up to kPrSeg, list2[lo, lo + cnt[2])
-// the rest. s_cnt: three ints of LDS, zeroed by the caller before a barrier.
-__device__ __forceinline__ void pagerank_lists(const GraphDev& g, int lo, int hi, int32_t* list, int32_t* list2,
-                                               int* s_cnt) {
+// This workgroup's long rows: from list[l0] on those of up to kPrMid edges, down
+// from list[l0 + hi - lo - 1] those of up to kPrSeg, from list2[l0] on the rest.
+// s_cnt: three ints of LDS, zeroed by the caller before a barrier.
+template <class P>
+__device__ __forceinline__ void pagerank_lists(const PrRows<P>& rows, int lo, int hi, int* s_cnt) {
   for (int v = lo + (int)threadIdx.x; v < hi; v += blockDim.x) {
-    const int deg = g.row_ptr[v + 1] - g.row_ptr[v];
+    const int deg = rows.row_ptr[v - rows.v0 + 1] - rows.row_ptr[v - rows.v0];
     if (deg <= kTopoEdges) continue;
     const int k = deg <= kPrMid ? 0 : deg <= kPrSeg ? 1 : 2;
     const int i = __hip_atomic_fetch_add(&s_cnt[k], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-    if (k == 0) list[lo + i] = v;
-    else if (k == 1) list[hi - 1 - i] = v;
-    else list2[lo + i] = v;
+    if (k == 0) rows.list[rows.l0 + i] = v;
+    else if (k == 1) rows.list[rows.l0 + hi - lo - 1 - i] = v;
+    else rows.list2[rows.l0 + i] = v;
   }
 }
 
-template <bool LONG>
-__device__ __forceinline__ void pagerank_pass(const GraphDev& g, const float* cin, float* cout, float* rank,
-                                              float damping, float base, bool last, int lo, int hi,
-                                              const int32_t* list, const int32_t* list2, const int* cnt,
+template <bool LONG, class P>
+__device__ __forceinline__ void pagerank_pass(const PrRows<P>& rows, const float* cin, float* cout, float* rank,
+                                              float damping, float base, bool last, int lo, int hi, const int* cnt,
                                               float* s_seg) {
+  const P row_ptr = rows.row_ptr, col = rows.col;
+  const int v0 = rows.v0;
   auto put = [&](int v, float sum, int deg) {
     const float r = __builtin_fmaf(damping, sum, base);
     if (last) rank[v] = r;
@@ -1246,14 +1260,14 @@ __device__ __forceinline__ void pagerank_pass(const GraphDev& g, const float* ci
   if (LONG) {  // the longest chains first
     const int wave = (int)threadIdx.x >> 6, nw = bd >> 6, lane = (int)threadIdx.x & 63;
     for (int i = 0; i < cnt[2]; i++) {
-      const int v = list2[lo + i];
-      const int beg = g.row_ptr[v], end = g.row_ptr[v + 1];
+      const int v = rows.list2[rows.l0 + i];
+      const int beg = row_ptr[v - v0], end = row_ptr[v - v0 + 1];
       float total = 0.0f;
       for (int a = beg; a < end; a += kPrSegs * kPrSeg) {
         const int ns = min(kPrSegs, (end - a + kPrSeg - 1) / kPrSeg);
         for (int s = wave; s < ns; s += nw) {
           const int sb = a + s * kPrSeg;
-          const float x = pagerank_group_sum<64>(g.col, cin, sb, min(sb + kPrSeg, end), lane);
+          const float x = pagerank_group_sum<64>(col, cin, sb, min(sb + kPrSeg, end), lane);
           if (lane == 0) s_seg[s] = x;
         }
         __syncthreads();
@@ -1268,15 +1282,15 @@ __device__ __forceinline__ void pagerank_pass(const GraphDev& g, const float* ci
       if (threadIdx.x == 0) put(v, total, end - beg);
     }
     for (int i = wave; i < cnt[1]; i += nw) {
-      const int v = list[hi - 1 - i];
-      const int beg = g.row_ptr[v], end = g.row_ptr[v + 1];
-      const float x = pagerank_group_sum<64>(g.col, cin, beg, end, lane);
+      const int v = rows.list[rows.l0 + hi - lo - 1 - i];
+      const int beg = row_ptr[v - v0], end = row_ptr[v - v0 + 1];
+      const float x = pagerank_group_sum<64>(col, cin, beg, end, lane);
       if (lane == 0) put(v, x, end - beg);
     }
     for (int i = (int)threadIdx.x >> 3; i < cnt[0]; i += bd >> 3) {
-      const int v = list[lo + i];
-      const int beg = g.row_ptr[v], end = g.row_ptr[v + 1];
-      const float x = pagerank_group_sum<8>(g.col, cin, beg, end, lane & 7);
+      const int v = rows.list[rows.l0 + i];
+      const int beg = row_ptr[v - v0], end = row_ptr[v - v0 + 1];
+      const float x = pagerank_group_sum<8>(col, cin, beg, end, lane & 7);
       if ((lane & 7) == 0) put(v, x, end - beg);
     }
   }
@@ -1286,8 +1300,8 @@ __device__ __forceinline__ void pagerank_pass(const GraphDev& g, const float* ci
     for (int k = 0; k < U; k++) {
       v[k] = b0 + k * bd;
       const bool in = v[k] < hi;
-      beg[k] = in ? g.row_ptr[v[k]] : 0;
-      end[k] = in ? g.row_ptr[v[k] + 1] : 0;
+      beg[k] = in ? row_ptr[v[k] - v0] : 0;
+      end[k] = in ? row_ptr[v[k] - v0 + 1] : 0;
       if (LONG && end[k] - beg[k] > kTopoEdges) v[k] = hi;  // summed above
     }
     int u[U][kTopoEdges];
@@ -1295,7 +1309,7 @@ __device__ __forceinline__ void pagerank_pass(const GraphDev& g, const float* ci
     for (int k = 0; k < U; k++)
 #pragma unroll
       for (int j = 0; j < kTopoEdges; j++)
-        u[k][j] = (!LONG || v[k] < hi) && beg[k] + j < end[k] ? g.col[beg[k] + j] : -1;
+        u[k][j] = (!LONG || v[k] < hi) && beg[k] + j < end[k] ? col[beg[k] + j] : -1;
     float cu[U][kTopoEdges];
 #pragma unroll
     for (int k = 0; k < U; k++)

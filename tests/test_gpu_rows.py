@@ -44,6 +44,34 @@ def test_pagerank_row_classes(rt):
     dg.close()
 
 
+def _hub_graph(n, hubs):
+    """Rows of degree `hubs`, spread evenly, and of up to 12 edges elsewhere."""
+    rng = np.random.default_rng(n)
+    src = [np.full(d, v * (n // len(hubs))) for v, d in enumerate(hubs)]
+    dst = [rng.permutation(n)[:d] for d in hubs]
+    rest = np.repeat(np.arange(n), rng.integers(0, 13, n))
+    to = rng.integers(0, n, len(rest))
+    return G.from_edges(n, np.concatenate(src + [rest]), np.concatenate(dst + [to]))
+
+
+@pytest.mark.parametrize("n,hubs", [
+    (7, (6,)), (1025, (64, 65, 5)), (16383, (2048, 2049, 4096, 4097)), (50001, (50000, 1023, 4)), (300001, (20000, 5)),
+])
+def test_pagerank_held_rows(rt, n, hubs):
+    """Ranges whose rows lie in LDS (many workgroups), in memory (few), and both in one launch (a row longer than the
+    LDS of a workgroup): the same bits, within the bound of the row classes above."""
+    g = _hub_graph(n, hubs)
+    ref = oracle.pagerank_f64(g.row_ptr, g.col, 0.85, 30)
+    dg = rt.graph(g)
+    base = None
+    for wg, wgs in ((64, 3), (64, 0), (192, 40), (1024, 1), (1024, 0), (1024, 300)):
+        r, _ = dg.pagerank(0.85, 30, wg_size=wg, num_wgs=wgs)
+        assert np.abs(r / ref - 1).max() <= 48 * 2.0 ** -24 / (1 - 0.85)
+        base = r if base is None else base
+        assert np.array_equal(r.view(np.uint32), base.view(np.uint32)), (wg, wgs)
+    dg.close()
+
+
 def _symmetric(g):
     return G.from_edges(g.n, np.repeat(np.arange(g.n), g.degrees()), g.col, symmetric=True)
 
