@@ -232,8 +232,8 @@ int64_t wgm_graph_bytes(const wgm_graph* g);
 /* Launch shape of a standalone persistent kernel. */
 typedef struct wgm_launch {
   int32_t wg_size;     /* threads per workgroup (64..1024, multiple of 64) */
-  int32_t num_wgs;     /* <= 0: discovered occupancy; of more than can be resident, as many as can (some apps take
-                          the threads asked for in fewer, larger workgroups) */
+  int32_t num_wgs;     /* <= 0: discovered occupancy, or fewer on small graphs; of more than can be resident, as
+                          many as can (some apps take the threads asked for in fewer, larger workgroups) */
   int32_t handshake;   /* 1: host flag handshake as in the reference's run_persistent */
   int32_t mode;        /* wgm_sssp's relaxation direction: WGM_SSSP_AUTO, _PUSH or _PULL */
 } wgm_launch;
