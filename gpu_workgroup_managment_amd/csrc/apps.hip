@@ -823,20 +823,23 @@ static int near_held(const wgm_runtime* rt, int n, int grid, int wg) {
   return std::min((lds_share(rt, grid, wg) - 1536) / 8, (n + grid - 1) / grid);
 }
 
-// Workgroups of the long-row form where the caller leaves the number open, of the
-// `fit` that can be resident. A barrier costs 6 us with 512 workgroups, 4 with
-// 256, 2.5 with 64, and an iteration of a small graph little else: four edges a
-// thread (a row counts kRowCost), from 65536 threads to half of those that fit;
-// all of them from kPrWide a thread of that half on. Whole calls of 50
-// iterations, all -> by the rule: 1024 threads, ER n = 4097 of degree 8, 434 -> 246
-// us, 30001 of 16, 489 -> 365, 131072 of 8, 647 -> 551; symmetrised RMAT scale 18
-// ef 8, 1257 -> 1316, ef 16 (just past the line) 1568 with half, 1689 with all, scale
-// 19 5290 and 4030; 256 threads, ER 16001 of degree 8, 1161 -> 369.
+// Workgroups where the caller leaves the number open, of the `fit` that can be
+// resident. A barrier costs 6 us with 512 workgroups, 4 with 256, 2.5 with 64, and
+// an iteration of a small graph little else: four units of `cost` a thread, from
+// 65536 threads to half of those that fit; all of them from `wide` a thread of that
+// half on. Units: edges (a row counts kRowCost) of the CSR forms, vertices of
+// k_pagerank_near. Whole calls of 50 iterations, all -> by the rule: 1024 threads,
+// ER n = 4097 of degree 8, 434 -> 246 us, 30001 of 16, 489 -> 365, 131072 of 8, 647
+// -> 551; symmetrised RMAT scale 18 ef 8, 1257 -> 1316, ef 16 (just past the line)
+// 1568 with half, 1689 with all, scale 19 5290 and 4030; 256 threads, ER 16001 of
+// degree 8, 1161 -> 369. Four random edges a vertex, n = 5001: 421 -> 233, 250001:
+// 695 -> 584, 700001: 1173 -> 1090. Meshes, 401^2: 478 -> 299, 1001^2: 692 -> 537,
+// 1401^2: 846 -> 756; 2047^2 (past the line) 1298 with half, 1273 with all.
 constexpr int kPrWide = 32;
-static int pagerank_grid(const wgm_runtime* rt, const wgm_graph* g, int fit, int wg) {
-  const int64_t cost = g->m + kRowCost * (int64_t)g->n;
+constexpr int kPrNearWide = 12;
+static int pagerank_grid(const wgm_runtime* rt, int64_t cost, int wide, int fit, int wg) {
   const int64_t half = (int64_t)rt->info.num_cus * 1024;
-  if (cost > kPrWide * half) return fit;
+  if (cost > wide * half) return fit;
   const int64_t threads = std::min(half, std::max<int64_t>(65536, cost / 4));
   return (int)std::min<int64_t>(fit, (threads + wg - 1) / wg);
 }
@@ -858,14 +861,16 @@ int wgm_pagerank(wgm_runtime* rt, wgm_graph* g, float damping, int32_t iteration
   int grid = 0, wg = 0;
   rc = launch_prologue(rt, WGM_K_PAGERANK, lc, &grid, &wg);
   if (rc) return rc;
+  const int64_t cost = g->m + kRowCost * (int64_t)g->n;
+  if (!lc || lc->num_wgs <= 0)
+    grid = g->near == 1 ? pagerank_grid(rt, g->n, kPrNearWide, grid, wg) : pagerank_grid(rt, cost, kPrWide, grid, wg);
   if (g->near == 1)
     hipLaunchKernelGGL(k_pagerank_near, dim3(grid), dim3(wg), 8 * (size_t)near_held(rt, g->n, grid, wg), rt->stream, rt->ctl,
                        wgm_graph_view(g), g->near_rows, near_held(rt, g->n, grid, wg), g->f0, g->f1, g->f2, damping, base,
                        r0, iterations, g->iters);
   else if (g->maxdeg > kTopoEdges) {
-    if (!lc || lc->num_wgs <= 0) grid = pagerank_grid(rt, g, grid, wg);
     // no more than an even share of the rows and edges could need, and a half of that
-    const int64_t even = (g->m + kRowCost * (int64_t)g->n) / grid;
+    const int64_t even = cost / grid;
     const int words = (int)std::min<int64_t>((lds_share(rt, grid, wg) - 3072) / 4, even + even / 2 + 64);
     hipLaunchKernelGGL(k_pagerank<true>, dim3(grid), dim3(wg), 4 * (size_t)words, rt->stream, rt->ctl, wgm_graph_view(g),
                        g->f0, g->f1, g->f2, damping, base, r0, iterations, g->wl, words, g->iters);
