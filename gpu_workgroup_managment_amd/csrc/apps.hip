@@ -685,6 +685,38 @@ static int low_rows(wgm_runtime* rt, wgm_graph* g) {
   return WGM_OK;
 }
 
+// Workgroups where the caller leaves the number open, of the `fit` that can be
+// resident. A barrier costs 6 us with 512 workgroups, 4 with 256, 2.5 with 64, and
+// a pass over a small graph little else: `each` units of cost a thread, from 65536
+// threads to 262144 on 256 CUs, half of what they hold; all that fit from `wide` a
+// thread of that half on. Units: edges and rows (kRowCost), vertices for
+// k_pagerank_near. Whole calls, all -> by the rule:
+// BFS, 1024 threads: ER n = 4097 of degree 8, 102 -> 94 us, RMAT 131072 ef 16, 148 ->
+// 142; 256 threads: 214 -> 101.
+// MIS, 1024 threads: ER n = 60001 of degree 8, 175 -> 139, 401^2 grid 170 -> 135, 801^2
+// 254 -> 238; 256 threads: ER 395 -> 173.
+// PageRank, 50 iterations, 1024 threads: ER n = 4097 of degree 8, 434 -> 246, 30001
+// of 16, 489 -> 365, 131072 of 8, 647 -> 551; symmetrised RMAT scale 18 ef 8, 1257 ->
+// 1316, ef 16 (just past the line) 1568 with half, 1689 with all, scale 19 5290 and
+// 4030; four random edges a vertex, n = 5001, 421 -> 233, 700001, 1173 -> 1090; meshes,
+// 401^2, 478 -> 299, 1401^2, 846 -> 756, 2047^2 (past the line) 1298 with half, 1273
+// with all; 256 threads, ER 16001 of degree 8, 1161 -> 369.
+struct FitRule {
+  int each, wide;
+};
+constexpr FitRule kFitBfs{16, 1 << 20};
+constexpr FitRule kFitMis{32, 1 << 20};
+constexpr FitRule kFitPr{4, 32};
+constexpr FitRule kFitPrNear{4, 12};
+static int fitted_grid(const wgm_runtime* rt, const wgm_launch* lc, int64_t cost, FitRule rule, int fit, int wg) {
+  if (lc && lc->num_wgs > 0) return fit;
+  const int64_t half = (int64_t)rt->info.num_cus * 1024;
+  if (cost > rule.wide * half) return fit;
+  const int64_t threads = std::min(half, std::max<int64_t>(65536, cost / rule.each));
+  return (int)std::min<int64_t>(fit, (threads + wg - 1) / wg);
+}
+static int64_t rows_and_edges(const wgm_graph* g) { return g->m + kRowCost * (int64_t)g->n; }
+
 // Enqueue k_low: the threads asked for, in workgroups of up to 1024 (one fits a
 // CU beside its LDS).
 static int enqueue_low(wgm_runtime* rt, const wgm_graph* g, const FrontierDev& s, const NearFar& nf, bool sssp, int src,
@@ -726,6 +758,7 @@ static int run_frontier(wgm_runtime* rt, wgm_graph* g, int32_t src, const wgm_la
   rc = low_rows(rt, g);
   if (rc) return rc;
   const bool low = sssp ? g->low_weights : g->low;
+  if (!sssp && !low) grid = fitted_grid(rt, lc, rows_and_edges(g), kFitBfs, grid, wg);
   GraphDev view = wgm_graph_view(g);
   if (!sssp && !low) {
     // BFS takes its wide levels bottom-up over the in-edges
@@ -784,6 +817,7 @@ int wgm_mis(wgm_runtime* rt, wgm_graph* g, const wgm_launch* lc, int32_t* s_out,
   int grid = 0, wg = 0;
   rc = launch_prologue(rt, WGM_K_MIS, lc, &grid, &wg);
   if (rc) return rc;
+  grid = fitted_grid(rt, lc, rows_and_edges(g), kFitMis, grid, wg);
   hipLaunchKernelGGL(g->maxdeg > kTopoEdges ? k_mis<true> : k_mis<false>, dim3(grid), dim3(wg), scan_lds_bytes(wg),
                      rt->stream, rt->ctl, wgm_graph_view(g), g->i32a, g->i32b, (void*)g->wl, g->iters);
   return launch_epilogue(rt, lc, g, g->i32b, s_out, st);
@@ -823,27 +857,6 @@ static int near_held(const wgm_runtime* rt, int n, int grid, int wg) {
   return std::min((lds_share(rt, grid, wg) - 1536) / 8, (n + grid - 1) / grid);
 }
 
-// Workgroups where the caller leaves the number open, of the `fit` that can be
-// resident. A barrier costs 6 us with 512 workgroups, 4 with 256, 2.5 with 64, and
-// an iteration of a small graph little else: four units of `cost` a thread, from
-// 65536 threads to half of those that fit; all of them from `wide` a thread of that
-// half on. Units: edges (a row counts kRowCost) of the CSR forms, vertices of
-// k_pagerank_near. Whole calls of 50 iterations, all -> by the rule: 1024 threads,
-// ER n = 4097 of degree 8, 434 -> 246 us, 30001 of 16, 489 -> 365, 131072 of 8, 647
-// -> 551; symmetrised RMAT scale 18 ef 8, 1257 -> 1316, ef 16 (just past the line)
-// 1568 with half, 1689 with all, scale 19 5290 and 4030; 256 threads, ER 16001 of
-// degree 8, 1161 -> 369. Four random edges a vertex, n = 5001: 421 -> 233, 250001:
-// 695 -> 584, 700001: 1173 -> 1090. Meshes, 401^2: 478 -> 299, 1001^2: 692 -> 537,
-// 1401^2: 846 -> 756; 2047^2 (past the line) 1298 with half, 1273 with all.
-constexpr int kPrWide = 32;
-constexpr int kPrNearWide = 12;
-static int pagerank_grid(const wgm_runtime* rt, int64_t cost, int wide, int fit, int wg) {
-  const int64_t half = (int64_t)rt->info.num_cus * 1024;
-  if (cost > wide * half) return fit;
-  const int64_t threads = std::min(half, std::max<int64_t>(65536, cost / 4));
-  return (int)std::min<int64_t>(fit, (threads + wg - 1) / wg);
-}
-
 int wgm_pagerank(wgm_runtime* rt, wgm_graph* g, float damping, int32_t iterations, const wgm_launch* lc,
                  float* rank_out, wgm_run_stats* st) {
   if (!rt || !g || g->rt != rt) return fail(rt, WGM_ERR_INVALID, "bad runtime/graph");
@@ -861,9 +874,8 @@ int wgm_pagerank(wgm_runtime* rt, wgm_graph* g, float damping, int32_t iteration
   int grid = 0, wg = 0;
   rc = launch_prologue(rt, WGM_K_PAGERANK, lc, &grid, &wg);
   if (rc) return rc;
-  const int64_t cost = g->m + kRowCost * (int64_t)g->n;
-  if (!lc || lc->num_wgs <= 0)
-    grid = g->near == 1 ? pagerank_grid(rt, g->n, kPrNearWide, grid, wg) : pagerank_grid(rt, cost, kPrWide, grid, wg);
+  const int64_t cost = rows_and_edges(g);
+  grid = g->near == 1 ? fitted_grid(rt, lc, g->n, kFitPrNear, grid, wg) : fitted_grid(rt, lc, cost, kFitPr, grid, wg);
   if (g->near == 1)
     hipLaunchKernelGGL(k_pagerank_near, dim3(grid), dim3(wg), 8 * (size_t)near_held(rt, g->n, grid, wg), rt->stream, rt->ctl,
                        wgm_graph_view(g), g->near_rows, near_held(rt, g->n, grid, wg), g->f0, g->f1, g->f2, damping, base,
