@@ -40,7 +40,7 @@ constexpr unsigned long long kBcSlotBytes = 8ull << 30;
 // in-edges in row order in blocks of 256, the last one padded.
 constexpr int kMpBlock = kRwtPad;
 struct MinplusDev {
-  const int32_t* sid;    // row of an edge's source; nrows: a vertex without in-edges, or padding
+  const int32_t* sid;    // row of an edge's source; none: a vertex without in-edges, or padding
   const int32_t* wt;
   const uint8_t* roff;   // row of an edge less the block's first
   const int32_t* bstart; // [nblk + 1] first row of a block; the last one: nrows
@@ -50,6 +50,7 @@ struct MinplusDev {
   const int32_t* owt;    // weights of the out-edges
   int32_t nblk;
   int32_t nrows;
+  int32_t none;          // a row number whose bit of the LDS map no row shares (mp_none)
   int32_t n;
   int32_t src;
   int32_t big;           // distance of an unreached vertex
@@ -58,7 +59,7 @@ struct MinplusDev {
   int32_t shift;         // rows per bit of the LDS map: 1 << shift
   int32_t map_words;
   int32_t bit_words;     // words of one bit set
-  int32_t* d;            // [nrows + 1] distances of the rows; the last one stays at big
+  int32_t* d;            // [nrows + 1] distances of the rows; the last one stays at big (a block's end is read there)
   uint32_t* bits;        // three bit sets: rows lowered in sweep s in set s % 3
   int32_t* dist;         // [n] result
 };
@@ -139,7 +140,7 @@ __device__ __forceinline__ bool minplus_step(const MinplusDev& p, int b, int b1,
   int c0[kMpU + 1];
 #pragma unroll
   for (int u = 0; u < kMpU; u++)
-    s[u] = b + u < b1 ? ((const i32x4*)p.sid)[(size_t)(b + u) * 64 + lane] : i32x4{p.nrows, p.nrows, p.nrows, p.nrows};
+    s[u] = b + u < b1 ? ((const i32x4*)p.sid)[(size_t)(b + u) * 64 + lane] : i32x4{p.none, p.none, p.none, p.none};
 #pragma unroll
   for (int u = 0; u <= kMpU; u++) c0[u] = p.bstart[min(b + u, b1)];
   const int first = c0[0], last = c0[kMpU];  // rows that other waves may lower too
@@ -310,13 +311,13 @@ __global__ void k_minplus_starts(const int32_t* rrow, const int32_t* cid, int n,
 // Rows of the edges and of their sources, padding included. *wild: 1 where a
 // weight is negative, or wraps when added to an unreached distance.
 __global__ void k_minplus_edges(const int32_t* rrow, const int32_t* rcol, const int32_t* rwt, const int32_t* cid,
-                                const int32_t* bstart, int n, int nblk, int nrows, int32_t* sid, uint8_t* roff,
+                                const int32_t* bstart, int n, int nblk, int none, int32_t* sid, uint8_t* roff,
                                 int* wild) {
   bool bad = false;
   const int64_t m = rrow[n], stride = (int64_t)gridDim.x * blockDim.x;
   for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < (int64_t)nblk * kMpBlock; e += stride) {
     const int c = e < m ? cid[rcol[e]] : -1;
-    sid[e] = c < 0 ? nrows : c;
+    sid[e] = c < 0 ? none : c;
     roff[e] = e < m ? (uint8_t)(cid[row_of(rrow, n, e)] - bstart[e / kMpBlock]) : 0;
     bad |= e < m && (uint32_t)rwt[e] > (uint32_t)(INT32_MAX - (int32_t)kInf);
   }
@@ -756,6 +757,23 @@ __global__ void __launch_bounds__(1024, LDS ? 8 : 4) k_bc(Ctl c, BcDev b, int* i
 
 namespace {
 
+// Rows per bit of the sweeps' LDS map, as a shift: one up to kMpMapBytes, above
+// that 2, 4, ...
+constexpr long long kMpMapBytes = 128 << 10;
+int mp_shift(int32_t rows) {
+  int shift = 0;
+  while (4ll * ((rows >> shift) / 32 + 4) > kMpMapBytes) shift++;
+  return shift;
+}
+// The row number for sources without in-edges: the first whose bit no row
+// shares. A bit's rows are followed when any of them was lowered, and such a
+// source's edges, followed from the unreached distance, would go wrong where a
+// weight wraps. (Unsigned: up to 2^31.)
+uint32_t mp_none(int32_t rows) {
+  const uint32_t per = 1u << mp_shift(rows);
+  return ((uint32_t)rows + per - 1u) / per * per;
+}
+
 // Edges of the min-plus graph, padding included.
 int64_t mp_edges(int64_t m) { return (m + kMpBlock - 1) / kMpBlock * kMpBlock; }
 
@@ -811,7 +829,7 @@ int minplus_rows(wgm_graph* g) {
   e = hipMemcpyAsync(g->iters, &wild, sizeof(int), hipMemcpyHostToDevice, rt->stream);
   hipLaunchKernelGGL(k_minplus_starts, dim3(1024), dim3(256), 0, rt->stream, g->rrow, g->mp_cid, n, nblk, rows, g->mp_start);
   hipLaunchKernelGGL(k_minplus_edges, dim3(4096), dim3(256), 0, rt->stream, g->rrow, g->rcol, g->rwt, g->mp_cid,
-                     g->mp_start, n, nblk, rows, sid, g->mp_roff, g->iters);
+                     g->mp_start, n, nblk, (int32_t)mp_none(rows), sid, g->mp_roff, g->iters);
   if (e == hipSuccess) e = hipGetLastError();
   if (e == hipSuccess) e = hipMemcpyAsync(&wild, g->iters, sizeof(int), hipMemcpyDeviceToHost, rt->stream);
   const hipError_t done = hipStreamSynchronize(rt->stream);
@@ -875,11 +893,8 @@ int bc_grid(wgm_runtime* rt, const wgm_graph* g, const wgm_launch* lc, int* grid
 }
 
 // Min-plus sweeps from src into dist (device, n entries; `big` where
-// unreached). The LDS map has a bit a row up to kMpMapBytes, above that a bit
-// for each 2, 4, ... rows. It takes a CU for a workgroup: more workgroups than
-// that are taken as one larger one on each CU, which also shortens the barrier.
-constexpr long long kMpMapBytes = 128 << 10;
-
+// unreached). The LDS map takes a CU for a workgroup: more workgroups than that
+// are taken as one larger one on each CU, which also shortens the barrier.
 int run_minplus(wgm_runtime* rt, wgm_graph* g, int32_t src, int32_t big, const wgm_launch* lc, int32_t* dist,
                 bool reached, void* dst, wgm_run_stats* st) {
   int rc = minplus_rows(g);
@@ -900,8 +915,9 @@ int run_minplus(wgm_runtime* rt, wgm_graph* g, int32_t src, int32_t big, const w
   p.big = big;
   p.all = g->wild_weights ? 1 : 0;
   p.max_sweeps = g->n + 1;
-  while (4ll * ((p.nrows >> p.shift) / 32 + 4) > kMpMapBytes) p.shift++;
-  p.map_words = ((p.nrows >> p.shift) / 32 + 4) / 4 * 4;
+  p.none = (int32_t)mp_none(p.nrows);
+  p.shift = mp_shift(p.nrows);
+  p.map_words = (int32_t)((mp_none(p.nrows) >> p.shift) / 32 + 4) / 4 * 4;
   p.bit_words = g->mp_words;
   p.d = g->mp_d;
   p.bits = g->mp_bits;

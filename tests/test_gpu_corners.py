@@ -1,0 +1,31 @@
+"""GPU parity at corners: weights that wrap, ids that share a word, shapes kept off before."""
+import numpy as np
+import pytest
+
+import oracle
+from gpu_workgroup_managment_amd import _lib as L
+from gpu_workgroup_managment_amd import graphs as G
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("n", [1200002, 1200003, 2500004])
+def test_minplus_source_without_in_edges(rt, n):
+    """More than 2^20 vertices with in-edges, so that a bit of the sweeps' map
+    stands for two or four of them. The source has no in-edge, one edge of a
+    weight that wraps when added to an unreached distance, and one to the last
+    vertex, the highest-numbered row: the first must never be followed."""
+    heavy = 2 ** 31 - 6
+    row = np.concatenate([[0], 2 + np.arange(n)]).astype(np.int32)  # the others have a loop each
+    col = np.concatenate([[1, n - 1], np.arange(1, n)]).astype(np.int32)
+    wt = np.concatenate([[heavy, 3], np.ones(n - 1)]).astype(np.int32)
+    g = G.CSR(row, col, wt)
+    ref, _ = oracle.sssp_minplus(g.row_ptr, g.col, g.wt, 0)
+    pull = np.where(ref == L.BIG_NUM, oracle.INF, ref)
+    dg = rt.graph(g)
+    for wg, wgs in ((512, 64), (1024, 0)):
+        d, _ = dg.sssp_minplus(0, wg_size=wg, num_wgs=wgs)
+        assert np.array_equal(d, ref), (wg, wgs)
+        d, _ = dg.sssp(0, wg_size=wg, num_wgs=wgs, mode=2)
+        assert np.array_equal(d, pull), (wg, wgs)
+    dg.close()
