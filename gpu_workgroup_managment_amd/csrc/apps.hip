@@ -175,14 +175,15 @@ __global__ void __launch_bounds__(1024) k_color(Ctl c, GraphDev g, int32_t* colo
   const int last = ld_relaxed(largest);
   if (mine == last) {
     const int lane = (int)threadIdx.x & 63;
-    for (int v0 = lo + ((int)threadIdx.x & ~63); v0 < hi; v0 += blockDim.x) {
-      unsigned long long m = __ballot(v0 + lane < hi && ld_agent(&color[min(v0 + lane, hi - 1)]) == last);
+    for (Span mine{(uint32_t)lo + (threadIdx.x & ~63u), (uint32_t)hi}; mine.has(); mine.next(blockDim.x)) {
+      unsigned long long m = __ballot(ld_agent(&color[mine.until(lane + 1) - 1]) == last && mine.has(lane));
       for (; m; m &= m - 1) {  // the wave walks each row
-        const int v = v0 + __ffsll((long long)m) - 1;
+        const int v = (int)mine.at + __ffsll((long long)m) - 1;
         const int beg = g.row_ptr[v], end = g.row_ptr[v + 1];
         if (end - beg == 1) continue;
         bool hit = false;
-        for (int e = beg + lane; e < end; e += 64) hit |= ld_agent(&color[g.col[e]]) == last;
+        for (Span row{(uint32_t)beg + lane, (uint32_t)end}; row.has(); row.next(64))
+          hit |= ld_agent(&color[g.col[row.at]]) == last;
         if (hit) st_relaxed(again, 1);
       }
     }
@@ -312,8 +313,8 @@ __global__ void __launch_bounds__(1024, 8) k_pagerank(Ctl c, GraphDev g, float* 
 constexpr int kNearNone = -32768;
 __global__ void k_near_rows(GraphDev g, uint2* rows, int* far) {
   bool bad = false;
-  for (int v = blockIdx.x * blockDim.x + threadIdx.x; v < g.n; v += gridDim.x * blockDim.x) {
-    const int beg = g.row_ptr[v], deg = g.row_ptr[v + 1] - beg;
+  for (Span mine{blockIdx.x * blockDim.x + threadIdx.x, (uint32_t)g.n}; mine.has(); mine.next(gridDim.x * blockDim.x)) {
+    const int v = (int)mine.at, beg = g.row_ptr[v], deg = g.row_ptr[v + 1] - beg;
     uint32_t w[4];
 #pragma unroll
     for (int k = 0; k < 4; k++) {
@@ -348,21 +349,23 @@ __global__ void __launch_bounds__(1024, 8) k_pagerank_near(Ctl c, GraphDev g, co
     float* cout = it == iters - 1 ? rank : (it & 1) ? c0 : c1;
     const bool last = it == iters - 1;
     auto rows_of = [&](int a, int z, auto&& row) {
-      for (int i0 = a + (int)threadIdx.x; i0 < z; i0 += U * bd) {
+      for (Span place{(uint32_t)a + threadIdx.x, (uint32_t)z}; place.has(); place.next(U * bd)) {
+        uint32_t i[U];  // beyond the range: its last row
+#pragma unroll
+        for (int k = 0; k < U; k++) i[k] = min(place.at + k * bd, place.stop - 1u);
         u32x2 r[U];
 #pragma unroll
-        for (int k = 0; k < U; k++) r[k] = row(min(i0 + k * bd, z - 1));
+        for (int k = 0; k < U; k++) r[k] = row(i[k]);
         float cu[U][4];
 #pragma unroll
         for (int k = 0; k < U; k++)
 #pragma unroll
           for (int j = 0; j < 4; j++) {
             const int step = (int)(int16_t)(r[k][j >> 1] >> (16 * (j & 1)));
-            cu[k][j] = step != kNearNone ? cin[lo + min(i0 + k * bd, z - 1) + step] : 0.0f;
+            cu[k][j] = step != kNearNone ? cin[lo + i[k] + step] : 0.0f;
           }
 #pragma unroll
         for (int k = 0; k < U; k++) {
-          const int i = i0 + k * bd;
           float sum = 0.0f;
           int deg = 0;
 #pragma unroll
@@ -372,12 +375,12 @@ __global__ void __launch_bounds__(1024, 8) k_pagerank_near(Ctl c, GraphDev g, co
             deg += edge ? 1 : 0;
           }
           const float x = __builtin_fmaf(damping, sum, base);
-          if (i < z) cout[lo + i] = last ? x : deg > 0 ? x / (float)deg : 0.0f;
+          if (place.has(k * bd)) cout[lo + i[k]] = last ? x : deg > 0 ? x / (float)deg : 0.0f;
         }
       }
     };
-    rows_of(0, held, [&](int i) { return mine[i]; });
-    rows_of(held, hi - lo, [&](int i) { return ((const u32x2*)rows)[lo + i]; });
+    rows_of(0, held, [&](uint32_t i) { return mine[i]; });
+    rows_of(held, hi - lo, [&](uint32_t i) { return ((const u32x2*)rows)[lo + i]; });
     xcd_barrier(c, t);
   }
   clock_end(c, t.id);
@@ -854,7 +857,7 @@ static int lds_share(const wgm_runtime* rt, int grid, int wg) {
 // Rows that a workgroup holds in LDS: its range, within the share of a CU's 160
 // KB that leaves 2048 threads (or the workgroup each CU has) resident.
 static int near_held(const wgm_runtime* rt, int n, int grid, int wg) {
-  return std::min((lds_share(rt, grid, wg) - 1536) / 8, (n + grid - 1) / grid);
+  return (int)std::min<int64_t>((lds_share(rt, grid, wg) - 1536) / 8, ((int64_t)n + grid - 1) / grid);
 }
 
 int wgm_pagerank(wgm_runtime* rt, wgm_graph* g, float damping, int32_t iterations, const wgm_launch* lc,

@@ -12,6 +12,7 @@
 // passes a team; the mega-kernel passes the resizable persistent ids.
 #pragma once
 
+#include "spans.hpp"
 #include "wgm_device.hpp"
 
 namespace wgm {
@@ -799,11 +800,11 @@ __device__ __forceinline__ int scan_row(const int32_t* col, int e, int stop, int
                                         int* w, int& acc) {
   const int shift = ((int)threadIdx.x & 63) & ~(G - 1);
   int at = -1;
-  for (; e < stop && at < 0; e += G * Q) {
+  for (Span row{(uint32_t)e, (uint32_t)stop}; row.has() && at < 0; row.next(G * Q)) {
     int u[Q];
     bool hit[Q];
 #pragma unroll
-    for (int q = 0; q < Q; q++) u[q] = e + q * G + lane < stop ? col[e + q * G + lane] : -1;
+    for (int q = 0; q < Q; q++) u[q] = row.has(q * G + lane) ? col[row.at + q * G + lane] : -1;
 #pragma unroll
     for (int q = 0; q < Q; q++) hit[q] = probe.test(max(u[q], 0), pv, u[q] >= 0, acc);
 #pragma unroll
@@ -813,7 +814,7 @@ __device__ __forceinline__ int scan_row(const int32_t* col, int e, int stop, int
       if (m && at < 0) {
         const int first = __ffsll((long long)m) - 1;
         *w = __shfl(u[q], first, G);
-        at = e + q * G + first;
+        at = (int)(row.at + q * G + first);
       }
     }
   }
@@ -843,7 +844,7 @@ __device__ __forceinline__ void scan_queued(const GraphDev& g, int* s_q, int* s_
     const int id = q1[i], e = q1[cap + i];
     int acc = q1[2 * cap + i], w = -1;
     const int v = row(id);
-    const int end = g.row_ptr[v + 1], stop = min(end, e + kScanMid);
+    const int end = g.row_ptr[v + 1], stop = (int)Span{(uint32_t)e, (uint32_t)end}.until(kScanMid);
     const int hit = scan_row<8, 2>(g.col, e, stop, lane & 7, g.prio[v], probe, &w, acc);
     if ((lane & 7) == 0) {
       if (hit >= 0 || stop == end) {
@@ -878,7 +879,7 @@ __device__ __forceinline__ void open_pass_long(const GraphDev& g, const Probe& p
                                                const int4* lin, int4* lout, int* ocnt, int* s_q, int* s_n,
                                                const Decide& decide, const Keep& keep) {
   const int bd = blockDim.x, cap = kScanU * bd;
-  for (int base = 0; base < cnt; base += kScanU * bd) {
+  for (Span chunk{0u, (uint32_t)cnt}; chunk.has(); chunk.next(kScanU * bd)) {
     if (threadIdx.x == 0) s_n[0] = s_n[1] = 0;
     __syncthreads();
     bool in[kScanU], scan[kScanU];
@@ -887,12 +888,12 @@ __device__ __forceinline__ void open_pass_long(const GraphDev& g, const Probe& p
     uint32_t pv[kScanU];
 #pragma unroll
     for (int k = 0; k < kScanU; k++) {
-      const int i = base + k * bd + (int)threadIdx.x;
-      in[k] = i < cnt;
+      const uint32_t i = (uint32_t)lo + chunk.at + k * bd + threadIdx.x;
+      in[k] = chunk.has(k * bd + threadIdx.x);
       en[k] = int4{0, 0, 0, 0};
       if (in[k]) {
-        if (lin) en[k] = lin[lo + i];
-        else en[k].x = lo + i;
+        if (lin) en[k] = lin[i];
+        else en[k].x = (int)i;
       }
     }
 #pragma unroll
@@ -908,7 +909,7 @@ __device__ __forceinline__ void open_pass_long(const GraphDev& g, const Probe& p
     for (int k = 0; k < kScanU; k++) {
       if (skip1 && !lin && end[k] - e[k] == 1) end[k] = e[k];
 #pragma unroll
-      for (int j = 0; j < 4; j++) u[k][j] = e[k] + j < end[k] ? g.col[e[k] + j] : -1;
+      for (int j = 0; j < 4; j++) u[k][j] = j < end[k] - e[k] ? g.col[e[k] + j] : -1;
     }
     bool hit[kScanU][4];
 #pragma unroll
@@ -925,7 +926,7 @@ __device__ __forceinline__ void open_pass_long(const GraphDev& g, const Probe& p
           en[k].y = e[k] + j;
           en[k].z = u[k][j];
         }
-      const bool more = scan[k] && !held && e[k] + 4 < end[k];
+      const bool more = scan[k] && !held && end[k] - e[k] > 4;
       if (in[k] && !held && !more) decide(en[k].x, en[k].w);
       if (held && !lin) keep(en[k].x);
       const int slot = wl_slot(held, ocnt);
@@ -956,18 +957,18 @@ __device__ __forceinline__ void open_pass_low(const GraphDev& g, const Probe& pr
                                               const int2* lin, int2* lout, int* ocnt, const Decide& decide,
                                               const Keep& keep) {
   const int bd = blockDim.x;
-  for (int base = (int)threadIdx.x; base < cnt; base += kTopoGroup * bd) {
+  for (Span mine{threadIdx.x, (uint32_t)cnt}; mine.has(); mine.next(kTopoGroup * bd)) {
     int2 en[kTopoGroup];
     bool in[kTopoGroup], scan[kTopoGroup];
     int beg[kTopoGroup], deg[kTopoGroup], acc[kTopoGroup];
     uint32_t pv[kTopoGroup];
 #pragma unroll
     for (int k = 0; k < kTopoGroup; k++) {
-      in[k] = base + k * bd < cnt;
+      in[k] = mine.has(k * bd);
       en[k] = int2{0, 0};
       if (in[k]) {
-        if (lin) en[k] = lin[lo + base + k * bd];
-        else en[k].x = lo + base + k * bd;
+        if (lin) en[k] = lin[(uint32_t)lo + mine.at + k * bd];
+        else en[k].x = (int)((uint32_t)lo + mine.at + k * bd);
       }
     }
 #pragma unroll
@@ -1047,7 +1048,7 @@ __device__ __forceinline__ void mis_phase_b_long(const GraphDev& g, int32_t* st,
                                                  const int4* lin, int4* lout, int* ocnt, int* s_q, int* s_n) {
   const int joined = 2 * round, bd = blockDim.x, cap = kScanU * bd;
   const JoinedProbe probe{st, joined};
-  for (int base = 0; base < cnt; base += kScanU * bd) {
+  for (Span chunk{0u, (uint32_t)cnt}; chunk.has(); chunk.next(kScanU * bd)) {
     if (threadIdx.x == 0) s_n[0] = s_n[1] = 0;
     __syncthreads();
     bool in[kScanU], gone[kScanU];
@@ -1055,9 +1056,8 @@ __device__ __forceinline__ void mis_phase_b_long(const GraphDev& g, int32_t* st,
     int beg[kScanU], end[kScanU];
 #pragma unroll
     for (int k = 0; k < kScanU; k++) {
-      const int i = base + k * bd + (int)threadIdx.x;
-      in[k] = i < cnt;
-      en[k] = in[k] ? lin[lo + i] : int4{0, 0, 0, 0};
+      in[k] = chunk.has(k * bd + threadIdx.x);
+      en[k] = in[k] ? lin[(uint32_t)lo + chunk.at + k * bd + threadIdx.x] : int4{0, 0, 0, 0};
     }
 #pragma unroll
     for (int k = 0; k < kScanU; k++) {
@@ -1069,7 +1069,7 @@ __device__ __forceinline__ void mis_phase_b_long(const GraphDev& g, int32_t* st,
 #pragma unroll
     for (int k = 0; k < kScanU; k++)
 #pragma unroll
-      for (int j = 0; j < 4; j++) u[k][j] = !gone[k] && beg[k] + j < end[k] ? g.col[beg[k] + j] : -1;
+      for (int j = 0; j < 4; j++) u[k][j] = !gone[k] && j < end[k] - beg[k] ? g.col[beg[k] + j] : -1;
     int none = 0;
 #pragma unroll
     for (int k = 0; k < kScanU; k++)
@@ -1080,13 +1080,13 @@ __device__ __forceinline__ void mis_phase_b_long(const GraphDev& g, int32_t* st,
 #pragma unroll
       for (int j = 0; j < 4; j++) gone[k] = gone[k] || u[k][j] != 0;
       if (gone[k]) st[en[k].x] = joined + 1;
-      const bool more = in[k] && !gone[k] && beg[k] + 4 < end[k];
+      const bool more = in[k] && !gone[k] && end[k] - beg[k] > 4;
       const bool stay = in[k] && !gone[k] && !more;
       const int slot = wl_slot(stay, ocnt);
       if (stay) lout[lo + slot] = en[k];
       const int qs = wl_slot(more, &s_n[0]);
       if (more) {
-        s_q[qs] = base + k * bd + (int)threadIdx.x;
+        s_q[qs] = (int)(chunk.at + k * bd + threadIdx.x);
         s_q[cap + qs] = beg[k] + 4;
         s_q[2 * cap + qs] = 0;
       }
@@ -1104,14 +1104,14 @@ __device__ __forceinline__ void mis_phase_b_low(const GraphDev& g, int32_t* st, 
                                                 const int2* lin, int2* lout, int* ocnt) {
   const int joined = 2 * round;
   const int bd = blockDim.x;
-  for (int base = (int)threadIdx.x; base < cnt; base += kTopoGroup * bd) {
+  for (Span mine{threadIdx.x, (uint32_t)cnt}; mine.has(); mine.next(kTopoGroup * bd)) {
     int2 en[kTopoGroup];
     bool in[kTopoGroup], gone[kTopoGroup];
     int beg[kTopoGroup], deg[kTopoGroup];
 #pragma unroll
     for (int k = 0; k < kTopoGroup; k++) {
-      in[k] = base + k * bd < cnt;
-      en[k] = in[k] ? lin[lo + base + k * bd] : int2{0, 0};
+      in[k] = mine.has(k * bd);
+      en[k] = in[k] ? lin[(uint32_t)lo + mine.at + k * bd] : int2{0, 0};
     }
 #pragma unroll
     for (int k = 0; k < kTopoGroup; k++) {
@@ -1146,8 +1146,8 @@ __device__ __forceinline__ void mis_phase_b_low(const GraphDev& g, int32_t* st, 
 // in a fixed order, so the result is bitwise reproducible. contrib holds
 // r(u)/deg(u) (0 for deg 0).
 __device__ __forceinline__ void pagerank_init(const GraphDev& g, float* contrib, float r0, int lo, int hi) {
-  for (int v = lo + (int)threadIdx.x; v < hi; v += blockDim.x) {
-    const int deg = g.row_ptr[v + 1] - g.row_ptr[v];
+  for (Span mine{(uint32_t)lo + threadIdx.x, (uint32_t)hi}; mine.has(); mine.next(blockDim.x)) {
+    const int v = (int)mine.at, deg = g.row_ptr[v + 1] - g.row_ptr[v];
     contrib[v] = deg ? r0 / (float)deg : 0.0f;
   }
 }
@@ -1203,12 +1203,12 @@ typedef __attribute__((address_space(3))) int32_t lds_i32;
 template <int G, class P>
 __device__ __forceinline__ float pagerank_group_sum(P col, const float* cin, int beg, int end, int lane) {
   float sum = 0.0f;
-  int e = beg + lane;
-  for (; e + 3 * G < end; e += 4 * G) {
+  Span row{(uint32_t)beg + lane, (uint32_t)end};
+  for (; row.has(3 * G); row.next(4 * G)) {
     int u[4];
     float x[4];
 #pragma unroll
-    for (int q = 0; q < 4; q++) u[q] = col[e + q * G];
+    for (int q = 0; q < 4; q++) u[q] = col[row.at + q * G];
 #pragma unroll
     for (int q = 0; q < 4; q++) x[q] = cin[u[q]];
 #pragma unroll
@@ -1217,7 +1217,7 @@ __device__ __forceinline__ float pagerank_group_sum(P col, const float* cin, int
   int u[3];
   float x[3];
 #pragma unroll
-  for (int q = 0; q < 3; q++) u[q] = e + q * G < end ? col[e + q * G] : -1;
+  for (int q = 0; q < 3; q++) u[q] = row.has(q * G) ? col[row.at + q * G] : -1;
 #pragma unroll
   for (int q = 0; q < 3; q++) x[q] = u[q] >= 0 ? cin[u[q]] : 0.0f;
 #pragma unroll
@@ -1233,8 +1233,8 @@ __device__ __forceinline__ float pagerank_group_sum(P col, const float* cin, int
 // s_cnt: three ints of LDS, zeroed by the caller before a barrier.
 template <class P>
 __device__ __forceinline__ void pagerank_lists(const PrRows<P>& rows, int lo, int hi, int* s_cnt) {
-  for (int v = lo + (int)threadIdx.x; v < hi; v += blockDim.x) {
-    const int deg = rows.row_ptr[v - rows.v0 + 1] - rows.row_ptr[v - rows.v0];
+  for (Span mine{(uint32_t)lo + threadIdx.x, (uint32_t)hi}; mine.has(); mine.next(blockDim.x)) {
+    const int v = (int)mine.at, deg = rows.row_ptr[v - rows.v0 + 1] - rows.row_ptr[v - rows.v0];
     if (deg <= kTopoEdges) continue;
     const int k = deg <= kPrMid ? 0 : deg <= kPrSeg ? 1 : 2;
     const int i = __hip_atomic_fetch_add(&s_cnt[k], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
@@ -1263,11 +1263,11 @@ __device__ __forceinline__ void pagerank_pass(const PrRows<P>& rows, const float
       const int v = rows.list2[rows.l0 + i];
       const int beg = row_ptr[v - v0], end = row_ptr[v - v0 + 1];
       float total = 0.0f;
-      for (int a = beg; a < end; a += kPrSegs * kPrSeg) {
-        const int ns = min(kPrSegs, (end - a + kPrSeg - 1) / kPrSeg);
+      for (Span row{(uint32_t)beg, (uint32_t)end}; row.has(); row.next(kPrSegs * kPrSeg)) {
+        const int ns = (int)min((uint32_t)kPrSegs, (row.stop - row.at + kPrSeg - 1) / kPrSeg);
         for (int s = wave; s < ns; s += nw) {
-          const int sb = a + s * kPrSeg;
-          const float x = pagerank_group_sum<64>(col, cin, sb, min(sb + kPrSeg, end), lane);
+          const Span seg{row.at + s * kPrSeg, row.stop};
+          const float x = pagerank_group_sum<64>(col, cin, (int)seg.at, (int)seg.until(kPrSeg), lane);
           if (lane == 0) s_seg[s] = x;
         }
         __syncthreads();
@@ -1294,22 +1294,23 @@ __device__ __forceinline__ void pagerank_pass(const PrRows<P>& rows, const float
       if ((lane & 7) == 0) put(v, x, end - beg);
     }
   }
-  for (int b0 = lo + (int)threadIdx.x; b0 < hi; b0 += U * bd) {
-    int v[U], beg[U], end[U];
+  for (Span mine{(uint32_t)lo + threadIdx.x, (uint32_t)hi}; mine.has(); mine.next(U * bd)) {
+    uint32_t v[U];
+    int beg[U], end[U];
 #pragma unroll
     for (int k = 0; k < U; k++) {
-      v[k] = b0 + k * bd;
-      const bool in = v[k] < hi;
+      v[k] = mine.at + k * bd;
+      const bool in = v[k] < mine.stop;
       beg[k] = in ? row_ptr[v[k] - v0] : 0;
       end[k] = in ? row_ptr[v[k] - v0 + 1] : 0;
-      if (LONG && end[k] - beg[k] > kTopoEdges) v[k] = hi;  // summed above
+      if (LONG && end[k] - beg[k] > kTopoEdges) v[k] = mine.stop;  // summed above
     }
     int u[U][kTopoEdges];
 #pragma unroll
     for (int k = 0; k < U; k++)
 #pragma unroll
       for (int j = 0; j < kTopoEdges; j++)
-        u[k][j] = (!LONG || v[k] < hi) && beg[k] + j < end[k] ? col[beg[k] + j] : -1;
+        u[k][j] = (!LONG || v[k] < mine.stop) && j < end[k] - beg[k] ? col[beg[k] + j] : -1;
     float cu[U][kTopoEdges];
 #pragma unroll
     for (int k = 0; k < U; k++)
@@ -1317,7 +1318,7 @@ __device__ __forceinline__ void pagerank_pass(const PrRows<P>& rows, const float
       for (int j = 0; j < kTopoEdges; j++) cu[k][j] = u[k][j] >= 0 ? cin[u[k][j]] : 0.0f;
 #pragma unroll
     for (int k = 0; k < U; k++) {
-      if (v[k] >= hi) continue;
+      if (v[k] >= mine.stop) continue;
       float sum = 0.0f;
 #pragma unroll
       for (int j = 0; j < kTopoEdges; j++)
@@ -1358,19 +1359,15 @@ __device__ __forceinline__ void block_range(int n, int rank, int nteam, int* lo,
 // an edge, reach `target`; called by a whole wave, 64 probes a round.
 constexpr int kRowCost = 4;
 __device__ __forceinline__ int balanced_split(const int32_t* row_ptr, int n, long long target) {
-  const int lane = (int)threadIdx.x & 63;
-  int a = 0, b = n;  // the answer is in [a, b]
-  while (a < b) {
-    const int step = (b - a + 63) >> 6;
-    const long long p = (long long)a + (long long)lane * step;  // probe: still below the target
-    const bool below = p < b && (long long)row_ptr[p] + (long long)kRowCost * p < target;
-    const int k = __popcll(__ballot(below));  // cost grows with the vertex: the first k probes are below
+  Split s{0u, (uint32_t)n};
+  while (s.open()) {
+    const uint32_t p = s.probe(threadIdx.x & 63u);
+    const bool below = p < s.b && (long long)row_ptr[p] + (long long)kRowCost * p < target;
+    const int k = __popcll(__ballot(below));  // cost grows with the vertex
     if (k == 0) break;
-    const int last = a + (k - 1) * step;
-    b = min(b, last + step);
-    a = last + 1;
+    s.narrow(k);
   }
-  return a;
+  return (int)s.a;
 }
 
 // Contiguous vertex range of workgroup `rank` among `nteam` with an even share

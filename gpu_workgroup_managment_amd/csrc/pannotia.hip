@@ -106,7 +106,7 @@ __device__ __forceinline__ void mp_load_map(const MinplusDev& p, const uint32_t*
 // anything, unless a weight is negative or so large that it wraps (p.all).
 __device__ __forceinline__ bool minplus_first(const MinplusDev& p, int id, int nteam) {
   uint32_t* next = p.bits + p.bit_words;
-  const int tid = id * (int)blockDim.x + (int)threadIdx.x, stride = nteam * (int)blockDim.x;
+  const uint32_t tid = (uint32_t)id * blockDim.x + threadIdx.x, stride = (uint32_t)nteam * blockDim.x;
   bool any = false;
   auto relax = [&](int e, int du) {
     const int c = p.cid[p.col[e]], cand = (int)((uint32_t)du + (uint32_t)p.owt[e]);
@@ -116,11 +116,11 @@ __device__ __forceinline__ bool minplus_first(const MinplusDev& p, int id, int n
     }
   };
   if (p.all) {
-    for (int u = tid; u < p.n; u += stride)
-      for (int e = p.row_ptr[u]; e < p.row_ptr[u + 1]; e++) relax(e, u == p.src ? 0 : p.big);
+    for (Span mine{tid, (uint32_t)p.n}; mine.has(); mine.next(stride))
+      for (int u = (int)mine.at, e = p.row_ptr[u]; e < p.row_ptr[u + 1]; e++) relax(e, u == p.src ? 0 : p.big);
   } else {
-    const int end = p.row_ptr[p.src + 1];
-    for (int e = p.row_ptr[p.src] + tid; e < end; e += stride) relax(e, 0);
+    Span row{(uint32_t)p.row_ptr[p.src] + tid, (uint32_t)p.row_ptr[p.src + 1]};
+    for (; row.has(); row.next(stride)) relax((int)row.at, 0);
   }
   return any;
 }
@@ -178,7 +178,7 @@ __device__ __forceinline__ bool minplus_step(const MinplusDev& p, int b, int b1,
     for (int q = 0; q < 4; q++) {
       dv[u][q] = 0;
       if (c0[u + 1] - c0[u] >= 64 * q)
-        dv[u][q] = __hip_atomic_load(&p.d[min(c0[u] + 64 * q + lane, p.nrows)], __ATOMIC_RELAXED,
+        dv[u][q] = __hip_atomic_load(&p.d[min((uint32_t)c0[u] + 64 * q + lane, (uint32_t)p.nrows)], __ATOMIC_RELAXED,
                                      __HIP_MEMORY_SCOPE_WORKGROUP);
     }
   }
@@ -281,8 +281,8 @@ __global__ void __launch_bounds__(1024) k_minplus(Ctl c, MinplusDev p, int* iter
       break;
     }
   }
-  for (int v = t.id * (int)blockDim.x + (int)threadIdx.x; v < p.n; v += t.n * (int)blockDim.x) {
-    const int r = p.cid[v];
+  for (Span mine{t.id * blockDim.x + threadIdx.x, (uint32_t)p.n}; mine.has(); mine.next(t.n * blockDim.x)) {
+    const int v = (int)mine.at, r = p.cid[v];
     p.dist[v] = r >= 0 ? p.d[r] : v == p.src ? 0 : p.big;
   }
   clock_end(c, t.id);
@@ -295,16 +295,19 @@ __global__ void __launch_bounds__(1024) k_minplus(Ctl c, MinplusDev p, int* iter
 __global__ void k_minplus_init(MinplusDev p) {
   const int tid = blockIdx.x * blockDim.x + threadIdx.x, stride = gridDim.x * blockDim.x;
   const int s = p.cid[p.src];
-  for (int r = tid; r <= p.nrows; r += stride) p.d[r] = r == s ? 0 : p.big;
+  for (Span rows{(uint32_t)tid, (uint32_t)p.nrows + 1u}; rows.has(); rows.next(stride))
+    p.d[rows.at] = (int)rows.at == s ? 0 : p.big;
   for (int i = tid; i < 3 * p.bit_words; i += stride) p.bits[i] = 0u;
 }
 
 // First rows of the blocks; one wave a vertex.
 __global__ void k_minplus_starts(const int32_t* rrow, const int32_t* cid, int n, int nblk, int nrows, int32_t* bstart) {
   const int waves = (int)(gridDim.x * blockDim.x) >> 6, lane = (int)threadIdx.x & 63;
-  for (int v = (int)(blockIdx.x * blockDim.x + threadIdx.x) >> 6; v < n; v += waves)
+  for (Span mine{(blockIdx.x * blockDim.x + threadIdx.x) >> 6, (uint32_t)n}; mine.has(); mine.next(waves)) {
+    const int v = (int)mine.at;
     for (long long b = ((long long)rrow[v] + kMpBlock - 1) / kMpBlock + lane; b * kMpBlock < rrow[v + 1]; b += 64)
       bstart[b] = cid[v];
+  }
   if (blockIdx.x == 0 && threadIdx.x == 0) bstart[nblk] = nrows;
 }
 
@@ -440,29 +443,30 @@ __device__ __forceinline__ void bc_mid(unsigned long long m, int v, int beg, int
   const int rank = __popcll(m & ((1ull << lane) - 1ull));
   const bool mine = (m >> lane) & 1ull;
   const int from = __builtin_amdgcn_ds_permute(4 * (mine ? rank : count + lane - rank), lane);
-  auto open = [&](int k, int& vv, int& e, int& b1) {
+  auto open = [&](int k, int& vv, Span& row) {
     const int src = __shfl(from, k & 63, 64);
     vv = __shfl(v, src, 64);
-    e = __shfl(beg, src, 64);
-    b1 = __shfl(end, src, 64);
-    if (k >= count) e = b1 = 0;
+    row.at = (uint32_t)__shfl(beg, src, 64);
+    row.stop = (uint32_t)__shfl(end, src, 64);
+    if (k >= count) row = Span{0u, 0u};
   };
   int k = lane >> 4;  // this group's row, and its next one
-  int vv, e, b1, ov, oe, ob1;
-  open(k, vv, e, b1);
-  int w = e + sub < b1 ? col[e + sub] : -1;
-  open(k + 4, ov, oe, ob1);
+  int vv, ov;
+  Span row, ahead;
+  open(k, vv, row);
+  int w = row.has(sub) ? col[row.at + sub] : -1;
+  open(k + 4, ov, ahead);
   bool first = true;
-  while (__ballot(e < b1)) {  // every lane takes part in the moves between lanes
-    const bool last = e + 16 >= b1;
+  while (__ballot(row.has())) {  // every lane takes part in the moves between lanes
+    const bool last = !row.has(16);
     const int cv = vv, cw = w;
-    const bool live = e < b1;
+    const bool live = row.has();
     vv = last ? ov : vv;
-    e = last ? oe : e + 16;
-    b1 = last ? ob1 : b1;
+    row.at = last ? ahead.at : row.at + 16;
+    row.stop = last ? ahead.stop : row.stop;
     k = last ? k + 4 : k;
-    w = e + sub < b1 ? col[e + sub] : -1;
-    if (__ballot(last)) open(k + 4, ov, oe, ob1);
+    w = row.has(sub) ? col[row.at + sub] : -1;
+    if (__ballot(last)) open(k + 4, ov, ahead);
     if (live) step(cv, cw, first, last);
     first = last;
   }
@@ -476,22 +480,22 @@ __device__ __forceinline__ void bc_wide(unsigned long long m, int beg, int end, 
   if (!m) return;
   const int lane = (int)threadIdx.x & 63;
   int l = __ffsll((long long)m) - 1;
-  int e = __builtin_amdgcn_readlane(beg, l), b1 = __builtin_amdgcn_readlane(end, l);
-  int w = e + lane < b1 ? col[e + lane] : -1;
+  Span row{(uint32_t)__builtin_amdgcn_readlane(beg, l), (uint32_t)__builtin_amdgcn_readlane(end, l)};
+  int w = row.has(lane) ? col[row.at + lane] : -1;
   bool first = true;
   while (true) {
     const int cl = l, cw = w;
-    const bool last = e + 64 >= b1;
-    e += 64;
+    const bool last = !row.has(64);
+    row.next(64);
     if (last) {
       m &= m - 1;
       if (m) {
         l = __ffsll((long long)m) - 1;
-        e = __builtin_amdgcn_readlane(beg, l);
-        b1 = __builtin_amdgcn_readlane(end, l);
+        row.at = (uint32_t)__builtin_amdgcn_readlane(beg, l);
+        row.stop = (uint32_t)__builtin_amdgcn_readlane(end, l);
       }
     }
-    w = m && e + lane < b1 ? col[e + lane] : -1;
+    w = m && row.has(lane) ? col[row.at + lane] : -1;
     step(cl, cw, first, last);
     if (!m) break;
     first = last;
@@ -546,7 +550,7 @@ __device__ __forceinline__ void bc_rows(const State& st, const int32_t* row, con
     const int deg = end - beg;
     int w[State::kRow];
 #pragma unroll
-    for (int k = 0; k < State::kRow; k++) w[k] = deg <= State::kRow && beg + k < end ? col[beg + k] : -1;
+    for (int k = 0; k < State::kRow; k++) w[k] = deg <= State::kRow && k < deg ? col[beg + k] : -1;
     if (in && deg <= State::kRow) {
       double acc = 0.0;
 #pragma unroll
@@ -604,7 +608,7 @@ __device__ __forceinline__ int bc_source(const BcDev& b, int s, const State& st,
       int w[State::kRow];
       bool open[State::kRow];
 #pragma unroll
-      for (int k = 0; k < State::kRow; k++) w[k] = deg <= State::kRow && beg + k < end ? b.col[beg + k] : -1;
+      for (int k = 0; k < State::kRow; k++) w[k] = deg <= State::kRow && k < deg ? b.col[beg + k] : -1;
 #pragma unroll
       for (int k = 0; k < State::kRow; k++) open[k] = w[k] >= 0 && st.fresh(w[k]);
 #pragma unroll
@@ -914,7 +918,7 @@ int run_minplus(wgm_runtime* rt, wgm_graph* g, int32_t src, int32_t big, const w
   p.src = src;
   p.big = big;
   p.all = g->wild_weights ? 1 : 0;
-  p.max_sweeps = g->n + 1;
+  p.max_sweeps = std::min(g->n, INT32_MAX - 1) + 1;
   p.none = (int32_t)mp_none(p.nrows);
   p.shift = mp_shift(p.nrows);
   p.map_words = (int32_t)((mp_none(p.nrows) >> p.shift) / 32 + 4) / 4 * 4;

@@ -114,7 +114,7 @@ __global__ void __launch_bounds__(kSortWg) k_sort_move(SortEdges in, SortEdges o
 // Row starts by search in the sorted targets, and the weights' padding.
 __global__ void k_sort_rows(const int32_t* key, int64_t m, int n, int32_t* rrow, int32_t* rwt, int64_t padded) {
   const int tid = blockIdx.x * blockDim.x + threadIdx.x, stride = gridDim.x * blockDim.x;
-  for (int v = tid; v <= n; v += stride) {
+  for (int64_t v = tid; v <= n; v += stride) {
     int64_t lo = 0, hi = m;
     while (lo < hi) {
       const int64_t mid = (lo + hi) >> 1;
@@ -127,13 +127,13 @@ __global__ void k_sort_rows(const int32_t* key, int64_t m, int n, int32_t* rrow,
 }
 
 // Whether a vertex has an in-edge (and zeros up to `padded`), to be summed.
-__global__ void k_row_flags(const int32_t* rrow, int n, int padded, int32_t* id) {
-  for (int v = blockIdx.x * blockDim.x + threadIdx.x; v < padded; v += gridDim.x * blockDim.x)
+__global__ void k_row_flags(const int32_t* rrow, int n, int64_t padded, int32_t* id) {
+  for (int64_t v = blockIdx.x * blockDim.x + threadIdx.x; v < padded; v += gridDim.x * blockDim.x)
     id[v] = v < n && rrow[v + 1] > rrow[v] ? 1 : 0;
 }
 __global__ void k_row_ids(const int32_t* rrow, int n, int32_t* id) {
-  for (int v = blockIdx.x * blockDim.x + threadIdx.x; v < n; v += gridDim.x * blockDim.x)
-    if (rrow[v + 1] == rrow[v]) id[v] = -1;
+  for (Span mine{blockIdx.x * blockDim.x + threadIdx.x, (uint32_t)n}; mine.has(); mine.next(gridDim.x * blockDim.x))
+    if (rrow[mine.at + 1] == rrow[mine.at]) id[mine.at] = -1;
 }
 
 }  // namespace wgm
@@ -244,9 +244,9 @@ int wgm_graph_in_edges(wgm_graph* g) {
 size_t wgm_row_id_words(int32_t n) { return ((size_t)n + 4) / 4 * 4; }
 int wgm_row_ids(wgm_graph* g, int32_t* id, int32_t* rows) {
   wgm_runtime* rt = g->rt;
-  const int padded = (int)wgm_row_id_words(g->n);
+  const int64_t padded = (int64_t)wgm_row_id_words(g->n);
   hipLaunchKernelGGL(k_row_flags, dim3(1024), dim3(256), 0, rt->stream, g->rrow, g->n, padded, id);
-  hipLaunchKernelGGL(k_sort_scan, dim3(1), dim3(kSortWg), 0, rt->stream, id, (int64_t)padded);
+  hipLaunchKernelGGL(k_sort_scan, dim3(1), dim3(kSortWg), 0, rt->stream, id, padded);
   hipLaunchKernelGGL(k_row_ids, dim3(1024), dim3(256), 0, rt->stream, g->rrow, g->n, id);
   HIPCHK(rt, hipGetLastError());
   HIPCHK(rt, hipMemcpyAsync(rows, id + g->n, sizeof(int32_t), hipMemcpyDeviceToHost, rt->stream));

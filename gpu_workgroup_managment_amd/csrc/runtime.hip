@@ -382,11 +382,11 @@ __global__ void __launch_bounds__(1024) k_finish(Ctl c, GraphDev g, const uint32
   __syncthreads();
   if (reached) {
     unsigned long long local = 0;
-    const int stride = (int)(gridDim.x * blockDim.x);
+    const uint32_t stride = gridDim.x * blockDim.x;
 #pragma unroll 4
-    for (int v = (int)(blockIdx.x * blockDim.x + threadIdx.x); v < g.n; v += stride) {
-      const int deg = g.row_ptr[v + 1] - g.row_ptr[v];
-      local += reached[v] != kInf ? (unsigned long long)deg : 0ull;
+    for (Span mine{blockIdx.x * blockDim.x + threadIdx.x, (uint32_t)g.n}; mine.has(); mine.next(stride)) {
+      const int deg = g.row_ptr[mine.at + 1] - g.row_ptr[mine.at];
+      local += reached[mine.at] != kInf ? (unsigned long long)deg : 0ull;
     }
     for (int d = 32; d > 0; d >>= 1) local += __shfl_down(local, d, 64);
     if ((threadIdx.x & 63) == 0 && local) atomicAdd(&s_part, local);

@@ -118,14 +118,14 @@ __device__ __forceinline__ void frontier_bottom_up(const GraphDev& g, const Fron
   int* s_found = lds + scan_lds_bytes(bd) / 4;
   int lo, hi;
   block_range(g.n, rank, nteam, &lo, &hi);
-  for (int base = lo; base < hi; base += kScanU * bd) {
-    if (base > lo) __syncthreads();  // the last chunk's found vertices are stored
+  for (Span chunk{(uint32_t)lo, (uint32_t)hi}; chunk.has(); chunk.next(kScanU * bd)) {
+    if (chunk.at > (uint32_t)lo) __syncthreads();  // the last chunk's found vertices are stored
     int v[kScanU], e[kScanU], end[kScanU], u[kScanU][4], none = 0;
     bool open[kScanU], hit[kScanU][4];
 #pragma unroll
     for (int k = 0; k < kScanU; k++) {
-      v[k] = base + k * bd + tid;
-      open[k] = v[k] < hi && ld_agent(&s.dist[min(v[k], hi - 1)]) == kInf;
+      v[k] = (int)min(chunk.at + k * bd + tid, chunk.stop - 1u);
+      open[k] = chunk.has(k * bd + tid) && ld_agent(&s.dist[v[k]]) == kInf;
     }
 #pragma unroll
     for (int k = 0; k < kScanU; k++) {
@@ -135,7 +135,7 @@ __device__ __forceinline__ void frontier_bottom_up(const GraphDev& g, const Fron
 #pragma unroll
     for (int k = 0; k < kScanU; k++)
 #pragma unroll
-      for (int j = 0; j < 4; j++) u[k][j] = e[k] + j < end[k] ? in.col[e[k] + j] : -1;
+      for (int j = 0; j < 4; j++) u[k][j] = j < end[k] - e[k] ? in.col[e[k] + j] : -1;
 #pragma unroll
     for (int k = 0; k < kScanU; k++)
 #pragma unroll
@@ -143,7 +143,7 @@ __device__ __forceinline__ void frontier_bottom_up(const GraphDev& g, const Fron
 #pragma unroll
     for (int k = 0; k < kScanU; k++) {
       const bool found = hit[k][0] || hit[k][1] || hit[k][2] || hit[k][3];
-      const bool more = !found && e[k] + 4 < end[k];
+      const bool more = !found && end[k] - e[k] > 4;
       const int fs = wl_slot(found, &s_n[2]);
       if (found) s_found[fs] = v[k];
       const int qs = wl_slot(more, &s_n[0]);
