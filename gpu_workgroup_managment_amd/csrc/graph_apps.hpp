@@ -739,12 +739,14 @@ __device__ __forceinline__ int wl_slot1(int* cnt) {
 // priority pv; held(w, acc) whether blocker w still does. acc collects what the
 // vertex's decision needs from its decided neighbours (colour: the largest
 // colour). The loads are issued for every call (u is a valid vertex also where
-// the lane has no edge), so several calls overlap.
+// the lane has no edge), so several calls overlap. kPrio: whether pv is looked at
+// (a BFS graph has no priorities to load).
 //
 // Colour: a vertex is coloured one above the largest colour among the
 // neighbours whose priority is not below its own, once they all have theirs
 // (negative: uncoloured).
 struct ColorProbe {
+  static constexpr bool kPrio = true;
   const int32_t* color;
   const uint32_t* prio;
   __device__ __forceinline__ bool test(int u, uint32_t pv, bool valid, int& acc) const {
@@ -762,6 +764,7 @@ struct ColorProbe {
 };
 // MIS phase A: undecided at the round's start (-1, or 2 * round: joined in it).
 struct MisProbe {
+  static constexpr bool kPrio = true;
   const int32_t* st;
   const uint32_t* prio;
   int joined;
@@ -778,6 +781,7 @@ struct MisProbe {
 // First pass of either: every neighbour is undecided.
 template <bool ABOVE>
 struct FirstProbe {
+  static constexpr bool kPrio = true;
   const uint32_t* prio;
   __device__ __forceinline__ bool test(int u, uint32_t pv, bool valid, int&) const {
     const uint32_t p = prio[u];
@@ -787,6 +791,7 @@ struct FirstProbe {
 };
 // MIS phase B: joined this round.
 struct JoinedProbe {
+  static constexpr bool kPrio = false;
   const int32_t* st;
   int joined;
   __device__ __forceinline__ bool test(int u, uint32_t, bool valid, int&) const { return valid & (st[u] == joined); }
@@ -845,7 +850,7 @@ __device__ __forceinline__ void scan_queued(const GraphDev& g, int* s_q, int* s_
     int acc = q1[2 * cap + i], w = -1;
     const int v = row(id);
     const int end = g.row_ptr[v + 1], stop = (int)Span{(uint32_t)e, (uint32_t)end}.until(kScanMid);
-    const int hit = scan_row<8, 2>(g.col, e, stop, lane & 7, g.prio[v], probe, &w, acc);
+    const int hit = scan_row<8, 2>(g.col, e, stop, lane & 7, Probe::kPrio ? g.prio[v] : 0u, probe, &w, acc);
     if ((lane & 7) == 0) {
       if (hit >= 0 || stop == end) {
         done(id, v, hit, w, acc);
@@ -863,7 +868,7 @@ __device__ __forceinline__ void scan_queued(const GraphDev& g, int* s_q, int* s_
     const int id = q2[i], e = q2[cap + i];
     int acc = q2[2 * cap + i], w = -1;
     const int v = row(id);
-    const int hit = scan_row<64, 4>(g.col, e, g.row_ptr[v + 1], lane, g.prio[v], probe, &w, acc);
+    const int hit = scan_row<64, 4>(g.col, e, g.row_ptr[v + 1], lane, Probe::kPrio ? g.prio[v] : 0u, probe, &w, acc);
     if (lane == 0) done(id, v, hit, w, acc);
   }
   __syncthreads();

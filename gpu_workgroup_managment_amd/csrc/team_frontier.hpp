@@ -77,6 +77,7 @@ __host__ __device__ constexpr int standalone_frontier_lds_bytes(int bd) {
 
 // Frontier membership (bottom-up): a vertex of distance `level`.
 struct FrontProbe {
+  static constexpr bool kPrio = false;
   const uint32_t* dist;
   uint32_t level;
   __device__ __forceinline__ bool test(int u, uint32_t, bool valid, int&) const {
