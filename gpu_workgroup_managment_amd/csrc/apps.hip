@@ -690,32 +690,28 @@ static int low_rows(wgm_runtime* rt, wgm_graph* g) {
 
 // Workgroups where the caller leaves the number open, of the `fit` that can be
 // resident. A barrier costs 6 us with 512 workgroups, 4 with 256, 2.5 with 64, and
-// a pass over a small graph little else: `each` units of cost a thread, from 65536
-// threads to 262144 on 256 CUs, half of what they hold; all that fit from `wide` a
-// thread of that half on. Units: edges and rows (kRowCost), vertices for
-// k_pagerank_near. Whole calls, all -> by the rule:
+// a pass over a small graph little else: a thread for every `each` units of cost
+// (edges and rows (kRowCost), vertices for k_pagerank_near), from 65536 threads to
+// 1024 a CU. (BFS and MIS hold no more than those in workgroups of 1024, in smaller
+// ones up to 1.75 times as many.)
+// Whole calls, all that fit -> by the rule:
 // BFS, 1024 threads: ER n = 4097 of degree 8, 102 -> 94 us, RMAT 131072 ef 16, 148 ->
-// 142; 256 threads: 214 -> 101.
+// 142; 512 threads: RMAT scale 20 ef 16, 374 -> 342, 1201 x 1303 grid, 24.4 -> 19.8
+// ms; 256 threads: ER n = 4097, 214 -> 101.
 // MIS, 1024 threads: ER n = 60001 of degree 8, 175 -> 139, 401^2 grid 170 -> 135, 801^2
-// 254 -> 238; 256 threads: ER 395 -> 173.
+// 254 -> 238; 256 threads: ER n = 60001, 395 -> 173, 524288 of 16, 656 -> 589, 2047^2
+// grid 968 -> 894.
 // PageRank, 50 iterations, 1024 threads: ER n = 4097 of degree 8, 434 -> 246, 30001
-// of 16, 489 -> 365, 131072 of 8, 647 -> 551; symmetrised RMAT scale 18 ef 8, 1257 ->
-// 1316, ef 16 (just past the line) 1568 with half, 1689 with all, scale 19 5290 and
-// 4030; four random edges a vertex, n = 5001, 421 -> 233, 700001, 1173 -> 1090; meshes,
-// 401^2, 478 -> 299, 1401^2, 846 -> 756, 2047^2 (past the line) 1298 with half, 1273
-// with all; 256 threads, ER 16001 of degree 8, 1161 -> 369.
-struct FitRule {
-  int each, wide;
-};
-constexpr FitRule kFitBfs{16, 1 << 20};
-constexpr FitRule kFitMis{32, 1 << 20};
-constexpr FitRule kFitPr{4, 32};
-constexpr FitRule kFitPrNear{4, 12};
-static int fitted_grid(const wgm_runtime* rt, const wgm_launch* lc, int64_t cost, FitRule rule, int fit, int wg) {
+// of 16, 489 -> 365, 131072 of 8, 638 -> 542; four random edges a vertex, n = 5001,
+// 421 -> 233; meshes, 401^2, 478 -> 299; 256 threads, ER 16001 of degree 8, 1161 ->
+// 369.
+constexpr int kFitBfs = 16;
+constexpr int kFitMis = 32;
+constexpr int kFitPr = 4;
+static int fitted_grid(const wgm_runtime* rt, const wgm_launch* lc, int64_t cost, int each, int fit, int wg) {
   if (lc && lc->num_wgs > 0) return fit;
-  const int64_t half = (int64_t)rt->info.num_cus * 1024;
-  if (cost > rule.wide * half) return fit;
-  const int64_t threads = std::min(half, std::max<int64_t>(65536, cost / rule.each));
+  const int64_t most = (int64_t)rt->info.num_cus * 1024;
+  const int64_t threads = std::min(most, std::max<int64_t>(65536, cost / each));
   return (int)std::min<int64_t>(fit, (threads + wg - 1) / wg);
 }
 static int64_t rows_and_edges(const wgm_graph* g) { return g->m + kRowCost * (int64_t)g->n; }
@@ -860,6 +856,39 @@ static int near_held(const wgm_runtime* rt, int n, int grid, int wg) {
   return (int)std::min<int64_t>((lds_share(rt, grid, wg) - 1536) / 8, ((int64_t)n + grid - 1) / grid);
 }
 
+// Words of dynamic LDS of k_pagerank<LONG>, for a range's rows.
+static int held_words(const wgm_runtime* rt, int grid, int wg) { return (lds_share(rt, grid, wg) - 3072) / 4; }
+
+// Workgroups of PageRank where left open: by fitted_grid, or all that fit. By
+// measurement of both (whole calls, 50 iterations, few / all, us):
+// Meshes: few up to 12 vertices a thread of theirs; 1024 threads, 1801 x 1701, 981 /
+// 1073, 2047^2, 1280 / 1254. Four random edges a vertex: few; 1024 threads, n =
+// 700001, 1097 / 1182, 4000001, 11310 / 11500.
+// With longer rows it is whether an average range's rows fit the LDS: ER n =
+// 524288, 1024 threads, of degree 16 (they do), 2099 / 2166, 512 threads, of degree 8
+// (only with all), 1898 / 1588; symmetrised RMAT scale 18, 1024 threads, ef 32 (with
+// neither), 4063 / 3100. Many rows of more than kPrSeg edges in a workgroup, which
+// sums them one after another, make all the better choice, if the longest fits
+// then (scale 18 ef 8, 1306 / 1242, scale 19 ef 4, 1597 / 1415) or the largest ranges,
+// up to 1.3 times the average there, do not with few (scale 19 ef 8, 2437 / 2302),
+// against scale 18 ef 16, 1566 / 1742, and scale 17 ef 32, 1198 / 1398. (How many meet
+// is an estimate: scale 17 ef 4, 841 / 745 and few taken.)
+// The barrier of more than four workgroups a CU costs too much, short of huge
+// graphs with longer rows: 256 threads, 3001 x 2903 mesh, 3793 / 3927, scale 18 ef 8,
+// 1580 / 1944, ER n = 2^20 of degree 32, 10190 / 11420, RMAT scale 20 ef 32, 15590 /
+// 15180.
+static int pagerank_grid(const wgm_runtime* rt, const wgm_launch* lc, const wgm_graph* g, int fit, int wg) {
+  const int64_t cus = rt->info.num_cus, cost = rows_and_edges(g);
+  const int few = fitted_grid(rt, lc, g->near == 1 ? g->n : cost, kFitPr, fit, wg);
+  if (g->near == 1) return fit <= 4 * cus && g->n > 12 * 1024 * cus ? fit : few;
+  if (g->maxdeg <= kTopoEdges) return few;
+  if (fit > 4 * cus) return cost > 192 * 1024 * cus ? fit : few;
+  const int64_t average = (g->m + 2 * (int64_t)g->n) / few;
+  if (g->maxdeg > kPrSeg && cost / few >= 9 * kPrSeg)
+    return g->maxdeg <= held_words(rt, fit, wg) || average + average / 4 > held_words(rt, few, wg) ? fit : few;
+  return average < held_words(rt, few, wg) ? few : fit;
+}
+
 int wgm_pagerank(wgm_runtime* rt, wgm_graph* g, float damping, int32_t iterations, const wgm_launch* lc,
                  float* rank_out, wgm_run_stats* st) {
   if (!rt || !g || g->rt != rt) return fail(rt, WGM_ERR_INVALID, "bad runtime/graph");
@@ -877,16 +906,13 @@ int wgm_pagerank(wgm_runtime* rt, wgm_graph* g, float damping, int32_t iteration
   int grid = 0, wg = 0;
   rc = launch_prologue(rt, WGM_K_PAGERANK, lc, &grid, &wg);
   if (rc) return rc;
-  const int64_t cost = rows_and_edges(g);
-  grid = g->near == 1 ? fitted_grid(rt, lc, g->n, kFitPrNear, grid, wg) : fitted_grid(rt, lc, cost, kFitPr, grid, wg);
+  grid = pagerank_grid(rt, lc, g, grid, wg);
   if (g->near == 1)
     hipLaunchKernelGGL(k_pagerank_near, dim3(grid), dim3(wg), 8 * (size_t)near_held(rt, g->n, grid, wg), rt->stream, rt->ctl,
                        wgm_graph_view(g), g->near_rows, near_held(rt, g->n, grid, wg), g->f0, g->f1, g->f2, damping, base,
                        r0, iterations, g->iters);
   else if (g->maxdeg > kTopoEdges) {
-    // no more than an even share of the rows and edges could need, and a half of that
-    const int64_t even = cost / grid;
-    const int words = (int)std::min<int64_t>((lds_share(rt, grid, wg) - 3072) / 4, even + even / 2 + 64);
+    const int words = held_words(rt, grid, wg);
     hipLaunchKernelGGL(k_pagerank<true>, dim3(grid), dim3(wg), 4 * (size_t)words, rt->stream, rt->ctl, wgm_graph_view(g),
                        g->f0, g->f1, g->f2, damping, base, r0, iterations, g->wl, words, g->iters);
   } else
