@@ -63,7 +63,12 @@ __global__ void __launch_bounds__(1024, 8) k_barrier_bench(Ctl c, int iterations
   const SpinBounded sp{abort, budget};
   if (id == 0 && threadIdx.x == 0) st_relaxed(c.bar_groups, n);
   if (threadIdx.x == 0) local_sense = 0;
-  global_barrier_disc(c, id, n, sp);
+  // Never the flat barrier and the two-level one on the same lines: a flat
+  // arrival (1) whose release (0) is still on its way reads as the two-level
+  // barrier's first, and a leader that counts it later writes its release (2)
+  // over the flat one, which the member then never sees.
+  if (variant == 2) xcd_barrier<true>(c, t, sp);
+  else global_barrier_disc(c, id, n, sp);
   clock_start(c, id);
   int b = 0;
   for (int i = 0; i < iterations; i++) {

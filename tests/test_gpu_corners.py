@@ -29,3 +29,13 @@ def test_minplus_source_without_in_edges(rt, n):
         d, _ = dg.sssp(0, wg_size=wg, num_wgs=wgs, mode=2)
         assert np.array_equal(d, pull), (wg, wgs)
     dg.close()
+
+
+@pytest.mark.parametrize("wg", [64, 256, 512, 1024])
+def test_two_level_barrier_at_full_occupancy(rt, wg):
+    """The two-level barrier with every workgroup that fits, each epoch checked
+    (every wait has a budget of spins: a wait that lasts too long ends the launch
+    with an error)."""
+    r = rt.barrier_bench(wg_size=wg, num_wgs=0, iterations=20, variant=L.BARRIER_XCD)
+    assert r["epoch_errors"] == 0
+    assert r["participating"] >= 256 and r["barriers"] == 200
