@@ -599,7 +599,7 @@ int wgm_graph_create(wgm_runtime* rt, const wgm_csr* h, const uint32_t* prio, wg
   if (!rc) rc = dev_alloc(rt, &g->col, (size_t)h->m);
   if (!rc && h->wt) rc = dev_alloc(rt, &g->wt, (size_t)h->m);
   if (!rc && prio) rc = dev_alloc(rt, &g->prio, (size_t)h->n);
-  if (!rc) rc = dev_alloc(rt, &g->iters, 1);
+  if (!rc) rc = dev_alloc(rt, &g->iters, 4);
   if (rc) return bail(rc);
   hipError_t e = hipMemcpy(g->row_ptr, h->row_ptr, sizeof(int32_t) * ((size_t)h->n + 1), hipMemcpyHostToDevice);
   if (e == hipSuccess && h->m) e = hipMemcpy(g->col, h->col, sizeof(int32_t) * (size_t)h->m, hipMemcpyHostToDevice);

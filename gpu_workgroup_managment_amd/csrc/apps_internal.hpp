@@ -23,7 +23,7 @@ struct wgm_graph {
   float* f0 = nullptr;
   float* f1 = nullptr;
   float* f2 = nullptr;
-  int* iters = nullptr;
+  int* iters = nullptr;   // the run's levels / rounds / sweeps; a 64-bit count at wgm_graph_extra
   int32_t* wl = nullptr;  // colour / MIS worklists, PageRank's long rows (wl_words in apps.hip)
   // low-degree graphs (k_low), looked at on first use: BFS may run on one
   // workgroup; the weights also fit the packed rows; the rows
@@ -75,6 +75,7 @@ struct wgm_graph {
 };
 
 wgm::GraphDev wgm_graph_view(const wgm_graph* g);
+inline unsigned long long* wgm_graph_extra(const wgm_graph* g) { return (unsigned long long*)(g->iters + 2); }
 // defined by the Pannotia unit (pannotia.hip)
 bool wgm_pannotia_kernel_info(int kernel, KernelInfo* out);
 int wgm_pannotia_probe(wgm_runtime* rt, int kernel, int grid, int wg_size);

@@ -62,6 +62,7 @@ struct MinplusDev {
   int32_t* d;            // [nrows + 1] distances of the rows; the last one stays at big (a block's end is read there)
   uint32_t* bits;        // three bit sets: rows lowered in sweep s in set s % 3
   int32_t* dist;         // [n] result
+  unsigned long long* first_edges;  // edges that the first sweep follows
 };
 
 typedef __attribute__((address_space(3))) int lds_i32;
@@ -291,13 +292,16 @@ __global__ void __launch_bounds__(1024) k_minplus(Ctl c, MinplusDev p, int* iter
 }
 
 // Distances of the rows (unreached ones at `big`: BIG_NUM for Pannotia SSSP,
-// MYINFINITY for Lonestar SSSP's pull direction) and the first two bit sets.
+// MYINFINITY for Lonestar SSSP's pull direction), the bit sets, and how many edges
+// the first sweep follows.
 __global__ void k_minplus_init(MinplusDev p) {
   const int tid = blockIdx.x * blockDim.x + threadIdx.x, stride = gridDim.x * blockDim.x;
   const int s = p.cid[p.src];
   for (Span rows{(uint32_t)tid, (uint32_t)p.nrows + 1u}; rows.has(); rows.next(stride))
     p.d[rows.at] = (int)rows.at == s ? 0 : p.big;
   for (int i = tid; i < 3 * p.bit_words; i += stride) p.bits[i] = 0u;
+  if (tid == 0)
+    *p.first_edges = (unsigned long long)(p.all ? p.row_ptr[p.n] : p.row_ptr[p.src + 1] - p.row_ptr[p.src]);
 }
 
 // First rows of the blocks; one wave a vertex.
@@ -926,6 +930,7 @@ int run_minplus(wgm_runtime* rt, wgm_graph* g, int32_t src, int32_t big, const w
   p.d = g->mp_d;
   p.bits = g->mp_bits;
   p.dist = dist;
+  p.first_edges = wgm_graph_extra(g);
   wgm_launch shape{256, 0, 0, 0};
   if (lc) shape = *lc;
   if (shape.wg_size <= 0) shape.wg_size = 256;
@@ -953,18 +958,21 @@ int run_minplus(wgm_runtime* rt, wgm_graph* g, int32_t src, int32_t big, const w
   void* args[] = {&ctl, &p, &g->iters};
   AppOut out;
   out.iters = g->iters;
+  out.extra = reached ? nullptr : p.first_edges;
   out.g = wgm_graph_view(g);
   out.reached = reached ? (const uint32_t*)dist : nullptr;
   out.src = dist;
   out.dst = dst;
   out.bytes = sizeof(int32_t) * (size_t)g->n;
   wgm_run_stats local{};
+  unsigned long long first = 0;
   rc = launch_standalone_app(rt, WGM_K_MINPLUS, (const void*)&k_minplus, &shape, &ctl, args, 0, out, &local,
-                             (size_t)minplus_tables(shape.wg_size) + 4 * (size_t)p.map_words);
+                             (size_t)minplus_tables(shape.wg_size) + 4 * (size_t)p.map_words, &first);
   if (rc) return rc;
   if (local.iterations < 0)
     return fail(rt, WGM_ERR_INVALID, "distances still fall after %d sweeps: negative cycle", g->n + 1);
-  if (!reached) local.edges_scanned = (int64_t)local.iterations * g->m;  // every sweep passes every in-edge
+  // every sweep after the first passes every in-edge
+  if (!reached) local.edges_scanned = (int64_t)first + (local.iterations - 1) * g->m;
   if (st) *st = local;
   return WGM_OK;
 }

@@ -309,7 +309,9 @@ int wgm_bfs_noalloc(wgm_runtime* rt, const int32_t* row_ptr, const int32_t* col,
  * in-edges (the reference reads its graph transposed, sssp.h:43; here the
  * in-edge CSR is built from the graph on first use and kept) until no
  * distance changes. dist_out: 0 at src, WGM_BIG_NUM (sssp.h:3) where
- * unreached. st->iterations = sweeps, st->edges_scanned = sweeps * m. */
+ * unreached. st->iterations = sweeps; st->edges_scanned = the edges the first
+ * sweep follows (src's; all where a weight is negative or above INT32_MAX -
+ * 10^9) + (sweeps - 1) * m. */
 #define WGM_BIG_NUM 99999999
 int wgm_sssp_minplus(wgm_runtime* rt, wgm_graph* g, int32_t src, const wgm_launch* lc, int32_t* dist_out,
                      wgm_run_stats* st);

@@ -39,3 +39,21 @@ def test_two_level_barrier_at_full_occupancy(rt, wg):
     r = rt.barrier_bench(wg_size=wg, num_wgs=0, iterations=20, variant=L.BARRIER_XCD)
     assert r["epoch_errors"] == 0
     assert r["participating"] >= 256 and r["barriers"] == 200
+
+
+@pytest.mark.parametrize("lowest", [1, -1])
+def test_minplus_edges_scanned(rt, lowest):
+    """The first sweep follows the source's edges (every edge where a weight is
+    negative), each later one passes every edge."""
+    n, src = 3001, 7
+    rng = np.random.default_rng(lowest + 2)
+    a, b = np.sort(rng.integers(0, n, (2, 9000)), axis=0)  # no cycles
+    g = G.from_edges(n, a[a != b], b[a != b])
+    g.wt = rng.integers(1, 256, g.m).astype(np.int32)
+    g.wt[g.m // 2] = lowest
+    dg = rt.graph(g)
+    d, st = dg.sssp_minplus(src, wg_size=256, num_wgs=8)
+    assert np.array_equal(d, oracle.sssp_minplus(g.row_ptr, g.col, g.wt, src)[0])
+    first = g.degrees()[src] if lowest > 0 else g.m
+    assert st["iterations"] > 1 and st["edges_scanned"] == first + (st["iterations"] - 1) * g.m
+    dg.close()
