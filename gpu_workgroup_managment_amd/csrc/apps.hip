@@ -48,7 +48,7 @@ __global__ void __launch_bounds__(1024) k_frontier(Ctl c, GraphDev g, FrontierDe
   if (!standalone_begin(c, t)) return;
   run_team<SSSP, SSSP ? kEdgeSlots : 1, true>(g, s, nf, src, t.id, t.n, lds, iters_out,
                                               [&]() { xcd_barrier<false>(c, t); },
-                                              lds + standalone_pass_lds_bytes(blockDim.x) / 4);
+                                              lds + standalone_pass_lds_bytes(SSSP, blockDim.x) / 4);
   clock_end(c, t.id);
   standalone_retire(c);
 }
@@ -530,13 +530,14 @@ static int team_frontier_state(wgm_graph* g, bool sssp, FrontierDev* s, NearFar*
 
 // Both forms of the colour and MIS kernels are launched with the long-row
 // form's LDS, so that the grid found for one holds for the other.
-static int wgm_frontier_lds(int wg) { return standalone_frontier_lds_bytes(wg); }
+template <bool SSSP>
+static int frontier_lds(int wg) { return standalone_frontier_lds_bytes(SSSP, wg); }
 static int scan_lds(int wg) { return scan_lds_bytes(wg); }
 
 bool wgm_app_kernel_info(int kernel, KernelInfo* out) {
   switch (kernel) {
-    case WGM_K_BFS: *out = KernelInfo{(const void*)&k_frontier<false>, wgm_frontier_lds}; return true;
-    case WGM_K_SSSP: *out = KernelInfo{(const void*)&k_frontier<true>, wgm_frontier_lds}; return true;
+    case WGM_K_BFS: *out = KernelInfo{(const void*)&k_frontier<false>, frontier_lds<false>}; return true;
+    case WGM_K_SSSP: *out = KernelInfo{(const void*)&k_frontier<true>, frontier_lds<true>}; return true;
     case WGM_K_COLOR: *out = KernelInfo{(const void*)&k_color<false>, scan_lds}; return true;
     case WGM_K_MIS: *out = KernelInfo{(const void*)&k_mis<false>, scan_lds}; return true;
     case WGM_K_PAGERANK: *out = KernelInfo{(const void*)&k_pagerank<false>, nullptr}; return true;
@@ -645,7 +646,7 @@ int wgm_enqueue_frontier(wgm_runtime* rt, const GraphDev& g, FrontierDev s, cons
                          int grid, int wg, int* iters_dev) {
   s.chunk = wg;  // frontier entries a workgroup claims at a time
   s.heavy = heavy_threshold(wg);
-  const size_t lds = standalone_frontier_lds_bytes(wg);
+  const size_t lds = standalone_frontier_lds_bytes(sssp, wg);
   if (sssp)
     hipLaunchKernelGGL(k_frontier<true>, dim3(grid), dim3(wg), lds, rt->stream, rt->ctl, g, s, nf, src, iters_dev);
   else

@@ -63,16 +63,16 @@ __device__ __forceinline__ void team_barrier(int* cnt, int* gen, int k, int& epo
   __syncthreads();
 }
 
-// LDS of the standalone frontier kernels: a frontier pass (frontier_batch) or a
-// bottom-up pass (the scan queues and its found vertices), then
+// LDS of the standalone frontier kernels: a frontier pass (frontier_batch) or, of
+// BFS, a bottom-up pass (the scan queues and its found vertices), then
 // kStandaloneWords words that outlast a pass.
 constexpr int kStandaloneWords = 4;
 __host__ __device__ constexpr int bottom_up_lds_bytes(int bd) { return scan_lds_bytes(bd) + kScanU * bd * 4; }
-__host__ __device__ constexpr int standalone_pass_lds_bytes(int bd) {
-  return frontier_lds_bytes(bd) > bottom_up_lds_bytes(bd) ? frontier_lds_bytes(bd) : bottom_up_lds_bytes(bd);
+__host__ __device__ constexpr int standalone_pass_lds_bytes(bool sssp, int bd) {
+  return sssp || frontier_lds_bytes(bd) > bottom_up_lds_bytes(bd) ? frontier_lds_bytes(bd) : bottom_up_lds_bytes(bd);
 }
-__host__ __device__ constexpr int standalone_frontier_lds_bytes(int bd) {
-  return standalone_pass_lds_bytes(bd) + 4 * kStandaloneWords;
+__host__ __device__ constexpr int standalone_frontier_lds_bytes(bool sssp, int bd) {
+  return standalone_pass_lds_bytes(sssp, bd) + 4 * kStandaloneWords;
 }
 
 // Frontier membership (bottom-up): a vertex of distance `level`.
