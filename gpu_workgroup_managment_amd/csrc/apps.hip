@@ -14,6 +14,7 @@
 
 #include <algorithm>
 #include <cstring>
+#include <utility>
 
 using namespace wgm;
 
@@ -623,15 +624,23 @@ int wgm_graph_destroy(wgm_graph* g) {
   return WGM_OK;
 }
 
+// Every array that the graph holds: itself, the layouts made from it and the
+// apps' state.
 int64_t wgm_graph_bytes(const wgm_graph* g) {
   if (!g) return 0;
-  int64_t b = 4 * ((int64_t)g->n + 1) + 4 * g->m;
-  if (g->wt) b += 4 * g->m;
-  if (g->prio) b += 4 * (int64_t)g->n;
-  if (g->near_rows) b += 8 * (int64_t)g->n;
-  if (g->ell) b += 4 * kLowDegree * (int64_t)g->n;
-  if (g->rrow) b += 4 * ((int64_t)g->n + 1) + (g->rwt ? 8 : 4) * g->m;
-  if (g->mp_sid) b += 5 * g->m + 4 * (g->m / 256 + (int64_t)g->n + g->mp_rows + 3 * (int64_t)g->mp_words);
+  const int64_t n = g->n, m = g->m, heavy = m / kHeavyMin + 2;
+  const std::pair<const void*, int64_t> arrays[] = {
+      {g->row_ptr, 4 * (n + 1)}, {g->col, 4 * m}, {g->wt, 4 * m}, {g->prio, 4 * n}, {g->iters, 16},
+      {g->near_rows, 8 * n}, {g->ell, 4 * kLowDegree * n},
+      // frontier state
+      {g->dist, 4 * n}, {g->stamp, 4 * n}, {g->q0, 4 * (n + 1)}, {g->q1, 4 * (n + 1)}, {g->counts, 12 * kLine},
+      {g->tq, 8 * g->tcap}, {g->tqa, 8 * g->tcap}, {g->claims, 12 * kLine}, {g->far, 8 * (n + 1)}, {g->in_far, 4 * n},
+      {g->fcnt, 12 * kLine}, {g->hv, 4 * heavy}, {g->hdu, 4 * heavy}, {g->hclaim, 4 * heavy}, {g->hcnt, 12 * kLine},
+      // colour, MIS, PageRank
+      {g->i32a, 4 * n}, {g->i32b, 4 * n}, {g->f0, 4 * n}, {g->f1, 4 * n}, {g->f2, 4 * n}, {g->wl, 4 * (int64_t)wl_words(g)}};
+  int64_t b = wgm_pannotia_bytes(g);
+  for (const auto& [p, bytes] : arrays)
+    if (p) b += bytes;
   return b;
 }
 

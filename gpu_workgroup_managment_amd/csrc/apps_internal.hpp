@@ -80,6 +80,7 @@ inline unsigned long long* wgm_graph_extra(const wgm_graph* g) { return (unsigne
 bool wgm_pannotia_kernel_info(int kernel, KernelInfo* out);
 int wgm_pannotia_probe(wgm_runtime* rt, int kernel, int grid, int wg_size);
 void wgm_pannotia_release(wgm_graph* g);
+int64_t wgm_pannotia_bytes(const wgm_graph* g);
 int wgm_graph_frontier_state(wgm_graph* g, bool sssp, wgm::FrontierDev* s);
 // per-run arrays of a topology-driven app: 1 colour (i32a), 2 MIS (i32a,
 // i32b), 3 PageRank (f0, f1, f2); 0 nothing

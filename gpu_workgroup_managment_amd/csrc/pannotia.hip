@@ -26,6 +26,7 @@
 #include "apps_internal.hpp"
 
 #include <algorithm>
+#include <utility>
 
 using namespace wgm;
 
@@ -1007,6 +1008,20 @@ void wgm_pannotia_release(wgm_graph* g) {
   void* ptrs[] = {g->rrow, g->rcol, g->rwt, g->mp_sid, g->mp_roff, g->mp_start, g->mp_cid, g->mp_d, g->mp_bits, g->bc_d, g->bc_sig, g->bc_del, g->bc_q, g->bc_lvl, g->bc_sum, g->bc_srcs};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
+}
+
+int64_t wgm_pannotia_bytes(const wgm_graph* g) {
+  const int64_t n = g->n, m = g->m, edges = mp_edges(m), slots = g->bc_slots;
+  const std::pair<const void*, int64_t> arrays[] = {
+      {g->rrow, 4 * (n + 1)}, {g->rcol, 4 * m}, {g->rwt, 4 * edges},
+      {g->mp_sid, 4 * edges}, {g->mp_roff, edges}, {g->mp_start, 4 * (edges / kMpBlock + 1)},
+      {g->mp_cid, 4 * (int64_t)wgm_row_id_words(g->n)}, {g->mp_d, 4 * ((int64_t)g->mp_rows + 1)}, {g->mp_bits, 12 * (int64_t)g->mp_words},
+      {g->bc_d, 4 * slots * n}, {g->bc_sig, 8 * slots * n}, {g->bc_del, 8 * g->bc_rows * n}, {g->bc_q, 4 * slots * n},
+      {g->bc_lvl, 4 * slots * (n + 2)}, {g->bc_sum, 8 * (n + 1)}, {g->bc_srcs, 4 * (n + 1)}};
+  int64_t b = 0;
+  for (const auto& [p, bytes] : arrays)
+    if (p) b += bytes;
+  return b;
 }
 
 extern "C" {

@@ -227,6 +227,15 @@ typedef struct wgm_graph wgm_graph;
  * instead of being re-uploaded per run. */
 int wgm_graph_create(wgm_runtime* rt, const wgm_csr* g, const uint32_t* prio, wgm_graph** out);
 int wgm_graph_destroy(wgm_graph* g);
+/* Device memory the graph holds now: itself, and the layouts and state that each
+ * app makes on its first run and keeps. In bytes, n vertices and m edges, in-edges
+ * 4 n + 4 m (8 m weighted) and the colour / MIS / PageRank lists 32 n (16 n up to
+ * out-degree 4, none for PageRank then) counted once: BFS 12 n + in-edges, or 28 n;
+ * SSSP push 16 n + 16 max(n, m) (16 n more up to out-degree 4), pull 13 n + 5 m +
+ * in-edges; colour 4 n + lists,
+ * MIS 8 n + lists; PageRank 12 n + lists, or 20 n; BC 12 n + in-edges + 4 n a
+ * workgroup + a row of 8 n a source, up to 1 GB of rows or one a workgroup (above
+ * 8900 vertices 16 n a workgroup more). */
 int64_t wgm_graph_bytes(const wgm_graph* g);
 
 /* Launch shape of a standalone persistent kernel. */

@@ -57,3 +57,27 @@ def test_minplus_edges_scanned(rt, lowest):
     first = g.degrees()[src] if lowest > 0 else g.m
     assert st["iterations"] > 1 and st["edges_scanned"] == first + (st["iterations"] - 1) * g.m
     dg.close()
+
+
+def test_graph_bytes_count_what_the_apps_keep(rt):
+    """The lists of the worklist apps (rows above 4 edges: two of 16 bytes a
+    vertex), the ranks, BC's rows and in-edges."""
+    n = 6007
+    rng = np.random.default_rng(3)
+    g = G.add_priorities(G.from_edges(n, rng.integers(0, n, 30000), rng.integers(0, n, 30000), symmetric=True))
+    assert g.degrees().max() > 4
+    dg = rt.graph(g)
+    want = 4 * (n + 1) + 4 * g.m + 4 * n + 16
+    assert dg.nbytes() == want
+    dg.color(wg_size=64, num_wgs=3)
+    want += 4 * n + 32 * n
+    assert dg.nbytes() == want
+    dg.mis(wg_size=64, num_wgs=3)
+    want += 4 * n
+    dg.pagerank(0.85, 2, wg_size=64, num_wgs=3)
+    want += 12 * n
+    assert dg.nbytes() == want
+    dg.bc(9, wg_size=64, num_wgs=3)
+    want += 4 * (n + 1) + 4 * g.m + 8 * 9 * n + 4 * 3 * (n + 2) + 8 * (n + 1) + 4 * (n + 1)
+    assert dg.nbytes() == want
+    dg.close()
