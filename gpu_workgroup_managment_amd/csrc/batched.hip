@@ -316,10 +316,7 @@ __global__ void __launch_bounds__(1024) k_batched(Ctl c, BatchDev b) {
     __syncthreads();
   }
   // the last workgroup to leave stamps the end of the batch
-  if (threadIdx.x == 0) {
-    fence_release();
-    if (add_acq_rel(&c.lines[0], 1) == n - 1) c.clock[1] = wall_clock64();
-  }
+  if (threadIdx.x == 0 && add_acq_rel(&c.lines[0], 1) == n - 1) c.clock[1] = wall_clock64();
 }
 
 // Per-launch reset of the work queue and team barriers (capture-safe: a

@@ -277,7 +277,6 @@ __device__ void np_task(const NPDev& t, int kind, int vid, int nwg, int* lds, un
   if (threadIdx.x == 0) {
     if (clk)
       __hip_atomic_fetch_max(&clk[1], (unsigned long long)wall_clock64(), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    fence_release();
     s_last = add_acq_rel(t.counter, 1) == nwg - 1;
   }
   __syncthreads();
@@ -290,11 +289,11 @@ __device__ void np_task(const NPDev& t, int kind, int vid, int nwg, int* lds, un
     if (threadIdx.x == 0) {
       unsigned h = 5381;
       for (int i = 0; i < t.dim; i++) h = h * 33u + (unsigned)t.C[i * t.dim + i];
-      __hip_atomic_store(t.h_result, (int)h, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+      sys_st_release(t.h_result, (int)h);
     }
   } else if (kind == WGM_NP_REDUCE_MIN) {
     if (threadIdx.x == 0)
-      __hip_atomic_store(t.h_result, ld_relaxed(t.dmin), __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+      sys_st_release(t.h_result, ld_relaxed(t.dmin));
   } else if (blockDim.x % 256 == 0 && t.dim % 64 == 0 && t.partial) {
     if (threadIdx.x == 0) {
       double sum = 0.0;
@@ -302,7 +301,7 @@ __device__ void np_task(const NPDev& t, int kind, int vid, int nwg, int* lds, un
       unsigned long long bits;
       __builtin_memcpy(&bits, &sum, 8);
       __hip_atomic_store(t.h_checksum, bits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-      __hip_atomic_store(t.h_result, 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+      sys_st_release(t.h_result, 1);
     }
   } else {
     // weighted checksum in FP64: sum_ij C[i][j] u(i) v(j)
@@ -320,11 +319,11 @@ __device__ void np_task(const NPDev& t, int kind, int vid, int nwg, int* lds, un
       unsigned long long bits;
       __builtin_memcpy(&bits, &red[0], 8);
       __hip_atomic_store(t.h_checksum, bits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-      __hip_atomic_store(t.h_result, 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+      sys_st_release(t.h_result, 1);
     }
   }
   __syncthreads();
-  if (executing && threadIdx.x == 0) __hip_atomic_fetch_add(executing, -1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
+  if (executing && threadIdx.x == 0) add_release(executing, -1);
 }
 
 }  // namespace wgm

@@ -248,7 +248,7 @@ __global__ void __launch_bounds__(1024) k_mega(Ctl c, SchedDev s, const MegaApp*
       drain_vmem();
       __syncthreads();
       if (threadIdx.x == 0) {
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "");
+        sys_fence_release();
         add_relaxed(s.p.executing, -1);
         sys_add_release(s.persistent_flag, -1);
       }

@@ -134,7 +134,8 @@ __device__ __forceinline__ bool offer_kill(const SchedDev& s, int vid) {
         // num_groups from the value it reads. If it got in first, the kill
         // unit is dropped (the scheduler no longer waits for it).
         int expect = vid + 1;
-        killed = __hip_atomic_compare_exchange_strong(s.p.num_groups, &expect, vid, __ATOMIC_RELEASE,
+        fence_release();
+        killed = __hip_atomic_compare_exchange_strong(s.p.num_groups, &expect, vid, __ATOMIC_RELAXED,
                                                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
                      ? 1
                      : 0;
@@ -174,11 +175,12 @@ __device__ __forceinline__ int offer_fork_thread0(const SchedDev& s, const R& to
       while (ld_relaxed(&s.task_array[(i + 1) * kLine]) != TASK_WAIT) {
       }
       *rslot<R>(s.r_ctx, i + 1) = to_fork;
-      st_release(&s.task_array[(i + 1) * kLine], TASK_PERSIST);
     }
+    fence_release();  // one write-back for all of them
+    for (int i = groups; i < groups + snapshot; i++) st_relaxed(&s.task_array[(i + 1) * kLine], TASK_PERSIST);
     add_relaxed(s.p.num_groups, snapshot);
     add_relaxed(s.p.executing, snapshot);
-    __hip_atomic_fetch_add(s.persistent_flag, snapshot, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    sys_add_release(s.persistent_flag, snapshot);
     add_relaxed(s.available, -snapshot);
     sched_unlock(s.pool_lock);
     *after = groups + snapshot;
@@ -253,12 +255,12 @@ __device__ __forceinline__ bool resize_barrier(const SchedDev& s, int vid, const
 // ------------------------------------------------- scheduler (WG 0, thread 0)
 // src/scheduler_rt/rt_device/cl_scheduler.cl:54-64
 __device__ __forceinline__ void scheduler_init(const SchedDev& s, int count) {
-  sys_st_release(s.participating, count - 1);
+  __hip_atomic_store(s.participating, count - 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
   st_relaxed(&s.task_array[0], count - 1);
-  st_release(s.pool_lock, 0);
-  st_release(s.np.executing, 0);
-  st_release(s.p.executing, 0);
-  sys_st_release(s.persistent_flag, 0);
+  st_relaxed(s.pool_lock, 0);
+  st_relaxed(s.np.executing, 0);
+  st_relaxed(s.p.executing, 0);
+  __hip_atomic_store(s.persistent_flag, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
   sys_st_release(s.scheduler_flag, DEVICE_WAITING);
 }
 
@@ -284,9 +286,10 @@ __device__ __forceinline__ void assign_np(const SchedDev& s, int k, int lpg) {
     s.np.group_ids[lpg - i] = i;
     while (ld_relaxed(&s.task_array[(lpg - i) * kLine]) != TASK_WAIT) {
     }
-    st_release(&s.task_array[(lpg - i) * kLine], TASK_MULT);
-    add_relaxed(s.available, -1);
   }
+  fence_release();  // one write-back for all of them
+  add_relaxed(s.available, -k);
+  for (int i = 0; i < k; i++) st_relaxed(&s.task_array[(lpg - i) * kLine], TASK_MULT);
 }
 
 // The persistent task takes discovered ids 1..k as virtual ids 0..k-1
@@ -297,9 +300,10 @@ __device__ __forceinline__ void assign_p(const SchedDev& s, int k) {
     while (ld_relaxed(&s.task_array[(i + 1) * kLine]) != TASK_WAIT) {
     }
     *(int*)rslot<RCtx>(s.r_ctx, i + 1) = 0;  // target 0: start from the top
-    st_release(&s.task_array[(i + 1) * kLine], TASK_PERSIST);
-    add_relaxed(s.available, -1);
   }
+  fence_release();  // one write-back for all of them
+  add_relaxed(s.available, -k);
+  for (int i = 0; i < k; i++) st_relaxed(&s.task_array[(i + 1) * kLine], TASK_PERSIST);
 }
 
 __device__ __forceinline__ int host_flag(const SchedDev& s) { return sys_ld_relaxed(s.scheduler_flag); }
@@ -337,9 +341,9 @@ __device__ __forceinline__ void serve_fork_back(const SchedDev& s, int lpg, int*
   *pos = i >= lpg ? 1 : i + 1;
   if (ld_relaxed(&s.task_array[i * kLine]) != TASK_WAIT) return;
   add_relaxed(s.p.executing, 1);
-  sys_add_release(s.persistent_flag, 1);
+  sys_add_release(s.persistent_flag, 1);  // releases to the member too
   add_relaxed(s.available, -1);
-  st_release(&s.task_array[i * kLine], TASK_PERSIST);
+  st_relaxed(&s.task_array[i * kLine], TASK_PERSIST);
 }
 
 // src/scheduler_rt/rt_device/cl_scheduler.cl:66-171
@@ -357,10 +361,11 @@ __device__ __forceinline__ void scheduler_loop(const SchedDev& s, int lpg) {
       }
       fence_acquire();
       sched_lock(s.pool_lock);
+      fence_release();
       for (int i = 1; i < lpg + 1; i++) {
         while (ld_acquire(&s.task_array[i * kLine]) != TASK_WAIT) {
         }
-        st_release(&s.task_array[i * kLine], TASK_QUIT);
+        st_relaxed(&s.task_array[i * kLine], TASK_QUIT);
         add_relaxed(s.available, -1);
       }
       sched_unlock(s.pool_lock);

@@ -269,8 +269,7 @@ __device__ bool serve_query(const SchedDev& s, const ServeDev& v, int slot, bool
           sv[3] = fi;
           sv[4] = s_far[fi];
           v.saved_pre[slot] += 1;
-          fence_release();
-          push_resume(v, slot);
+          push_resume(v, slot);  // releases what was saved
         }
         __syncthreads();
         return true;
@@ -361,7 +360,7 @@ __device__ bool serve_query(const SchedDev& s, const ServeDev& v, int slot, bool
     __hip_atomic_store(rw + 6, (unsigned long long)(unsigned)v.saved_pre[slot], __ATOMIC_RELAXED,
                        __HIP_MEMORY_SCOPE_SYSTEM);
     const unsigned long long head = ((unsigned long long)(unsigned)level << 32) | (unsigned)rq.seq;
-    __hip_atomic_store(rw + 0, head, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    sys_st_release(rw + 0, head);
   }
   __syncthreads();
   return false;
@@ -413,14 +412,14 @@ __device__ void doorbell_loop(const SchedDev& s, const ServeDev& v) {
     if (t != last_tail) {
       // the ring entries and descriptors are read by the claimer with
       // system-scope loads after its own acquire; order the mirror after
-      // this load of the tail
+      // this load of the tail (this wave has written nothing to release)
       __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-      st_release(v.ring_tail, t);
+      st_relaxed(v.ring_tail, t);
       last_tail = t;
     }
     const int st = sys_ld_relaxed(s.stop);
     if (st != last_stop) {
-      st_release(v.stop_dev, st);
+      st_relaxed(v.stop_dev, st);
       last_stop = st;
     }
     __builtin_amdgcn_s_sleep(1);
@@ -440,7 +439,7 @@ __global__ void __launch_bounds__(1024) k_serve(Ctl c, SchedDev s, ServeDev v, N
     if (threadIdx.x == 0) {
       scheduler_init(s, n);
       scheduler_loop(s, n - 1);
-      st_release(v.quit_dev, 1);
+      st_relaxed(v.quit_dev, 1);
     } else if (threadIdx.x == 64) {
       doorbell_loop(s, v);
     }

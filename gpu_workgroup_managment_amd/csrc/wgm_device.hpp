@@ -23,6 +23,26 @@ namespace wgm {
 
 constexpr int kLine = 32;  // ints per 128-byte line
 
+// ------------------------------------------------------------------- fences
+// A release writes the XCD's L2 back (buffer_wbl2) and the flag that publishes it
+// must wait for that. The compiler's own wait is lost where it knows of no other
+// memory operation on its way (ROCm 7.2 does not count the write-back it has just
+// emitted): every release after a drain_vmem or a completed load became
+// `buffer_wbl2 sc1` with the flag's store right behind it. So every release here
+// is a fence with a wait of its own, and the atomic after it is relaxed; none is
+// left to an atomic's release order (tests/test_release_waits.py reads the built
+// code for it).
+__device__ __forceinline__ void wait_written_back() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+__device__ __forceinline__ void fence_acquire() { __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent"); }
+__device__ __forceinline__ void fence_release() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+  wait_written_back();
+}
+__device__ __forceinline__ void sys_fence_release() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "");
+  wait_written_back();
+}
+
 // ------------------------------------------------------------------ atomics
 __device__ __forceinline__ int ld_relaxed(const int* p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -34,7 +54,8 @@ __device__ __forceinline__ void st_relaxed(int* p, int v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 __device__ __forceinline__ void st_release(int* p, int v) {
-  __hip_atomic_store(p, v, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
+  fence_release();
+  st_relaxed(p, v);
 }
 template <class T>
 __device__ __forceinline__ T ld_agent(const T* p) {
@@ -47,17 +68,21 @@ __device__ __forceinline__ void st_agent(T* p, T v) {
 __device__ __forceinline__ int add_relaxed(int* p, int v) {
   return __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
+__device__ __forceinline__ void add_release(int* p, int v) {
+  fence_release();
+  add_relaxed(p, v);
+}
 __device__ __forceinline__ int add_acq_rel(int* p, int v) {
-  return __hip_atomic_fetch_add(p, v, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
+  fence_release();
+  return __hip_atomic_fetch_add(p, v, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT);
 }
 __device__ __forceinline__ int or_acq_rel(int* p, int v) {
-  return __hip_atomic_fetch_or(p, v, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
+  fence_release();
+  return __hip_atomic_fetch_or(p, v, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT);
 }
 __device__ __forceinline__ int xchg_acquire(int* p, int v) {
   return __hip_atomic_exchange(p, v, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT);
 }
-__device__ __forceinline__ void fence_acquire() { __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent"); }
-__device__ __forceinline__ void fence_release() { __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent"); }
 
 // System scope: cells shared with the host through coherent host memory.
 __device__ __forceinline__ int sys_ld_acquire(const int* p) {
@@ -66,11 +91,14 @@ __device__ __forceinline__ int sys_ld_acquire(const int* p) {
 __device__ __forceinline__ int sys_ld_relaxed(const int* p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
-__device__ __forceinline__ void sys_st_release(int* p, int v) {
-  __hip_atomic_store(p, v, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+template <class T>
+__device__ __forceinline__ void sys_st_release(T* p, T v) {
+  sys_fence_release();
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 __device__ __forceinline__ int sys_add_release(int* p, int v) {
-  return __hip_atomic_fetch_add(p, v, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+  sys_fence_release();
+  return __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 __device__ __forceinline__ void sys_st_u64(unsigned long long* p, unsigned long long v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);

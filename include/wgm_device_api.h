@@ -250,4 +250,66 @@ __device__ inline R wgm_restoration_ctx(const wgm_mega_args& ma) {
     }                                                                                 \
   } while (0)
 
+/* ------------------------------------------------------- release operations
+ * A release at agent or system scope has to wait until the L2 is written back.
+ * The compiler (ROCm 7.2) drops that wait where it knows of no other memory
+ * operation on its way, for instance behind a load that has returned, and a lock's
+ * release can then be seen before the data it guards (wgm_device.hpp, "fences").
+ * In kernels that include this header the release half of an atomic, and a
+ * thread fence, are therefore a fence with its own wait; orders without a release,
+ * narrower scopes and host code are as they were. */
+namespace wgm_api {
+constexpr bool releases(int order, int scope) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return (order == __ATOMIC_RELEASE || order == __ATOMIC_ACQ_REL || order == __ATOMIC_SEQ_CST) &&
+         (scope == __HIP_MEMORY_SCOPE_AGENT || scope == __HIP_MEMORY_SCOPE_SYSTEM);
+#else
+  return false;
+#endif
+}
+template <int order, int scope>
+__host__ __device__ inline void release_first() {
+#if defined(__HIP_DEVICE_COMPILE__)
+  if constexpr (releases(order, scope)) {
+    if constexpr (scope == __HIP_MEMORY_SCOPE_SYSTEM) wgm::sys_fence_release();
+    else wgm::fence_release();
+  }
+#endif
+}
+/* The order of the operation behind that fence. */
+constexpr int order_left(int order, int scope) {
+  return !releases(order, scope) || order == __ATOMIC_SEQ_CST ? order
+         : order == __ATOMIC_ACQ_REL                          ? __ATOMIC_ACQUIRE
+                                                              : __ATOMIC_RELAXED;
+}
+__device__ inline void agent_fence() {
+  wgm::fence_release();
+  wgm::fence_acquire();
+}
+__device__ inline void system_fence() {
+  wgm::sys_fence_release();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "");
+}
+}  // namespace wgm_api
+
+#define WGM_RELEASED(op, p, v, order, scope) \
+  (wgm_api::release_first<(order), (scope)>(), op(p, v, wgm_api::order_left(order, scope), scope))
+#define __hip_atomic_store(p, v, order, scope) WGM_RELEASED(__hip_atomic_store, p, v, order, scope)
+#define __hip_atomic_exchange(p, v, order, scope) WGM_RELEASED(__hip_atomic_exchange, p, v, order, scope)
+#define __hip_atomic_fetch_add(p, v, order, scope) WGM_RELEASED(__hip_atomic_fetch_add, p, v, order, scope)
+#define __hip_atomic_fetch_sub(p, v, order, scope) WGM_RELEASED(__hip_atomic_fetch_sub, p, v, order, scope)
+#define __hip_atomic_fetch_and(p, v, order, scope) WGM_RELEASED(__hip_atomic_fetch_and, p, v, order, scope)
+#define __hip_atomic_fetch_or(p, v, order, scope) WGM_RELEASED(__hip_atomic_fetch_or, p, v, order, scope)
+#define __hip_atomic_fetch_xor(p, v, order, scope) WGM_RELEASED(__hip_atomic_fetch_xor, p, v, order, scope)
+#define __hip_atomic_fetch_min(p, v, order, scope) WGM_RELEASED(__hip_atomic_fetch_min, p, v, order, scope)
+#define __hip_atomic_fetch_max(p, v, order, scope) WGM_RELEASED(__hip_atomic_fetch_max, p, v, order, scope)
+#define __hip_atomic_compare_exchange_strong(p, e, v, order, fail, scope) \
+  (wgm_api::release_first<(order), (scope)>(),                             \
+   __hip_atomic_compare_exchange_strong(p, e, v, wgm_api::order_left(order, scope), fail, scope))
+#define __hip_atomic_compare_exchange_weak(p, e, v, order, fail, scope) \
+  (wgm_api::release_first<(order), (scope)>(),                           \
+   __hip_atomic_compare_exchange_weak(p, e, v, wgm_api::order_left(order, scope), fail, scope))
+#define __threadfence() wgm_api::agent_fence()
+#define __threadfence_system() wgm_api::system_fence()
+
 #endif /* WGM_DEVICE_API_H */
