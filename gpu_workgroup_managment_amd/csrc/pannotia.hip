@@ -7,9 +7,9 @@
 // relax, compare). Here one sweep relaxes in place and flags any decrease, with
 // one barrier per sweep: values only decrease and every one stays an upper
 // bound, so the sweeps reach the same unique fixpoint (the shortest
-// distances; BIG_NUM where unreached) in at most as many sweeps. The in-edge
-// rows are cut into tasks of at most 16 * G edges, G lanes per task, so a hub's
-// row is shared by several lane groups and meets at one atomic min.
+// distances; BIG_NUM where unreached) in at most as many sweeps. A sweep follows
+// only the edges whose source the last one lowered; the in-edges lie in blocks of
+// 256, so a hub's row is shared by several waves and meets at one atomic min.
 //
 // Pannotia BC (bc_combined, src/pannotia/graph_apps/bc/device/bc.cl:186-235,
 // plugin src/pannotia/graph_apps/bc/bc.h): Brandes' betweenness. The reference

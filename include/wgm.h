@@ -232,17 +232,29 @@ int wgm_graph_destroy(wgm_graph* g);
  * 4 n + 4 m (8 m weighted) and the colour / MIS / PageRank lists 32 n (16 n up to
  * out-degree 4, none for PageRank then) counted once: BFS 12 n + in-edges, or 28 n;
  * SSSP push 16 n + 16 max(n, m) (16 n more up to out-degree 4), pull 13 n + 5 m +
- * in-edges; colour 4 n + lists,
- * MIS 8 n + lists; PageRank 12 n + lists, or 20 n; BC 12 n + in-edges + 4 n a
- * workgroup + a row of 8 n a source, up to 1 GB of rows or one a workgroup (above
- * 8900 vertices 16 n a workgroup more). */
+ * in-edges; colour 4 n + lists, MIS 8 n + lists; PageRank 12 n + lists, or 20 n;
+ * BC 12 n + in-edges + 4 n a workgroup + a row of 8 n a source, up to 1 GB of rows
+ * or one a workgroup (above 8900 vertices 16 n a workgroup more). */
 int64_t wgm_graph_bytes(const wgm_graph* g);
 
-/* Launch shape of a standalone persistent kernel. */
+/* Launch shape of a standalone persistent kernel. The result arrays do not depend
+ * on it; st->participating says how many workgroups ran. A shape asked for is
+ * kept, except:
+ * - of more workgroups than can be resident, as many as can take part;
+ * - wgm_sssp_minplus and wgm_sssp's pull direction take more than a workgroup a CU
+ *   as one larger one on each, and on small graphs fewer: up to 64 where a wave
+ *   then has a block of 256 in-edges, more only where it has four, of 512 threads
+ *   where those suffice;
+ * - wgm_bfs and wgm_sssp's push direction on low-degree graphs of narrow levels
+ *   (out-degree <= 4, n <= 2^18, edges spanning <= 768 places of the vertex order
+ *   or n <= 16384) take the threads in workgroups of 1024; the first runs the whole
+ *   traversal and the others end at once;
+ * - wgm_bc, with a source's state in LDS (up to about 8900 vertices), takes the
+ *   threads in as many larger workgroups as fit. */
 typedef struct wgm_launch {
   int32_t wg_size;     /* threads per workgroup (64..1024, multiple of 64) */
-  int32_t num_wgs;     /* <= 0: discovered occupancy, or fewer on small graphs; of more than can be resident, as
-                          many as can (some apps take the threads asked for in fewer, larger workgroups) */
+  int32_t num_wgs;     /* <= 0, left open: the discovered occupancy, or fewer where BFS, MIS, PageRank and the
+                          min-plus sweeps are faster with fewer */
   int32_t handshake;   /* 1: host flag handshake as in the reference's run_persistent */
   int32_t mode;        /* wgm_sssp's relaxation direction: WGM_SSSP_AUTO, _PUSH or _PULL */
 } wgm_launch;
@@ -275,8 +287,9 @@ typedef struct wgm_run_stats {
  * wgm_sssp: Lonestar SSSP (src/lonestar/graph_apps/sssp/sssp.h:16-382,
  *   src/lonestar/graph_apps/sssp/device/standalone.cl), same distances: by
  *   default pull sweeps over the in-edges on graphs with an out-degree above
- *   4, and on the others push in near-far bands of width 1024 (lc->mode;
- *   a push on a graph of out-degree above 4 takes bands of width 128);
+ *   4, and on the others push in near-far bands of width 1024, 512 where one
+ *   workgroup runs it (lc->mode; a push on a graph of out-degree above 4 takes
+ *   bands of width 128);
  *   st->edges_scanned counts the reached vertices' out-edges either way;
  * wgm_color: Pannotia color (src/pannotia/graph_apps/color/color.h:41-195,
  *   src/pannotia/graph_apps/color/device/standalone.cl:10-126);
