@@ -281,7 +281,8 @@ typedef struct wgm_run_stats {
 
 /* Standalone persistent apps: run_persistent (src/host_skeleton/skel.cpp:250-385)
  * with one plugin each. Outputs are host arrays of n entries (may be NULL to
- * leave the result on the device).
+ * leave the result on the device); a runtime keeps up to 16 MB of pinned host
+ * memory that they are copied through.
  * wgm_bfs: Lonestar BFS (src/lonestar/graph_apps/bfs/bfs.h:16-370,
  *   src/lonestar/graph_apps/bfs/device/standalone.cl:218-320);
  * wgm_sssp: Lonestar SSSP (src/lonestar/graph_apps/sssp/sssp.h:16-382,
